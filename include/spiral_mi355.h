@@ -108,8 +108,7 @@ int sp_clock_sample(uint64_t* out, void* stream);
  *   alpha must be non-zero (kernel.spi:49).  beta == 0 means C is never read, so NaNs in the
  *   old C do not propagate (kernel.spi:152-154).
  *   K must be a multiple of 8 (16-bit) / 4 (f32): rows of A and B are whole 16-byte chunks.  Every such
- *   shape with N a multiple of 4 runs on the tiled MFMA kernels (tiles that overhang M, N or K are
- *   masked); only N not a multiple of 4 falls back to a slow one-thread-per-output kernel.
+ *   shape runs on the MFMA kernels (tiles that overhang M, N or K are masked).
  */
 int sp_gemm_abt(int dtype_in, int dtype_out, const void* A, const void* B, void* C, const float* bias,
                 int64_t M, int64_t N, int64_t K, float alpha, float beta, uint32_t flags, void* stream);
@@ -128,8 +127,7 @@ int sp_gemm_abt_batched(int dtype_in, int dtype_out, const void* A, const void* 
                         int64_t stride_c, float alpha, float beta, uint32_t flags, void* stream);
 
 /* Which tile configuration sp_gemm_abt picks for a shape (the counterpart of
- * `matmul_config_tf32`, ml/matmul/run.spi:8-19).  Writes block tile sizes and the workgroup size;
- * tile_m == 0 means the general kernel. */
+ * `matmul_config_tf32`, ml/matmul/run.spi:8-19).  Writes block tile sizes and the workgroup size. */
 int sp_gemm_config(int dtype_in, int64_t M, int64_t N, int64_t K,
                    int32_t* tile_m, int32_t* tile_n, int32_t* tile_k, int32_t* threads);
 

@@ -3,7 +3,7 @@
 // A (M,K) and B (N,K) are both K-contiguous, so neither operand needs a transposing read: a
 // 32x32 MFMA fragment of either one is "32 rows x one 16-byte K-chunk per lane".
 //
-// Two tiled kernels: gemm_abt_w4_kernel (four waves, 16x16x32 MFMAs; large 16-bit shapes) and gemm_abt_kernel (eight or
+// Here the workgroup tiles (small and narrow outputs: gemm_wave.hip).  Two kernels: gemm_abt_w4_kernel (four waves, 16x16x32 MFMAs; large 16-bit shapes) and gemm_abt_kernel (eight or
 // four waves, 32x32 MFMAs; f32, small tiles, single-column outputs).
 //
 // Data movement per workgroup and K-tile (128 bytes of K per row: 64 bf16/f16 or 32 f32):
@@ -15,86 +15,9 @@
 //
 // Semantics follow matmul_tf32_template (ml/matmul/kernel.spi:25-240) with a_trans=false,
 // b_trans=true; the f32 path multiplies in full f32 (v_mfma_f32_32x32x2_f32), not TF32.
-#include "common.h"
-#include <type_traits>
+#include "gemm_common.h"
 
 namespace sp {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
-
-struct GemmArgs {
-    const void* A;
-    const void* B;
-    void* C;
-    const float* bias;
-    long M, N, K;
-    float alpha, beta;
-    int relu;
-    int out_dtype;
-    int tiles_m, tiles_n;
-    long stride_a, stride_b, stride_c;   // bytes between the matrices of a batch (0: shared)
-    int batch;
-    int group_m;   // tile rows per group of the block -> tile walk (4: an XCD's 32 concurrent tiles form a 4 x 8 patch)
-    int ragged;    // M or N is not a multiple of the tile: tiles_m / tiles_n are rounded up
-    int k_rotate;  // workgroup t starts its K loop at K-tile (t * k_rotate) % nk and wraps around (0: everyone at 0)
-    int store_policy;   // ST_THROUGH or ST_STREAM for the stores of C when beta == 0 (with beta != 0 C is read here: ST_PLAIN)
-    int phase_groups;   // persistent four-wave kernel: workgroup w starts ((w / 8) % phase_groups) * phase_skew
-    int phase_skew;     // sleeps of ~2048 cycles late (0 / 1 groups: everybody at once)
-};
-
-// The tiled kernels take the fields their first fetches need (operand addresses, K, batch strides, the tile grid) once
-// more as leading scalar parameters: the library is built with kernel-argument preloading, which hands the first
-// dwords of scalar parameters to a wave in registers when it starts (a struct is not preloaded), so the first
-// fetches do not wait for a scalar load from the argument block (~900 cycles).
-#define SP_GEMM_PRELOADED const void *A_first, const void *B_first, long K_first, long stride_a_first, long stride_b_first, \
-                          int tiles_m_first, int tiles_n_first, int group_m_first
-#define SP_GEMM_PRELOADED_ARGS(g) (g).A, (g).B, (g).K, (g).stride_a, (g).stride_b, (g).tiles_m, (g).tiles_n, (g).group_m
-__device__ __forceinline__ GemmArgs with_preloaded(const GemmArgs& g0, SP_GEMM_PRELOADED) {
-    GemmArgs g = g0;
-    g.A = A_first; g.B = B_first; g.K = K_first; g.stride_a = stride_a_first; g.stride_b = stride_b_first;
-    g.tiles_m = tiles_m_first; g.tiles_n = tiles_n_first; g.group_m = group_m_first;
-    return g;
-}
-#define SP_GEMM_TAKE_PRELOADED                                                                                          \
-    const GemmArgs g = with_preloaded(g_rest, A_first, B_first, K_first, stride_a_first, stride_b_first, tiles_m_first, \
-                                      tiles_n_first, group_m_first)
-
-constexpr int ROW_BYTES = 128;  // bytes of K per LDS row and K-tile
-constexpr int CHUNKS = 8;       // 16-byte chunks per LDS row
-
-// 16-byte chunk `kc` of LDS row `row` lives at chunk slot kc ^ swz(row): any 8 consecutive rows
-// read at the same kc touch 8 different slots, and rows r, r+8 land in different 128-byte halves.
-__device__ __forceinline__ int lds_offset(int row, int kc) {
-    return row * ROW_BYTES + (((kc ^ row ^ (row >> 3)) & 7) << 4);
-}
-
-template <int T>
-__device__ __forceinline__ float half_bits_to_f32(unsigned bits) {
-    if constexpr (T == SP_BF16) return __uint_as_float(bits << 16);
-    else return (float)__builtin_bit_cast(_Float16, (unsigned short)bits);
-}
-
-__device__ __forceinline__ unsigned short f32_to_bf16_rne(float x) {
-    unsigned u = __float_as_uint(x);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (unsigned short)((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
-}
-
-// Two f32 values rounded to nearest even and packed into one register (v_cvt_pk_{f16,bf16}_f32).
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-template <int T>
-__device__ __forceinline__ unsigned pack_halves(float a, float b) {
-    if constexpr (T == SP_BF16) return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2));
-    else return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, f16x2));
-}
 
 // Map the linear workgroup id to an output tile.  Workgroups are dealt round-robin to the 8 XCDs
 // (each with a private L2), so id % 8 selects the XCD; each XCD gets a contiguous range of the
@@ -116,52 +39,11 @@ __device__ __forceinline__ void tile_of_block(int pid, int tiles_m, int tiles_n,
     tn = in_group / gsz;
 }
 
-// A store of C with a cache policy.  ST_PLAIN: the compiler's store (write-back in the XCD's L2).  ST_THROUGH
-// (sc1): written through the L2 as it is issued, instead of leaving the L2 in bursts when lines are evicted or the
-// kernel ends -- the C of a GEMM is written once and read by nobody in this launch.  ST_STREAM (nt): streaming, for
-// outputs that should not take room in the caches from operands that are read again.  The host picks one per launch
-// (`store_policy`).  Measured (bf16, f32 C, us, plain / through / stream): 65536 x 256 x 256 20.8 / 18.0 / 20.7;
-// 131072 x 256 x 256 36.5 / 33.3 / 37.3; 65536 x 256 x 2048 76.0 / 75.2 / 65.0; 8192^3 731 / 730 / 689;
-// 16384 x 4096 x 4096 383 / 390 / 364; 65536 x 2048 x 512 178 / 177 / 158; 65536 x 1024 x 512 91 / 91 / 96;
-// 8192 x 8192 x 1024 123 / 128 / 132; 4096^3 92.6 / 91.8 / 92.2.
-enum { ST_PLAIN = 0, ST_THROUGH = 1, ST_STREAM = 2 };
-template <int POLICY, typename V>
-__device__ __forceinline__ void store_c(V* p, V v) {
-    static_assert(sizeof(V) == 16 || sizeof(V) == 8, "16- or 8-byte pieces of C");
-    if constexpr (POLICY == ST_STREAM) __builtin_nontemporal_store(v, p);
-    else if constexpr (POLICY == ST_PLAIN) *p = v;
-    else if constexpr (sizeof(V) == 16) store16_through(p, v);
-    else asm volatile("global_store_dwordx2 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
-}
-
-// One wave-wide DMA: every lane copies 16 bytes from global memory (uniform base + per-lane
-// 32-bit offset) to LDS byte m0 + 16 * lane.  Completion is tracked by vmcnt; the instruction is
-// issued from inline assembly so that the tile in flight does not make the compiler wait before
-// LDS reads of the tile being multiplied (it cannot tell the two buffers apart).
-__device__ __forceinline__ void dma_to_lds(const unsigned char* base, unsigned lane_offset, unsigned lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(lane_offset), "s"(base), "s"(lds_addr)
-                 : "memory", "m0");
-}
-
-// The same with a full address per lane (the last, partial K-tile of a ragged K: chunks past the end of a row
-// are fetched from a block of zeros instead).
-__device__ __forceinline__ void dma_to_lds_addr(const unsigned char* addr, unsigned lds_addr) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(addr), "s"(lds_addr) : "memory", "m0");
-}
-__device__ __attribute__((aligned(16))) const unsigned kZeroChunk[4] = {0u, 0u, 0u, 0u};
-
-__device__ __forceinline__ const unsigned char* uniform_ptr(const unsigned char* p) {
-    const unsigned long long v = (unsigned long long)p;
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
-    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-    return (const unsigned char*)(((unsigned long long)hi << 32) | lo);
-}
-
-// RAGGED: M, N and K need not be multiples of the tile (N a multiple of 4, K of 16 bytes).  Rows past the end are
-// fetched as copies of the last row and the chunks of the last K-tile that lie past the end of a row as zeros, so
-// every load stays inside the matrices, and the epilogue skips what lies outside C.
+// RAGGED: M, N and K need not be multiples of the tile (K a multiple of 16 bytes).  Rows past the end are fetched as
+// copies of the last row and the chunks of the last K-tile that lie past the end of a row as zeros, so every load stays
+// inside the matrices, and the epilogue skips what lies outside C.  With N not a multiple of 4 the rows of C start at any
+// element: the same wide stores at element alignment, and one to three single elements at the end of a row (5001 x 1003
+// x 1000 f16 846 -> 29 us against one thread per output).
 template <int DT, int OT, int BM, int BN, int WM, int WN, int NS = 2, int NSA = NS, bool RAGGED = false>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_abt_kernel(SP_GEMM_PRELOADED, const GemmArgs g_rest) {
     SP_GEMM_TAKE_PRELOADED;
@@ -489,7 +371,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_abt_kernel(SP_GEMM_PRELOADED
 #pragma unroll
             for (int js = 0; js < TN / SF; ++js) {
                 const long col = n0 + wn * WTN + js * SW + ec;
-                const bool col_ok = !RAGGED || col < g.N;
+                const bool col_ok = !RAGGED || col + 3 < g.N;          // all four columns of this lane
                 f32x4 bias4 = {0.f, 0.f, 0.f, 0.f};
                 if (g.bias && col_ok) bias4 = *reinterpret_cast<const f32x4*>(g.bias + col);
 #pragma unroll
@@ -502,28 +384,64 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_abt_kernel(SP_GEMM_PRELOADED
                     }
                 const long row_first = m0 + wm * WTM + i * 32 + er;
                 long idx = row_first * g.N + col;     // advanced by RPP rows per pass
-#pragma unroll
-                for (int p = 0; p < 32 / RPP; ++p, idx += row_step) {
-                    const int rl = p * RPP + er;
-                    const f32x4 v = *reinterpret_cast<const f32x4*>(stg + rl * EPI_STRIDE + ec * 4);
-                    if (RAGGED && !(col_ok && row_first + p * RPP < g.M)) continue;
-                    f32x4 old = {0.f, 0.f, 0.f, 0.f};
+                // one 4-column piece: what C held there, and the store
+                typedef typename std::conditional<RAGGED, f32x4_unaligned, f32x4>::type c32_t;
+                typedef typename std::conditional<RAGGED, u32x2_unaligned, u32x2>::type c16_t;
+                auto read_old = [&](long at) {
                     if constexpr (OT == SP_F32) {
-                        f32x4* c = reinterpret_cast<f32x4*>((float*)Cb + idx);
-                        if constexpr (HAS_BETA) old = *c;
-                        store_c<POLICY>(c, finish(v, old, bias4));
+                        return (f32x4)*reinterpret_cast<const c32_t*>((const float*)Cb + at);
                     } else {
-                        u32x2* c = reinterpret_cast<u32x2*>((unsigned short*)Cb + idx);
-                        if constexpr (HAS_BETA) {
-                            const u32x2 o = *c;
-                            old = f32x4{half_bits_to_f32<OT>(o.x & 0xffffu), half_bits_to_f32<OT>(o.x >> 16),
-                                        half_bits_to_f32<OT>(o.y & 0xffffu), half_bits_to_f32<OT>(o.y >> 16)};
-                        }
-                        const f32x4 r = finish(v, old, bias4);
+                        const u32x2 o = *reinterpret_cast<const c16_t*>((const unsigned short*)Cb + at);
+                        return f32x4{half_bits_to_f32<OT>(o.x & 0xffffu), half_bits_to_f32<OT>(o.x >> 16),
+                                     half_bits_to_f32<OT>(o.y & 0xffffu), half_bits_to_f32<OT>(o.y >> 16)};
+                    }
+                };
+                auto write = [&](long at, const f32x4& r) {
+                    if constexpr (OT == SP_F32) {
+                        store_c<POLICY>(reinterpret_cast<c32_t*>((float*)Cb + at), r);
+                    } else {
                         u32x2 o;
                         o.x = pack_halves<OT>(r.x, r.y);
                         o.y = pack_halves<OT>(r.z, r.w);
-                        store_c<POLICY>(c, o);
+                        store_c<POLICY>(reinterpret_cast<c16_t*>((unsigned short*)Cb + at), o);
+                    }
+                };
+                constexpr int PASSES = 32 / RPP;
+                if constexpr (RAGGED) {
+                    // The masks split every pass into blocks of its own, so nothing may wait inside them: all of LDS (and
+                    // of the old C) is read first, then everything is stored (63 x 223 x 24 f32 with beta: one read, one
+                    // store per pass 7.4 us, this form 4.4).
+                    f32x4 v[PASSES], old[PASSES];
+                    const long rows_left = g.M - row_first;
+#pragma unroll
+                    for (int p = 0; p < PASSES; ++p) {
+                        v[p] = *reinterpret_cast<const f32x4*>(stg + (p * RPP + er) * EPI_STRIDE + ec * 4);
+                        if constexpr (HAS_BETA) {
+                            old[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+                            if (col_ok && p * RPP < rows_left) old[p] = read_old(idx + p * row_step);
+                        }
+                    }
+                    const bool row_end = g.N % 4 != 0 && n0 + wn * WTN + js * SW < g.N && g.N < n0 + wn * WTN + (js + 1) * SW;
+                    if (row_end) {                       // the last one to three columns of this strip's 32 rows
+                        const int first = (int)(g.N / 4 * 4 - (n0 + wn * WTN + js * SW)), count = (int)(g.N % 4);
+                        const long row = m0 + wm * WTM + i * 32 + (lane & 31);
+                        for (int e = lane >> 5; e < count && row < g.M; e += 2) {
+                            const long c = n0 + wn * WTN + js * SW + first + e;
+                            const float sum = *reinterpret_cast<const float*>(stg + (lane & 31) * EPI_STRIDE + (first + e) * 4);
+                            store_element(Cb, OT, row * g.N + c, sum * alpha, HAS_BETA ? beta : 0.f, g.bias ? g.bias[c] : 0.f, RELU);
+                        }
+                    }
+#pragma unroll
+                    for (int p = 0; p < PASSES; ++p)
+                        if (col_ok && p * RPP < rows_left)
+                            write(idx + p * row_step, finish(v[p], HAS_BETA ? old[p] : f32x4{0.f, 0.f, 0.f, 0.f}, bias4));
+                } else {
+#pragma unroll
+                    for (int p = 0; p < PASSES; ++p, idx += row_step) {
+                        const f32x4 v = *reinterpret_cast<const f32x4*>(stg + (p * RPP + er) * EPI_STRIDE + ec * 4);
+                        f32x4 old = {0.f, 0.f, 0.f, 0.f};
+                        if constexpr (HAS_BETA) old = read_old(idx);
+                        write(idx, finish(v, old, bias4));
                     }
                 }
             }
@@ -958,8 +876,8 @@ __global__ __launch_bounds__(256) void gemm_abt_w4_kernel(SP_GEMM_PRELOADED, con
     }
 }
 
-// Shape-agnostic kernel: one thread per output element, 16-byte loads along K.  Used for shapes
-// the tiled kernels do not divide (the MLP's K = 32 or N = 3 for instance).
+// Shape-agnostic kernel: one thread per output element, 16-byte loads along K.  Only SP_GEMM_FORCE_GENERIC comes here
+// (every shape has an MFMA kernel): a second opinion for tests.
 template <int DT>
 __global__ __launch_bounds__(256) void gemm_abt_generic_kernel(const GemmArgs g) {
     constexpr int ES = (DT == SP_F32) ? 4 : 2;
@@ -1055,19 +973,75 @@ static int choose_cfg(int dtype_in, long M, long N, long K, long batch = 1) {
     return smallest;
 }
 
-// Shapes no tile divides: the same tiled kernels with rows clamped in the loader, zeros for the missing part of the
-// last K-tile and a masked epilogue, provided N is a multiple of 4 (16-byte accesses to C and the bias).  Tile choice
-// as above, on tile counts rounded up.
-static int choose_cfg_ragged(int dtype_in, long M, long N, long K, long batch) {
-    (void)K;   // any K that passed validation (a multiple of 16 bytes)
-    if (N % 4 != 0) return -1;
-    const int cus = device_cu_count();
-    for (int i = 0; i < kNumCfgs; ++i) {
-        const TileCfg& c = kTileCfgs[i];
-        const long tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * batch;
-        if (tiles * 5 >= (long)cus * 4) return i;
+// The tile a GEMM runs on: a workgroup tile of kTileCfgs (cfg 0..2) or a split-K tile of gemm_wave.hip (cfg < 0).
+// `ragged`: the tile does not divide M, N and K -- rows clamped in the loader, zeros for the missing part of the last
+// K-tile, a masked epilogue.
+struct TileChoice {
+    int cfg, bm, bn, threads;
+    bool ragged;
+};
+
+// Estimated time of the most loaded compute unit on a tile, in us: n = ceil(tiles / units) tiles one after the other,
+// each nk K-tiles of `tk` plus `overhead` (prologue, epilogue, padding of its stores), and never less than `latency` per
+// K-tile (what a lone workgroup per unit waits for its loads).  Fitted to every tile on ~60 shapes; the estimate is within
+// 15 % for f32 and 30 % for 16-bit, and what matters is the order (us, 256 / 128 / 64 / split 32 x 32): f32 6928 x 624 x 680
+// 176 / 94 / 66 / 74; 43712 x 48 x 336 98 / 54 / 25 / 33; 4000 x 4000 x 1000 251 / 258 / 269 / 338; 6160 x 192 x 2984
+// 696 / 202 / 103 / 80; 3072 x 1024 x 1024 237 / 71 / 58 / 67; bf16 3000^3 80 / 109 / 125 / 257; 54928 x 80 x 5504 180 /
+// 157 / 189 / 213; 4784 x 912 x 64 f32 34 / 22 / 15 / 28; f16 5001 x 1003 x 1000 44 / 29 / 33 / 40.  16-bit rows that
+// do not start on 128-byte lines cost every fetch a second line, hence two sets of numbers.
+struct TileCost {
+    int cfg, bm, bn;
+    float tk, overhead, latency;
+};
+static const TileCost kCostF32[] = {{0, 256, 256, 7.85f, 10.f, 0.f}, {1, 128, 128, 2.13f, 3.f, 0.f}, {2, 64, 64, 0.57f, 1.f, 0.f},
+                                    {-1, 32, 32, 0.184f, 0.5f, 0.f}, {-1, 16, 16, 0.089f, 0.3f, 0.f}};
+static const TileCost kCostLines[] = {{0, 256, 256, 1.75f, 8.f, 0.f}, {1, 128, 128, 0.55f, 3.5f, 1.05f}, {2, 64, 64, 0.22f, 0.8f, 0.25f},
+                                      {-1, 64, 64, 0.22f, 1.5f, 0.f}, {-1, 64, 32, 0.17f, 0.8f, 0.f}, {-1, 32, 32, 0.09f, 0.5f, 0.f},
+                                      {-1, 16, 16, 0.05f, 0.3f, 0.f}};
+static const TileCost kCostCrossing[] = {{0, 256, 256, 1.5f, 14.f, 0.f}, {1, 128, 128, 0.65f, 4.f, 1.05f}, {2, 64, 64, 0.29f, 0.8f, 0.5f},
+                                         {-1, 64, 64, 0.27f, 1.5f, 0.f}, {-1, 64, 32, 0.19f, 0.8f, 0.f}, {-1, 32, 32, 0.11f, 0.5f, 0.f},
+                                         {-1, 16, 16, 0.055f, 0.3f, 0.f}};
+
+static TileChoice choose_tile(int dtype_in, long M, long N, long K, long batch) {
+    const int es = dtype_in == SP_F32 ? 4 : 2, bk = ROW_BYTES / es;
+    const long cus = device_cu_count(), nk = (K + bk - 1) / bk;
+    // 16-bit shapes that a 256 or 128 tile divides: choose_cfg.  The rest, and f32, by the estimate.
+    const int whole = dtype_in == SP_F32 ? -1 : choose_cfg(dtype_in, M, N, K, batch);
+    int best = whole;
+    float best_us = 0.f;
+    int bm = 0, bn = 0;
+    if (whole != 0 && whole != 1) {
+        best = -2;
+        // K split over four waves: from seven K-tiles up.  Below that (where a large output wants the workgroup tiles
+        // whatever the estimate says, and where a member of a batch and a plain call of its shape take the same sums) only
+        // for small outputs, whose time is the chain behind one of them (us, 64 x 64 tile / split: 181 x 39 x 96 f32 6.9 /
+        // 3.9; 86 x 61 x 56 5.6 / 3.6; 16 x 21 x 144 bf16 4.4 / 3.4), and for odd widths, where the split form's stores
+        // cost less (5371 x 45 x 48 f16 5.4 / 4.5).
+        const double small = (double)((M + 15) / 16) * (double)((N + 15) / 16);
+        const bool may_split = nk >= 7 || (batch <= 64 && small <= (N % 4 ? 1024 : 64));
+        auto consider = [&](const TileCost& c) {
+            if (whole == 2 && (c.cfg == 0 || c.cfg == 1)) return;
+            if (c.cfg < 0 && (!may_split || K * es > kWaveMaxRowBytes || M > 2147483000l || N > 2147483000l)) return;
+            const double tiles = (double)((M + c.bm - 1) / c.bm) * (double)((N + c.bn - 1) / c.bn) * (double)batch;
+            const float n = (float)((tiles + cus - 1) / cus >= 1e9 ? 1e9 : (double)(long)((tiles + cus - 1) / cus));
+            const float per_k = n * c.tk > c.latency ? n * c.tk : c.latency;
+            const float us = n * c.overhead + (float)nk * per_k;
+            if (best == -2 || us < best_us) {
+                best = c.cfg;
+                best_us = us;
+                bm = c.bm;
+                bn = c.bn;
+            }
+        };
+        if (dtype_in == SP_F32) for (const TileCost& c : kCostF32) consider(c);
+        else if (K % bk == 0) for (const TileCost& c : kCostLines) consider(c);
+        else for (const TileCost& c : kCostCrossing) consider(c);
     }
-    return kNumCfgs - 1;
+    if (best < 0) return {-1, bm, bn, 256, true};
+    const TileCfg& t = kTileCfgs[best];
+    const bool ragged = M % t.bm != 0 || N % t.bn != 0 || K % bk != 0;
+    const int threads = best == 0 && !ragged && use_four_waves(dtype_in, N, K) ? 256 : t.wm * t.wn * 64;
+    return {best, t.bm, t.bn, threads, ragged};
 }
 
 template <int DT, int OT, int BM, int BN, int WM, int WN, int NS, int NSA = NS, bool RAGGED = false>
@@ -1256,19 +1230,11 @@ extern "C" int sp_gemm_config(int dtype_in, int64_t M, int64_t N, int64_t K, int
     if (!tile_m || !tile_n || !tile_k || !threads) return fail(SP_ERR_NULL, "sp_gemm_config: NULL output");
     int rc = validate_gemm(dtype_in, SP_F32, M, N, K);
     if (rc != SP_OK) return rc;
-    int cfg = choose_cfg(dtype_in, M, N, K);
-    bool ragged = false;
-    if (cfg < 0) {
-        cfg = choose_cfg_ragged(dtype_in, M, N, K, 1);
-        ragged = cfg >= 0;
-    }
-    if (cfg < 0) {
-        *tile_m = 0; *tile_n = 0; *tile_k = 0; *threads = 256;
-    } else {
-        *tile_m = kTileCfgs[cfg].bm; *tile_n = kTileCfgs[cfg].bn; *tile_k = dtype_in == SP_F32 ? 32 : 64;
-        *threads = kTileCfgs[cfg].wm * kTileCfgs[cfg].wn * 64;
-        if (cfg == 0 && !ragged && use_four_waves(dtype_in, N, K)) *threads = 256;
-    }
+    const TileChoice t = choose_tile(dtype_in, M, N, K, 1);
+    *tile_m = t.bm;
+    *tile_n = t.bn;
+    *tile_k = dtype_in == SP_F32 ? 32 : 64;
+    *threads = t.threads;
     return SP_OK;
 }
 
@@ -1286,7 +1252,6 @@ static int gemm_entry(const char* fn, int dtype_in, int dtype_out, const void* A
     if (batch > 1 && stride_c < M * N) return fail(SP_ERR_ARG, "%s: the outputs of a batch must not overlap", fn);
     rc = require_gfx950(fn);
     if (rc != SP_OK) return rc;
-    int cfg = (flags & SP_GEMM_FORCE_GENERIC) ? -1 : choose_cfg(dtype_in, M, N, K, batch);
     GemmArgs g{};
     g.A = A; g.B = B; g.C = C; g.bias = bias; g.M = M; g.N = N; g.K = K; g.alpha = alpha; g.beta = beta;
     g.relu = (flags & SP_GEMM_RELU) ? 1 : 0;
@@ -1303,15 +1268,16 @@ static int gemm_entry(const char* fn, int dtype_in, int dtype_out, const void* A
         g.store_policy = (in_bytes >= 140 * MiB || out_bytes >= 384 * MiB) ? ST_STREAM : ST_THROUGH;
     }
     g.stride_a = stride_a * es_in; g.stride_b = stride_b * es_in; g.stride_c = stride_c * es_out;
-    if (cfg < 0 && !(flags & SP_GEMM_FORCE_GENERIC)) {
-        cfg = choose_cfg_ragged(dtype_in, M, N, K, batch);
-        g.ragged = cfg >= 0;
-    }
-    if (cfg >= 0) {
-        g.tiles_m = (int)((M + kTileCfgs[cfg].bm - 1) / kTileCfgs[cfg].bm);
-        g.tiles_n = (int)((N + kTileCfgs[cfg].bn - 1) / kTileCfgs[cfg].bn);
-    }
     hipStream_t s = (hipStream_t)stream;
+    int cfg = -1;                                         // the generic kernel
+    if (!(flags & SP_GEMM_FORCE_GENERIC)) {
+        const TileChoice t = choose_tile(dtype_in, M, N, K, batch);
+        cfg = t.cfg;
+        g.ragged = t.ragged;
+        g.tiles_m = (int)((M + t.bm - 1) / t.bm);
+        g.tiles_n = (int)((N + t.bn - 1) / t.bn);
+        if (cfg < 0) return launch_gemm_wave(dtype_in, t.bm, t.bn, g, s);
+    }
     switch (dtype_in) {
         case SP_F32: return launch_dtype<SP_F32, SP_F32>(cfg, g, s);
         case SP_F16:

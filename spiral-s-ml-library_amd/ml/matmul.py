@@ -16,7 +16,7 @@ from ._lib import check, lib, ptr, stream_ptr
 
 def matmul_config_tf32(a_trans, b_trans, m, n, k, dtype=torch.float32):
     """Tile configuration chosen for a shape (counterpart of ml/matmul/run.spi:8-19).
-    Returns dict(m_tile, n_tile, k_tile, threads); m_tile == 0 means the general kernel."""
+    Returns dict(m_tile, n_tile, k_tile, threads)."""
     out = [C.c_int32() for _ in range(4)]
     check(lib.sp_gemm_config(_lib.DTYPES[dtype], m, n, k, *[C.byref(o) for o in out]))
     return dict(zip(("m_tile", "n_tile", "k_tile", "threads"), (o.value for o in out)))

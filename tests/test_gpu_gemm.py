@@ -109,6 +109,37 @@ def test_ragged_m_and_n(MM, dtype, m, n, k):
     assert (got[pad:pad + m * n].reshape(m, n).astype(np.float64) == np.maximum(want + 2 * c0 + bias, 0)).all()
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("m,n,kt", [(1, 1, 1), (17, 3, 6), (31, 33, 6), (130, 31, 5.5), (5000, 5, 2), (16, 4096, 7), (33, 15, 7),
+                                    (257, 16, 7.5), (250, 250, 8), (500, 331, 9), (1900, 241, 11), (331, 65, 27.5), (1, 9001, 13),
+                                    (9001, 2, 30), (1027, 1027, 3.5), (4099, 259, 6), (2049, 2051, 7.5)])
+def test_split_k_and_odd_widths_are_exact(MM, dtype, m, n, kt):
+    """Small and narrow outputs (K split over the waves of a workgroup, tiles of 16 x 16 to 64 x 64) and widths that are not
+    a multiple of 4, there and on the workgroup tiles: integer operands give the exact product in every output type, with
+    bias + ReLU and beta, and nothing outside C is touched."""
+    k = int(kt * (32 if dtype == "f32" else 64))
+    announce("gemm split K / odd widths %s %dx%dx%d" % (dtype, m, n, k))
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    ai = rng.integers(-3, 4, size=(m, k)).astype(np.float32)
+    bi = rng.integers(-3, 4, size=(n, k)).astype(np.float32)
+    want = ai.astype(np.float64) @ bi.astype(np.float64).T
+    bias = rng.integers(-5, 6, size=n).astype(np.float32)
+    c0 = rng.integers(-4, 5, size=(m, n)).astype(np.float32)
+    a, b = dev(ai, TORCH[dtype]), dev(bi, TORCH[dtype])
+    pad = 64
+    for out in {"f32", dtype}:
+        exact = lambda x: x if out == "f32" else ogemm.round_to(x.astype(np.float32), dtype)
+        for beta in (0.0, 2.0):
+            buf = torch.full((pad + m * n + pad,), -77.0, dtype=TORCH[out], device="cuda")
+            c = buf[pad:pad + m * n].view(m, n)
+            c.copy_(dev(c0))
+            MM.matmul_abt(a, b, c=c, beta=beta, bias=dev(bias) if beta else None, relu=beta != 0)
+            got = host(buf.float())
+            assert (got[:pad] == -77).all() and (got[pad + m * n:] == -77).all()
+            full = np.maximum(want + 2 * c0 + bias, 0) if beta else want
+            assert (got[pad:pad + m * n].reshape(m, n) == exact(full)).all(), (out, beta)
+
+
 def test_random_small_shapes_are_exact(MM):
     """120 seeded shapes around the tile boundaries (M, N up to 330, K up to 45 chunks), all three dtypes, integer
     operands: the tiled kernels' masking of M, N and K must give the exact product, with and without bias + ReLU."""
