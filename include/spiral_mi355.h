@@ -427,6 +427,21 @@ int sp_mlp_forward_ensemble(int dtype, const void* x, int32_t n_layers, const vo
                             int32_t members, const float* u, const sp_philox_t* philox, float* policy_out,
                             int32_t* action_out, int64_t batch, int32_t head, int32_t mask_size, void* stream);
 
+/* Fused forward of a stack of f32 layers with a row head, for one model (members = 1) or every member of an ensemble on one
+ * shared input, one launch:
+ *   h_0 = x,  h_{l+1} = act_l(h_l . W_l[e]^T),  policy[e] = head(h_{n-1} . W_{n-1}[e]^T), action[e] sampled from it.
+ * x: (batch, dims[0]); weights[l]: (members, dims[l + 1], dims[l]); dims[0] a multiple of 4 up to 128, hidden widths multiples
+ * of 16 up to 128, the output width a multiple of 4 up to 64; 1 to 8 layers whose weights (16 x 16 blocks of 1 KiB; of a
+ * masked head only the valid columns) fit 144 KiB of LDS, else SP_ERR_UNSUPPORTED.  acts[l] (l < n_layers - 1): an sp_map_op,
+ * plus SP_STACK_LN_L2 for ln_l2 in front of it.  head_op: SP_ROW_SOFTMAX, SP_ROW_MASKED_SOFTMAX, SP_ROW_REGRET_MATCHING or
+ * SP_ROW_MASKED_REGRET_MATCHING, with the results of sp_row_sample on the logits.  u, philox, policy_out, action_out as for
+ * sp_mlp_forward_ensemble; members x batch below 2^31.
+ * Replaces: the node-by-node run (ml/layers.spi:194-240, 336-344) of the graphs of ml/layers.spi:564-665. */
+#define SP_STACK_LN_L2 0x100
+int sp_stack_forward_f32(const void* x, int32_t n_layers, const void* const* weights, const int32_t* dims, const int32_t* acts,
+                         int32_t members, const float* u, const sp_philox_t* philox, float* policy_out, int32_t* action_out,
+                         int64_t batch, int32_t head_op, int32_t mask_size, void* stream);
+
 /* out[e][r] = (OR over j of (not (y[r, j] <= 0)) << j) mod modulo with y = x . W[e]^T: one ensemble layer and the hash
  * head `binarize` in one launch; y is never written.  x: (batch, k0) f32, k0 a multiple of 8 in [8, 256]; weights:
  * (members, n, k0) f32; out: (members, batch) u32.  As in sp_row_binarize the shift is the device's 32-bit shift

@@ -1,6 +1,7 @@
 // What the GEMM kernels share: arguments, the swizzled LDS tile, the DMA loads and the stores of C.
 #pragma once
 #include "common.h"
+#include "gemm_dma.h"
 #include <type_traits>
 
 namespace sp {
@@ -129,13 +130,6 @@ __device__ __forceinline__ void dma_to_lds(const unsigned char* base, unsigned l
                  : "v"(lane_offset), "s"(base), "s"(lds_addr)
                  : "memory", "m0");
 }
-
-// The same with a full address per lane (the last, partial K-tile of a ragged K: chunks past the end of a row
-// are fetched from a block of zeros instead).
-__device__ __forceinline__ void dma_to_lds_addr(const unsigned char* addr, unsigned lds_addr) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(addr), "s"(lds_addr) : "memory", "m0");
-}
-__device__ __attribute__((aligned(16))) const unsigned kZeroChunk[4] = {0u, 0u, 0u, 0u};
 
 __device__ __forceinline__ const unsigned char* uniform_ptr(const unsigned char* p) {
     const unsigned long long v = (unsigned long long)p;

@@ -1,0 +1,333 @@
+// Fused forward of a stack of small f32 layers -- matmul [-> ln_l2] [-> relu | tanh | sigmoid] -> ... -> matmul -> row head
+// [-> sampling] -- for one model or for every member of an ensemble on one shared input, in one launch.  These are the graphs
+// of ml/layers.spi test3 - test5 (:564-665), which the interpreter (:194-240, 336-344) runs node by node.
+//
+// A wave owns 16 batch rows and takes them through the whole stack; the activations never leave its registers.  The product
+// is v_mfma_f32_16x16x4 with the WEIGHTS as the row operand, so lane (r, q) -- r = lane % 16 the batch row, q = lane / 16 --
+// ends up with features 16 t + 4 q + i of row r in register i of tile t.  Which K-index an MFMA step takes from lane group q
+// is free as long as both operands agree: step i of K-block j stands for k = 16 j + 4 q + i, so a layer's result registers
+// ARE the next layer's second operand.  The norm of a row is 4 registers x tiles and two cross-lane adds.
+//   The weights of all layers sit in LDS in the order they are consumed (one 1 KiB block per 16 x 16 of W, lane l's 16 bytes
+// at 16 l: conflict-free reads, and the DMA's natural layout), so the walk over a stack is one pointer that advances by
+// 1 KiB per four MFMAs, one block ahead of them.  Features and K past a layer's widths are zeros.
+//   The logits cross LDS once more, from the feature-major registers into one row per 16 lanes: the head and the sampling
+// are the row primitives' own operations in their order, and the stores are whole rows.
+//
+// What bounds it: the f32 matrix pipe (157 TFLOP/s), 32 cycles per MFMA and SIMD; a 64-64-64-64 stack is 6144 of them for
+// 16 rows.  16-row tiles because a batch of 16384 rows is then one tile per SIMD.
+// Measured (node by node / this kernel, us): 64-64-64-64 with ln_l2 and relu, softmax and sampling over 16384 rows 32.8 / 13.8,
+// 16 members of it 206 / 87 (41 on the matrix pipe alone).
+#include "mlp_common.h"
+#include "row_common.h"
+#include "gemm_dma.h"
+
+#pragma clang fp contract(off)
+
+namespace sp {
+
+constexpr int ST_ROWS = 16;            // batch rows per tile
+constexpr int ST_MAX_LAYERS = 8;
+constexpr int ST_MAX_WIDTH = 128;
+constexpr int ST_MAX_OUT = 64;
+constexpr int ST_MAX_THREADS = 512;
+constexpr int ST_BLOCK = 1024;         // bytes of a 16 x 16 block of weights
+constexpr int ST_SCRATCH = ST_ROWS * ST_MAX_OUT * 4;   // per wave: the logits on their way into rows
+constexpr int ST_LDS = 160 * 1024;
+
+struct StackArgs {
+    const float* x;
+    const float* u;                    // (members, batch) uniforms, or nullptr
+    float* policy;                     // (members, batch, n)
+    int* action;                       // (members, batch), or nullptr
+    const float* w[ST_MAX_LAYERS];     // (members, dims[l + 1], dims[l])
+    int dims[ST_MAX_LAYERS + 1];       // the last one: the computed outputs (a mask leaves only its own)
+    int acts[ST_MAX_LAYERS];           // sp_map_op, plus SP_STACK_LN_L2
+    int n_layers, n, mask_size;        // n: output width; mask_size: the valid columns of the head
+    int w_bytes;                       // weights in LDS
+    int batch, tiles;
+    long out_stride;                   // floats between two members' weights of the last layer
+    PhiloxStream ph;
+};
+
+template <typename F>
+__device__ __forceinline__ void map_tiles(f32x4* y, int nt, int count, F f) {
+#pragma unroll
+    for (int t = 0; t < count; ++t)
+        if (t < nt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[t][i] = f(y[t][i]);
+}
+
+// HT: 16-wide tiles of the widest layer (4 or 8).  OPK: 0 softmax, 1 masked softmax, 2 regret matching (mask_size columns).
+template <int HT, int OPK>
+__global__ __launch_bounds__(ST_MAX_THREADS) void mlp_stack_kernel(const StackArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int waves = blockDim.x >> 6;
+    const int r = lane & 15, q = lane >> 4;
+    const int e = blockIdx.y;
+    const float NEG_INF = -__builtin_inff();
+    const int layers = a.n_layers, k0 = a.dims[0], kt0 = (k0 + 15) >> 4;
+
+    auto load_x = [&](int tile, f32x4 (&x)[HT]) {
+        int row = tile * ST_ROWS + r;
+        row = row < a.batch ? row : a.batch - 1;
+        const float* xr = a.x + (long)row * k0;
+#pragma unroll
+        for (int j = 0; j < HT; ++j) {
+            x[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const int col = 16 * j + 4 * q;
+            if (j < kt0 && col < k0) x[j] = *reinterpret_cast<const f32x4*>(xr + col);
+        }
+    };
+    int tile = blockIdx.x * waves + wave;
+    f32x4 x[HT];
+    if (tile < a.tiles) load_x(tile, x);
+
+    // ---- the member's weights, once per workgroup ----
+    const unsigned lds0 = (unsigned)(size_t)lds;
+    {
+        unsigned dst = lds0;
+        for (int l = 0; l < layers; ++l) {
+            const int K = a.dims[l], F = a.dims[l + 1], kt = (K + 15) >> 4, nt = (F + 15) >> 4;
+            const float* W = a.w[l] + (long)e * (l + 1 < layers ? (long)F * K : a.out_stride);
+            for (int b = wave; b < kt * nt; b += waves) {
+                const int t = b / kt, row = 16 * t + r, col = 16 * (b - t * kt) + 4 * q;
+                const unsigned char* at = (const unsigned char*)(W + (long)row * K + col);
+                dma_to_lds_addr(row < F && col < K ? at : (const unsigned char*)kZeroChunk, __builtin_amdgcn_readfirstlane(dst + b * ST_BLOCK));
+            }
+            dst += kt * nt * ST_BLOCK;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+    unsigned char* const scratch = lds + a.w_bytes + wave * ST_SCRATCH;
+    const int stride = gridDim.x * waves;
+
+    for (; tile < a.tiles; tile += stride) {
+        const int my_row = tile * ST_ROWS + r;
+        float u = 1.f;
+        if (a.action != nullptr) {
+            const int row = my_row < a.batch ? my_row : a.batch - 1;
+            if (a.ph.philox_mode < 0) u = a.u[(long)e * a.batch + row];
+            else if (a.ph.member_rows > 0) u = run_row_uniform<unsigned>(a.ph, row, a.ph.draw_offset + (unsigned long long)e * a.ph.member_draws);
+            else u = run_row_uniform<unsigned>(a.ph, (unsigned)e * a.batch + row, a.ph.draw_offset);
+        }
+
+        const unsigned char* wp = lds + lane * 16;
+        f32x4 w = *reinterpret_cast<const f32x4*>(wp);
+        f32x4 xn[HT];
+        load_x(tile + stride < a.tiles ? tile + stride : tile, xn);
+        int nt = 0;
+        for (int l = 0; l < layers; ++l) {
+            const int kt = (a.dims[l] + 15) >> 4;
+            nt = (a.dims[l + 1] + 15) >> 4;
+            f32x4 y[HT];
+#pragma unroll
+            for (int t = 0; t < HT; ++t) {
+                y[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (t < nt) {
+#pragma unroll
+                    for (int j = 0; j < HT; ++j)
+                        if (j < kt) {
+                            // (behind the last block of the stack lies the scratch: read, not used)
+                            wp += ST_BLOCK;
+                            const f32x4 next = *reinterpret_cast<const f32x4*>(wp);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) y[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[j][i], y[t], 0, 0, 0);
+                            w = next;
+                        }
+                }
+            }
+            if (l + 1 < layers) {
+                const int act = a.acts[l];
+                if (act & SP_STACK_LN_L2) {       // local_ln_l2 (ml/primitives.spi:701-703)
+                    float s = 0.f;
+#pragma unroll
+                    for (int t = 0; t < HT; ++t) {
+                        float sq[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) sq[i] = y[t][i] * y[t][i];
+                        s = t == 0 ? sum4(sq) : s + sum4(sq);
+                    }
+                    s += __shfl_xor(s, 16);
+                    s += __shfl_xor(s, 32);
+                    const RowDivisor over_s(s);
+                    map_tiles(y, nt, HT, [&](float v) { return s != 0.f ? over_s(v) : 0.f; });
+                }
+                const int map = act & ~SP_STACK_LN_L2;
+                if (map == SP_MAP_RELU) map_tiles(y, nt, HT, [](float v) { return fmaxf(v, 0.f); });
+                else if (map == SP_MAP_TANH) map_tiles(y, nt, HT, [](float v) { return tanhf(v); });
+                else if (map == SP_MAP_SIGMOID) map_tiles(y, nt, HT, [](float v) { return 1.f / (1.f + expf(-v)); });
+            }
+#pragma unroll
+            for (int t = 0; t < HT; ++t) x[t] = y[t];
+        }
+
+        // ---- logits into rows: quad c of row r at slot c ^ r of its 256 bytes ----
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (t < nt) *reinterpret_cast<f32x4*>(scratch + r * 256 + (((4 * t + q) ^ r) & 15) * 16) = x[t];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+        // ---- the head and the sampling: lane l of 16 holds columns 4 l .. of its row, as in the row primitives ----
+        const int lq = r;                         // (lane % 16 again: here the column quad)
+        const int limit = a.mask_size;
+#pragma unroll
+        for (int pass = 0; pass < 4; ++pass) {
+            const int rr = 4 * pass + q;
+            const int row = tile * ST_ROWS + rr;
+            f32x4 v = *reinterpret_cast<const f32x4*>(scratch + rr * 256 + ((lq ^ rr) & 15) * 16);
+            // columns past the head's width, or its mask, enter as -inf (an exact 0 after the exponential) or 0
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (4 * lq + k >= limit) v[k] = NEG_INF;
+            float p[4];
+            if constexpr (OPK == 2) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) p[k] = 4 * lq + k < limit ? fmaxf(v[k], 0.f) : 0.f;
+                const float s = group_reduce<16>(sum4(p), [](float m, float n) { return m + n; });
+                const float inv_len = 1.f / (float)limit;
+                const RowDivisor over_s(s);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) p[k] = 4 * lq + k < limit ? (s != 0.f ? over_s(p[k]) : inv_len) : 0.f;
+            } else {
+                const float m = group_max<16>(vmax(vmax(v[0], v[1]), vmax(v[2], v[3])));
+#pragma unroll
+                for (int k = 0; k < 4; ++k) p[k] = fast_exp(v[k] - m);
+                const float s = group_reduce<16>(sum4(p), [](float m, float n) { return m + n; });
+                const float inv = 1.f / s;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) p[k] = p[k] * inv;
+            }
+            const bool row_ok = row < a.batch;
+            const long out_row = (long)e * a.batch + row;
+            if (row_ok && 4 * lq < a.n)
+                store16_through(reinterpret_cast<f32x4*>(a.policy + out_row * a.n + 4 * lq), f32x4{p[0], p[1], p[2], p[3]});
+            if (a.action != nullptr) {            // local_discrete_sampling (ml/primitives.spi:782-798)
+                const float incl = group_inclusive_scan<16>(sum4(p), lq);
+                float run = dpp_move<0x138>(incl);
+                if (lq == 0) run = 0.f;
+                float c[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    run = run + p[k];
+                    c[k] = run;
+                }
+                const float m = group_max<16>(sum4(p) > 0.f ? c[3] : NEG_INF);
+                const float thr = __shfl(u, rr) * m;
+                int pick = 2147483647;
+#pragma unroll
+                for (int k = 3; k >= 0; --k)
+                    if (p[k] > 0.f && c[k] >= thr) pick = 4 * lq + k;
+                pick = group_reduce<16>(pick, [](int m, int n) { return m < n ? m : n; });
+                if (row_ok && lq == 0) a.action[out_row] = pick;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < HT; ++j) x[j] = xn[j];
+    }
+}
+
+}  // namespace sp
+
+using namespace sp;
+
+template <int HT>
+static const void* pick_stack_kernel(int opk) {
+    return opk == 0 ? (const void*)mlp_stack_kernel<HT, 0> : opk == 1 ? (const void*)mlp_stack_kernel<HT, 1> : (const void*)mlp_stack_kernel<HT, 2>;
+}
+
+// Bytes of LDS the weights take (dims[n_layers] = the computed outputs).
+static long stack_weight_bytes(int n_layers, const int* dims) {
+    long blocks = 0;
+    for (int l = 0; l < n_layers; ++l) blocks += (long)((dims[l] + 15) / 16) * ((dims[l + 1] + 15) / 16);
+    return blocks * ST_BLOCK;
+}
+
+// Reference role: the body of `graph_run_host model` (ml/layers.spi:336-344) for the chains named at the top.
+extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void* const* weights, const int32_t* dims,
+                                    const int32_t* acts, int32_t members, const float* u, const sp_philox_t* philox,
+                                    float* policy_out, int32_t* action_out, int64_t batch, int32_t head_op, int32_t mask_size,
+                                    void* stream) {
+    SP_REQUIRE_PTR(x);
+    SP_REQUIRE_PTR(policy_out);
+    SP_OPTIONAL_PTR(u); SP_OPTIONAL_PTR(action_out);
+    if (weights == nullptr || dims == nullptr || acts == nullptr) return fail(SP_ERR_NULL, "sp_stack_forward_f32: weights/dims/acts is NULL");
+    if (n_layers < 1 || n_layers > ST_MAX_LAYERS) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: 1 to %d layers, got %d", ST_MAX_LAYERS, n_layers);
+    if (members <= 0 || members > 65535) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: members must be in [1, 65535]");
+    if (batch <= 0 || batch >= (1ll << 31) / members - ST_ROWS) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: batch must be positive and members x batch below 2^31");
+    const int opk = head_op == SP_ROW_SOFTMAX ? 0 : head_op == SP_ROW_MASKED_SOFTMAX ? 1
+                  : head_op == SP_ROW_REGRET_MATCHING || head_op == SP_ROW_MASKED_REGRET_MATCHING ? 2 : -1;
+    if (opk < 0) return fail(SP_ERR_ARG, "sp_stack_forward_f32: unknown head %d", head_op);
+    if (action_out != nullptr && u == nullptr && philox == nullptr)
+        return fail(SP_ERR_NULL, "sp_stack_forward_f32: action requested but u and philox are NULL");
+    if (u != nullptr && philox != nullptr) return fail(SP_ERR_ARG, "sp_stack_forward_f32: at most one of u and philox may be given");
+    const int n = dims[n_layers];
+    if (dims[0] < 4 || dims[0] % 4 != 0 || dims[0] > ST_MAX_WIDTH)
+        return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: input width %d must be a multiple of 4 in [4, %d]", dims[0], ST_MAX_WIDTH);
+    for (int l = 1; l < n_layers; ++l)
+        if (dims[l] < 16 || dims[l] % 16 != 0 || dims[l] > ST_MAX_WIDTH)
+            return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: hidden width %d must be a multiple of 16 in [16, %d]", dims[l], ST_MAX_WIDTH);
+    if (n < 4 || n % 4 != 0 || n > ST_MAX_OUT)
+        return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: output width %d must be a multiple of 4 in [4, %d]", n, ST_MAX_OUT);
+    const bool masked = head_op == SP_ROW_MASKED_SOFTMAX || head_op == SP_ROW_MASKED_REGRET_MATCHING;
+    if (masked && (mask_size <= 0 || mask_size > n)) return fail(SP_ERR_ARG, "sp_stack_forward_f32: mask_size must be in [1, %d], got %d", n, mask_size);
+    StackArgs a{};
+    int widest = 0;
+    for (int l = 0; l < n_layers; ++l) {
+        if (weights[l] == nullptr) return fail(SP_ERR_NULL, "sp_stack_forward_f32: weights[%d] is NULL", l);
+        if (!aligned16(weights[l])) return fail(SP_ERR_ALIGN, "sp_stack_forward_f32: weights[%d] is not 16-byte aligned", l);
+        const int map = acts[l] & ~SP_STACK_LN_L2;
+        if (map != SP_MAP_COPY && map != SP_MAP_RELU && map != SP_MAP_TANH && map != SP_MAP_SIGMOID)
+            return fail(SP_ERR_ARG, "sp_stack_forward_f32: unknown activation %d of layer %d", acts[l], l);
+        a.w[l] = (const float*)weights[l];
+        a.acts[l] = acts[l];
+        a.dims[l] = dims[l];
+        if (dims[l] > widest) widest = dims[l];
+    }
+    a.ph.philox_mode = -1;
+    int rc = mlp_set_philox(a.ph, philox, (int64_t)members * batch, n, __func__);
+    if (rc != SP_OK) return rc;
+    if (philox != nullptr && philox->member_rows > 0 && philox->member_rows != batch)
+        return fail(SP_ERR_ARG, "sp_stack_forward_f32: member_rows must be the batch");
+    a.mask_size = masked ? mask_size : n;
+    a.dims[n_layers] = a.mask_size;
+    a.out_stride = (long)n * dims[n_layers - 1];
+    const long w_bytes = stack_weight_bytes(n_layers, a.dims);
+    if (w_bytes > ST_LDS - 4 * ST_SCRATCH)
+        return fail(SP_ERR_UNSUPPORTED, "sp_stack_forward_f32: %ld bytes of weights exceed the LDS", w_bytes);
+    rc = require_gfx950(__func__);
+    if (rc != SP_OK) return rc;
+    a.x = (const float*)x; a.u = u; a.policy = policy_out; a.action = action_out;
+    a.n_layers = n_layers; a.n = n; a.w_bytes = (int)w_bytes; a.batch = (int)batch;
+    a.tiles = (int)((batch + ST_ROWS - 1) / ST_ROWS);
+    // Four waves a workgroup while that is one tile per SIMD; beyond it eight, so that one wave's norms and head run beside
+    // another's products, and as many workgroups per unit as the LDS holds (at most two).
+    const long cus = device_cu_count();
+    const int waves = (long)a.tiles * members > 4 * cus && w_bytes + 8 * ST_SCRATCH <= ST_LDS ? 8 : 4;
+    const int lds_bytes = (int)w_bytes + waves * ST_SCRATCH;
+    const int resident = 2 * lds_bytes <= ST_LDS ? 2 : 1;
+    long gx = (cus * resident + members - 1) / members;
+    const long most = (a.tiles + waves - 1) / waves;
+    if (gx > most) gx = most;
+    const long each = (a.tiles + gx * waves - 1) / (gx * waves);      // tiles per wave: no more workgroups than give that
+    gx = (a.tiles + each * waves - 1) / (each * waves);
+    const void* kernel = widest <= 64 ? pick_stack_kernel<4>(opk) : pick_stack_kernel<8>(opk);
+    rc = ensure_dynamic_lds(kernel, ST_LDS);
+    if (rc != SP_OK) return rc;
+    void* args[] = {(void*)&a};
+    const hipError_t err = hipLaunchKernel(kernel, dim3((unsigned)gx, (unsigned)members), dim3(64 * waves), args, lds_bytes, (hipStream_t)stream);
+    if (err != hipSuccess) return fail(SP_ERR_DEVICE, "sp_stack_forward_f32: launch failed: %s", hipGetErrorString(err));
+    return check_launch(__func__);
+}
+
+namespace {
+struct MlpStackKernelNames {
+    MlpStackKernelNames() { register_kernel("stack_forward_f32", (const void*)mlp_stack_kernel<4, 0>, ST_MAX_THREADS); }
+} mlp_stack_kernel_names;
+}  // namespace

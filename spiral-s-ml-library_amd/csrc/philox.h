@@ -55,6 +55,34 @@ __device__ __forceinline__ float philox_uniform(unsigned long long seed, unsigne
 // Which (subsequence, 4-word group) the reference's sampling op uses for row r: every thread of
 // the row draws once per element it holds and the draw attached to column 0 wins
 // (ml/primitives.spi:786-791), i.e. the first draw of the row's lane 0 in that row-iteration.
+// I: the type of the row arithmetic -- `unsigned` where the rows of a run are known to fit (a 64-bit division is some 150
+// instructions, a 32-bit one 20).  run_row_uniform: row r of one run whose generator is draw_offset draws in.
+template <typename I, typename A>
+__device__ __forceinline__ float run_row_uniform(const A& a, I r, unsigned long long draw_offset) {
+    const I t = a.cols / 4;               // threads per row in the reference
+    const I tpb = a.tpb;
+    const I per_iter = tpb / t;           // rows per block-iteration
+    unsigned long long sub, group;
+    if (a.philox_mode == SP_PHILOX_BLOCK) {
+        sub = (r % per_iter) * t;
+        group = r / per_iter;
+    } else if (a.philox_mode == SP_PHILOX_GRID) {
+        const I it = r / per_iter;
+        sub = (unsigned long long)(it % (I)a.blocks) * tpb + (r % per_iter) * t;
+        group = it / (I)a.blocks;
+    } else if (a.philox_mode == SP_PHILOX_GATHER) {  // row r belongs to thread r
+        const I lt = r % tpb;
+        sub = (unsigned long long)(r / tpb) * tpb + (lt % per_iter) * t;
+        group = lt / per_iter;
+    } else {  // SP_PHILOX_LAYER: block b = r / rows_per_block walks its own slice (ml/layers.spi:339-344)
+        const I b = r / (I)a.rows_per_block, rb = r % (I)a.rows_per_block;
+        sub = (unsigned long long)b * tpb + (rb % per_iter) * t;
+        group = rb / per_iter;
+    }
+    // the generator is `draw_offset` draws in; this row uses the first draw of its 4-draw group
+    return philox_uniform(a.seed, sub, group + draw_offset / 4, (int)(draw_offset % 4));
+}
+
 template <typename A>
 __device__ __forceinline__ float reference_row_uniform(const A& a, long r) {
     unsigned long long draw_offset = a.draw_offset;
@@ -62,27 +90,7 @@ __device__ __forceinline__ float reference_row_uniform(const A& a, long r) {
         draw_offset += (unsigned long long)(r / a.member_rows) * a.member_draws;
         r = r % a.member_rows;
     }
-    const long t = a.cols / 4;            // threads per row in the reference
-    const long per_iter = a.tpb / t;      // rows per block-iteration
-    unsigned long long sub, group;
-    if (a.philox_mode == SP_PHILOX_BLOCK) {
-        sub = (r % per_iter) * t;
-        group = r / per_iter;
-    } else if (a.philox_mode == SP_PHILOX_GRID) {
-        const long it = r / per_iter;
-        sub = (it % a.blocks) * a.tpb + (r % per_iter) * t;
-        group = it / a.blocks;
-    } else if (a.philox_mode == SP_PHILOX_GATHER) {  // row r belongs to thread r
-        const long lt = r % a.tpb;
-        sub = (r / a.tpb) * a.tpb + (lt % per_iter) * t;
-        group = lt / per_iter;
-    } else {  // SP_PHILOX_LAYER: block b = r / rows_per_block walks its own slice (ml/layers.spi:339-344)
-        const long b = r / a.rows_per_block, rb = r % a.rows_per_block;
-        sub = b * a.tpb + (rb % per_iter) * t;
-        group = rb / per_iter;
-    }
-    // the generator is `draw_offset` draws in; this row uses the first draw of its 4-draw group
-    return philox_uniform(a.seed, sub, group + draw_offset / 4, (int)(draw_offset % 4));
+    return run_row_uniform<long>(a, r, draw_offset);
 }
 
 #endif

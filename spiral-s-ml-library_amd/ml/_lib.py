@@ -17,6 +17,7 @@ MAP_COPY, MAP_RELU, MAP_TANH, MAP_SIGMOID = 0, 1, 2, 3
 REDUCE_SUM, REDUCE_PROD, REDUCE_MAX, REDUCE_MIN, REDUCE_AVERAGE = 0, 1, 2, 3, 4
 MAP_IN_IDENTITY, MAP_IN_SQUARE, MAP_IN_ABS = 0, 1, 2
 MAP_OUT_IDENTITY, MAP_OUT_SQRT = 0, 1
+STACK_LN_L2 = 0x100
 HEAD_NONE, HEAD_SOFTMAX, HEAD_REGRET_MATCHING, HEAD_SOFTMAX_RM = 0, 1, 2, 3
 
 ERROR_NAMES = {0: "SP_OK", -1: "SP_ERR_NULL", -2: "SP_ERR_SHAPE", -3: "SP_ERR_ALIGN", -4: "SP_ERR_DTYPE",
@@ -88,6 +89,8 @@ SIGNATURES = {
                                         C.POINTER(PhiloxConfig), _P, _P, _P, _I64, _I32, _I32, _P]),
     "sp_mlp_forward_ensemble": (C.c_int, [C.c_int, _P, _I32, C.POINTER(_P), C.POINTER(C.c_int32), _I32, _P,
                                           C.POINTER(PhiloxConfig), _P, _P, _I64, _I32, _I32, _P]),
+    "sp_stack_forward_f32": (C.c_int, [_P, _I32, C.POINTER(_P), C.POINTER(C.c_int32), C.POINTER(C.c_int32), _I32, _P,
+                                       C.POINTER(PhiloxConfig), _P, _P, _I64, _I32, _I32, _P]),
     "sp_ensemble_binarize": (C.c_int, [C.c_int, _P, _P, _P, _I32, _I64, _I32, _I32, _U32, _P]),
 }
 
@@ -109,7 +112,7 @@ LAUNCHES = frozenset(("sp_gemm_abt", "sp_gemm_abt_batched", "sp_row_ops", "sp_ro
                       "sp_row_sample", "sp_philox_uniforms", "sp_row_get_prob", "sp_cem_resample", "sp_cem_resample_philox",
                       "sp_row_reduce_f32", "sp_cem_update_mask",
                       "sp_row_binarize", "sp_map_f32", "sp_reduce_sum", "sp_reduce", "sp_row_l1_normalize", "sp_reduce_sum_static", "sp_transpose_inner_b32", "sp_mlp_forward", "sp_mlp_pack_weights",
-                      "sp_mlp_forward_packed", "sp_mlp_forward_ensemble", "sp_ensemble_binarize"))
+                      "sp_mlp_forward_packed", "sp_mlp_forward_ensemble", "sp_ensemble_binarize", "sp_stack_forward_f32"))
 
 
 class Tape:

@@ -933,6 +933,130 @@ def _run_fused_ensemble(model, key, count, ls):
     return True
 
 
+_STACK_HEADS = {"softmax": _lib.ROW_SOFTMAX, "masked_softmax": _lib.ROW_MASKED_SOFTMAX,
+                "regret_matching": _lib.ROW_REGRET_MATCHING, "masked_regret_matching": _lib.ROW_MASKED_REGRET_MATCHING}
+_STACK_MAPS = {"copy": _lib.MAP_COPY, "relu": _lib.MAP_RELU, "tanh": _lib.MAP_TANH, "sigmoid": _lib.MAP_SIGMOID}
+_STACK_LDS = 144 * 1024          # bytes of weights sp_stack_forward_f32 keeps on chip
+
+
+def _stack_plan(model, key):
+    """`input -> matmul [-> ln_l2] [-> map] -> ... -> matmul -> row head`, the graphs of ml/layers.spi test3 - test5
+    (:564-665), with every weight and output of one member (key None) or stacked under `apply key`:
+    (x node, [weight nodes], [activation codes], head name, mask size, output node or None) or None.  A node in the middle
+    that has a name (`key_graph`) or an output tensor of its own is one the caller can look at: such a graph is not taken."""
+    top = model.graph
+    sampling = isinstance(top, BlockRowMapReduce)
+    if not isinstance(top, (BlockRowMap, BlockRowMapReduce)):
+        return None
+    head = top.f[:-len("_and_discrete_sample")] if sampling else top.f
+    if head not in _STACK_HEADS or head.startswith("masked") != (top.size > 0):
+        return None
+
+    def tensor_node(k):
+        while isinstance(k, (KeyGraph, Fst)):
+            if isinstance(k, Fst):
+                k = k.x
+                while isinstance(k, KeyGraph):
+                    k = k.x
+                if not isinstance(k, Pair):
+                    return None
+                k = k.a
+            else:
+                k = k.x
+        return k if isinstance(k, Layer) else None
+
+    def member(k):
+        while isinstance(k, KeyGraph):
+            k = k.x
+        if key is None:
+            return tensor_node(k)
+        return tensor_node(k.a) if isinstance(k, Apply) and isinstance(k.b, KeyScalar) and k.b.key == key else None
+
+    weights, acts, node = [], [], top.a
+    while isinstance(node, BlockMatmul):
+        w = member(node.b)
+        if w is None:
+            return None
+        weights.insert(0, w)
+        node, act = node.a, 0
+        if isinstance(node, BlockMap) and node.out is None and node.f in _STACK_MAPS:
+            node, act = node.a, _STACK_MAPS[node.f]
+        if isinstance(node, BlockRowMap) and node.out is None and node.f == "ln_l2":
+            node, act = node.a, act | _lib.STACK_LN_L2
+        if not isinstance(node, BlockMatmul):
+            if act:
+                return None
+            break
+        acts.insert(0, act)
+    x = tensor_node(node)
+    if not weights or x is None:
+        return None
+    out = top.out
+    while isinstance(out, KeyGraph):
+        out = out.x
+    if out is None:
+        outs = None if key is None else ()
+    elif sampling:
+        outs = (member(out.a), member(out.b)) if isinstance(out, Pair) else ()
+    else:
+        outs = (member(out),)
+    if outs is not None and (not outs or any(o is None for o in outs)):
+        return None
+    return x, weights, acts + [0], head, top.size, outs
+
+
+def _overlap(a, b):
+    end = lambda t: t.data_ptr() + t.numel() * t.element_size()
+    return a.data_ptr() < end(b) and b.data_ptr() < end(a)
+
+
+def _run_fused_stack(model, key, count, ls):
+    """One sp_stack_forward_f32 launch in place of a walk over the nodes, where the graph is of that shape, its widths are
+    ones the kernel takes and its weights fit on chip.  (The inner nodes' tensors are not written then.)"""
+    plan = _stack_plan(model, key)
+    if plan is None:
+        return False
+    x_node, w_nodes, acts, head, mask, out_nodes = plan
+    if len(w_nodes) > 8:
+        return False
+    tensor = lambda node: graph_extract(Model(node, model.dims, model.data))
+    x, ws = tensor(x_node), [tensor(w) for w in w_nodes]
+    outs = graph_extract(model) if out_nodes is None else tuple(tensor(o) for o in out_nodes)
+    outs = outs if isinstance(outs, tuple) else (outs,)
+    lead = () if key is None else (count,)
+    if x.dim() != 3 or any(t.dtype != torch.float32 for t in [x, outs[0]] + ws):
+        return False
+    if any(w.dim() != 2 + len(lead) or w.shape[:-2] != lead for w in ws):
+        return False
+    q, w, k0 = x.shape
+    dims = [k0] + [t.shape[-2] for t in ws]
+    cols, computed = dims[-1], mask or dims[-1]
+    if any(t.shape[-1] != d for t, d in zip(ws, dims)):
+        return False
+    if dims[0] % 4 or dims[0] > 128 or any(d % 16 or d > 128 for d in dims[1:-1]) or cols % 4 or cols > 64 or mask > cols:
+        return False
+    blocks = [(d + 15) // 16 for d in dims[:-1]] + [(computed + 15) // 16]
+    if 1024 * builtins.sum(i * o for i, o in zip(blocks[:-1], blocks[1:])) > _STACK_LDS or count * q * w >= (1 << 31) - (1 << 21):
+        return False
+    if outs[0].shape != lead + (q, w, cols) or (len(outs) == 2 and (outs[1].shape != lead + (q, w) or outs[1].dtype != torch.int32)):
+        return False
+    if any(_overlap(o, t) for o in outs for t in [x] + ws) or (len(outs) == 2 and _overlap(*outs)):
+        return False          # node by node, an output may take the place of what has been read
+    rng = None
+    if len(outs) == 2:
+        draws = _sampling_draws(w, cols)
+        rng = _prim.philox(_lib.PHILOX_LAYER, seed=ls.seed, threads_per_block=THREADS_PER_BLOCK, blocks_per_grid=q,
+                           rows_per_block=w, offset=ls.draws, member_rows=q * w if key is not None else 0, member_draws=draws)
+        ls.draws += draws
+    n = len(ws)
+    check(lib.sp_stack_forward_f32(
+        ptr(x, name="x"), n, (C.c_void_p * n)(*[ptr(t, name="weights[%d]" % i) for i, t in enumerate(ws)]),
+        (C.c_int32 * (n + 1))(*dims), (C.c_int32 * n)(*acts), count, None, C.byref(rng) if rng is not None else None,
+        ptr(outs[0], name="policy"), ptr(outs[1], name="action") if len(outs) == 2 else None, q * w, _STACK_HEADS[head], mask,
+        stream_ptr()))
+    return True
+
+
 def _graph_run_batched(model, key, count, ls):
     """`loop.linear {key=count} fun indices => graph_run_device m ls indices` (ml/layers.spi:343-344) as ONE
     pass: `apply key t` yields the whole tensor, every node downstream works on `count` stacked members
@@ -1062,7 +1186,8 @@ def graph_run_host(model, sizes=None, seed=_prim.CONSTANT_SEED, fuse=True, batch
     """Runs the graph for every combination of the key indices in `sizes`, e.g. {"ensemble": 16}
     (ml/layers.spi:336-344).  Uniforms come from the reference's per-thread Philox streams.  A loop over
     one key that only indexes leading dimensions runs as a single batched pass with the same results
-    (`batched=False` keeps the member-by-member loop).  `static_weights=True` says that the weights have not
+    (`batched=False` keeps the member-by-member loop).  A dense stack under a row head runs as one launch, whose f32 sums
+    add up in another order and which does not write the unnamed nodes in the middle; `fuse=False` runs node by node.  `static_weights=True` says that the weights have not
     changed since the previous such run (or since `weights_changed(model)`): a fused relu-MLP then keeps a copy
     of them packed for the faster kernel instead of reading the arena on every run."""
     if fuse and not sizes:
@@ -1116,8 +1241,10 @@ def _graph_run_walk(model, sizes, seed, batched, fuse=True):
     ls = create_layer_state(seed)
     key = _batchable_key(model, sizes) if batched and sizes else None
     if key is not None and sizes[key] > 1:
-        if not (fuse and _run_fused_ensemble(model, key, sizes[key], ls)):
+        if not (fuse and (_run_fused_ensemble(model, key, sizes[key], ls) or _run_fused_stack(model, key, sizes[key], ls))):
             _graph_run_batched(model, key, sizes[key], ls)
+        return
+    if fuse and not sizes and _run_fused_stack(model, None, 1, ls):
         return
     keys = list(sizes)
     for combo in itertools.product(*[range(sizes[k]) for k in keys]):

@@ -308,6 +308,54 @@ def test_replayed_runs_see_new_inputs_and_weights(L, kind):
         previous = got[0]
 
 
+@pytest.mark.parametrize("rows,widths,act,ensemble,head", [
+    (64, (64, 64, 64, 64), "ln_l2_relu", 1, "softmax"),      # test3 of ml/layers.spi
+    (1, (4, 16, 4), "tanh", 1, "softmax"),                   # the narrowest: one row a block, padded K, a quarter of a tile out
+    (17, (100, 128, 96, 64), "ln_l2_relu", 5, "masked"),   # 110 KiB of weights, the mask leaves one tile of outputs
+    (7, (36, 48, 64), "sigmoid", 3, "softmax"),              # a last tile of 8 rows, an odd number of tiles per member
+    (130, (128, 16), "relu", 2, "regret"),                   # one layer
+    (33, (64, 128, 16), "relu", 1, "masked_regret")])
+def test_dense_stack_runs_as_one_launch(L, rows, widths, act, ensemble, head):
+    """A stack of dense layers under a row head (sp_stack_forward_f32) against the node-by-node run: sums in another order
+    (f32 bar: 1e-5), the draws bit-exact given the probabilities and the stream."""
+    announce("layers dense stack %s x%d %s %s" % (widths, ensemble, act, head))
+    x = L.input("input", (Q, rows, widths[0]))
+    for i, (a, b) in enumerate(zip(widths[:-1], widths[1:])):
+        x = L.matmul((a, b), x) if ensemble == 1 else L.matmul_ensemble((ensemble, a, b), x)
+        if i + 2 < len(widths):
+            x = L.relu(L.ln_l2(x)) if act == "ln_l2_relu" else getattr(L, act)(x)
+    wrap = (lambda t: t) if ensemble == 1 else lambda t: L.apply("ensemble", t)
+    lead, n = ((ensemble,) if ensemble > 1 else ()), widths[-1]
+    out = L.pair(wrap(L.input("probs", lead + (Q, rows, n))), wrap(L.input("picks", lead + (Q, rows), "int")))
+    if ensemble == 1 and head in ("softmax", "masked_regret"):
+        g = L.softmax_and_discrete_sample(x) if head == "softmax" else L.BlockRowMapReduce(
+            "masked_regret_matching_and_discrete_sample", x, None, 3)
+    else:
+        g = {"softmax": lambda: L.softmax_and_discrete_sample_(out, x),
+             "masked": lambda: L.masked_softmax_and_discrete_sample_(3, out, x),
+             "regret": lambda: L.BlockRowMapReduce("regret_matching_and_discrete_sample", x, out)}[head]()
+    m = L.create_model(g)
+    sizes = {"ensemble": ensemble} if ensemble > 1 else {}
+    rng = np.random.default_rng(rows)
+    for t in [L.key_extract(m, "input")] + [t for _, t, _ in L.extract_layers_(m, L.weight_id())]:
+        fill(t, rng, 1.0 if t.shape[-2:] == (rows, widths[0]) else 0.2)
+    outs = lambda: tuple(host(t) for t in (L.graph_extract(m) if g.out is None else (L.key_extract(m, "probs"), L.key_extract(m, "picks"))))
+    L.graph_run_host(m, sizes, fuse=False)
+    want = outs()[0].copy()
+    for _ in range(2):                       # the second run replays the recorded launch
+        (L.graph_extract(m)[0] if g.out is None else L.key_extract(m, "probs")).fill_(7)
+        L.graph_run_host(m, sizes)
+        probs, picks = outs()
+        assert ogemm.rel_frobenius(probs.reshape(-1, n), want.reshape(-1, n)) < 1e-5
+        per_node = ophilox.draws_per_sampling_node(rows, n)
+        for e in range(ensemble):
+            u = ophilox.row_uniforms_layer(Q, rows, n, offset=e * per_node)
+            pe, ie = (probs[e], picks[e]) if ensemble > 1 else (probs, picks)
+            assert (ie.reshape(-1) == orow.discrete_sampling(pe.reshape(-1, n), u, order="wave")).all()
+    tape = m._tapes[(L._prim.CONSTANT_SEED, True, True, tuple(sizes.items()))][1]
+    assert [c[0].__name__ for c in tape.calls] == ["sp_stack_forward_f32"]
+
+
 @pytest.mark.parametrize("sampling", [False, True])
 def test_leduc_policy_graph_runs_as_one_launch(L, sampling):
     """The graph of the reference's Leduc policy (game/leduc/model_cem.spi:55-63: input -> matmul_ensemble_with_adjoint
