@@ -7,16 +7,19 @@
 // ends up with features 16 t + 4 q + i of row r in register i of tile t.  Which K-index an MFMA step takes from lane group q
 // is free as long as both operands agree: step i of K-block j stands for k = 16 j + 4 q + i, so a layer's result registers
 // ARE the next layer's second operand.  The norm of a row is 4 registers x tiles and two cross-lane adds.
-//   The weights of all layers sit in LDS in the order they are consumed (one 1 KiB block per 16 x 16 of W, lane l's 16 bytes
-// at 16 l: conflict-free reads, and the DMA's natural layout), so the walk over a stack is one pointer that advances by
-// 1 KiB per four MFMAs, one block ahead of them.  Features and K past a layer's widths are zeros.
+//   The weights of all layers sit in LDS in the order they are consumed (one 1 KiB block per 16 x 16 of W,
+// lane l's 16 bytes at 16 l: conflict-free reads, and the DMA's natural layout), so the walk over a stack is one
+// pointer that advances by 1 KiB per four MFMAs.  Features and K past a layer's widths are zeros.
 //   The logits cross LDS once more, from the feature-major registers into one row per 16 lanes: the head and the sampling
 // are the row primitives' own operations in their order, and the stores are whole rows.
 //
-// What bounds it: the f32 matrix pipe (157 TFLOP/s), 32 cycles per MFMA and SIMD; a 64-64-64-64 stack is 6144 of them for
-// 16 rows.  16-row tiles because a batch of 16384 rows is then one tile per SIMD.
-// Measured (node by node / this kernel, us): 64-64-64-64 with ln_l2 and relu, softmax and sampling over 16384 rows 32.8 / 13.8,
-// 16 members of it 206 / 87 (41 on the matrix pipe alone).
+// What bounds it: the f32 matrix pipe, 32 cycles per MFMA and SIMD (a 64-64-64-64 stack is 6144 of them for 16 rows), and the
+// vector ALU, whose instructions do not hide behind f32 MFMAs whichever wave they come from (800 instructions, 3200 cycles, per
+// 16 rows of that stack with ln_l2, relu, softmax and sampling).  Hence the products in a straight line where a layer is full,
+// the uniforms of four tiles in one go, one reciprocal per norm.  16-row tiles because a batch of 16384 rows is then one
+// tile per SIMD.
+// Measured, that stack over 16384 rows (node by node / every layer through part_product, a draw per tile / this kernel, us):
+// one model 32.8 / 13.8 / 10.3, 16 members 206 / 87 / 68.8 (the matrix pipe alone: 41).
 #include "mlp_common.h"
 #include "row_common.h"
 #include "gemm_dma.h"
@@ -49,18 +52,68 @@ struct StackArgs {
     PhiloxStream ph;
 };
 
-template <typename F>
-__device__ __forceinline__ void map_tiles(f32x4* y, int nt, int count, F f) {
+template <int HT, typename F>
+__device__ __forceinline__ void map_tiles(f32x4 (&y)[HT], int nt, F f) {
 #pragma unroll
-    for (int t = 0; t < count; ++t)
+    for (int t = 0; t < HT; ++t) {
         if (t < nt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) y[t][i] = f(y[t][i]);
+        __builtin_amdgcn_sched_barrier(0);      // (a tile at a time: registers)
+    }
 }
 
-// HT: 16-wide tiles of the widest layer (4 or 8).  OPK: 0 softmax, 1 masked softmax, 2 regret matching (mask_size columns).
-template <int HT, int OPK>
-__global__ __launch_bounds__(ST_MAX_THREADS) void mlp_stack_kernel(const StackArgs a) {
+// y (NT tiles of features) = W . x for the weights at wp, K-blocks outermost; advances wp behind them.
+// A full layer is a straight line, the weights of one K-block read ahead of the products of the one before.
+template <int KT, int NT>
+__device__ __forceinline__ void full_product(const unsigned char*& wp, const f32x4 (&x)[KT], f32x4 (&y)[NT]) {
+    f32x4 w[2][NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        y[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        w[0][t] = *reinterpret_cast<const f32x4*>(wp + t * ST_BLOCK);
+    }
+#pragma unroll
+    for (int j = 0; j < KT; ++j) {
+        __builtin_amdgcn_sched_barrier(0);      // (else every load of the layer moves up here: registers)
+        if (j + 1 < KT) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) w[(j + 1) & 1][t] = *reinterpret_cast<const f32x4*>(wp + ((j + 1) * NT + t) * ST_BLOCK);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) y[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j & 1][t][i], x[j][i], y[t], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    wp += KT * NT * ST_BLOCK;
+}
+
+// The same for kt <= KT blocks of K and nt <= NT tiles of features, feature tiles outermost, the weights one block ahead
+// (behind the last block of the stack lies the scratch: read, not used).
+template <int KT, int NT>
+__device__ __forceinline__ void part_product(const unsigned char*& wp, const f32x4 (&x)[KT], f32x4 (&y)[NT], int kt, int nt) {
+    f32x4 w = *reinterpret_cast<const f32x4*>(wp);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        y[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (t < nt) {
+#pragma unroll
+            for (int j = 0; j < KT; ++j)
+                if (j < kt) {
+                    wp += ST_BLOCK;
+                    const f32x4 next = *reinterpret_cast<const f32x4*>(wp);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) y[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[j][i], y[t], 0, 0, 0);
+                    w = next;
+                }
+        }
+    }
+}
+
+// HT: 16-wide tiles of the widest layer (4 or 8).  FULL: the input and every hidden layer have exactly that many.  OPK: 0 softmax, 1 masked softmax, 2 regret matching (mask_size columns).
+template <int HT, int OPK, bool FULL>
+__global__ __launch_bounds__(ST_MAX_THREADS, HT == 4 ? 4 : 2) void mlp_stack_kernel(const StackArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -83,7 +136,7 @@ __global__ __launch_bounds__(ST_MAX_THREADS) void mlp_stack_kernel(const StackAr
     };
     int tile = blockIdx.x * waves + wave;
     f32x4 x[HT];
-    if (tile < a.tiles) load_x(tile, x);
+    load_x(tile < a.tiles ? tile : 0, x);
 
     // ---- the member's weights, once per workgroup ----
     const unsigned lds0 = (unsigned)(size_t)lds;
@@ -92,8 +145,11 @@ __global__ __launch_bounds__(ST_MAX_THREADS) void mlp_stack_kernel(const StackAr
         for (int l = 0; l < layers; ++l) {
             const int K = a.dims[l], F = a.dims[l + 1], kt = (K + 15) >> 4, nt = (F + 15) >> 4;
             const float* W = a.w[l] + (long)e * (l + 1 < layers ? (long)F * K : a.out_stride);
+            const bool k_outer = FULL && (l + 1 < layers || nt == ST_MAX_OUT / 16);      // as full_product reads them
+            const int inner = k_outer ? nt : kt;
             for (int b = wave; b < kt * nt; b += waves) {
-                const int t = b / kt, row = 16 * t + r, col = 16 * (b - t * kt) + 4 * q;
+                const int hi = b / inner, lo = b - hi * inner;
+                const int row = 16 * (k_outer ? lo : hi) + r, col = 16 * (k_outer ? hi : lo) + 4 * q;
                 const unsigned char* at = (const unsigned char*)(W + (long)row * K + col);
                 dma_to_lds_addr(row < F && col < K ? at : (const unsigned char*)kZeroChunk, __builtin_amdgcn_readfirstlane(dst + b * ST_BLOCK));
             }
@@ -102,73 +158,73 @@ __global__ __launch_bounds__(ST_MAX_THREADS) void mlp_stack_kernel(const StackAr
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     }
+#pragma unroll
+    for (int j = 0; j < HT; ++j) asm volatile("" : "+v"(x[j]));       // (the compiler's own wait for the first inputs: here, not in the loop)
     unsigned char* const scratch = lds + a.w_bytes + wave * ST_SCRATCH;
     const int stride = gridDim.x * waves;
 
-    for (; tile < a.tiles; tile += stride) {
-        const int my_row = tile * ST_ROWS + r;
-        float u = 1.f;
-        if (a.action != nullptr) {
-            const int row = my_row < a.batch ? my_row : a.batch - 1;
-            if (a.ph.philox_mode < 0) u = a.u[(long)e * a.batch + row];
-            else if (a.ph.member_rows > 0) u = run_row_uniform<unsigned>(a.ph, row, a.ph.draw_offset + (unsigned long long)e * a.ph.member_draws);
-            else u = run_row_uniform<unsigned>(a.ph, (unsigned)e * a.batch + row, a.ph.draw_offset);
+    float* const policy = a.policy + (long)e * a.batch * a.n;
+    int* const action = a.action + (long)e * a.batch;       // (only used where a.action is not null)
+    float u4 = 1.f;
+    for (int turn = 0; tile < a.tiles; tile += stride, ++turn) {
+        // The uniforms of four tiles at once, lane group q those of tile q from here: a draw is 250 vector instructions.
+        if (a.action != nullptr && (turn & 3) == 0) {
+            const long at = (long)(tile + (long)q * stride) * ST_ROWS + r;
+            const int row = at < a.batch ? (int)at : a.batch - 1;
+            if (a.ph.philox_mode < 0) u4 = a.u[(long)e * a.batch + row];
+            else if (a.ph.member_rows > 0) u4 = run_row_uniform<unsigned>(a.ph, row, a.ph.draw_offset + (unsigned long long)e * a.ph.member_draws);
+            else u4 = run_row_uniform<unsigned>(a.ph, (unsigned)e * a.batch + row, a.ph.draw_offset);
         }
 
         const unsigned char* wp = lds + lane * 16;
-        f32x4 w = *reinterpret_cast<const f32x4*>(wp);
         f32x4 xn[HT];
         load_x(tile + stride < a.tiles ? tile + stride : tile, xn);
-        int nt = 0;
-        for (int l = 0; l < layers; ++l) {
-            const int kt = (a.dims[l] + 15) >> 4;
-            nt = (a.dims[l + 1] + 15) >> 4;
+        for (int l = 0; l + 1 < layers; ++l) {
+            const int nt = a.dims[l + 1] >> 4;
             f32x4 y[HT];
+            if constexpr (FULL) full_product<HT, HT>(wp, x, y);
+            else part_product<HT, HT>(wp, x, y, (a.dims[l] + 15) >> 4, nt);
+            const int act = a.acts[l];
+            if (act & SP_STACK_LN_L2) {       // local_ln_l2 (ml/primitives.spi:701-703)
+                float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-            for (int t = 0; t < HT; ++t) {
-                y[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                if (t < nt) {
-#pragma unroll
-                    for (int j = 0; j < HT; ++j)
-                        if (j < kt) {
-                            // (behind the last block of the stack lies the scratch: read, not used)
-                            wp += ST_BLOCK;
-                            const f32x4 next = *reinterpret_cast<const f32x4*>(wp);
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) y[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[j][i], y[t], 0, 0, 0);
-                            w = next;
-                        }
+                for (int t = 0; t < HT; ++t) {
+                    s0 = __builtin_fmaf(y[t][0], y[t][0], s0);
+                    s1 = __builtin_fmaf(y[t][1], y[t][1], s1);
+                    s0 = __builtin_fmaf(y[t][2], y[t][2], s0);
+                    s1 = __builtin_fmaf(y[t][3], y[t][3], s1);
                 }
+                float s = s0 + s1;
+                s += __shfl_xor(s, 16);
+                s += __shfl_xor(s, 32);
+                const RowDivisor over_s(s);
+                // (no row of the wave is zero or needs the scale, as nearly always: the same quotients by one multiplication)
+                if (__all(s != 0.f && over_s.scale == 1.f)) map_tiles<HT>(y, FULL ? HT : nt, [&](float v) { return v * over_s.inv; });
+                else map_tiles<HT>(y, FULL ? HT : nt, [&](float v) { return s != 0.f ? over_s(v) : 0.f; });
             }
-            if (l + 1 < layers) {
-                const int act = a.acts[l];
-                if (act & SP_STACK_LN_L2) {       // local_ln_l2 (ml/primitives.spi:701-703)
-                    float s = 0.f;
-#pragma unroll
-                    for (int t = 0; t < HT; ++t) {
-                        float sq[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) sq[i] = y[t][i] * y[t][i];
-                        s = t == 0 ? sum4(sq) : s + sum4(sq);
-                    }
-                    s += __shfl_xor(s, 16);
-                    s += __shfl_xor(s, 32);
-                    const RowDivisor over_s(s);
-                    map_tiles(y, nt, HT, [&](float v) { return s != 0.f ? over_s(v) : 0.f; });
-                }
-                const int map = act & ~SP_STACK_LN_L2;
-                if (map == SP_MAP_RELU) map_tiles(y, nt, HT, [](float v) { return fmaxf(v, 0.f); });
-                else if (map == SP_MAP_TANH) map_tiles(y, nt, HT, [](float v) { return tanhf(v); });
-                else if (map == SP_MAP_SIGMOID) map_tiles(y, nt, HT, [](float v) { return 1.f / (1.f + expf(-v)); });
-            }
+            const int map = act & ~SP_STACK_LN_L2;
+            if (map == SP_MAP_RELU) map_tiles<HT>(y, FULL ? HT : nt, [](float v) { return fmaxf(v, 0.f); });
+            else if (map == SP_MAP_TANH) map_tiles<HT>(y, FULL ? HT : nt, [](float v) { return tanhf(v); });
+            else if (map == SP_MAP_SIGMOID) map_tiles<HT>(y, FULL ? HT : nt, [](float v) { return 1.f / (1.f + expf(-v)); });
 #pragma unroll
             for (int t = 0; t < HT; ++t) x[t] = y[t];
         }
+        f32x4 logits[ST_MAX_OUT / 16];
+        const int nt = (a.dims[layers] + 15) >> 4;
+        if (FULL && nt == ST_MAX_OUT / 16) full_product<HT, ST_MAX_OUT / 16>(wp, x, logits);
+        else part_product<HT, ST_MAX_OUT / 16>(wp, x, logits, (a.dims[layers - 1] + 15) >> 4, nt);
 
         // ---- logits into rows: quad c of row r at slot c ^ r of its 256 bytes ----
 #pragma unroll
         for (int t = 0; t < 4; ++t)
-            if (t < nt) *reinterpret_cast<f32x4*>(scratch + r * 256 + (((4 * t + q) ^ r) & 15) * 16) = x[t];
+            if (t < nt) *reinterpret_cast<f32x4*>(scratch + r * 256 + (((4 * t + q) ^ r) & 15) * 16) = logits[t];
+        // the next tile's inputs are waited for here, in front of the stores: the counter of outstanding accesses runs in
+        // order, and behind them that wait would be one for the stores
+#pragma unroll
+        for (int j = 0; j < HT; ++j) {
+            x[j] = xn[j];
+            asm volatile("" : "+v"(x[j]));
+        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -176,15 +232,18 @@ __global__ __launch_bounds__(ST_MAX_THREADS) void mlp_stack_kernel(const StackAr
         // ---- the head and the sampling: lane l of 16 holds columns 4 l .. of its row, as in the row primitives ----
         const int lq = r;                         // (lane % 16 again: here the column quad)
         const int limit = a.mask_size;
+        const int rows_here = a.batch - tile * ST_ROWS;
+        float* const tile_policy = policy + (long)tile * (ST_ROWS * a.n);
 #pragma unroll
         for (int pass = 0; pass < 4; ++pass) {
             const int rr = 4 * pass + q;
-            const int row = tile * ST_ROWS + rr;
             f32x4 v = *reinterpret_cast<const f32x4*>(scratch + rr * 256 + ((lq ^ rr) & 15) * 16);
             // columns past the head's width, or its mask, enter as -inf (an exact 0 after the exponential) or 0
+            if (limit < ST_MAX_OUT) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (4 * lq + k >= limit) v[k] = NEG_INF;
+                for (int k = 0; k < 4; ++k)
+                    if (4 * lq + k >= limit) v[k] = NEG_INF;
+            }
             float p[4];
             if constexpr (OPK == 2) {
 #pragma unroll
@@ -203,10 +262,9 @@ __global__ __launch_bounds__(ST_MAX_THREADS) void mlp_stack_kernel(const StackAr
 #pragma unroll
                 for (int k = 0; k < 4; ++k) p[k] = p[k] * inv;
             }
-            const bool row_ok = row < a.batch;
-            const long out_row = (long)e * a.batch + row;
+            const bool row_ok = rr < rows_here;
             if (row_ok && 4 * lq < a.n)
-                store16_through(reinterpret_cast<f32x4*>(a.policy + out_row * a.n + 4 * lq), f32x4{p[0], p[1], p[2], p[3]});
+                store16_through(reinterpret_cast<f32x4*>(tile_policy + rr * a.n + 4 * lq), f32x4{p[0], p[1], p[2], p[3]});
             if (a.action != nullptr) {            // local_discrete_sampling (ml/primitives.spi:782-798)
                 const float incl = group_inclusive_scan<16>(sum4(p), lq);
                 float run = dpp_move<0x138>(incl);
@@ -218,18 +276,16 @@ __global__ __launch_bounds__(ST_MAX_THREADS) void mlp_stack_kernel(const StackAr
                     c[k] = run;
                 }
                 const float m = group_max<16>(sum4(p) > 0.f ? c[3] : NEG_INF);
-                const float thr = __shfl(u, rr) * m;
+                const float thr = __shfl(u4, rr + 16 * (turn & 3)) * m;
                 int pick = 2147483647;
 #pragma unroll
                 for (int k = 3; k >= 0; --k)
                     if (p[k] > 0.f && c[k] >= thr) pick = 4 * lq + k;
                 pick = group_reduce<16>(pick, [](int m, int n) { return m < n ? m : n; });
-                if (row_ok && lq == 0) a.action[out_row] = pick;
+                if (row_ok && lq == 0) action[tile * ST_ROWS + rr] = pick;
             }
         }
         __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int j = 0; j < HT; ++j) x[j] = xn[j];
     }
 }
 
@@ -237,9 +293,10 @@ __global__ __launch_bounds__(ST_MAX_THREADS) void mlp_stack_kernel(const StackAr
 
 using namespace sp;
 
-template <int HT>
+template <int HT, bool FULL>
 static const void* pick_stack_kernel(int opk) {
-    return opk == 0 ? (const void*)mlp_stack_kernel<HT, 0> : opk == 1 ? (const void*)mlp_stack_kernel<HT, 1> : (const void*)mlp_stack_kernel<HT, 2>;
+    return opk == 0 ? (const void*)mlp_stack_kernel<HT, 0, FULL> : opk == 1 ? (const void*)mlp_stack_kernel<HT, 1, FULL>
+                                                                            : (const void*)mlp_stack_kernel<HT, 2, FULL>;
 }
 
 // Bytes of LDS the weights take (dims[n_layers] = the computed outputs).
@@ -317,7 +374,11 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
     if (gx > most) gx = most;
     const long each = (a.tiles + gx * waves - 1) / (gx * waves);      // tiles per wave: no more workgroups than give that
     gx = (a.tiles + each * waves - 1) / (each * waves);
-    const void* kernel = widest <= 64 ? pick_stack_kernel<4>(opk) : pick_stack_kernel<8>(opk);
+    const int ht = widest <= 64 ? 4 : 8;
+    bool full = true;
+    for (int l = 0; l < n_layers; ++l) full = full && (dims[l] + 15) / 16 == ht;
+    const void* kernel = ht == 4 ? (full ? pick_stack_kernel<4, true>(opk) : pick_stack_kernel<4, false>(opk))
+                                 : (full ? pick_stack_kernel<8, true>(opk) : pick_stack_kernel<8, false>(opk));
     rc = ensure_dynamic_lds(kernel, ST_LDS);
     if (rc != SP_OK) return rc;
     void* args[] = {(void*)&a};
@@ -328,6 +389,6 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
 
 namespace {
 struct MlpStackKernelNames {
-    MlpStackKernelNames() { register_kernel("stack_forward_f32", (const void*)mlp_stack_kernel<4, 0>, ST_MAX_THREADS); }
+    MlpStackKernelNames() { register_kernel("stack_forward_f32", (const void*)mlp_stack_kernel<4, 0, true>, ST_MAX_THREADS); }
 } mlp_stack_kernel_names;
 }  // namespace
