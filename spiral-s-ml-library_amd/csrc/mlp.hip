@@ -227,13 +227,36 @@ __global__ __launch_bounds__(NW * 64) void mlp_forward_kernel(const MlpArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // drain the dummy DMAs before the LDS is released
 
     // ---- head: lanes 0..15 of every wave own one batch row each (the staging is wave private) ----
+    const int N = a.dims[a.n_layers];
+    const int limit = a.mask_size > 0 ? a.mask_size : N;
+    float past = 0.f;
     if (lane < 16 && row_ok) {
-        const int N = a.dims[a.n_layers];
-        const int limit = a.mask_size > 0 ? a.mask_size : N;
         float* p = head_rows + lane * MLP_MAX_OUT;   // this row's outputs
         const float u = a.ph.philox_mode >= 0 ? reference_row_uniform(a.ph, row) : a.action != nullptr ? a.u[row] : 1.f;
-        if (N <= 8) head_row<8>(head_out(a), p, row, N, limit, u);      // narrow heads run in registers
+        if (N <= 8) head_row<8>(head_out(a), p, row, N, limit, u, N, &past);      // narrow heads run in registers
         else head_row<MLP_MAX_OUT>(head_out(a), p, row, N, limit, u);
+    }
+    if (a.out_stride > N) {
+        // a masked head computed for its valid columns only (N < 8): the wave fills the rest of its 16 policy rows, 16 bytes
+        // per lane where rows are whole pieces, the columns in front of the first whole piece by the row's own lane
+        const int stride = a.out_stride, s4 = stride >> 2, c0 = stride % 4 == 0 ? (N + 3) >> 2 : s4 + 1;
+        if (lane < 16 && row_ok)
+            for (int c = N; c < stride && c < 4 * c0; ++c) a.policy[row * stride + c] = past;
+        if (c0 < s4) {
+            const long first = (long)blockIdx.x * MLP_ROWS + wave * 16;
+            int r = lane / s4, c = lane - r * s4;
+            const int dr = 64 / s4, dc = 64 - dr * s4;
+            for (int idx = lane; idx < 16 * s4; idx += 64) {      // (16 s4 is a multiple of 16: the lanes of the rows stay in)
+                const float v = __shfl(past, r);
+                if (c >= c0 && first + r < a.batch) *reinterpret_cast<float4*>(a.policy + (first + r) * stride + 4 * c) = make_float4(v, v, v, v);
+                r += dr;
+                c += dc;
+                if (c >= s4) {
+                    c -= s4;
+                    ++r;
+                }
+            }
+        }
     }
 }
 
@@ -1035,6 +1058,11 @@ extern "C" int sp_mlp_forward(int dtype, const void* x, int32_t n_layers, const 
     if (h256 && head != SP_HEAD_NONE && logits_out == nullptr && mask_size > 0 && mask_size <= 16 &&
         mask_size < dims[n_layers])
         a.nout = mask_size;
+    // The same in the kernel of the other hidden widths, whose head walks its outputs column by column in one lane (bf16
+    // 128-64-64 masked to 3, regret matching and a sample, 64 rows: 14.4 us with all 64 columns, 9.3 so).  Seven at most, so that the
+    // head has a column past the mask of its own: what the rest of the row is filled with.
+    if (!h256 && head != SP_HEAD_NONE && logits_out == nullptr && mask_size > 0 && mask_size <= 7 && mask_size < dims[n_layers])
+        a.dims[n_layers] = mask_size;
     if (h256 && mlp_resident_takes(n_layers, dims, a.nout) &&
         (batch + 63) / 64 >= (long)(mlp_pipe_takes(n_layers, dims, a.nout) ? SP_MLP_PIPE_MIN_TILES_ROWMAJOR
                                                                            : SP_MLP_RESIDENT_MIN_TILES_ROWMAJOR) * cus) {

@@ -160,6 +160,27 @@ def test_masked_head_without_logits(LY, dtype, batch, dims, head, mask):
     assert (action == orow.discrete_sampling(policy, u)).all() and (action < mask).all() and (action >= 0).all()
 
 
+@pytest.mark.parametrize("dims,head,mask,batch,dtype", [([128, 64, 64], "regret_matching", 3, 64, "bf16"),
+                                                        ([48, 96, 128, 10], "softmax", 4, 37, "f16"),      # rows of no whole pieces
+                                                        ([16, 32, 12], "softmax_regret_matching", 7, 130, "bf16"),
+                                                        ([32, 64, 160, 64], "softmax", 1, 20000, "f16")])  # 128 rows a workgroup
+def test_masked_head_of_other_stacks_without_logits(LY, dims, head, mask, batch, dtype):
+    """The same for hidden widths other than 256: bit for bit what the run that writes the logits (and computes every
+    column) gives, a row of NaNs among them."""
+    announce("mlp masked head, no logits: %s %s batch=%d mask=%d %s" % (dims, head, batch, mask, dtype))
+    rng = np.random.default_rng(batch + mask)
+    t = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    x = rng.standard_normal((batch, dims[0])).astype(np.float32)
+    x[batch // 2] = np.nan
+    xd = dev(x, t)
+    wd = [dev((rng.standard_normal((o, i)) / np.sqrt(i)).astype(np.float32), t) for i, o in zip(dims[:-1], dims[1:])]
+    ud = dev((1 - rng.random(batch)).astype(np.float32))
+    policy_t = torch.full((batch, dims[-1]), 7.0, device="cuda")
+    _, action = LY.mlp_forward(xd, wd, None, head, ud, mask, False, policy_out=policy_t)
+    full_p, full_a, _ = LY.mlp_forward(xd, wd, None, head, ud, mask, True)
+    assert torch.equal(policy_t.view(torch.int32), full_p.view(torch.int32)) and torch.equal(action, full_a)
+
+
 @pytest.mark.parametrize("dims,head,mask,batch,dtype,with_bias", [
     ([32, 256, 256, 256, 3], "softmax_regret_matching", 0, 16384, "f16", False),     # the benchmark's policy network
     ([32, 256, 256, 256, 3], "softmax", 0, 1, "bf16", False),                        # a single row
