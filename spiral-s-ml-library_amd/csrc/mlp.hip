@@ -233,7 +233,11 @@ __global__ __launch_bounds__(NW * 64) void mlp_forward_kernel(const MlpArgs a) {
     if (lane < 16 && row_ok) {
         float* p = head_rows + lane * MLP_MAX_OUT;   // this row's outputs
         const float u = a.ph.philox_mode >= 0 ? reference_row_uniform(a.ph, row) : a.action != nullptr ? a.u[row] : 1.f;
-        if (N <= 8) head_row<8>(head_out(a), p, row, N, limit, u, N, &past);      // narrow heads run in registers
+        // narrow heads run in registers, at the smallest width that holds them: the head is a chain of this lane's own (batch
+        // 64, us, always 64 columns / these widths: 64-64-64-10 14.9 / 10.0, 64-96-96-16 16.7 / 11.8, 128-64-24 14.1 / 10.2)
+        if (N <= 8) head_row<8>(head_out(a), p, row, N, limit, u, N, &past);
+        else if (N <= 16) head_row<16>(head_out(a), p, row, N, limit, u);
+        else if (N <= 32) head_row<32>(head_out(a), p, row, N, limit, u);
         else head_row<MLP_MAX_OUT>(head_out(a), p, row, N, limit, u);
     }
     if (a.out_stride > N) {

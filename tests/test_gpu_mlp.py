@@ -160,6 +160,16 @@ def test_masked_head_without_logits(LY, dtype, batch, dims, head, mask):
     assert (action == orow.discrete_sampling(policy, u)).all() and (action < mask).all() and (action >= 0).all()
 
 
+@pytest.mark.parametrize("dims,head,mask", [([32, 64, 9], "softmax", 0), ([16, 96, 16], "regret_matching", 0),
+                                            ([64, 32, 17], "softmax_regret_matching", 11), ([48, 160, 32], "softmax", 0),
+                                            ([32, 64, 33], "softmax", 0)])
+def test_head_widths_of_other_stacks(LY, dims, head, mask):
+    """The widths at which the head of the kernel for any hidden width changes its instance."""
+    announce("mlp head width %s head=%s mask=%d" % (dims, head, mask))
+    x, ws, u = make_problem(np.random.default_rng(dims[-1]), 70, dims, "f16")
+    check(LY, x, ws, u, "f16", head, mask)
+
+
 @pytest.mark.parametrize("dims,head,mask,batch,dtype", [([128, 64, 64], "regret_matching", 3, 64, "bf16"),
                                                         ([48, 96, 128, 10], "softmax", 4, 37, "f16"),      # rows of no whole pieces
                                                         ([16, 32, 12], "softmax_regret_matching", 7, 130, "bf16"),
