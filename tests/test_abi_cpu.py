@@ -233,3 +233,19 @@ def test_ensemble_argument_errors(L):
     assert hash_call(modulo=0) == -5 and "modulo" in _err(L)
     assert hash_call(members=70000) == -2
     assert hash_call(w=C.c_void_p(0x6008)) == -3
+
+
+def test_stack_argument_errors(L):
+    p = C.c_void_p(0x6000)
+    ints = lambda *d: (C.c_int32 * len(d))(*d)
+    call = lambda x=p, n=2, w=(C.c_void_p * 2)(p, p), d=ints(64, 64, 16), acts=ints(1, 0), members=1, pol=p, act=None, batch=64, head=1, mask=0, ph=None: \
+        L.lib.sp_stack_forward_f32(x, n, w, d, acts, members, None, ph, pol, act, batch, head, mask, None)
+    assert call(x=None) == -1 and call(pol=None) == -1 and call(w=None) == -1 and call(w=(C.c_void_p * 2)(p, None)) == -1
+    assert call(act=p) == -1                                          # an action without uniforms
+    assert call(x=C.c_void_p(0x6004)) == -3
+    assert call(n=9) == -2 and call(members=0) == -2 and call(batch=0) == -2 and call(batch=1 << 31) == -2
+    assert call(d=ints(66, 64, 16)) == -2 and call(d=ints(64, 72, 16)) == -2 and call(d=ints(64, 64, 68)) == -2 and call(d=ints(64, 144, 16)) == -2
+    assert call(head=3) == -5 and call(acts=ints(9, 0)) == -5 and call(head=2, mask=0) == -5 and call(head=2, mask=17) == -5
+    ph = L.PhiloxConfig(1, 0, L.PHILOX_LAYER, 256, 8, 8, 32, 0)
+    assert call(act=p, ph=C.byref(ph)) == -5 and "member_rows" in _err(L)
+    assert call(n=4, w=(C.c_void_p * 4)(p, p, p, p), d=ints(128, 128, 128, 128, 64), acts=ints(1, 1, 1, 0)) == -6 and "LDS" in _err(L)

@@ -147,3 +147,17 @@ def test_ensemble_with_adjoint_places_the_dual_in_the_adjoint_arena():
     assert w.data_ptr() == L.key_extract(m, "weights").data_ptr()
     assert wt.data_ptr() == L.model_to_model_ptrs(m)[L.weight_adjoint_id()].data_ptr()
     assert L.get_dim({}, x).dim == (24, 64, n)
+
+
+def test_stack_plan_takes_whole_chains_only():
+    """The graphs that run as one launch of the f32 stack kernel: a chain whose inner nodes nobody can look at."""
+    plan = lambda g, key=None: L._stack_plan(L.Model(g, {}, []), key)
+    x, ws, acts, head, mask, outs = plan(graph_of_test3())
+    assert len(ws) == 3 and head == "softmax" and mask == 0 and outs is None and acts[0] == acts[1] != 0 and acts[2] == 0
+    assert plan(ensemble_graph(4, True), "ensemble")[5] is not None and plan(ensemble_graph(4, True)) is None
+    inp = lambda: L.input("input", (24, 64, 64))
+    named = L.pipe(L.key_graph("hidden", L.pipe(inp(), L.matmul((64, 64)))), L.relu, L.matmul((64, 64)), L.softmax_and_discrete_sample)
+    kept = L.pipe(L.copy_(L.input("kept", (24, 64, 64)), L.pipe(inp(), L.matmul((64, 64)))), L.matmul((64, 64)), L.softmax_and_discrete_sample)
+    swapped = L.pipe(inp(), L.matmul((64, 64)), L.relu, L.ln_l2, L.matmul((64, 64)), L.softmax_and_discrete_sample)   # norm behind the map
+    first = L.pipe(inp(), L.relu, L.matmul((64, 64)), L.softmax_and_discrete_sample)                                    # a map of the input
+    assert [plan(g) for g in (named, kept, swapped, first)] == [None] * 4
