@@ -1023,6 +1023,7 @@ static TileChoice choose_tile(int dtype_in, long M, long N, long K, long batch) 
             if (whole == 2 && (c.cfg == 0 || c.cfg == 1)) return;
             if (c.cfg < 0 && (!may_split || K * es > kWaveMaxRowBytes || M > 2147483000l || N > 2147483000l)) return;
             const double tiles = (double)((M + c.bm - 1) / c.bm) * (double)((N + c.bn - 1) / c.bn) * (double)batch;
+            if (c.cfg < 0 && tiles >= 4294967296.0) return;     // the split form numbers the tiles of a whole batch in 32 bits
             const float n = (float)((tiles + cus - 1) / cus >= 1e9 ? 1e9 : (double)(long)((tiles + cus - 1) / cus));
             const float per_k = n * c.tk > c.latency ? n * c.tk : c.latency;
             const float us = n * c.overhead + (float)nk * per_k;

@@ -37,7 +37,7 @@ __device__ __forceinline__ f32x4 mma(const u32x4& b, const u32x4& a, f32x4 c) {
 
 template <int DT, int TM, int TN, int NS>
 __global__ __launch_bounds__(256) void gemm_wave_kernel(const void* A_first, const void* B_first, int M, int N, int K, int tiles_m,
-                                                        int tiles_n, long stride_a, long stride_b, const GemmArgs g) {
+                                                        int tiles_n, int batch, long stride_a, long stride_b, const GemmArgs g) {
     constexpr int KS = 4;                                   // waves, each with every KS-th K-tile
     constexpr int ES = DT == SP_F32 ? 4 : 2;
     constexpr int BK = ROW_BYTES / ES;
@@ -48,19 +48,25 @@ __global__ __launch_bounds__(256) void gemm_wave_kernel(const void* A_first, con
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // workgroups are dealt round-robin to the 8 XCDs: each XCD walks a contiguous range of tiles, along the longer side
-    // of the tile grid last, so that the panel its neighbours share stays in its L2
-    const unsigned tiles = (unsigned)tiles_m * (unsigned)tiles_n;
-    const unsigned t = (blockIdx.x & 7u) * ((tiles + 7u) / 8u) + (blockIdx.x >> 3);
-    if (t >= tiles) return;
+    // workgroups are dealt round-robin to the 8 XCDs: each XCD walks a contiguous range of the tiles of the whole batch,
+    // along the longer side of a member's tile grid last, so that the panel its neighbours share stays in its L2.  (With
+    // ranges within every member, members of one to seven tiles all began on the first XCDs: bf16 71 x (112 x 48 x 952)
+    // 25.2 us, numbered through 7.4; f32 103 x (64 x 64 x 448) 16.6 / 7.8; the same tiles without a batch unchanged.)
+    const unsigned tiles = (unsigned)tiles_m * (unsigned)tiles_n, all = tiles * (unsigned)batch;
+    const unsigned block = blockIdx.y * tiles + blockIdx.x, xcd = block & 7u;
+    unsigned t = xcd * (all / 8u) + (xcd < (all & 7u) ? xcd : (all & 7u)) + (block >> 3), member = 0;
+    if (batch > 1) {
+        member = t / tiles;
+        t -= member * tiles;
+    }
     const bool m_last = tiles_m >= tiles_n;
     const unsigned inner = m_last ? (unsigned)tiles_n : (unsigned)tiles_m;
     const unsigned hi = t / inner, lo = t - hi * inner;
     const long m0 = (long)(m_last ? hi : lo) * (16 * TM), n0 = (long)(m_last ? lo : hi) * (16 * TN);
 
     const long row_bytes = (long)K * ES;
-    const unsigned char* pA = uniform_ptr((const unsigned char*)A_first + (long)blockIdx.y * stride_a + m0 * row_bytes);
-    const unsigned char* pB = uniform_ptr((const unsigned char*)B_first + (long)blockIdx.y * stride_b + n0 * row_bytes);
+    const unsigned char* pA = uniform_ptr((const unsigned char*)A_first + (long)member * stride_a + m0 * row_bytes);
+    const unsigned char* pB = uniform_ptr((const unsigned char*)B_first + (long)member * stride_b + n0 * row_bytes);
     const unsigned my_lds = __builtin_amdgcn_readfirstlane((unsigned)(size_t)lds + wave * (NS * STAGE));
     const int nk = (K + BK - 1) / BK;
     const bool k_tail = K % BK != 0;
@@ -140,7 +146,7 @@ __global__ __launch_bounds__(256) void gemm_wave_kernel(const void* A_first, con
     // One quad of registers: C[row][col .. col + 3], the last one to three columns of a row element by element.  All
     // that is read is requested before any of it is waited for.
     constexpr int OT16 = DT == SP_BF16 ? SP_BF16 : SP_F16;
-    unsigned char* const Cb = (unsigned char*)g.C + (long)blockIdx.y * g.stride_c;
+    unsigned char* const Cb = (unsigned char*)g.C + (long)member * g.stride_c;
     const bool half = g.out_dtype != SP_F32;
     auto put = [&](long row, long col, f32x4 v) {
         if (row >= M || col >= N) return;
@@ -224,9 +230,9 @@ static int launch_wave(const GemmArgs& g, hipStream_t stream) {
     constexpr int lds_bytes = ring > partial ? ring : partial;
     const int rc = ensure_dynamic_lds((const void*)kernel, lds_bytes);
     if (rc != SP_OK) return rc;
-    const long blocks = ((long)g.tiles_m * g.tiles_n + 7) / 8 * 8;    // a whole number per XCD
+    const long blocks = (long)g.tiles_m * g.tiles_n;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks, (unsigned)g.batch), dim3(256), lds_bytes, stream, g.A, g.B, (int)g.M,
-                       (int)g.N, (int)g.K, g.tiles_m, g.tiles_n, g.stride_a, g.stride_b, g);
+                       (int)g.N, (int)g.K, g.tiles_m, g.tiles_n, g.batch, g.stride_a, g.stride_b, g);
     return check_launch("sp_gemm_abt");
 }
 

@@ -140,6 +140,26 @@ def test_split_k_and_odd_widths_are_exact(MM, dtype, m, n, kt):
             assert (got[pad:pad + m * n].reshape(m, n) == exact(full)).all(), (out, beta)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("e,m,n,kt", [(239, 64, 64, 1), (5, 16, 16, 7), (17, 64, 16, 9.5), (3, 132, 35, 30), (9, 84, 61, 8), (7, 212, 100, 7.5),
+                                      (70, 48, 33, 3), (2, 500, 331, 9)])
+def test_batched_split_k_and_odd_widths_are_exact(MM, dtype, e, m, n, kt):
+    """The tiles of a whole batch are numbered through, whatever a member has of them (one, a few, an odd number): integer
+    operands give the exact products of every member, odd widths and partial K-tiles among them, with bias, ReLU and beta."""
+    k = int(kt * (32 if dtype == "f32" else 64))
+    announce("gemm batched split K %s e=%d %dx%dx%d" % (dtype, e, m, n, k))
+    rng = np.random.default_rng(e + m + 3 * n + 7 * k)
+    ai = rng.integers(-3, 4, size=(e, m, k)).astype(np.float32)
+    bi = rng.integers(-3, 4, size=(e, n, k)).astype(np.float32)
+    want = np.matmul(ai, bi.transpose(0, 2, 1)).astype(np.float64)          # exact: every sum is below 2^24
+    bias = rng.integers(-5, 6, size=n).astype(np.float32)
+    c0 = rng.integers(-4, 5, size=(e, m, n)).astype(np.float32)
+    a, b = dev(ai, TORCH[dtype]), dev(bi, TORCH[dtype])
+    assert (host(MM.matmul_abt_batched(a, b)) == want).all()
+    got = host(MM.matmul_abt_batched(a, b, c=dev(c0), beta=2.0, bias=dev(bias), relu=True))
+    assert (got == np.maximum(want + 2 * c0 + bias, 0)).all()
+
+
 def test_random_small_shapes_are_exact(MM):
     """120 seeded shapes around the tile boundaries (M, N up to 330, K up to 45 chunks), all three dtypes, integer
     operands: the tiled kernels' masking of M, N and K must give the exact product, with and without bias + ReLU."""
