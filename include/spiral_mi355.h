@@ -121,6 +121,8 @@ int sp_gemm_abt(int dtype_in, int dtype_out, const void* A, const void* B, void*
  * (ml/layers.spi:227-240,336-344,468-471): A = the shared input, stride_a = 0, B = the (E, out, in)
  * weight tensor, stride_b = out * in.  The tile is chosen for the whole batch, so many small members
  * fill the chip.  bias (N,) is shared by all members.
+ * f32: every member's C is bit-identical to sp_gemm_abt on that member (the shape of one member alone decides the order
+ * in which K is added up).  16-bit inputs: equal to the rounding of the sums; a large batch may add up K in another order.
  */
 int sp_gemm_abt_batched(int dtype_in, int dtype_out, const void* A, const void* B, void* C, const float* bias,
                         int64_t M, int64_t N, int64_t K, int64_t batch, int64_t stride_a, int64_t stride_b,
@@ -130,6 +132,11 @@ int sp_gemm_abt_batched(int dtype_in, int dtype_out, const void* A, const void* 
  * `matmul_config_tf32`, ml/matmul/run.spi:8-19).  Writes block tile sizes and the workgroup size. */
 int sp_gemm_config(int dtype_in, int64_t M, int64_t N, int64_t K,
                    int32_t* tile_m, int32_t* tile_n, int32_t* tile_k, int32_t* threads);
+
+/* The same for one launch over `batch` matrices (sp_gemm_abt_batched); k_parts: the partial sums over K that an output is
+ * added up from (4 on the split-K tiles, 1 on the workgroup tiles). */
+int sp_gemm_batched_config(int dtype_in, int64_t M, int64_t N, int64_t K, int64_t batch,
+                           int32_t* tile_m, int32_t* tile_n, int32_t* tile_k, int32_t* threads, int32_t* k_parts);
 
 /* ------------------------------------------------------------------------------------------ */
 /* Row primitives                                                                              */

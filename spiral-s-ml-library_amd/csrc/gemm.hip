@@ -957,10 +957,9 @@ static bool use_four_waves(int dtype_in, long N, long K) {
 // of the compute units, except for the four-wave kernel, which does per unit so much more than the 128 x 128 tiles
 // that 9/16 of the units are enough (3072^3 bf16: 144 tiles of 256 x 256 take 56 us, 576 tiles of 128 x 128 76 us; at
 // 128 tiles the two are level, below that the smaller tiles win).
-static int choose_cfg(int dtype_in, long M, long N, long K, long batch = 1) {
+static int choose_cfg(int dtype_in, long M, long N, long K, long batch, long cus) {
     const int bk = dtype_in == SP_F32 ? 32 : 64;
     if (K % bk != 0) return -1;
-    const int cus = device_cu_count();
     int smallest = -1;
     for (int i = 0; i < kNumCfgs; ++i) {
         const TileCfg& c = kTileCfgs[i];
@@ -968,7 +967,7 @@ static int choose_cfg(int dtype_in, long M, long N, long K, long batch = 1) {
         smallest = i;
         const long tiles = (M / c.bm) * (N / c.bn) * batch;
         const bool four_waves = i == 0 && use_four_waves(dtype_in, N, K);
-        if (four_waves ? tiles * 16 >= (long)cus * 9 : tiles * 5 >= (long)cus * 4) return i;
+        if (four_waves ? tiles * 16 >= cus * 9 : tiles * 5 >= cus * 4) return i;
     }
     return smallest;
 }
@@ -979,6 +978,7 @@ static int choose_cfg(int dtype_in, long M, long N, long K, long batch = 1) {
 struct TileChoice {
     int cfg, bm, bn, threads;
     bool ragged;
+    float us;      // the estimate
 };
 
 // Estimated time of the most loaded compute unit on a tile, in us: n = ceil(tiles / units) tiles one after the other,
@@ -1002,47 +1002,59 @@ static const TileCost kCostCrossing[] = {{0, 256, 256, 1.5f, 14.f, 0.f}, {1, 128
                                          {-1, 64, 64, 0.27f, 1.5f, 0.f}, {-1, 64, 32, 0.19f, 0.8f, 0.f}, {-1, 32, 32, 0.11f, 0.5f, 0.f},
                                          {-1, 16, 16, 0.055f, 0.3f, 0.f}};
 
-static TileChoice choose_tile(int dtype_in, long M, long N, long K, long batch) {
+enum TileKind { TILE_ANY, TILE_WORKGROUP, TILE_SPLIT };
+
+static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, long cus, TileKind kind) {
     const int es = dtype_in == SP_F32 ? 4 : 2, bk = ROW_BYTES / es;
-    const long cus = device_cu_count(), nk = (K + bk - 1) / bk;
+    const long nk = (K + bk - 1) / bk;
     // 16-bit shapes that a 256 or 128 tile divides: choose_cfg.  The rest, and f32, by the estimate.
-    const int whole = dtype_in == SP_F32 ? -1 : choose_cfg(dtype_in, M, N, K, batch);
-    int best = whole;
+    const int whole = dtype_in == SP_F32 || kind == TILE_SPLIT ? -1 : choose_cfg(dtype_in, M, N, K, batch, cus);
+    // K split over four waves: from seven K-tiles up.  Below that (where a large output wants the workgroup tiles
+    // whatever the estimate says) only for small outputs, whose time is the chain behind one of them (us, 64 x 64 tile /
+    // split: 181 x 39 x 96 f32 6.2 / 2.8; 64 x 64 x 128 4.5 / 2.6; 16 x 21 x 128 bf16 3.1 / 2.5), and for odd widths,
+    // where the split form's stores cost less (1371 x 45 x 64 bf16 4.4 / 2.8).
+    const double small = (double)((M + 15) / 16) * (double)((N + 15) / 16);
+    const bool may_split = kind == TILE_SPLIT || nk >= 7 || (batch <= 64 && small <= (N % 4 ? 1024 : 64));
+    const TileCost* best = nullptr;
     float best_us = 0.f;
-    int bm = 0, bn = 0;
-    if (whole != 0 && whole != 1) {
-        best = -2;
-        // K split over four waves: from seven K-tiles up.  Below that (where a large output wants the workgroup tiles
-        // whatever the estimate says, and where a member of a batch and a plain call of its shape take the same sums) only
-        // for small outputs, whose time is the chain behind one of them (us, 64 x 64 tile / split: 181 x 39 x 96 f32 6.9 /
-        // 3.9; 86 x 61 x 56 5.6 / 3.6; 16 x 21 x 144 bf16 4.4 / 3.4), and for odd widths, where the split form's stores
-        // cost less (5371 x 45 x 48 f16 5.4 / 4.5).
-        const double small = (double)((M + 15) / 16) * (double)((N + 15) / 16);
-        const bool may_split = nk >= 7 || (batch <= 64 && small <= (N % 4 ? 1024 : 64));
-        auto consider = [&](const TileCost& c) {
-            if (whole == 2 && (c.cfg == 0 || c.cfg == 1)) return;
-            if (c.cfg < 0 && (!may_split || K * es > kWaveMaxRowBytes || M > 2147483000l || N > 2147483000l)) return;
-            const double tiles = (double)((M + c.bm - 1) / c.bm) * (double)((N + c.bn - 1) / c.bn) * (double)batch;
-            if (c.cfg < 0 && tiles >= 4294967296.0) return;     // the split form numbers the tiles of a whole batch in 32 bits
-            const float n = (float)((tiles + cus - 1) / cus >= 1e9 ? 1e9 : (double)(long)((tiles + cus - 1) / cus));
-            const float per_k = n * c.tk > c.latency ? n * c.tk : c.latency;
-            const float us = n * c.overhead + (float)nk * per_k;
-            if (best == -2 || us < best_us) {
-                best = c.cfg;
-                best_us = us;
-                bm = c.bm;
-                bn = c.bn;
-            }
-        };
-        if (dtype_in == SP_F32) for (const TileCost& c : kCostF32) consider(c);
-        else if (K % bk == 0) for (const TileCost& c : kCostLines) consider(c);
-        else for (const TileCost& c : kCostCrossing) consider(c);
-    }
-    if (best < 0) return {-1, bm, bn, 256, true};
-    const TileCfg& t = kTileCfgs[best];
+    auto consider = [&](const TileCost& c) {
+        if (whole == 0 || whole == 1 ? c.cfg != whole : whole == 2 && (c.cfg == 0 || c.cfg == 1)) return;
+        if (c.cfg < 0 ? kind == TILE_WORKGROUP : kind == TILE_SPLIT) return;
+        if (c.cfg < 0 && (!may_split || K * es > kWaveMaxRowBytes || M > 2147483000l || N > 2147483000l)) return;
+        const double tiles = (double)((M + c.bm - 1) / c.bm) * (double)((N + c.bn - 1) / c.bn) * (double)batch;
+        if (c.cfg < 0 && tiles >= 4294967296.0) return;     // the split form numbers the tiles of a whole batch in 32 bits
+        const float n = (float)((tiles + cus - 1) / cus >= 1e9 ? 1e9 : (double)(long)((tiles + cus - 1) / cus));
+        const float per_k = n * c.tk > c.latency ? n * c.tk : c.latency;
+        const float us = n * c.overhead + (float)nk * per_k;
+        if (best == nullptr || us < best_us) {
+            best = &c;
+            best_us = us;
+        }
+    };
+    if (dtype_in == SP_F32) for (const TileCost& c : kCostF32) consider(c);
+    else if (K % bk == 0) for (const TileCost& c : kCostLines) consider(c);
+    else for (const TileCost& c : kCostCrossing) consider(c);
+    if (best == nullptr) return best_tile(dtype_in, M, N, K, batch, cus, TILE_WORKGROUP);   // (a split form that cannot be numbered)
+    if (best->cfg < 0) return {-1, best->bm, best->bn, 256, true, best_us};
+    const TileCfg& t = kTileCfgs[best->cfg];
     const bool ragged = M % t.bm != 0 || N % t.bn != 0 || K % bk != 0;
-    const int threads = best == 0 && !ragged && use_four_waves(dtype_in, N, K) ? 256 : t.wm * t.wn * 64;
-    return {best, t.bm, t.bn, threads, ragged};
+    const int threads = best->cfg == 0 && !ragged && use_four_waves(dtype_in, N, K) ? 256 : t.wm * t.wn * 64;
+    return {best->cfg, t.bm, t.bn, threads, ragged, best_us};
+}
+
+// The members of a batch are to add up like a plain launch of each.  The split-K tiles all add an output's products in one
+// order and the workgroup tiles of f32 in another, so the shape of ONE member decides between the two kinds and the batch
+// between the tiles of that kind.  Always for f32, whose batched and member-by-member runs are bit-identical; it costs most
+// where small whole tiles come in large numbers (us, workgroup tiles / split K: 300 x (128 x 128 x 224) 28.8 / 31.7,
+// 37 x (960 x 384 x 320) 78 / 104, 300 x (64 x 64 x 64) 4.8 / 7.8).  For 16-bit inputs, whose 256 wide tiles have MFMAs and
+// K walks of their own anyway, as long as the other kind is not a quarter faster by the estimate.
+static TileChoice choose_tile(int dtype_in, long M, long N, long K, long batch, long cus) {
+    const TileChoice member = best_tile(dtype_in, M, N, K, 1, cus, TILE_ANY);
+    if (batch == 1) return member;
+    const TileChoice alike = best_tile(dtype_in, M, N, K, batch, cus, member.cfg < 0 ? TILE_SPLIT : TILE_WORKGROUP);
+    if (dtype_in == SP_F32) return alike;
+    const TileChoice any = best_tile(dtype_in, M, N, K, batch, cus, TILE_ANY);
+    return alike.us <= 1.25f * any.us ? alike : any;
 }
 
 template <int DT, int OT, int BM, int BN, int WM, int WN, int NS, int NSA = NS, bool RAGGED = false>
@@ -1226,17 +1238,30 @@ struct GemmKernelNames {
 
 using namespace sp;
 
-extern "C" int sp_gemm_config(int dtype_in, int64_t M, int64_t N, int64_t K, int32_t* tile_m, int32_t* tile_n,
-                              int32_t* tile_k, int32_t* threads) {
-    if (!tile_m || !tile_n || !tile_k || !threads) return fail(SP_ERR_NULL, "sp_gemm_config: NULL output");
+static int gemm_config(const char* fn, int dtype_in, int64_t M, int64_t N, int64_t K, int64_t batch, int32_t* tile_m,
+                       int32_t* tile_n, int32_t* tile_k, int32_t* threads, int32_t* k_parts) {
+    if (!tile_m || !tile_n || !tile_k || !threads || !k_parts) return fail(SP_ERR_NULL, "%s: NULL output", fn);
     int rc = validate_gemm(dtype_in, SP_F32, M, N, K);
     if (rc != SP_OK) return rc;
-    const TileChoice t = choose_tile(dtype_in, M, N, K, 1);
+    if (batch < 1 || batch > 65535) return fail(SP_ERR_SHAPE, "%s: batch must be in [1, 65535], got %lld", fn, (long long)batch);
+    const TileChoice t = choose_tile(dtype_in, M, N, K, batch, device_cu_count());
     *tile_m = t.bm;
     *tile_n = t.bn;
     *tile_k = dtype_in == SP_F32 ? 32 : 64;
     *threads = t.threads;
+    *k_parts = t.cfg < 0 ? 4 : 1;
     return SP_OK;
+}
+
+extern "C" int sp_gemm_config(int dtype_in, int64_t M, int64_t N, int64_t K, int32_t* tile_m, int32_t* tile_n,
+                              int32_t* tile_k, int32_t* threads) {
+    int32_t k_parts = 0;
+    return gemm_config(__func__, dtype_in, M, N, K, 1, tile_m, tile_n, tile_k, threads, &k_parts);
+}
+
+extern "C" int sp_gemm_batched_config(int dtype_in, int64_t M, int64_t N, int64_t K, int64_t batch, int32_t* tile_m,
+                                      int32_t* tile_n, int32_t* tile_k, int32_t* threads, int32_t* k_parts) {
+    return gemm_config(__func__, dtype_in, M, N, K, batch, tile_m, tile_n, tile_k, threads, k_parts);
 }
 
 static int gemm_entry(const char* fn, int dtype_in, int dtype_out, const void* A, const void* B, void* C,
@@ -1272,12 +1297,13 @@ static int gemm_entry(const char* fn, int dtype_in, int dtype_out, const void* A
     hipStream_t s = (hipStream_t)stream;
     int cfg = -1;                                         // the generic kernel
     if (!(flags & SP_GEMM_FORCE_GENERIC)) {
-        const TileChoice t = choose_tile(dtype_in, M, N, K, batch);
+        const long cus = device_cu_count();
+        const TileChoice t = choose_tile(dtype_in, M, N, K, batch, cus);
         cfg = t.cfg;
         g.ragged = t.ragged;
         g.tiles_m = (int)((M + t.bm - 1) / t.bm);
         g.tiles_n = (int)((N + t.bn - 1) / t.bn);
-        if (cfg < 0) return launch_gemm_wave(dtype_in, t.bm, t.bn, g, s);
+        if (cfg < 0) return launch_gemm_wave(dtype_in, t.bm, t.bn, cus, g, s);
     }
     switch (dtype_in) {
         case SP_F32: return launch_dtype<SP_F32, SP_F32>(cfg, g, s);

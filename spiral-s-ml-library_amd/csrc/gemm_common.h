@@ -140,8 +140,8 @@ __device__ __forceinline__ const unsigned char* uniform_ptr(const unsigned char*
 
 // The split-K kernel of gemm_wave.hip on a tile of its menu (16 x 16, 32 x 32; 16-bit inputs also 64 x 32, 64 x 64), with
 // tiles_m / tiles_n set for that tile, rows of at most 32 MiB (per-lane byte offsets of up to 63 rows in 32 bits) and fewer
-// than 2^32 tiles in the batch.
-int launch_gemm_wave(int dtype_in, int tile_m, int tile_n, const GemmArgs& g, hipStream_t stream);
+// than 2^32 tiles in the batch; cus: the compute units of the device.
+int launch_gemm_wave(int dtype_in, int tile_m, int tile_n, long cus, const GemmArgs& g, hipStream_t stream);
 constexpr long kWaveMaxRowBytes = 1l << 25;
 
 }  // namespace sp

@@ -237,23 +237,28 @@ static int launch_wave(const GemmArgs& g, hipStream_t stream) {
 }
 
 // LDS rings: two stages of 8 KiB per wave leave room for two workgroups on a compute unit, four of 4 KiB likewise; the
-// larger tiles, one workgroup per unit, take all of the LDS they can use.
+// larger tiles, one workgroup per unit, take all of the LDS they can use.  With more tiles than those places a ring of ONE
+// stage: what a wave no longer has in flight, five workgroups (of 32 x 32; three and two of the larger tiles) on a unit
+// have between them, and a workgroup's prologue and last sums hide behind the others' K loops.  (us, rings / one stage:
+// f32 37 x (960 x 384 x 320), 52 tiles a unit, 130 / 104, 300 x (256 x 32 x 128), 9 a unit, 17.3 / 14.0; bf16
+// 172 x (695 x 100 x 320) 69 / 43.5, 29 x (1528 x 176 x 2240) 89 / 66.  At one or two tiles a unit the rings are 5 % faster.)
 template <int DT>
-static int launch_wave_dtype(int tile_m, int tile_n, const GemmArgs& g, hipStream_t stream) {
+static int launch_wave_dtype(int tile_m, int tile_n, long cus, const GemmArgs& g, hipStream_t stream) {
+    const long tiles = (long)g.tiles_m * g.tiles_n * g.batch;
     if (tile_m == 16) return launch_wave<DT, 1, 1, 4>(g, stream);
-    if (tile_m == 32) return launch_wave<DT, 2, 2, 2>(g, stream);
+    if (tile_m == 32) return tiles > 2 * cus ? launch_wave<DT, 2, 2, 1>(g, stream) : launch_wave<DT, 2, 2, 2>(g, stream);
     if constexpr (DT != SP_F32) {
-        if (tile_m == 64 && tile_n == 32) return launch_wave<DT, 4, 2, 3>(g, stream);
-        if (tile_m == 64) return launch_wave<DT, 4, 4, 2>(g, stream);
+        if (tile_m == 64 && tile_n == 32) return tiles > cus ? launch_wave<DT, 4, 2, 1>(g, stream) : launch_wave<DT, 4, 2, 3>(g, stream);
+        if (tile_m == 64) return tiles > cus ? launch_wave<DT, 4, 4, 1>(g, stream) : launch_wave<DT, 4, 4, 2>(g, stream);
     }
     return fail(SP_ERR_UNSUPPORTED, "sp_gemm_abt: no split-K kernel for a %d x %d tile", tile_m, tile_n);
 }
 
-int launch_gemm_wave(int dtype_in, int tile_m, int tile_n, const GemmArgs& g, hipStream_t stream) {
+int launch_gemm_wave(int dtype_in, int tile_m, int tile_n, long cus, const GemmArgs& g, hipStream_t stream) {
     switch (dtype_in) {
-        case SP_F32: return launch_wave_dtype<SP_F32>(tile_m, tile_n, g, stream);
-        case SP_F16: return launch_wave_dtype<SP_F16>(tile_m, tile_n, g, stream);
-        default: return launch_wave_dtype<SP_BF16>(tile_m, tile_n, g, stream);
+        case SP_F32: return launch_wave_dtype<SP_F32>(tile_m, tile_n, cus, g, stream);
+        case SP_F16: return launch_wave_dtype<SP_F16>(tile_m, tile_n, cus, g, stream);
+        default: return launch_wave_dtype<SP_BF16>(tile_m, tile_n, cus, g, stream);
     }
 }
 

@@ -60,6 +60,7 @@ SIGNATURES = {
     "sp_gemm_abt_batched": (C.c_int, [C.c_int, C.c_int, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _F, _F,
                                       _U32, _P]),
     "sp_gemm_config": (C.c_int, [C.c_int, _I64, _I64, _I64] + [C.POINTER(C.c_int32)] * 4),
+    "sp_gemm_batched_config": (C.c_int, [C.c_int, _I64, _I64, _I64, _I64] + [C.POINTER(C.c_int32)] * 5),
     "sp_row_ops": (C.c_int, [_P] * 8 + [_I64, _I64, _U32, _P]),
     "sp_row_map_f32": (C.c_int, [C.c_int, _P, _P, _I64, _I64, _I32, _P]),
     "sp_row_map_i32": (C.c_int, [C.c_int, _P, _P, _I64, _I64, _P]),

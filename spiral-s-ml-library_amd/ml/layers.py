@@ -1185,8 +1185,9 @@ def weights_changed(model):
 def graph_run_host(model, sizes=None, seed=_prim.CONSTANT_SEED, fuse=True, batched=True, static_weights=False):
     """Runs the graph for every combination of the key indices in `sizes`, e.g. {"ensemble": 16}
     (ml/layers.spi:336-344).  Uniforms come from the reference's per-thread Philox streams.  A loop over
-    one key that only indexes leading dimensions runs as a single batched pass with the same results
-    (`batched=False` keeps the member-by-member loop).  A dense stack under a row head runs as one launch, whose f32 sums
+    one key that only indexes leading dimensions runs as a single batched pass (`batched=False` keeps the
+    member-by-member loop): node by node the two are bit-identical in f32, in 16 bit equal to the rounding of the
+    sums.  A dense stack under a row head runs as one launch, whose f32 sums
     add up in another order and which does not write the unnamed nodes in the middle; `fuse=False` runs node by node.  `static_weights=True` says that the weights have not
     changed since the previous such run (or since `weights_changed(model)`): a fused relu-MLP then keeps a copy
     of them packed for the faster kernel instead of reading the arena on every run."""

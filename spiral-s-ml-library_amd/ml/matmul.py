@@ -22,6 +22,13 @@ def matmul_config_tf32(a_trans, b_trans, m, n, k, dtype=torch.float32):
     return dict(zip(("m_tile", "n_tile", "k_tile", "threads"), (o.value for o in out)))
 
 
+def matmul_config_batched(batch, m, n, k, dtype=torch.float32):
+    """The same for one launch over `batch` matrices, with k_parts, the partial sums over K behind an output."""
+    out = [C.c_int32() for _ in range(5)]
+    check(lib.sp_gemm_batched_config(_lib.DTYPES[dtype], m, n, k, batch, *[C.byref(o) for o in out]))
+    return dict(zip(("m_tile", "n_tile", "k_tile", "threads", "k_parts"), (o.value for o in out)))
+
+
 def matmul_abt(a, b, c=None, alpha=1.0, beta=0.0, bias=None, relu=False, out_dtype=None, force_generic=False):
     """C = alpha * A . B^T + beta * C (+ bias, ReLU).  a: (M, K), b: (N, K), both row-major and of
     the same dtype (f32, f16 or bf16).  `c` is updated in place and returned; when it is None a new
@@ -49,7 +56,8 @@ def matmul_abt(a, b, c=None, alpha=1.0, beta=0.0, bias=None, relu=False, out_dty
 def matmul_abt_batched(a, b, c=None, alpha=1.0, beta=0.0, bias=None, relu=False, out_dtype=None, force_generic=False):
     """C[e] = alpha * A[e] . B[e]^T + beta * C[e] for every batch member in ONE launch.  a: (E, M, K) or (M, K)
     (shared by all members), b: (E, N, K) or (N, K), at least one of them batched; c: (E, M, N).  This is the
-    loop `graph_run_host model {ensemble}` makes around a `matmul_ensemble` layer (ml/layers.spi:336-344,468-471)."""
+    loop `graph_run_host model {ensemble}` makes around a `matmul_ensemble` layer (ml/layers.spi:336-344,468-471).
+    In f32 every member is bit-identical to `matmul_abt` on it alone; in 16 bit a batch may add up K in another order."""
     if a.dtype != b.dtype or a.dtype not in _lib.DTYPES:
         raise TypeError("a and b must share one of the dtypes f32/f16/bf16")
     if a.dim() not in (2, 3) or b.dim() not in (2, 3) or (a.dim() == 2 and b.dim() == 2):

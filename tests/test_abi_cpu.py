@@ -62,6 +62,37 @@ def test_gemm_argument_errors(L):
     assert lib.sp_gemm_abt(*args(M=(1 << 31) + 1)) == -2
 
 
+def test_a_batch_adds_up_like_a_launch_per_member(L):
+    """Split-K or workgroup tiles is a matter of one member's shape, for f32 always, for 16-bit inputs unless the other kind
+    is estimated to be a quarter faster (large batches).  Shapes around the edges of tiles, of the K rule and of the estimate."""
+    import random
+    def config(dtype, m, n, k, e):
+        out = [C.c_int32() for _ in range(5)]
+        assert L.lib.sp_gemm_batched_config(dtype, m, n, k, e, *[C.byref(o) for o in out]) == 0
+        return [o.value for o in out]
+    rng = random.Random(3)
+    shapes = [(0, 1536, 64, 256), (0, 64, 64, 64), (0, 128, 128, 192), (2, 1536, 128, 512), (0, 336, 304, 2256), (1, 86, 61, 56)]
+    for _ in range(3000):
+        dtype = rng.choice([0, 1, 2])
+        m, n = (max(1, int(2 ** rng.uniform(0, 13)) // a * a) for a in (rng.choice([1, 16, 64]), rng.choice([1, 4, 64])))
+        shapes.append((dtype, m, n, max(8, int(2 ** rng.uniform(3, 13)) // 8 * 8)))
+    kinds, alike = {1: 0, 4: 0}, {e: [] for e in (2, 4, 16, 33, 64, 65, 100, 300)}
+    for dtype, m, n, k in shapes:
+        one = config(dtype, m, n, k, 1)
+        single = [C.c_int32() for _ in range(4)]
+        assert L.lib.sp_gemm_config(dtype, m, n, k, *[C.byref(o) for o in single]) == 0 and [o.value for o in single] == one[:4]
+        kinds[one[4]] += 1
+        for e in alike:
+            many = config(dtype, m, n, k, e)
+            assert dtype != 0 or many[4] == one[4], (m, n, k, e, one, many)
+            alike[e].append(many[4] == one[4])
+    assert kinds[1] > 300 and kinds[4] > 300
+    share = lambda e: sum(alike[e]) / len(alike[e])
+    assert share(2) > 0.95 and share(16) > 0.85, {e: share(e) for e in alike}
+    assert L.lib.sp_gemm_batched_config(0, 64, 64, 64, 0, *[C.byref(C.c_int32()) for _ in range(5)]) == -2
+    assert L.lib.sp_gemm_batched_config(0, 64, 64, 64, 2, None, *[C.byref(C.c_int32()) for _ in range(4)]) == -1
+
+
 def test_batched_gemm_argument_errors(L):
     lib = L.lib
     p = C.c_void_p(0x1000)

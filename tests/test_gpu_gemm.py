@@ -492,7 +492,10 @@ def test_clock_sample_gives_the_shader_clock():
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("e,m,n,k,shared", [(16, 1536, 64, 64, "a"), (5, 256, 256, 128, None), (3, 100, 24, 40, "a"),
-                                            (4, 128, 512, 64, "b"), (40, 64, 64, 64, "a")])
+                                            (4, 128, 512, 64, "b"), (40, 64, 64, 64, "a"),
+                                            # shapes whose plain launch splits K over waves; odd widths
+                                            (16, 1536, 64, 256, "a"), (64, 128, 128, 192, None), (65, 64, 64, 64, "b"),
+                                            (3, 132, 35, 1000, None), (8, 76, 21, 488, "a"), (5, 300, 147, 240, "b")])
 def test_batched(MM, dtype, e, m, n, k, shared):
     """One launch for a whole ensemble (`matmul_ensemble`: E weight matrices, one shared input)."""
     announce("gemm batched %s e=%d %dx%dx%d shared=%s" % (dtype, e, m, n, k, shared))
@@ -510,9 +513,15 @@ def test_batched(MM, dtype, e, m, n, k, shared):
         want = ogemm.gemm_abt(a[0 if shared == "a" else i], b[0 if shared == "b" else i], c=c0[i], alpha=0.5, beta=2.0,
                               bias=bias, relu=True)
         assert ogemm.rel_frobenius(got[i], want) < TOL[dtype]
-    # every member equals the plain launch on its own operands, bit for bit
-    one = host(MM.matmul_abt(dev(a[0], t), dev(b[0], t)))
-    many = host(MM.matmul_abt_batched(ad, bd))
-    assert (many[0] == one).all()
     with pytest.raises(AssertionError, match="K dimension"):
         MM.matmul_abt_batched(ad, dev(np.zeros((e, n, k + 8), dtype=np.float32), t))
+    # every member equals the plain launch on its own operands, bit for bit: always in f32, in 16 bit where both add up K
+    # in the same number of parts
+    parts = lambda members: MM.matmul_config_batched(members, m, n, k, t)["k_parts"]
+    assert dtype != "f32" or parts(e) == parts(1)
+    if parts(e) != parts(1):
+        return
+    many = host(MM.matmul_abt_batched(ad, bd))
+    for i in (0, e - 1):
+        one = host(MM.matmul_abt(dev(a[0 if shared == "a" else i], t), dev(b[0 if shared == "b" else i], t)))
+        assert (many[i] == one).all()

@@ -120,6 +120,27 @@ def test_batched_ensemble_pass_equals_member_by_member_loop(L):
     assert (want_i < 17).all() and len(np.unique(want_i)) > 5
 
 
+@pytest.mark.parametrize("ensemble,rows", [(16, 64), (100, 2)])
+def test_batched_ensemble_pass_of_wide_layers_equals_the_loop(L, ensemble, rows):
+    """The same for a hidden layer of 256, whose products are long enough for the tiles that split K: the batch must not
+    change the order in which a member's sums add up."""
+    announce("layers batched ensemble pass, wide: %d members, %d rows a block" % (ensemble, rows))
+    out = L.pair(L.apply("ensemble", L.input("probs", (ensemble, Q, rows, 64))),
+                 L.apply("ensemble", L.input("picks", (ensemble, Q, rows), "int")))
+    x = L.pipe(L.input("input", (Q, rows, 64)), L.matmul_ensemble((ensemble, 64, 256)), L.ln_l2, L.relu,
+               L.matmul_ensemble((ensemble, 256, 64)))
+    m = L.create_model(L.softmax_and_discrete_sample_(out, x))
+    rng = np.random.default_rng(ensemble)
+    for t in [L.key_extract(m, "input")] + [t for _, t, _ in L.extract_layers_(m, L.weight_id())]:
+        fill(t, rng, 1.0 if t.shape[-2:] == (rows, 64) else 0.2)
+    outs = lambda: [host(L.key_extract(m, key)).copy() for key in ("probs", "picks")]
+    L.graph_run_host(m, {"ensemble": ensemble}, batched=False)
+    want = outs()
+    L.key_extract(m, "probs").zero_()
+    L.graph_run_host(m, {"ensemble": ensemble})
+    assert all((a == b).all() for a, b in zip(outs(), want))
+
+
 def test_ensemble_with_adjoint_and_the_cem_update(L):
     """`matmul_ensemble_with_adjoint` keeps every ensemble layer as the pair (weights, transposed dual in the adjoint
     arena); the product is the one `matmul_ensemble` computes, and the reference's CEM update walks the pair:
