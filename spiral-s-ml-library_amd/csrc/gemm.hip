@@ -385,25 +385,24 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_abt_kernel(SP_GEMM_PRELOADED
                 const long row_first = m0 + wm * WTM + i * 32 + er;
                 long idx = row_first * g.N + col;     // advanced by RPP rows per pass
                 // one 4-column piece: what C held there, and the store
-                typedef typename std::conditional<RAGGED, f32x4_unaligned, f32x4>::type c32_t;
-                typedef typename std::conditional<RAGGED, u32x2_unaligned, u32x2>::type c16_t;
+                constexpr int AT32 = RAGGED ? 4 : 16, AT16 = RAGGED ? 2 : 8;      // ragged rows begin at any element
                 auto read_old = [&](long at) {
                     if constexpr (OT == SP_F32) {
-                        return (f32x4)*reinterpret_cast<const c32_t*>((const float*)Cb + at);
+                        return load_aligned<AT32, f32x4>((const float*)Cb + at);
                     } else {
-                        const u32x2 o = *reinterpret_cast<const c16_t*>((const unsigned short*)Cb + at);
+                        const u32x2 o = load_aligned<AT16, u32x2>((const unsigned short*)Cb + at);
                         return f32x4{half_bits_to_f32<OT>(o.x & 0xffffu), half_bits_to_f32<OT>(o.x >> 16),
                                      half_bits_to_f32<OT>(o.y & 0xffffu), half_bits_to_f32<OT>(o.y >> 16)};
                     }
                 };
                 auto write = [&](long at, const f32x4& r) {
                     if constexpr (OT == SP_F32) {
-                        store_c<POLICY>(reinterpret_cast<c32_t*>((float*)Cb + at), r);
+                        store_c<POLICY, AT32>((float*)Cb + at, r);
                     } else {
                         u32x2 o;
                         o.x = pack_halves<OT>(r.x, r.y);
                         o.y = pack_halves<OT>(r.z, r.w);
-                        store_c<POLICY>(reinterpret_cast<c16_t*>((unsigned short*)Cb + at), o);
+                        store_c<POLICY, AT16>((unsigned short*)Cb + at, o);
                     }
                 };
                 constexpr int PASSES = 32 / RPP;
@@ -820,7 +819,7 @@ __global__ __launch_bounds__(256) void gemm_abt_w4_kernel(SP_GEMM_PRELOADED, con
                     const f32x4 v = *reinterpret_cast<const f32x4*>(strip + strip_at(rl, ec / 4));
                     f32x4* c = reinterpret_cast<f32x4*>((float*)Cb + idx);
                     if constexpr (HAS_BETA) old0 = *c;
-                    store_c<POLICY>(c, finish(v, old0, bias4[0]));
+                    store_c<POLICY, alignof(f32x4)>(c, finish(v, old0, bias4[0]));
                 } else {
                     const f32x4 v0 = *reinterpret_cast<const f32x4*>(strip + strip_at(rl, ec / 4));
                     const f32x4 v1 = *reinterpret_cast<const f32x4*>(strip + strip_at(rl, ec / 4 + 1));
@@ -838,7 +837,7 @@ __global__ __launch_bounds__(256) void gemm_abt_w4_kernel(SP_GEMM_PRELOADED, con
                     o.y = pack_halves<OT>(r0.z, r0.w);
                     o.z = pack_halves<OT>(r1.x, r1.y);
                     o.w = pack_halves<OT>(r1.z, r1.w);
-                    store_c<POLICY>(c, o);
+                    store_c<POLICY, alignof(decltype(o))>(c, o);
                 }
             }
         }

@@ -91,11 +91,21 @@ __device__ __forceinline__ unsigned pack_halves(float a, float b) {
 // 16384 x 4096 x 4096 383 / 390 / 364; 65536 x 2048 x 512 178 / 177 / 158; 65536 x 1024 x 512 91 / 91 / 96;
 // 8192 x 8192 x 1024 123 / 128 / 132; 4096^3 92.6 / 91.8 / 92.2.
 enum { ST_PLAIN = 0, ST_THROUGH = 1, ST_STREAM = 2 };
-template <int POLICY, typename P, typename V>
-__device__ __forceinline__ void store_c(P* p, V v) {
+// ALIGN: what the address is known to be aligned to (the attribute of a typedef is lost where that type is a template
+// argument, so it is put on inside).
+template <int ALIGN, typename V>
+__device__ __forceinline__ V load_aligned(const void* p) {
+    typedef V W __attribute__((aligned(ALIGN)));
+    static_assert(alignof(W) == ALIGN, "alignment lost");
+    return *reinterpret_cast<const W*>(p);
+}
+template <int POLICY, int ALIGN, typename V>
+__device__ __forceinline__ void store_c(void* p, V v) {
+    typedef V W __attribute__((aligned(ALIGN)));
+    static_assert(alignof(W) == ALIGN, "alignment lost");
     static_assert(sizeof(V) == 16 || sizeof(V) == 8, "16- or 8-byte pieces of C");
-    if constexpr (POLICY == ST_STREAM) __builtin_nontemporal_store(v, p);
-    else if constexpr (POLICY == ST_PLAIN) *p = v;
+    if constexpr (POLICY == ST_STREAM) __builtin_nontemporal_store(v, reinterpret_cast<W*>(p));
+    else if constexpr (POLICY == ST_PLAIN) *reinterpret_cast<W*>(p) = v;
     else if constexpr (sizeof(V) == 16) store16_through((V*)p, v);
     else asm volatile("global_store_dwordx2 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
 }
