@@ -980,20 +980,21 @@ struct TileChoice {
     float us;      // the estimate
 };
 
-// Estimated time of the most loaded compute unit on a tile, in us: n = ceil(tiles / units) tiles one after the other,
-// each nk K-tiles of `tk` plus `overhead` (prologue, epilogue, padding of its stores), and never less than `latency` per
-// K-tile (what a lone workgroup per unit waits for its loads).  Fitted to every tile on ~60 shapes; the estimate is within
-// 15 % for f32 and 30 % for 16-bit, and what matters is the order (us, 256 / 128 / 64 / split 32 x 32): f32 6928 x 624 x 680
-// 176 / 94 / 66 / 74; 43712 x 48 x 336 98 / 54 / 25 / 33; 4000 x 4000 x 1000 251 / 258 / 269 / 338; 6160 x 192 x 2984
-// 696 / 202 / 103 / 80; 3072 x 1024 x 1024 237 / 71 / 58 / 67; bf16 3000^3 80 / 109 / 125 / 257; 54928 x 80 x 5504 180 /
-// 157 / 189 / 213; 4784 x 912 x 64 f32 34 / 22 / 15 / 28; f16 5001 x 1003 x 1000 44 / 29 / 33 / 40.  16-bit rows that
-// do not start on 128-byte lines cost every fetch a second line, hence two sets of numbers.
+// Estimated time of the most loaded compute unit on a tile, in us, without the launch: n tiles one after the other, each nk
+// K-tiles of `tk` plus `overhead` (prologue, epilogue, padding of its stores), and never less than `latency` per K-tile (what a
+// lone workgroup per unit waits for its loads).  n is ceil(tiles / units) for 16-bit inputs; for f32, whose tiles hold a unit's
+// matrix pipes busy side by side, the mean of that and of tiles / units.  Fitted to every tile on some 330 shapes
+// (profiles/gemm_tiles.txt has them, with what each tile takes and which one the estimate picks); what matters is the order.
+// The f32 line is the second fit: the first had too little overhead for the large tiles and cost short K up to 1.6 times
+// (us, 256 / 128 / 64 wide tiles: 11200 x 1792 x 32 44 / 33 / 20, 2688 x 5760 x 64 31 / 25 / 23, 2112 x 1536 x 96 36 / 15 / 9.6;
+// 10688 x 768 x 3648, 824 / 467 / 485, keeps its 128).  16-bit rows that do not start on 128-byte lines cost every fetch a
+// second line, hence two sets of numbers.
 struct TileCost {
     int cfg, bm, bn;
     float tk, overhead, latency;
 };
-static const TileCost kCostF32[] = {{0, 256, 256, 7.85f, 10.f, 0.f}, {1, 128, 128, 2.13f, 3.f, 0.f}, {2, 64, 64, 0.57f, 1.f, 0.f},
-                                    {-1, 32, 32, 0.184f, 0.5f, 0.f}, {-1, 16, 16, 0.089f, 0.3f, 0.f}};
+static const TileCost kCostF32[] = {{0, 256, 256, 7.86f, 22.f, 0.f}, {1, 128, 128, 2.17f, 3.6f, 0.f}, {2, 64, 64, 0.556f, 0.52f, 0.f},
+                                    {-1, 32, 32, 0.151f, 0.45f, 0.f}, {-1, 16, 16, 0.079f, 0.24f, 0.f}};
 static const TileCost kCostLines[] = {{0, 256, 256, 1.75f, 8.f, 0.f}, {1, 128, 128, 0.55f, 3.5f, 1.05f}, {2, 64, 64, 0.22f, 0.8f, 0.25f},
                                       {-1, 64, 64, 0.22f, 1.5f, 0.f}, {-1, 64, 32, 0.17f, 0.8f, 0.f}, {-1, 32, 32, 0.09f, 0.5f, 0.f},
                                       {-1, 16, 16, 0.05f, 0.3f, 0.f}};
@@ -1022,7 +1023,8 @@ static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, lo
         if (c.cfg < 0 && (!may_split || K * es > kWaveMaxRowBytes || M > 2147483000l || N > 2147483000l)) return;
         const double tiles = (double)((M + c.bm - 1) / c.bm) * (double)((N + c.bn - 1) / c.bn) * (double)batch;
         if (c.cfg < 0 && tiles >= 4294967296.0) return;     // the split form numbers the tiles of a whole batch in 32 bits
-        const float n = (float)((tiles + cus - 1) / cus >= 1e9 ? 1e9 : (double)(long)((tiles + cus - 1) / cus));
+        const float rounds = (float)((tiles + cus - 1) / cus >= 1e9 ? 1e9 : (double)(long)((tiles + cus - 1) / cus));
+        const float n = dtype_in == SP_F32 && tiles > cus ? 0.5f * (rounds + (float)(tiles / cus)) : rounds;
         const float per_k = n * c.tk > c.latency ? n * c.tk : c.latency;
         const float us = n * c.overhead + (float)nk * per_k;
         if (best == nullptr || us < best_us) {

@@ -62,6 +62,15 @@ def test_gemm_argument_errors(L):
     assert lib.sp_gemm_abt(*args(M=(1 << 31) + 1)) == -2
 
 
+@pytest.mark.parametrize("m,n,k,tile", [(11200, 1792, 32, 64), (2688, 5760, 64, 64), (2112, 1536, 96, 64), (7872, 448, 1888, 64),
+                                        (10688, 768, 3648, 128), (8192, 8192, 4096, 256)])
+def test_f32_tile_choice_by_the_length_of_k(L, m, n, k, tile):
+    """The tile that was measured to be the fastest, where the large ones do not pay for their prologue (256 units)."""
+    out = [C.c_int32() for _ in range(4)]
+    assert L.lib.sp_gemm_config(0, m, n, k, *[C.byref(o) for o in out]) == 0
+    assert [o.value for o in out[:2]] == [tile, tile]
+
+
 def test_a_batch_adds_up_like_a_launch_per_member(L):
     """Split-K or workgroup tiles is a matter of one member's shape, for f32 always, for 16-bit inputs unless the other kind
     is estimated to be a quarter faster (large batches).  Shapes around the edges of tiles, of the K rule and of the estimate."""
