@@ -950,6 +950,11 @@ static bool use_four_waves(int dtype_in, long N, long K) {
     return dtype_in != SP_F32 && K % 128 == 0 && K <= (1l << 22) && N >= 512;
 }
 
+// A launch holds fewer than 2^32 work items along x: tiles that small are not for outputs that tall (M = 1.2e9 rows of 16
+// columns are 18.75 million 64 x 64 tiles of 256 threads).  The 256 wide tiles hold every M x N that validate_gemm lets
+// through, but for the last 255 row counts below 2^31.
+static bool launch_holds(double tiles, int threads) { return tiles * threads < 4294967296.0; }
+
 // The counterpart of the reference's tile search (`frame` / `frame_iter`, ml/primitives.spi:17-33, as used by
 // matmul_config_tf32, ml/matmul/run.spi:8-19: tiles doubled from 16 x 16 under the shared-memory budget): a fixed menu
 // of three tiles.  Largest tile whose grid still fills the chip; otherwise the smallest tile that divides the shape.  "Fills" is 80 %
@@ -963,6 +968,7 @@ static int choose_cfg(int dtype_in, long M, long N, long K, long batch, long cus
     for (int i = 0; i < kNumCfgs; ++i) {
         const TileCfg& c = kTileCfgs[i];
         if (M % c.bm != 0 || N % c.bn != 0) continue;
+        if (i > 0 && !launch_holds((double)(M / c.bm) * (double)(N / c.bn), c.wm * c.wn * 64)) continue;
         smallest = i;
         const long tiles = (M / c.bm) * (N / c.bn) * batch;
         const bool four_waves = i == 0 && use_four_waves(dtype_in, N, K);
@@ -1021,7 +1027,9 @@ static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, lo
         if (whole == 0 || whole == 1 ? c.cfg != whole : whole == 2 && (c.cfg == 0 || c.cfg == 1)) return;
         if (c.cfg < 0 ? kind == TILE_WORKGROUP : kind == TILE_SPLIT) return;
         if (c.cfg < 0 && (!may_split || K * es > kWaveMaxRowBytes || M > 2147483000l || N > 2147483000l)) return;
-        const double tiles = (double)((M + c.bm - 1) / c.bm) * (double)((N + c.bn - 1) / c.bn) * (double)batch;
+        const double of_member = (double)((M + c.bm - 1) / c.bm) * (double)((N + c.bn - 1) / c.bn);
+        const double tiles = of_member * (double)batch;
+        if (c.cfg != 0 && !launch_holds(of_member, 256)) return;
         if (c.cfg < 0 && tiles >= 4294967296.0) return;     // the split form numbers the tiles of a whole batch in 32 bits
         const float rounds = (float)((tiles + cus - 1) / cus >= 1e9 ? 1e9 : (double)(long)((tiles + cus - 1) / cus));
         const float n = dtype_in == SP_F32 && tiles > cus ? 0.5f * (rounds + (float)(tiles / cus)) : rounds;

@@ -71,6 +71,21 @@ def test_f32_tile_choice_by_the_length_of_k(L, m, n, k, tile):
     assert [o.value for o in out[:2]] == [tile, tile]
 
 
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_tall_outputs_get_tiles_a_launch_can_number(L, dtype):
+    """HIP launches fewer than 2^32 work items along a dimension: outputs of a few columns and up to 2^31 - 256 rows are within the
+    limits of the entry point and must not be cut into tiles too small for that."""
+    for m in (1 << 20, 1 << 28, (1 << 30) - 64, 1 << 30, 1200000000, (1 << 31) - 256):
+        for n in (1, 4, 15, 16, 64, 128, 256):
+            for k in (8, 16, 64, 128, 512, 1000):
+                out = [C.c_int32() for _ in range(4)]
+                if ((m + 15) // 16) * ((n + 15) // 16) > (1 << 31) - 1:
+                    continue
+                assert L.lib.sp_gemm_config(dtype, m, n, k, *[C.byref(o) for o in out]) == 0
+                bm, bn, _, threads = [o.value for o in out]
+                assert -(-m // bm) * -(-n // bn) * threads < 1 << 32, (m, n, k, bm, bn, threads)
+
+
 def test_a_batch_adds_up_like_a_launch_per_member(L):
     """Split-K or workgroup tiles is a matter of one member's shape, for f32 always, for 16-bit inputs unless the other kind
     is estimated to be a quarter faster (large batches).  Shapes around the edges of tiles, of the K rule and of the estimate."""
