@@ -20,6 +20,7 @@ MAP_OUT_IDENTITY, MAP_OUT_SQRT = 0, 1
 STACK_LN_L2 = 0x100
 HEAD_NONE, HEAD_SOFTMAX, HEAD_REGRET_MATCHING, HEAD_SOFTMAX_RM = 0, 1, 2, 3
 
+ERR_SHAPE, ERR_UNSUPPORTED = -2, -6
 ERROR_NAMES = {0: "SP_OK", -1: "SP_ERR_NULL", -2: "SP_ERR_SHAPE", -3: "SP_ERR_ALIGN", -4: "SP_ERR_DTYPE",
                -5: "SP_ERR_ARG", -6: "SP_ERR_UNSUPPORTED", -7: "SP_ERR_DEVICE"}
 

@@ -936,7 +936,6 @@ def _run_fused_ensemble(model, key, count, ls):
 _STACK_HEADS = {"softmax": _lib.ROW_SOFTMAX, "masked_softmax": _lib.ROW_MASKED_SOFTMAX,
                 "regret_matching": _lib.ROW_REGRET_MATCHING, "masked_regret_matching": _lib.ROW_MASKED_REGRET_MATCHING}
 _STACK_MAPS = {"copy": _lib.MAP_COPY, "relu": _lib.MAP_RELU, "tanh": _lib.MAP_TANH, "sigmoid": _lib.MAP_SIGMOID}
-_STACK_LDS = 144 * 1024          # bytes of weights sp_stack_forward_f32 keeps on chip
 
 
 def _stack_plan(model, key):
@@ -1011,14 +1010,12 @@ def _overlap(a, b):
 
 
 def _run_fused_stack(model, key, count, ls):
-    """One sp_stack_forward_f32 launch in place of a walk over the nodes, where the graph is of that shape, its widths are
-    ones the kernel takes and its weights fit on chip.  (The inner nodes' tensors are not written then.)"""
+    """One sp_stack_forward_f32 launch in place of a walk over the nodes, where the graph is of that shape and the entry point
+    takes its sizes (it says so itself, before anything is launched).  (The inner nodes' tensors are not written then.)"""
     plan = _stack_plan(model, key)
     if plan is None:
         return False
     x_node, w_nodes, acts, head, mask, out_nodes = plan
-    if len(w_nodes) > 8:
-        return False
     tensor = lambda node: graph_extract(Model(node, model.dims, model.data))
     x, ws = tensor(x_node), [tensor(w) for w in w_nodes]
     outs = graph_extract(model) if out_nodes is None else tuple(tensor(o) for o in out_nodes)
@@ -1030,30 +1027,28 @@ def _run_fused_stack(model, key, count, ls):
         return False
     q, w, k0 = x.shape
     dims = [k0] + [t.shape[-2] for t in ws]
-    cols, computed = dims[-1], mask or dims[-1]
-    if any(t.shape[-1] != d for t, d in zip(ws, dims)):
-        return False
-    if dims[0] % 4 or dims[0] > 128 or any(d % 16 or d > 128 for d in dims[1:-1]) or cols % 4 or cols > 64 or mask > cols:
-        return False
-    blocks = [(d + 15) // 16 for d in dims[:-1]] + [(computed + 15) // 16]
-    if 1024 * builtins.sum(i * o for i, o in zip(blocks[:-1], blocks[1:])) > _STACK_LDS or count * q * w >= (1 << 31) - (1 << 21):
+    cols = dims[-1]
+    if any(t.shape[-1] != d for t, d in zip(ws, dims)) or cols % 4:
         return False
     if outs[0].shape != lead + (q, w, cols) or (len(outs) == 2 and (outs[1].shape != lead + (q, w) or outs[1].dtype != torch.int32)):
         return False
     if any(_overlap(o, t) for o in outs for t in [x] + ws) or (len(outs) == 2 and _overlap(*outs)):
         return False          # node by node, an output may take the place of what has been read
-    rng = None
+    rng, draws = None, 0
     if len(outs) == 2:
         draws = _sampling_draws(w, cols)
         rng = _prim.philox(_lib.PHILOX_LAYER, seed=ls.seed, threads_per_block=THREADS_PER_BLOCK, blocks_per_grid=q,
                            rows_per_block=w, offset=ls.draws, member_rows=q * w if key is not None else 0, member_draws=draws)
-        ls.draws += draws
     n = len(ws)
-    check(lib.sp_stack_forward_f32(
+    rc = lib.sp_stack_forward_f32(
         ptr(x, name="x"), n, (C.c_void_p * n)(*[ptr(t, name="weights[%d]" % i) for i, t in enumerate(ws)]),
         (C.c_int32 * (n + 1))(*dims), (C.c_int32 * n)(*acts), count, None, C.byref(rng) if rng is not None else None,
         ptr(outs[0], name="policy"), ptr(outs[1], name="action") if len(outs) == 2 else None, q * w, _STACK_HEADS[head], mask,
-        stream_ptr()))
+        stream_ptr())
+    if rc in (_lib.ERR_SHAPE, _lib.ERR_UNSUPPORTED):
+        return False
+    check(rc)
+    ls.draws += draws
     return True
 
 

@@ -161,3 +161,31 @@ def test_stack_plan_takes_whole_chains_only():
     swapped = L.pipe(inp(), L.matmul((64, 64)), L.relu, L.ln_l2, L.matmul((64, 64)), L.softmax_and_discrete_sample)   # norm behind the map
     first = L.pipe(inp(), L.relu, L.matmul((64, 64)), L.softmax_and_discrete_sample)                                    # a map of the input
     assert [plan(g) for g in (named, kept, swapped, first)] == [None] * 4
+
+
+def test_a_stack_the_entry_point_refuses_runs_node_by_node(monkeypatch):
+    """Which sizes run as one launch is sp_stack_forward_f32's own answer: refused sizes fall back to the walk and leave the
+    generator where it was, every other error is raised."""
+    g = L.pipe(L.input("input", (24, 64, 64)), L.matmul((64, 64)), L.relu, L.matmul((64, 16)), L.softmax_and_discrete_sample)
+    model, answer, calls = L.create_model(g, device="cpu"), [0], []
+
+    class Refusing:
+        def sp_stack_forward_f32(self, *args):
+            calls.append(args)
+            return answer[0]
+
+    monkeypatch.setattr(L, "lib", Refusing())
+    monkeypatch.setattr(L, "ptr", lambda t, dtype=None, name="": None if t is None else t.data_ptr())
+    monkeypatch.setattr(L, "stream_ptr", lambda: None)
+    ls = L.create_layer_state()
+    for answer[0] in (-2, -6):
+        assert L._run_fused_stack(model, None, 1, ls) is False and ls.draws == 0
+    answer[0] = -5
+    with pytest.raises(L._lib.SpiralError):
+        L._run_fused_stack(model, None, 1, ls)
+    answer[0] = 0
+    assert L._run_fused_stack(model, None, 1, ls) is True and ls.draws > 0 and len(calls) == 4
+    # sizes that no kernel takes are asked about all the same: the limits stand in one place
+    wide = L.create_model(L.pipe(L.input("input", (24, 64, 64)), L.matmul((64, 256)), L.relu, L.matmul((256, 16)), L.softmax), device="cpu")
+    answer[0] = -2
+    assert L._run_fused_stack(wide, None, 1, ls) is False and len(calls) == 5
