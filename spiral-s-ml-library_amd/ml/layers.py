@@ -508,6 +508,7 @@ class LayerState:
 
     def __init__(self, seed=_prim.CONSTANT_SEED):
         self.seed, self.draws = seed, 0
+        self.not_written = frozenset()      # nodes of the model that the run left out (a fused stack)
 
     def rng(self, q, w, cols):
         cfg = _prim.philox(_lib.PHILOX_LAYER, seed=self.seed, threads_per_block=THREADS_PER_BLOCK, blocks_per_grid=q,
@@ -542,6 +543,8 @@ def graph_extract_(layer_state, model, indices):
     views = cached[1]
 
     def extract_current(node):
+        if layer_state is None and not isinstance(node, Layer):
+            _looked_up(model, node)
         v = views.get(node)
         if v is not None:
             return v
@@ -622,6 +625,18 @@ def graph_extract_(layer_state, model, indices):
         raise TypeError("unknown graph node %r" % (graph,))
 
     return loop(model.graph)
+
+
+def _looked_up(model, node):
+    """The caller is handed the tensor of a computed node.  A fused stack leaves the nodes in its middle out; those that
+    somebody has looked at are written by every run from then on (the stack then runs node by node), and one that is looked
+    at for the first time behind a fused run is computed here, from what the arenas hold."""
+    arena = model.data[workspace_id()]
+    seen = arena.setdefault("looked_up", set())
+    if node not in seen:
+        seen.add(node)
+        if node in arena.get("not_written", ()):
+            graph_run(Model(node, model.dims, model.data), create_layer_state(), {})
 
 
 def graph_extract(model, indices=None):
@@ -941,8 +956,8 @@ _STACK_MAPS = {"copy": _lib.MAP_COPY, "relu": _lib.MAP_RELU, "tanh": _lib.MAP_TA
 def _stack_plan(model, key):
     """`input -> matmul [-> ln_l2] [-> map] -> ... -> matmul -> row head`, the graphs of ml/layers.spi test3 - test5
     (:564-665), with every weight and output of one member (key None) or stacked under `apply key`:
-    (x node, [weight nodes], [activation codes], head name, mask size, output node or None) or None.  A node in the middle
-    that has a name (`key_graph`) or an output tensor of its own is one the caller can look at: such a graph is not taken."""
+    (x node, [weight nodes], [activation codes], head name, mask size, output node or None, nodes in the middle) or None.  A
+    node in the middle that has a name (`key_graph`) or an output tensor of its own is one to be looked at: not taken."""
     top = model.graph
     sampling = isinstance(top, BlockRowMapReduce)
     if not isinstance(top, (BlockRowMap, BlockRowMapReduce)):
@@ -971,16 +986,19 @@ def _stack_plan(model, key):
             return tensor_node(k)
         return tensor_node(k.a) if isinstance(k, Apply) and isinstance(k.b, KeyScalar) and k.b.key == key else None
 
-    weights, acts, node = [], [], top.a
+    weights, acts, middle, node = [], [], set(), top.a
     while isinstance(node, BlockMatmul):
         w = member(node.b)
         if w is None:
             return None
         weights.insert(0, w)
+        middle.add(node)
         node, act = node.a, 0
         if isinstance(node, BlockMap) and node.out is None and node.f in _STACK_MAPS:
+            middle.add(node)
             node, act = node.a, _STACK_MAPS[node.f]
         if isinstance(node, BlockRowMap) and node.out is None and node.f == "ln_l2":
+            middle.add(node)
             node, act = node.a, act | _lib.STACK_LN_L2
         if not isinstance(node, BlockMatmul):
             if act:
@@ -1001,7 +1019,7 @@ def _stack_plan(model, key):
         outs = (member(out),)
     if outs is not None and (not outs or any(o is None for o in outs)):
         return None
-    return x, weights, acts + [0], head, top.size, outs
+    return x, weights, acts + [0], head, top.size, outs, middle
 
 
 def _overlap(a, b):
@@ -1011,11 +1029,16 @@ def _overlap(a, b):
 
 def _run_fused_stack(model, key, count, ls):
     """One sp_stack_forward_f32 launch in place of a walk over the nodes, where the graph is of that shape and the entry point
-    takes its sizes (it says so itself, before anything is launched).  (The inner nodes' tensors are not written then.)"""
+    takes its sizes (it says so itself, before anything is launched).  The tensors of the nodes in the middle are not written
+    then, so a model whose caller has looked at one of them is not taken.  (A batched pass has none: its nodes are temporaries.)"""
     plan = _stack_plan(model, key)
     if plan is None:
         return False
-    x_node, w_nodes, acts, head, mask, out_nodes = plan
+    x_node, w_nodes, acts, head, mask, out_nodes, middle = plan
+    arena = model.data[workspace_id()]
+    if key is None and not middle.isdisjoint(arena.get("looked_up", ())):
+        arena.get("not_written", set()).difference_update(middle)      # the walk writes them
+        return False
     tensor = lambda node: graph_extract(Model(node, model.dims, model.data))
     x, ws = tensor(x_node), [tensor(w) for w in w_nodes]
     outs = graph_extract(model) if out_nodes is None else tuple(tensor(o) for o in out_nodes)
@@ -1049,6 +1072,9 @@ def _run_fused_stack(model, key, count, ls):
         return False
     check(rc)
     ls.draws += draws
+    if key is None:
+        ls.not_written = frozenset(middle)
+        arena.setdefault("not_written", set()).update(middle)
     return True
 
 
@@ -1183,7 +1209,9 @@ def graph_run_host(model, sizes=None, seed=_prim.CONSTANT_SEED, fuse=True, batch
     one key that only indexes leading dimensions runs as a single batched pass (`batched=False` keeps the
     member-by-member loop): node by node the two are bit-identical in f32, in 16 bit equal to the rounding of the
     sums.  A dense stack under a row head runs as one launch, whose f32 sums
-    add up in another order and which does not write the unnamed nodes in the middle; `fuse=False` runs node by node.  `static_weights=True` says that the weights have not
+    add up in another order and which writes the nodes in the middle only if they are looked at: by name (`key_graph`), or
+    with `graph_extract` on the node, before or after the run (before it is captured into a graph, if it is);
+    `fuse=False` runs node by node.  `static_weights=True` says that the weights have not
     changed since the previous such run (or since `weights_changed(model)`): a fused relu-MLP then keeps a copy
     of them packed for the faster kernel instead of reading the arena on every run."""
     if fuse and not sizes:
@@ -1220,31 +1248,32 @@ def graph_run_host(model, sizes=None, seed=_prim.CONSTANT_SEED, fuse=True, batch
     tape_key = (seed, fuse, batched, tuple(sorted(sizes.items())))
     entry = tapes.get(tape_key)
     data = model.data
-    if entry is not None and len(entry[0]) == len(data) and all(a is d["array"] for a, d in zip(entry[0], data)):
+    if entry is not None and len(entry[0]) == len(data) and all(a is d["array"] for a, d in zip(entry[0], data)) and \
+            entry[2].isdisjoint(data[workspace_id()].get("looked_up", ())):
         entry[1].replay()
         return
     tape = _lib.start_tape()
     try:
-        _graph_run_walk(model, sizes, seed, batched, fuse)
+        not_written = _graph_run_walk(model, sizes, seed, batched, fuse)
     finally:
         _lib.stop_tape()
-    tapes[tape_key] = (tuple(d["array"] for d in data), tape)
+    tapes[tape_key] = (tuple(d["array"] for d in data), tape, not_written)
 
 
 def _graph_run_walk(model, sizes, seed, batched, fuse=True):
     """One run by walking the graph: a single batched pass over one key where that is possible (a single fused launch
-    where the graph is a two-layer relu stack per member), else every combination of the key indices in turn."""
+    where the graph is a two-layer relu stack per member), else every combination of the key indices in turn.  Returns the
+    nodes whose tensors it left out."""
     ls = create_layer_state(seed)
     key = _batchable_key(model, sizes) if batched and sizes else None
     if key is not None and sizes[key] > 1:
         if not (fuse and (_run_fused_ensemble(model, key, sizes[key], ls) or _run_fused_stack(model, key, sizes[key], ls))):
             _graph_run_batched(model, key, sizes[key], ls)
-        return
-    if fuse and not sizes and _run_fused_stack(model, None, 1, ls):
-        return
-    keys = list(sizes)
-    for combo in itertools.product(*[range(sizes[k]) for k in keys]):
-        graph_run_device(model, ls, dict(zip(keys, combo)))
+    elif not (fuse and not sizes and _run_fused_stack(model, None, 1, ls)):
+        keys = list(sizes)
+        for combo in itertools.product(*[range(sizes[k]) for k in keys]):
+            graph_run_device(model, ls, dict(zip(keys, combo)))
+    return ls.not_written
 
 
 # ---- node constructors (ml/layers.spi:346-484) ------------------------------------------------

@@ -377,6 +377,36 @@ def test_dense_stack_runs_as_one_launch(L, rows, widths, act, ensemble, head):
     assert [c[0].__name__ for c in tape.calls] == ["sp_stack_forward_f32"]
 
 
+@pytest.mark.parametrize("look", ["before", "behind"])
+def test_nodes_in_the_middle_of_a_stack_hold_their_values_when_looked_at(L, look):
+    """A caller that keeps an inner node and reads it gets what the last run computed, whether it looked the node up before
+    the run or behind it, and again after the inputs have changed."""
+    announce("layers dense stack, inner nodes looked up %s the run" % look)
+    x = L.input("input", (Q, 5, 64))
+    product = L.matmul((64, 32), x)
+    hidden = L.relu(L.ln_l2(product))
+    logits = L.matmul((32, 16), hidden)
+    m = L.create_model(L.softmax_and_discrete_sample(logits))
+    node = lambda n: L.graph_extract(L.Model(n, m.dims, m.data))
+    inner = [product, hidden.a, hidden, logits]
+    rng = np.random.default_rng(5)
+    views = [node(n) for n in inner] if look == "before" else None
+    for t in [L.key_extract(m, "input")] + [t for _, t, _ in L.extract_layers_(m, L.weight_id())]:
+        fill(t, rng, 0.3)
+    for turn in range(3):
+        xh = fill(L.key_extract(m, "input"), rng)
+        for t in views or []:
+            t.fill_(7)
+        L.graph_run_host(m)
+        views = views or [node(n) for n in inner]
+        ws = [host(t) for _, t, _ in L.extract_layers_(m, L.weight_id())]
+        p = xh.reshape(-1, 64).astype(np.float64) @ ws[0].T.astype(np.float64)
+        n2 = p / (p * p).sum(axis=1, keepdims=True)
+        r = np.maximum(n2, 0)
+        for t, want in zip(views, (p, n2, r, r @ ws[1].T.astype(np.float64))):
+            assert ogemm.rel_frobenius(host(t).reshape(want.shape), want) < 1e-5, turn
+
+
 @pytest.mark.parametrize("sampling", [False, True])
 def test_leduc_policy_graph_runs_as_one_launch(L, sampling):
     """The graph of the reference's Leduc policy (game/leduc/model_cem.spi:55-63: input -> matmul_ensemble_with_adjoint

@@ -152,8 +152,8 @@ def test_ensemble_with_adjoint_places_the_dual_in_the_adjoint_arena():
 def test_stack_plan_takes_whole_chains_only():
     """The graphs that run as one launch of the f32 stack kernel: a chain whose inner nodes nobody can look at."""
     plan = lambda g, key=None: L._stack_plan(L.Model(g, {}, []), key)
-    x, ws, acts, head, mask, outs = plan(graph_of_test3())
-    assert len(ws) == 3 and head == "softmax" and mask == 0 and outs is None and acts[0] == acts[1] != 0 and acts[2] == 0
+    x, ws, acts, head, mask, outs, middle = plan(graph_of_test3())
+    assert len(ws) == 3 and head == "softmax" and mask == 0 and outs is None and acts[0] == acts[1] != 0 and acts[2] == 0 and len(middle) == 7
     assert plan(ensemble_graph(4, True), "ensemble")[5] is not None and plan(ensemble_graph(4, True)) is None
     inp = lambda: L.input("input", (24, 64, 64))
     named = L.pipe(L.key_graph("hidden", L.pipe(inp(), L.matmul((64, 64)))), L.relu, L.matmul((64, 64)), L.softmax_and_discrete_sample)
@@ -189,3 +189,45 @@ def test_a_stack_the_entry_point_refuses_runs_node_by_node(monkeypatch):
     wide = L.create_model(L.pipe(L.input("input", (24, 64, 64)), L.matmul((64, 256)), L.relu, L.matmul((256, 16)), L.softmax), device="cpu")
     answer[0] = -2
     assert L._run_fused_stack(wide, None, 1, ls) is False and len(calls) == 5
+
+
+def test_a_node_somebody_looks_at_is_written(monkeypatch):
+    """A fused stack leaves the tensors in its middle out.  Looked up before the run, such a node keeps the model on the walk;
+    looked up behind a fused run for the first time, it is computed then, and the recorded launch is not replayed any more."""
+    calls, walked = [], []
+
+    class Taking:
+        def sp_stack_forward_f32(self, *args):
+            calls.append(args)
+            return 0
+
+    monkeypatch.setattr(L, "lib", Taking())
+    monkeypatch.setattr(L, "ptr", lambda t, dtype=None, name="": None if t is None else t.data_ptr())
+    monkeypatch.setattr(L, "stream_ptr", lambda: None)
+    monkeypatch.setattr(L._lib, "stream_ptr", lambda: None)
+    monkeypatch.setattr(L, "graph_run", lambda model, ls, indices: walked.append(model.graph))
+    hidden = L.pipe(L.input("input", (24, 64, 64)), L.matmul((64, 64)), L.relu)
+    build = lambda: L.create_model(L.pipe(hidden, L.matmul((64, 16)), L.softmax), device="cpu")
+    run = lambda m: L.graph_run_host(m)
+    look = lambda m: L.graph_extract(L.Model(hidden, m.dims, m.data))
+
+    first = build()
+    look(first)
+    run(first)
+    assert walked == [first.graph] and not calls
+
+    then = build()
+    run(then)
+    assert len(calls) == 1 and len(walked) == 1                 # one launch, nothing computed besides
+    L.graph_extract(then)                                       # the result: always written
+    L.key_extract(then, "input")
+    assert len(walked) == 1
+    look(then)
+    assert walked[1] is hidden                                  # computed for the first look
+    look(then)
+    run(then)
+    run(then)
+    assert len(calls) == 1 and walked[2] is then.graph and hidden not in walked[2:]
+    other = build()
+    run(other)
+    assert len(calls) == 2                                      # another model of the same graph is not concerned
