@@ -1,0 +1,142 @@
+"""sp_stack_forward_f32 on the launch shapes a graph of ordinary size does not reach: several tiles per wave (inputs read
+ahead, one draw for four tiles, the scratch used again), eight waves a workgroup, every instance of the kernel, uniforms given or
+drawn.  Probabilities against float64 (f32 sums of up to 128 terms in up to three layers and an exponential to 1e-6: 1e-5 in the
+Frobenius norm); sampled indices bit for bit given the kernel's own probabilities and the uniforms."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import philox as ophilox, row_ops as orow
+from gpu_util import announce, dev, host
+
+pytestmark = pytest.mark.gpu
+
+ACT = {"copy": 0, "relu": 1, "tanh": 2, "sigmoid": 3}
+LN = 0x100
+
+
+@pytest.fixture(scope="module")
+def S():
+    from ml import _lib
+    return _lib
+
+
+def forward(S, x, ws, acts, head, mask=0, u=None, rng=None, sample=True):
+    members, rows, n = ws[0].shape[0], x.shape[0], ws[-1].shape[1]
+    policy = torch.full((members, rows, n), 7.0, device="cuda")
+    action = torch.full((members, rows), -7, dtype=torch.int32, device="cuda") if sample else None
+    k, dims = len(ws), [x.shape[1]] + [w.shape[1] for w in ws]
+    codes = [sum(ACT.get(part, LN) for part in act.split("+")) for act in acts] + [0]
+    S.check(S.lib.sp_stack_forward_f32(S.ptr(x), k, (C.c_void_p * k)(*[S.ptr(w) for w in ws]), (C.c_int32 * (k + 1))(*dims),
+                                       (C.c_int32 * k)(*codes), members, S.ptr(u), C.byref(rng) if rng is not None else None,
+                                       S.ptr(policy), S.ptr(action), rows, head, mask, S.stream_ptr()))
+    return policy, action
+
+
+def probabilities(x, ws, acts, regret, mask):
+    """In float64, a member at a time."""
+    out = []
+    for e in range(ws[0].shape[0]):
+        h = x.double()
+        for w, act in zip(ws, acts + [""]):
+            h = h @ w[e].double().T
+            for part in [p for p in act.split("+") if p]:
+                if part == "ln":
+                    s = (h * h).sum(-1, keepdim=True)
+                    h = torch.where(s != 0, h / s, torch.zeros_like(h))
+                else:
+                    h = {"copy": lambda t: t, "relu": torch.relu, "tanh": torch.tanh, "sigmoid": torch.sigmoid}[part](h)
+        valid = torch.arange(h.shape[-1], device=h.device) < (mask or h.shape[-1])
+        if regret:
+            p = torch.where(valid, torch.relu(h), torch.zeros_like(h))
+            s = p.sum(-1, keepdim=True)
+            p = torch.where(s != 0, p / s, valid.double() / valid.sum())
+        else:
+            p = torch.softmax(torch.where(valid, h, torch.full_like(h, -np.inf)), -1)
+        out.append(p)
+    return torch.stack(out)
+
+
+def make(rng, members, rows, widths, scale=0.3):
+    x = dev(rng.standard_normal((rows, widths[0]), dtype=np.float32))
+    return x, [dev(rng.standard_normal((members, o, i), dtype=np.float32) * np.float32(scale / np.sqrt(i / 16)))
+               for i, o in zip(widths[:-1], widths[1:])]
+
+
+def check(S, x, ws, acts, head, mask, u, rng):
+    """u: (members * rows,) uniforms the run is to use, given as they are (rng None) or drawn on the device."""
+    members, rows, n = ws[0].shape[0], x.shape[0], ws[-1].shape[1]
+    policy, action = forward(S, x, ws, acts, head, mask, dev(u) if rng is None else None, rng)
+    want = probabilities(x, ws, acts, head in (S.ROW_REGRET_MATCHING, S.ROW_MASKED_REGRET_MATCHING), mask)
+    assert float((policy.double() - want).norm() / want.norm()) < 1e-5
+    p, a = host(policy).reshape(-1, n), host(action).reshape(-1)
+    assert (p[:, mask or n:] == 0).all()
+    assert (a == orow.discrete_sampling(p, u, order="wave")).all()
+    again, none = forward(S, x, ws, acts, head, mask, sample=False)
+    assert torch.equal(again, policy) and none is None
+
+
+def uniforms(rng, n):
+    return (1 - rng.random(n, dtype=np.float32)).astype(np.float32)
+
+
+# 64 wide stacks: 512 workgroups of eight waves, 16 rows a wave and turn; 128 wide ones: 256 workgroups
+@pytest.mark.parametrize("members,rows,widths,acts,head,mask", [
+    (1, 5 * 65536 + 37, (64, 64, 64, 64), "ln+relu", "ROW_SOFTMAX", 0),                 # six turns, the last tile of five rows
+    (3, 8 * 21888 + 3, (64, 64, 16), "relu", "ROW_SOFTMAX", 0),                         # nine turns a member: two refills of the draws
+    (16, 16384, (64, 64, 64, 64), "ln+relu", "ROW_MASKED_SOFTMAX", 17),                 # eight waves, two tiles a wave
+    (1, 5 * 32768 + 9, (128, 128, 64), "ln+tanh", "ROW_SOFTMAX", 0),                    # full_product of 128 x 128 and 128 x 64
+    (2, 40000, (128, 128, 64), "sigmoid", "ROW_REGRET_MATCHING", 0),
+    (5, 33000, (36, 48, 96, 24), "relu", "ROW_SOFTMAX", 0)])                            # narrow layers, several turns
+def test_many_tiles_per_wave(S, members, rows, widths, acts, head, mask):
+    announce("stack, many tiles: %d x %d rows %s %s" % (members, rows, widths, head))
+    rng = np.random.default_rng(rows)
+    x, ws = make(rng, members, rows, widths)
+    check(S, x, ws, [acts] * (len(widths) - 2), getattr(S, head), mask, uniforms(rng, members * rows), None)
+
+
+@pytest.mark.parametrize("widths,head,mask", [
+    ((64, 64, 64, 64), "ROW_SOFTMAX", 0), ((52, 64, 64), "ROW_REGRET_MATCHING", 0),      # full, the second with a part of a K-block
+    ((64, 64, 20), "ROW_MASKED_REGRET_MATCHING", 9), ((4, 16, 4), "ROW_SOFTMAX", 0),     # a narrow head behind full layers; not full
+    ((128, 128, 64), "ROW_MASKED_SOFTMAX", 64), ((116, 128, 48), "ROW_REGRET_MATCHING", 0), ((128, 64), "ROW_SOFTMAX", 0),
+    ((100, 32, 128, 40), "ROW_MASKED_SOFTMAX", 33), ((128, 16, 16, 16, 16, 16, 16, 16, 8), "ROW_SOFTMAX", 0)])
+@pytest.mark.parametrize("rows", [1, 16, 47])
+def test_every_instance(S, rows, widths, head, mask):
+    announce("stack instance %s %s rows=%d" % (widths, head, rows))
+    rng = np.random.default_rng(rows + widths[0])
+    x, ws = make(rng, 3, rows, widths)
+    check(S, x, ws, ["ln+relu", "tanh", "copy", "ln+sigmoid", "ln+copy", "sigmoid", "relu"][:len(widths) - 2], getattr(S, head), mask,
+          uniforms(rng, 3 * rows), None)
+
+
+@pytest.mark.parametrize("members,blocks,rows_per_block,widths", [(3, 24, 9101, (64, 64, 64)), (2, 7, 5, (128, 128, 16)), (1, 24, 13655, (32, 64, 8))])
+def test_uniforms_drawn_on_the_device(S, members, blocks, rows_per_block, widths):
+    """A run per member (member_rows), later in the stream each, and one run over all members' rows."""
+    from ml import primitives as P
+    rows, n = blocks * rows_per_block, widths[-1]
+    announce("stack draws: %d x %d rows %s" % (members, rows, widths))
+    rng = np.random.default_rng(rows)
+    x, ws = make(rng, members, rows, widths)
+    draws = ophilox.draws_per_sampling_node(rows_per_block, n)
+    layer = P.philox(S.PHILOX_LAYER, blocks_per_grid=blocks, rows_per_block=rows_per_block, offset=4, member_rows=rows, member_draws=draws)
+    u = np.concatenate([ophilox.row_uniforms_layer(blocks, rows_per_block, n, offset=4 + e * draws) for e in range(members)])
+    check(S, x, ws, ["relu"] * (len(widths) - 2), S.ROW_SOFTMAX, 0, u, layer)
+    grid = P.philox(S.PHILOX_GRID, blocks_per_grid=24)
+    check(S, x, ws, ["relu"] * (len(widths) - 2), S.ROW_SOFTMAX, 0, ophilox.row_uniforms_grid(members * rows, n), grid)
+
+
+def test_rows_of_nan_and_infinity_stay_their_own(S):
+    announce("stack, NaN and infinite rows")
+    rng = np.random.default_rng(1)
+    x, ws = make(rng, 2, 100, (64, 64, 64, 16))
+    u = dev(uniforms(rng, 200))
+    clean, picks = forward(S, x, ws, ["ln+relu", "ln+relu"], S.ROW_SOFTMAX, 0, u)
+    bad = x.clone()
+    bad[17], bad[40, 3], bad[99] = float("nan"), float("inf"), float("-inf")
+    policy, action = forward(S, bad, ws, ["ln+copy", "ln+copy"], S.ROW_SOFTMAX, 0, u)
+    mixed, mixed_picks = forward(S, bad, ws, ["ln+relu", "ln+relu"], S.ROW_SOFTMAX, 0, u)
+    rest = [r for r in range(100) if r not in (17, 40, 99)]
+    assert torch.equal(mixed[:, rest], clean[:, rest]) and torch.equal(mixed_picks[:, rest], picks[:, rest])
+    assert bool(policy[:, [17, 40, 99]].isnan().all()) and bool((action[:, [17, 40, 99]] == 2147483647).all())
