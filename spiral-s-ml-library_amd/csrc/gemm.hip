@@ -957,13 +957,12 @@ static bool launch_holds(double tiles, int threads) { return tiles * threads < 4
 
 // The counterpart of the reference's tile search (`frame` / `frame_iter`, ml/primitives.spi:17-33, as used by
 // matmul_config_tf32, ml/matmul/run.spi:8-19: tiles doubled from 16 x 16 under the shared-memory budget): a fixed menu
-// of three tiles.  Largest tile whose grid still fills the chip; otherwise the smallest tile that divides the shape.  "Fills" is 80 %
+// of three tiles, for 16-bit inputs.  Largest tile whose grid still fills the chip; otherwise the smallest that divides the shape.  "Fills" is 80 %
 // of the compute units, except for the four-wave kernel, which does per unit so much more than the 128 x 128 tiles
 // that 9/16 of the units are enough (3072^3 bf16: 144 tiles of 256 x 256 take 56 us, 576 tiles of 128 x 128 76 us; at
 // 128 tiles the two are level, below that the smaller tiles win).
 static int choose_cfg(int dtype_in, long M, long N, long K, long batch, long cus) {
-    const int bk = dtype_in == SP_F32 ? 32 : 64;
-    if (K % bk != 0) return -1;
+    if (K % 64 != 0) return -1;
     int smallest = -1;
     for (int i = 0; i < kNumCfgs; ++i) {
         const TileCfg& c = kTileCfgs[i];

@@ -111,8 +111,9 @@ __device__ __forceinline__ void part_product(const unsigned char*& wp, const f32
     }
 }
 
-// HT: 16-wide tiles of the widest layer (4 or 8).  FULL: the input and every hidden layer have exactly that many.  OPK: 0 softmax, 1 masked softmax, 2 regret matching (mask_size columns).
-template <int HT, int OPK, bool FULL>
+// HT: 16-wide tiles of the widest layer (4 or 8).  FULL: the input and every hidden layer have exactly that many.  REGRET:
+// regret matching instead of softmax as the head (of mask_size columns, either).
+template <int HT, bool REGRET, bool FULL>
 __global__ __launch_bounds__(ST_MAX_THREADS, HT == 4 ? 4 : 2) void mlp_stack_kernel(const StackArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int lane = threadIdx.x & 63;
@@ -245,7 +246,7 @@ __global__ __launch_bounds__(ST_MAX_THREADS, HT == 4 ? 4 : 2) void mlp_stack_ker
                     if (4 * lq + k >= limit) v[k] = NEG_INF;
             }
             float p[4];
-            if constexpr (OPK == 2) {
+            if constexpr (REGRET) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k) p[k] = 4 * lq + k < limit ? fmaxf(v[k], 0.f) : 0.f;
                 const float s = group_reduce<16>(sum4(p), [](float m, float n) { return m + n; });
@@ -294,9 +295,8 @@ __global__ __launch_bounds__(ST_MAX_THREADS, HT == 4 ? 4 : 2) void mlp_stack_ker
 using namespace sp;
 
 template <int HT, bool FULL>
-static const void* pick_stack_kernel(int opk) {
-    return opk == 0 ? (const void*)mlp_stack_kernel<HT, 0, FULL> : opk == 1 ? (const void*)mlp_stack_kernel<HT, 1, FULL>
-                                                                            : (const void*)mlp_stack_kernel<HT, 2, FULL>;
+static const void* pick_stack_kernel(bool regret) {
+    return regret ? (const void*)mlp_stack_kernel<HT, true, FULL> : (const void*)mlp_stack_kernel<HT, false, FULL>;
 }
 
 // Bytes of LDS the weights take (dims[n_layers] = the computed outputs).
@@ -318,9 +318,8 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
     if (n_layers < 1 || n_layers > ST_MAX_LAYERS) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: 1 to %d layers, got %d", ST_MAX_LAYERS, n_layers);
     if (members <= 0 || members > 65535) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: members must be in [1, 65535]");
     if (batch <= 0 || batch >= (1ll << 31) / members - ST_ROWS) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: batch must be positive and members x batch below 2^31");
-    const int opk = head_op == SP_ROW_SOFTMAX ? 0 : head_op == SP_ROW_MASKED_SOFTMAX ? 1
-                  : head_op == SP_ROW_REGRET_MATCHING || head_op == SP_ROW_MASKED_REGRET_MATCHING ? 2 : -1;
-    if (opk < 0) return fail(SP_ERR_ARG, "sp_stack_forward_f32: unknown head %d", head_op);
+    const bool regret = head_op == SP_ROW_REGRET_MATCHING || head_op == SP_ROW_MASKED_REGRET_MATCHING;
+    if (!regret && head_op != SP_ROW_SOFTMAX && head_op != SP_ROW_MASKED_SOFTMAX) return fail(SP_ERR_ARG, "sp_stack_forward_f32: unknown head %d", head_op);
     if (action_out != nullptr && u == nullptr && philox == nullptr)
         return fail(SP_ERR_NULL, "sp_stack_forward_f32: action requested but u and philox are NULL");
     if (u != nullptr && philox != nullptr) return fail(SP_ERR_ARG, "sp_stack_forward_f32: at most one of u and philox may be given");
@@ -377,8 +376,8 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
     const int ht = widest <= 64 ? 4 : 8;
     bool full = true;
     for (int l = 0; l < n_layers; ++l) full = full && (dims[l] + 15) / 16 == ht;
-    const void* kernel = ht == 4 ? (full ? pick_stack_kernel<4, true>(opk) : pick_stack_kernel<4, false>(opk))
-                                 : (full ? pick_stack_kernel<8, true>(opk) : pick_stack_kernel<8, false>(opk));
+    const void* kernel = ht == 4 ? (full ? pick_stack_kernel<4, true>(regret) : pick_stack_kernel<4, false>(regret))
+                                 : (full ? pick_stack_kernel<8, true>(regret) : pick_stack_kernel<8, false>(regret));
     rc = ensure_dynamic_lds(kernel, ST_LDS);
     if (rc != SP_OK) return rc;
     void* args[] = {(void*)&a};
@@ -389,6 +388,6 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
 
 namespace {
 struct MlpStackKernelNames {
-    MlpStackKernelNames() { register_kernel("stack_forward_f32", (const void*)mlp_stack_kernel<4, 0, true>, ST_MAX_THREADS); }
+    MlpStackKernelNames() { register_kernel("stack_forward_f32", (const void*)mlp_stack_kernel<4, false, true>, ST_MAX_THREADS); }
 } mlp_stack_kernel_names;
 }  // namespace
