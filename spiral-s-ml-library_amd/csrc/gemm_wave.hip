@@ -262,4 +262,21 @@ int launch_gemm_wave(int dtype_in, int tile_m, int tile_n, long cus, const GemmA
     }
 }
 
+namespace {
+struct GemmWaveKernelNames {
+    GemmWaveKernelNames() {
+        register_kernel("gemm_f32_split_16x16", (const void*)gemm_wave_kernel<SP_F32, 1, 1, 4>, 256);
+        register_kernel("gemm_f32_split_32x32", (const void*)gemm_wave_kernel<SP_F32, 2, 2, 2>, 256);
+        register_kernel("gemm_f32_split_32x32_1", (const void*)gemm_wave_kernel<SP_F32, 2, 2, 1>, 256);
+        register_kernel("gemm_bf16_split_16x16", (const void*)gemm_wave_kernel<SP_BF16, 1, 1, 4>, 256);
+        register_kernel("gemm_bf16_split_32x32", (const void*)gemm_wave_kernel<SP_BF16, 2, 2, 2>, 256);
+        register_kernel("gemm_bf16_split_32x32_1", (const void*)gemm_wave_kernel<SP_BF16, 2, 2, 1>, 256);
+        register_kernel("gemm_bf16_split_64x32", (const void*)gemm_wave_kernel<SP_BF16, 4, 2, 3>, 256);
+        register_kernel("gemm_bf16_split_64x32_1", (const void*)gemm_wave_kernel<SP_BF16, 4, 2, 1>, 256);
+        register_kernel("gemm_bf16_split_64x64", (const void*)gemm_wave_kernel<SP_BF16, 4, 4, 2>, 256);
+        register_kernel("gemm_bf16_split_64x64_1", (const void*)gemm_wave_kernel<SP_BF16, 4, 4, 1>, 256);
+    }
+} gemm_wave_kernel_names;
+}  // namespace
+
 }  // namespace sp

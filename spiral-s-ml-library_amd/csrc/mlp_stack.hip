@@ -388,6 +388,15 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
 
 namespace {
 struct MlpStackKernelNames {
-    MlpStackKernelNames() { register_kernel("stack_forward_f32", (const void*)mlp_stack_kernel<4, false, true>, ST_MAX_THREADS); }
+    MlpStackKernelNames() {
+        register_kernel("stack_forward_f32", (const void*)mlp_stack_kernel<4, false, true>, ST_MAX_THREADS);
+        register_kernel("stack_forward_f32_regret", (const void*)mlp_stack_kernel<4, true, true>, ST_MAX_THREADS);
+        register_kernel("stack_forward_f32_part", (const void*)mlp_stack_kernel<4, false, false>, ST_MAX_THREADS);
+        register_kernel("stack_forward_f32_part_regret", (const void*)mlp_stack_kernel<4, true, false>, ST_MAX_THREADS);
+        register_kernel("stack_forward_f32_128", (const void*)mlp_stack_kernel<8, false, true>, ST_MAX_THREADS);
+        register_kernel("stack_forward_f32_128_regret", (const void*)mlp_stack_kernel<8, true, true>, ST_MAX_THREADS);
+        register_kernel("stack_forward_f32_128_part", (const void*)mlp_stack_kernel<8, false, false>, ST_MAX_THREADS);
+        register_kernel("stack_forward_f32_128_part_regret", (const void*)mlp_stack_kernel<8, true, false>, ST_MAX_THREADS);
+    }
 } mlp_stack_kernel_names;
 }  // namespace

@@ -466,6 +466,17 @@ def test_device_and_kernel_info():
         _lib.kernel_info("no_such_kernel")
 
 
+@pytest.mark.parametrize("name,threads", [("stack_forward_f32" + part, 512) for part in (
+    "", "_regret", "_part", "_part_regret", "_128", "_128_regret", "_128_part", "_128_part_regret")] + [
+    ("gemm_" + part, 256) for part in ("f32_split_16x16", "f32_split_32x32", "f32_split_32x32_1", "bf16_split_16x16", "bf16_split_32x32",
+                                       "bf16_split_32x32_1", "bf16_split_64x32", "bf16_split_64x32_1", "bf16_split_64x64", "bf16_split_64x64_1")])
+def test_every_instance_of_the_split_and_stack_kernels_is_named(name, threads):
+    announce("kernel info " + name)
+    from ml import _lib
+    info = _lib.kernel_info(name)
+    assert info["threads_per_block"] == threads and 0 < info["vgprs"] <= (256 if threads == 512 else 512)
+
+
 def test_clock_sample_gives_the_shader_clock():
     """Two sp_clock_sample results around a stretch of work: per SIMD sampled both times the cycle counter's advance
     over the 100 MHz counter's is the shader clock; the SIMDs of the chip agree on it, and it lies in the part's range."""
