@@ -314,7 +314,7 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
     SP_REQUIRE_PTR(x);
     SP_REQUIRE_PTR(policy_out);
     SP_OPTIONAL_PTR(u); SP_OPTIONAL_PTR(action_out);
-    if (weights == nullptr || dims == nullptr || acts == nullptr) return fail(SP_ERR_NULL, "sp_stack_forward_f32: weights/dims/acts is NULL");
+    if (weights == nullptr || dims == nullptr || (acts == nullptr && n_layers != 1)) return fail(SP_ERR_NULL, "sp_stack_forward_f32: weights/dims/acts is NULL");
     if (n_layers < 1 || n_layers > ST_MAX_LAYERS) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: 1 to %d layers, got %d", ST_MAX_LAYERS, n_layers);
     if (members <= 0 || members > 65535) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: members must be in [1, 65535]");
     if (batch <= 0 || batch >= (1ll << 31) / members - ST_ROWS) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: batch must be positive and members x batch below 2^31");
@@ -338,11 +338,13 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
     for (int l = 0; l < n_layers; ++l) {
         if (weights[l] == nullptr) return fail(SP_ERR_NULL, "sp_stack_forward_f32: weights[%d] is NULL", l);
         if (!aligned16(weights[l])) return fail(SP_ERR_ALIGN, "sp_stack_forward_f32: weights[%d] is not 16-byte aligned", l);
-        const int map = acts[l] & ~SP_STACK_LN_L2;
-        if (map != SP_MAP_COPY && map != SP_MAP_RELU && map != SP_MAP_TANH && map != SP_MAP_SIGMOID)
-            return fail(SP_ERR_ARG, "sp_stack_forward_f32: unknown activation %d of layer %d", acts[l], l);
+        if (l + 1 < n_layers) {                            // (behind the last layer stands the head)
+            const int map = acts[l] & ~SP_STACK_LN_L2;
+            if (map != SP_MAP_COPY && map != SP_MAP_RELU && map != SP_MAP_TANH && map != SP_MAP_SIGMOID)
+                return fail(SP_ERR_ARG, "sp_stack_forward_f32: unknown activation %d of layer %d", acts[l], l);
+            a.acts[l] = acts[l];
+        }
         a.w[l] = (const float*)weights[l];
-        a.acts[l] = acts[l];
         a.dims[l] = dims[l];
         if (dims[l] > widest) widest = dims[l];
     }

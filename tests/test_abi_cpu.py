@@ -304,3 +304,14 @@ def test_stack_argument_errors(L):
     ph = L.PhiloxConfig(1, 0, L.PHILOX_LAYER, 256, 8, 8, 32, 0)
     assert call(act=p, ph=C.byref(ph)) == -5 and "member_rows" in _err(L)
     assert call(n=4, w=(C.c_void_p * 4)(p, p, p, p), d=ints(128, 128, 128, 128, 64), acts=ints(1, 1, 1, 0)) == -6 and "LDS" in _err(L)
+
+
+def test_a_stack_reads_no_activation_behind_its_last_layer(L):
+    """acts holds n_layers - 1 codes: what lies behind them is not looked at (here a code that is refused anywhere else, in a stack
+    that is refused for its size, so nothing is launched)."""
+    p = C.c_void_p(0x6000)
+    ints = lambda *d: (C.c_int32 * len(d))(*d)
+    call = lambda *acts: L.lib.sp_stack_forward_f32(p, 4, (C.c_void_p * 4)(p, p, p, p), ints(128, 128, 128, 128, 64), ints(*acts), 1, None,
+                                                    None, p, None, 64, 1, 0, None)
+    assert call(1, 1, 1, 9) == -6 and "LDS" in _err(L)
+    assert call(1, 1, 9, 0) == -5 and "activation" in _err(L)
