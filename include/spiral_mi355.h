@@ -445,6 +445,8 @@ int sp_mlp_forward_ensemble(int dtype, const void* x, int32_t n_layers, const vo
  * sp_mlp_forward_ensemble; members x batch below 2^31.
  * Replaces: the node-by-node run (ml/layers.spi:194-240, 336-344) of the graphs of ml/layers.spi:564-665. */
 #define SP_STACK_LN_L2 0x100
+/* Whether a call of these sizes and this head is taken: SP_OK, or the error it would be refused with.  A host query. */
+int sp_stack_forward_takes(int32_t n_layers, const int32_t* dims, int32_t members, int64_t batch, int32_t head_op, int32_t mask_size);
 int sp_stack_forward_f32(const void* x, int32_t n_layers, const void* const* weights, const int32_t* dims, const int32_t* acts,
                          int32_t members, const float* u, const sp_philox_t* philox, float* policy_out, int32_t* action_out,
                          int64_t batch, int32_t head_op, int32_t mask_size, void* stream);

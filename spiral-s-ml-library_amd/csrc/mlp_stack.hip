@@ -299,11 +299,38 @@ static const void* pick_stack_kernel(bool regret) {
     return regret ? (const void*)mlp_stack_kernel<HT, true, FULL> : (const void*)mlp_stack_kernel<HT, false, FULL>;
 }
 
-// Bytes of LDS the weights take (dims[n_layers] = the computed outputs).
-static long stack_weight_bytes(int n_layers, const int* dims) {
+// Bytes of LDS the weights take; computed: the outputs that a mask leaves.
+static long stack_weight_bytes(int n_layers, const int32_t* dims, int computed) {
     long blocks = 0;
-    for (int l = 0; l < n_layers; ++l) blocks += (long)((dims[l] + 15) / 16) * ((dims[l + 1] + 15) / 16);
+    for (int l = 0; l < n_layers; ++l) blocks += (long)((dims[l] + 15) / 16) * (((l + 1 < n_layers ? dims[l + 1] : computed) + 15) / 16);
     return blocks * ST_BLOCK;
+}
+
+// The sizes and the head of a call: what sp_stack_forward_takes answers for and sp_stack_forward_f32 checks.
+static bool head_is_masked(int head_op) { return head_op == SP_ROW_MASKED_SOFTMAX || head_op == SP_ROW_MASKED_REGRET_MATCHING; }
+static bool head_is_regret(int head_op) { return head_op == SP_ROW_REGRET_MATCHING || head_op == SP_ROW_MASKED_REGRET_MATCHING; }
+static int check_stack_sizes(const char* fn, int n_layers, const int32_t* dims, int members, int64_t batch, int head_op, int mask_size) {
+    if (n_layers < 1 || n_layers > ST_MAX_LAYERS) return fail(SP_ERR_SHAPE, "%s: 1 to %d layers, got %d", fn, ST_MAX_LAYERS, n_layers);
+    if (members <= 0 || members > 65535) return fail(SP_ERR_SHAPE, "%s: members must be in [1, 65535]", fn);
+    if (batch <= 0 || batch >= (1ll << 31) / members - ST_ROWS) return fail(SP_ERR_SHAPE, "%s: batch must be positive and members x batch below 2^31", fn);
+    if (!head_is_regret(head_op) && head_op != SP_ROW_SOFTMAX && head_op != SP_ROW_MASKED_SOFTMAX) return fail(SP_ERR_ARG, "%s: unknown head %d", fn, head_op);
+    const int n = dims[n_layers];
+    if (dims[0] < 4 || dims[0] % 4 != 0 || dims[0] > ST_MAX_WIDTH)
+        return fail(SP_ERR_SHAPE, "%s: input width %d must be a multiple of 4 in [4, %d]", fn, dims[0], ST_MAX_WIDTH);
+    for (int l = 1; l < n_layers; ++l)
+        if (dims[l] < 16 || dims[l] % 16 != 0 || dims[l] > ST_MAX_WIDTH)
+            return fail(SP_ERR_SHAPE, "%s: hidden width %d must be a multiple of 16 in [16, %d]", fn, dims[l], ST_MAX_WIDTH);
+    if (n < 4 || n % 4 != 0 || n > ST_MAX_OUT)
+        return fail(SP_ERR_SHAPE, "%s: output width %d must be a multiple of 4 in [4, %d]", fn, n, ST_MAX_OUT);
+    if (head_is_masked(head_op) && (mask_size <= 0 || mask_size > n)) return fail(SP_ERR_ARG, "%s: mask_size must be in [1, %d], got %d", fn, n, mask_size);
+    const long w_bytes = stack_weight_bytes(n_layers, dims, head_is_masked(head_op) ? mask_size : n);
+    if (w_bytes > ST_LDS - 4 * ST_SCRATCH) return fail(SP_ERR_UNSUPPORTED, "%s: %ld bytes of weights exceed the LDS", fn, w_bytes);
+    return SP_OK;
+}
+
+extern "C" int sp_stack_forward_takes(int32_t n_layers, const int32_t* dims, int32_t members, int64_t batch, int32_t head_op, int32_t mask_size) {
+    if (dims == nullptr) return fail(SP_ERR_NULL, "sp_stack_forward_takes: dims is NULL");
+    return check_stack_sizes(__func__, n_layers, dims, members, batch, head_op, mask_size);
 }
 
 // Reference role: the body of `graph_run_host model` (ml/layers.spi:336-344) for the chains named at the top.
@@ -315,24 +342,13 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
     SP_REQUIRE_PTR(policy_out);
     SP_OPTIONAL_PTR(u); SP_OPTIONAL_PTR(action_out);
     if (weights == nullptr || dims == nullptr || (acts == nullptr && n_layers != 1)) return fail(SP_ERR_NULL, "sp_stack_forward_f32: weights/dims/acts is NULL");
-    if (n_layers < 1 || n_layers > ST_MAX_LAYERS) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: 1 to %d layers, got %d", ST_MAX_LAYERS, n_layers);
-    if (members <= 0 || members > 65535) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: members must be in [1, 65535]");
-    if (batch <= 0 || batch >= (1ll << 31) / members - ST_ROWS) return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: batch must be positive and members x batch below 2^31");
-    const bool regret = head_op == SP_ROW_REGRET_MATCHING || head_op == SP_ROW_MASKED_REGRET_MATCHING;
-    if (!regret && head_op != SP_ROW_SOFTMAX && head_op != SP_ROW_MASKED_SOFTMAX) return fail(SP_ERR_ARG, "sp_stack_forward_f32: unknown head %d", head_op);
+    int rc = check_stack_sizes(__func__, n_layers, dims, members, batch, head_op, mask_size);
+    if (rc != SP_OK) return rc;
     if (action_out != nullptr && u == nullptr && philox == nullptr)
         return fail(SP_ERR_NULL, "sp_stack_forward_f32: action requested but u and philox are NULL");
     if (u != nullptr && philox != nullptr) return fail(SP_ERR_ARG, "sp_stack_forward_f32: at most one of u and philox may be given");
     const int n = dims[n_layers];
-    if (dims[0] < 4 || dims[0] % 4 != 0 || dims[0] > ST_MAX_WIDTH)
-        return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: input width %d must be a multiple of 4 in [4, %d]", dims[0], ST_MAX_WIDTH);
-    for (int l = 1; l < n_layers; ++l)
-        if (dims[l] < 16 || dims[l] % 16 != 0 || dims[l] > ST_MAX_WIDTH)
-            return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: hidden width %d must be a multiple of 16 in [16, %d]", dims[l], ST_MAX_WIDTH);
-    if (n < 4 || n % 4 != 0 || n > ST_MAX_OUT)
-        return fail(SP_ERR_SHAPE, "sp_stack_forward_f32: output width %d must be a multiple of 4 in [4, %d]", n, ST_MAX_OUT);
-    const bool masked = head_op == SP_ROW_MASKED_SOFTMAX || head_op == SP_ROW_MASKED_REGRET_MATCHING;
-    if (masked && (mask_size <= 0 || mask_size > n)) return fail(SP_ERR_ARG, "sp_stack_forward_f32: mask_size must be in [1, %d], got %d", n, mask_size);
+    const bool masked = head_is_masked(head_op), regret = head_is_regret(head_op);
     StackArgs a{};
     int widest = 0;
     for (int l = 0; l < n_layers; ++l) {
@@ -349,16 +365,14 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
         if (dims[l] > widest) widest = dims[l];
     }
     a.ph.philox_mode = -1;
-    int rc = mlp_set_philox(a.ph, philox, (int64_t)members * batch, n, __func__);
+    rc = mlp_set_philox(a.ph, philox, (int64_t)members * batch, n, __func__);
     if (rc != SP_OK) return rc;
     if (philox != nullptr && philox->member_rows > 0 && philox->member_rows != batch)
         return fail(SP_ERR_ARG, "sp_stack_forward_f32: member_rows must be the batch");
     a.mask_size = masked ? mask_size : n;
     a.dims[n_layers] = a.mask_size;
     a.out_stride = (long)n * dims[n_layers - 1];
-    const long w_bytes = stack_weight_bytes(n_layers, a.dims);
-    if (w_bytes > ST_LDS - 4 * ST_SCRATCH)
-        return fail(SP_ERR_UNSUPPORTED, "sp_stack_forward_f32: %ld bytes of weights exceed the LDS", w_bytes);
+    const long w_bytes = stack_weight_bytes(n_layers, dims, a.mask_size);
     rc = require_gfx950(__func__);
     if (rc != SP_OK) return rc;
     a.x = (const float*)x; a.u = u; a.policy = policy_out; a.action = action_out;

@@ -93,6 +93,7 @@ SIGNATURES = {
                                           C.POINTER(PhiloxConfig), _P, _P, _I64, _I32, _I32, _P]),
     "sp_stack_forward_f32": (C.c_int, [_P, _I32, C.POINTER(_P), C.POINTER(C.c_int32), C.POINTER(C.c_int32), _I32, _P,
                                        C.POINTER(PhiloxConfig), _P, _P, _I64, _I32, _I32, _P]),
+    "sp_stack_forward_takes": (C.c_int, [_I32, C.POINTER(C.c_int32), _I32, _I64, _I32, _I32]),
     "sp_ensemble_binarize": (C.c_int, [C.c_int, _P, _P, _P, _I32, _I64, _I32, _I32, _U32, _P]),
 }
 

@@ -1029,7 +1029,7 @@ def _overlap(a, b):
 
 def _run_fused_stack(model, key, count, ls):
     """One sp_stack_forward_f32 launch in place of a walk over the nodes, where the graph is of that shape and the entry point
-    takes its sizes (it says so itself, before anything is launched).  The tensors of the nodes in the middle are not written
+    takes its sizes (sp_stack_forward_takes says so, the limits stand there alone).  The tensors of the nodes in the middle are not written
     then, so a model whose caller has looked at one of them is not taken.  (A batched pass has none: its nodes are temporaries.)"""
     plan = _stack_plan(model, key)
     if plan is None:
@@ -1039,39 +1039,40 @@ def _run_fused_stack(model, key, count, ls):
     if key is None and not middle.isdisjoint(arena.get("looked_up", ())):
         arena.get("not_written", set()).difference_update(middle)      # the walk writes them
         return False
+    spec, w_specs, lead = x_node.spec, [w.spec for w in w_nodes], () if key is None else (count,)
+    if len(spec.dim) != 3 or any(t.dtype != torch.float32 for t in [spec] + w_specs):
+        return False
+    if any(len(t.dim) != 2 + len(lead) or t.dim[:-2] != lead for t in w_specs):
+        return False
+    q, w, k0 = spec.dim
+    dims = [k0] + [t.dim[-2] for t in w_specs]
+    cols, n = dims[-1], len(w_specs)
+    if any(t.dim[-1] != d for t, d in zip(w_specs, dims)) or cols % 4:
+        return False
+    dims_c, head_op = (C.c_int32 * (n + 1))(*dims), _STACK_HEADS[head]
+    if lib.sp_stack_forward_takes(n, dims_c, count, q * w, head_op, mask) in (_lib.ERR_SHAPE, _lib.ERR_UNSUPPORTED):
+        return False
     tensor = lambda node: graph_extract(Model(node, model.dims, model.data))
     x, ws = tensor(x_node), [tensor(w) for w in w_nodes]
     outs = graph_extract(model) if out_nodes is None else tuple(tensor(o) for o in out_nodes)
     outs = outs if isinstance(outs, tuple) else (outs,)
-    lead = () if key is None else (count,)
-    if x.dim() != 3 or any(t.dtype != torch.float32 for t in [x, outs[0]] + ws):
+    if outs[0].dtype != torch.float32 or outs[0].shape != lead + (q, w, cols):
         return False
-    if any(w.dim() != 2 + len(lead) or w.shape[:-2] != lead for w in ws):
-        return False
-    q, w, k0 = x.shape
-    dims = [k0] + [t.shape[-2] for t in ws]
-    cols = dims[-1]
-    if any(t.shape[-1] != d for t, d in zip(ws, dims)) or cols % 4:
-        return False
-    if outs[0].shape != lead + (q, w, cols) or (len(outs) == 2 and (outs[1].shape != lead + (q, w) or outs[1].dtype != torch.int32)):
+    if len(outs) == 2 and (outs[1].shape != lead + (q, w) or outs[1].dtype != torch.int32):
         return False
     if any(_overlap(o, t) for o in outs for t in [x] + ws) or (len(outs) == 2 and _overlap(*outs)):
         return False          # node by node, an output may take the place of what has been read
-    rng, draws = None, 0
+    rng = None
     if len(outs) == 2:
         draws = _sampling_draws(w, cols)
         rng = _prim.philox(_lib.PHILOX_LAYER, seed=ls.seed, threads_per_block=THREADS_PER_BLOCK, blocks_per_grid=q,
                            rows_per_block=w, offset=ls.draws, member_rows=q * w if key is not None else 0, member_draws=draws)
-    n = len(ws)
-    rc = lib.sp_stack_forward_f32(
-        ptr(x, name="x"), n, (C.c_void_p * n)(*[ptr(t, name="weights[%d]" % i) for i, t in enumerate(ws)]),
-        (C.c_int32 * (n + 1))(*dims), (C.c_int32 * n)(*acts), count, None, C.byref(rng) if rng is not None else None,
-        ptr(outs[0], name="policy"), ptr(outs[1], name="action") if len(outs) == 2 else None, q * w, _STACK_HEADS[head], mask,
-        stream_ptr())
-    if rc in (_lib.ERR_SHAPE, _lib.ERR_UNSUPPORTED):
-        return False
-    check(rc)
-    ls.draws += draws
+        ls.draws += draws
+    check(lib.sp_stack_forward_f32(
+        ptr(x, name="x"), n, (C.c_void_p * n)(*[ptr(t, name="weights[%d]" % i) for i, t in enumerate(ws)]), dims_c,
+        (C.c_int32 * n)(*acts), count, None, C.byref(rng) if rng is not None else None,
+        ptr(outs[0], name="policy"), ptr(outs[1], name="action") if len(outs) == 2 else None, q * w, head_op, mask,
+        stream_ptr()))
     if key is None:
         ls.not_written = frozenset(middle)
         arena.setdefault("not_written", set()).update(middle)

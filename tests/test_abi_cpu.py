@@ -307,11 +307,22 @@ def test_stack_argument_errors(L):
 
 
 def test_a_stack_reads_no_activation_behind_its_last_layer(L):
-    """acts holds n_layers - 1 codes: what lies behind them is not looked at (here a code that is refused anywhere else, in a stack
-    that is refused for its size, so nothing is launched)."""
+    """acts holds n_layers - 1 codes: what lies behind them is not looked at (here a code that is refused anywhere else, in a call
+    that is refused for its random stream, so nothing is launched)."""
     p = C.c_void_p(0x6000)
     ints = lambda *d: (C.c_int32 * len(d))(*d)
-    call = lambda *acts: L.lib.sp_stack_forward_f32(p, 4, (C.c_void_p * 4)(p, p, p, p), ints(128, 128, 128, 128, 64), ints(*acts), 1, None,
-                                                    None, p, None, 64, 1, 0, None)
-    assert call(1, 1, 1, 9) == -6 and "LDS" in _err(L)
-    assert call(1, 1, 9, 0) == -5 and "activation" in _err(L)
+    stream = L.PhiloxConfig(1, 0, L.PHILOX_LAYER, 256, 8, 8, 32, 0)      # member_rows is not the batch
+    call = lambda *acts: L.lib.sp_stack_forward_f32(p, 2, (C.c_void_p * 2)(p, p), ints(64, 64, 16), ints(*acts), 1, None,
+                                                    C.byref(stream), p, p, 64, 1, 0, None)
+    assert call(1, 9) == -5 and "member_rows" in _err(L)
+    assert call(9, 0) == -5 and "activation" in _err(L)
+
+
+def test_stack_sizes_are_asked_without_a_call(L):
+    ints = lambda *d: (C.c_int32 * len(d))(*d)
+    takes = lambda *d, members=1, batch=64, head=1, mask=0: L.lib.sp_stack_forward_takes(len(d) - 1, ints(*d), members, batch, head, mask)
+    assert takes(64, 64, 64, 64) == 0 and takes(4, 16, 4) == 0 and takes(128, 128, 128, 64) == -6 and takes(128, 128, 128, 64, head=2, mask=16) == 0
+    assert takes(66, 64, 16) == -2 and takes(64, 72, 16) == -2 and takes(64, 144, 16) == -2 and takes(64, 64, 68) == -2
+    assert takes(64, 16, members=70000) == -2 and takes(64, 16, batch=0) == -2 and takes(64, 16, members=2, batch=1 << 30) == -2
+    assert takes(64, 16, head=3) == -5 and takes(64, 16, head=2, mask=17) == -5 and takes(*([64] * 10)) == -2
+    assert L.lib.sp_stack_forward_takes(1, None, 1, 64, 1, 0) == -1

@@ -163,48 +163,54 @@ def test_stack_plan_takes_whole_chains_only():
     assert [plan(g) for g in (named, kept, swapped, first)] == [None] * 4
 
 
-def test_a_stack_the_entry_point_refuses_runs_node_by_node(monkeypatch):
-    """Which sizes run as one launch is sp_stack_forward_f32's own answer: refused sizes fall back to the walk and leave the
-    generator where it was, every other error is raised."""
-    g = L.pipe(L.input("input", (24, 64, 64)), L.matmul((64, 64)), L.relu, L.matmul((64, 16)), L.softmax_and_discrete_sample)
-    model, answer, calls = L.create_model(g, device="cpu"), [0], []
+class Answering:
+    """Stands in for the library: sizes are answered by the real one or with a code, launches are recorded."""
 
-    class Refusing:
-        def sp_stack_forward_f32(self, *args):
-            calls.append(args)
-            return answer[0]
+    def __init__(self, takes=None, launch=0):
+        self.takes, self.launch, self.calls = takes, launch, []
 
-    monkeypatch.setattr(L, "lib", Refusing())
+    def sp_stack_forward_takes(self, *args):
+        return L._lib.lib.sp_stack_forward_takes(*args) if self.takes is None else self.takes
+
+    def sp_stack_forward_f32(self, *args):
+        self.calls.append(args)
+        return self.launch
+
+
+def without_a_gpu(monkeypatch, lib):
+    monkeypatch.setattr(L, "lib", lib)
     monkeypatch.setattr(L, "ptr", lambda t, dtype=None, name="": None if t is None else t.data_ptr())
     monkeypatch.setattr(L, "stream_ptr", lambda: None)
-    ls = L.create_layer_state()
-    for answer[0] in (-2, -6):
-        assert L._run_fused_stack(model, None, 1, ls) is False and ls.draws == 0
-    answer[0] = -5
+    monkeypatch.setattr(L._lib, "stream_ptr", lambda: None)
+    return lib
+
+
+def test_a_stack_the_entry_point_refuses_runs_node_by_node(monkeypatch):
+    """Which sizes run as one launch is sp_stack_forward_takes' answer alone: what it refuses for its size falls back to the
+    walk and leaves the generator where it was, errors of a launch are raised."""
+    lib = without_a_gpu(monkeypatch, Answering())
+    build = lambda *widths: L.create_model(L.softmax_and_discrete_sample(L.pipe(L.input("input", (24, 64, widths[0])), *[
+        L.matmul(pair) for pair in zip(widths[:-1], widths[1:])])), device="cpu")
+    model, ls = build(64, 64, 16), L.create_layer_state()
+    for lib.takes in (-2, -6):
+        assert L._run_fused_stack(model, None, 1, ls) is False and ls.draws == 0 and not lib.calls
+    lib.takes = 0
+    lib.launch = -5
     with pytest.raises(L._lib.SpiralError):
         L._run_fused_stack(model, None, 1, ls)
-    answer[0] = 0
-    assert L._run_fused_stack(model, None, 1, ls) is True and ls.draws > 0 and len(calls) == 4
-    # sizes that no kernel takes are asked about all the same: the limits stand in one place
-    wide = L.create_model(L.pipe(L.input("input", (24, 64, 64)), L.matmul((64, 256)), L.relu, L.matmul((256, 16)), L.softmax), device="cpu")
-    answer[0] = -2
-    assert L._run_fused_stack(wide, None, 1, ls) is False and len(calls) == 5
+    lib.takes, lib.launch = None, 0
+    assert L._run_fused_stack(model, None, 1, ls) is True and ls.draws > 0
+    # the real answers: widths, depth, the LDS
+    for widths in ((4, 16, 4), (128, 64), (100, 128, 96, 64), (64,) * 9):
+        assert L._run_fused_stack(build(*widths), None, 1, ls) is True, widths
+    for widths in ((132, 64, 16), (64, 72, 16), (64, 256, 16), (64, 64, 68), (64,) * 10, (128, 128, 128, 128, 64)):
+        assert L._run_fused_stack(build(*widths), None, 1, ls) is False, widths
 
 
 def test_a_node_somebody_looks_at_is_written(monkeypatch):
     """A fused stack leaves the tensors in its middle out.  Looked up before the run, such a node keeps the model on the walk;
     looked up behind a fused run for the first time, it is computed then, and the recorded launch is not replayed any more."""
-    calls, walked = [], []
-
-    class Taking:
-        def sp_stack_forward_f32(self, *args):
-            calls.append(args)
-            return 0
-
-    monkeypatch.setattr(L, "lib", Taking())
-    monkeypatch.setattr(L, "ptr", lambda t, dtype=None, name="": None if t is None else t.data_ptr())
-    monkeypatch.setattr(L, "stream_ptr", lambda: None)
-    monkeypatch.setattr(L._lib, "stream_ptr", lambda: None)
+    calls, walked = without_a_gpu(monkeypatch, Answering()).calls, []
     monkeypatch.setattr(L, "graph_run", lambda model, ls, indices: walked.append(model.graph))
     hidden = L.pipe(L.input("input", (24, 64, 64)), L.matmul((64, 64)), L.relu)
     build = lambda: L.create_model(L.pipe(hidden, L.matmul((64, 16)), L.softmax), device="cpu")
