@@ -1016,10 +1016,11 @@ static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, lo
     const int whole = dtype_in == SP_F32 || kind == TILE_SPLIT ? -1 : choose_cfg(dtype_in, M, N, K, batch, cus);
     // K split over four waves: from seven K-tiles up.  Below that (where a large output wants the workgroup tiles
     // whatever the estimate says) only for small outputs, whose time is the chain behind one of them (us, 64 x 64 tile /
-    // split: 181 x 39 x 96 f32 6.2 / 2.8; 64 x 64 x 128 4.5 / 2.6; 16 x 21 x 128 bf16 3.1 / 2.5), and for odd widths,
-    // where the split form's stores cost less (1371 x 45 x 64 bf16 4.4 / 2.8).
+    // split: 181 x 39 x 96 f32 6.3 / 2.8; 64 x 64 x 128 4.5 / 2.6; 16 x 21 x 144 bf16 3.6 / 2.5), and for odd widths,
+    // where the split form's stores cost less (1371 x 45 x 64 bf16 4.4 / 2.8, 1745 x 163 x 64 4.3 / 3.4; level from about
+    // 3000 tiles of 16 x 16 up: 1134 x 583 x 24 4.4 / 4.2, 1650 x 1102 x 192 5.8 / 7.7).
     const double small = (double)((M + 15) / 16) * (double)((N + 15) / 16);
-    const bool may_split = kind == TILE_SPLIT || nk >= 7 || (batch <= 64 && small <= (N % 4 ? 1024 : 64));
+    const bool may_split = kind == TILE_SPLIT || nk >= 7 || (batch <= 64 && small <= (N % 4 ? 2048 : 64));
     const TileCost* best = nullptr;
     float best_us = 0.f;
     auto consider = [&](const TileCost& c) {

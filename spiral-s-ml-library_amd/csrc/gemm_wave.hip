@@ -11,10 +11,10 @@
 // The loads are the DMA of the other GEMM kernels (8 rows x 128 bytes of K per instruction, swizzled chunks), N and M
 // are ragged (rows clamped, stores masked) and K may end in a partial K-tile (chunks past the end come from zeros).
 //
-// Measured (us, gemm_abt_kernel on 64 x 64 tiles / this kernel; f32 unless said otherwise): 336 x 304 x 2256 48.5 / 11.7,
-// 865 x 147 x 4136 86.9 / 23.7, 700 x 700 x 4096 84.9 / 41.5, 512^3 12.3 / 6.1, 20031 x 15 x 1800 78.8 / 33.3,
-// 50372 x 4 x 1208 168 / 46 (5.3 TB/s); bf16 16 x 4096 x 4096 32.6 / 8.2, 2027 x 6 x 1688 12.2 / 4.3, 52020 x 17 x 1472
-// 39.1 / 29.8 (5.2 TB/s), 1019 x 622 x 6392 56.6 / 30.4; f16 362 x 669 x 4352 36.8 / 10.6, 1882 x 241 x 3152 28.2 / 12.9.
+// Measured (us, gemm_abt_kernel on 64 x 64 tiles / this kernel; f32 unless said otherwise): 336 x 304 x 2256 48.3 / 9.5,
+// 865 x 147 x 4136 86.8 / 24.1, 700 x 700 x 4096 87.0 / 43.1, 512^3 11.6 / 5.7, 20031 x 15 x 1800 63.7 / 24.6,
+// 50372 x 4 x 1208 79.1 / 43.8 (5.6 TB/s); bf16 16 x 4096 x 4096 31.3 / 5.8, 2027 x 6 x 1688 11.1 / 3.6, 52020 x 17 x 1472
+// 25.3 / 25.8 (5.9 TB/s either way), 1019 x 622 x 6392 55.5 / 30.4; f16 362 x 669 x 4352 33.4 / 8.7, 1882 x 241 x 3152 27.0 / 11.6.
 #include "gemm_common.h"
 
 namespace sp {

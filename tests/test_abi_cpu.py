@@ -71,6 +71,13 @@ def test_f32_tile_choice_by_the_length_of_k(L, m, n, k, tile):
     assert [o.value for o in out[:2]] == [tile, tile]
 
 
+def test_odd_widths_of_short_k_split_as_long_as_that_is_faster(L):
+    out = [C.c_int32() for _ in range(5)]
+    for m, n, k, parts in ((375, 793, 16, 4), (1745, 163, 64, 4), (1650, 1102, 192, 1), (1304, 1979, 40, 1), (376, 792, 16, 1)):
+        assert L.lib.sp_gemm_batched_config(2, m, n, k, 1, *[C.byref(o) for o in out]) == 0
+        assert out[4].value == parts, (m, n, k)
+
+
 @pytest.mark.parametrize("dtype", [0, 1, 2])
 def test_tall_outputs_get_tiles_a_launch_can_number(L, dtype):
     """HIP launches fewer than 2^32 work items along a dimension: outputs of a few columns and up to 2^31 - 256 rows are within the
