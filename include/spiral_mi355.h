@@ -129,12 +129,13 @@ int sp_gemm_abt_batched(int dtype_in, int dtype_out, const void* A, const void* 
                         int64_t stride_c, float alpha, float beta, uint32_t flags, void* stream);
 
 /* Which tile configuration sp_gemm_abt picks for a shape (the counterpart of
- * `matmul_config_tf32`, ml/matmul/run.spi:8-19).  Writes block tile sizes and the workgroup size. */
+ * `matmul_config_tf32`, ml/matmul/run.spi:8-19).  Writes block tile sizes and the workgroup size; tile_m == 0 means one thread
+ * per output (odd widths of the shortest K). */
 int sp_gemm_config(int dtype_in, int64_t M, int64_t N, int64_t K,
                    int32_t* tile_m, int32_t* tile_n, int32_t* tile_k, int32_t* threads);
 
 /* The same for one launch over `batch` matrices (sp_gemm_abt_batched); k_parts: the partial sums over K that an output is
- * added up from (4 on the split-K tiles, 1 on the workgroup tiles). */
+ * added up from (4 on the split-K tiles, 1 on the workgroup tiles, 0 where one thread adds them up in order). */
 int sp_gemm_batched_config(int dtype_in, int64_t M, int64_t N, int64_t K, int64_t batch,
                            int32_t* tile_m, int32_t* tile_n, int32_t* tile_k, int32_t* threads, int32_t* k_parts);
 

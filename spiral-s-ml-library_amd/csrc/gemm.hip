@@ -875,8 +875,8 @@ __global__ __launch_bounds__(256) void gemm_abt_w4_kernel(SP_GEMM_PRELOADED, con
     }
 }
 
-// Shape-agnostic kernel: one thread per output element, 16-byte loads along K.  Only SP_GEMM_FORCE_GENERIC comes here
-// (every shape has an MFMA kernel): a second opinion for tests.
+// Shape-agnostic kernel: one thread per output element, 16-byte loads along K.  For odd widths of the shortest K (one_thread_each
+// below), where it has neither a prologue nor sums to gather, and for SP_GEMM_FORCE_GENERIC, a second opinion for tests.
 template <int DT>
 __global__ __launch_bounds__(256) void gemm_abt_generic_kernel(const GemmArgs g) {
     constexpr int ES = (DT == SP_F32) ? 4 : 2;
@@ -976,7 +976,8 @@ static int choose_cfg(int dtype_in, long M, long N, long K, long batch, long cus
     return smallest;
 }
 
-// The tile a GEMM runs on: a workgroup tile of kTileCfgs (cfg 0..2) or a split-K tile of gemm_wave.hip (cfg < 0).
+// The tile a GEMM runs on: a workgroup tile of kTileCfgs (cfg 0..2), a split-K tile of gemm_wave.hip (cfg -1) or none, one
+// thread per output (cfg -2).
 // `ragged`: the tile does not divide M, N and K -- rows clamped in the loader, zeros for the missing part of the last
 // K-tile, a masked epilogue.
 struct TileChoice {
@@ -1051,16 +1052,26 @@ static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, lo
     return {best->cfg, t.bm, t.bn, threads, ragged, best_us};
 }
 
+// Odd widths of at most 64 bytes of K: one thread per output, up to 2^19 of them, of 64 bytes up to 2^17 (us, the fastest tile /
+// so: bf16 18043 x 3 x 16 5.2 / 2.6, 375 x 793 x 16 3.8 / 3.1, 20 x 33 x 8 2.3 / 2.0, f32 25058 x 6 x 4 5.3 / 2.7,
+// 1154 x 382 x 12 4.8 / 3.6, 667 x 134 x 16 2.9 / 2.6; beyond: f32 810 x 1377 x 16 5.2 / 9.4, bf16 1405 x 718 x 24 4.7 / 6.1,
+// 1527 x 218 x 32 3.9 / 4.2, 270 x 47 x 48 2.5 / 2.7).  Its time over a batch is that of its outputs, some 4 us a million.
+static bool one_thread_each(int dtype_in, long M, long N, long K) {
+    const long row = K * (dtype_in == SP_F32 ? 4 : 2);
+    return N % 4 != 0 && row <= 64 && (double)M * (double)N <= (row <= 48 ? 524288.0 : 131072.0);
+}
+
 // The members of a batch are to add up like a plain launch of each.  The split-K tiles all add an output's products in one
-// order and the workgroup tiles of f32 in another, so the shape of ONE member decides between the two kinds and the batch
+// order and the workgroup tiles of f32 in another, so the shape of ONE member decides between the kinds and the batch
 // between the tiles of that kind.  Always for f32, whose batched and member-by-member runs are bit-identical; it costs most
 // where small whole tiles come in large numbers (us, workgroup tiles / split K: 300 x (128 x 128 x 224) 28.8 / 31.7,
 // 37 x (960 x 384 x 320) 78 / 104, 300 x (64 x 64 x 64) 4.8 / 7.8).  For 16-bit inputs, whose 256 wide tiles have MFMAs and
 // K walks of their own anyway, as long as the other kind is not a quarter faster by the estimate.
 static TileChoice choose_tile(int dtype_in, long M, long N, long K, long batch, long cus) {
-    const TileChoice member = best_tile(dtype_in, M, N, K, 1, cus, TILE_ANY);
+    const TileChoice each = {-2, 0, 0, 256, true, 4e-6f * (float)M * (float)N * (float)batch};
+    const TileChoice member = one_thread_each(dtype_in, M, N, K) ? each : best_tile(dtype_in, M, N, K, 1, cus, TILE_ANY);
     if (batch == 1) return member;
-    const TileChoice alike = best_tile(dtype_in, M, N, K, batch, cus, member.cfg < 0 ? TILE_SPLIT : TILE_WORKGROUP);
+    const TileChoice alike = member.cfg == -2 ? each : best_tile(dtype_in, M, N, K, batch, cus, member.cfg < 0 ? TILE_SPLIT : TILE_WORKGROUP);
     if (dtype_in == SP_F32) return alike;
     const TileChoice any = best_tile(dtype_in, M, N, K, batch, cus, TILE_ANY);
     return alike.us <= 1.25f * any.us ? alike : any;
@@ -1258,7 +1269,7 @@ static int gemm_config(const char* fn, int dtype_in, int64_t M, int64_t N, int64
     *tile_n = t.bn;
     *tile_k = dtype_in == SP_F32 ? 32 : 64;
     *threads = t.threads;
-    *k_parts = t.cfg < 0 ? 4 : 1;
+    *k_parts = t.cfg == -1 ? 4 : t.cfg == -2 ? 0 : 1;
     return SP_OK;
 }
 
@@ -1304,15 +1315,17 @@ static int gemm_entry(const char* fn, int dtype_in, int dtype_out, const void* A
     }
     g.stride_a = stride_a * es_in; g.stride_b = stride_b * es_in; g.stride_c = stride_c * es_out;
     hipStream_t s = (hipStream_t)stream;
-    int cfg = -1;                                         // the generic kernel
+    int cfg = -2;                                         // one thread per output
     if (!(flags & SP_GEMM_FORCE_GENERIC)) {
         const long cus = device_cu_count();
         const TileChoice t = choose_tile(dtype_in, M, N, K, batch, cus);
         cfg = t.cfg;
-        g.ragged = t.ragged;
-        g.tiles_m = (int)((M + t.bm - 1) / t.bm);
-        g.tiles_n = (int)((N + t.bn - 1) / t.bn);
-        if (cfg < 0) return launch_gemm_wave(dtype_in, t.bm, t.bn, cus, g, s);
+        if (cfg != -2) {
+            g.ragged = t.ragged;
+            g.tiles_m = (int)((M + t.bm - 1) / t.bm);
+            g.tiles_n = (int)((N + t.bn - 1) / t.bn);
+        }
+        if (cfg == -1) return launch_gemm_wave(dtype_in, t.bm, t.bn, cus, g, s);
     }
     switch (dtype_in) {
         case SP_F32: return launch_dtype<SP_F32, SP_F32>(cfg, g, s);

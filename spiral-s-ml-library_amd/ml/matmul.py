@@ -16,14 +16,14 @@ from ._lib import check, lib, ptr, stream_ptr
 
 def matmul_config_tf32(a_trans, b_trans, m, n, k, dtype=torch.float32):
     """Tile configuration chosen for a shape (counterpart of ml/matmul/run.spi:8-19).
-    Returns dict(m_tile, n_tile, k_tile, threads)."""
+    Returns dict(m_tile, n_tile, k_tile, threads); m_tile == 0 means one thread per output."""
     out = [C.c_int32() for _ in range(4)]
     check(lib.sp_gemm_config(_lib.DTYPES[dtype], m, n, k, *[C.byref(o) for o in out]))
     return dict(zip(("m_tile", "n_tile", "k_tile", "threads"), (o.value for o in out)))
 
 
 def matmul_config_batched(batch, m, n, k, dtype=torch.float32):
-    """The same for one launch over `batch` matrices, with k_parts, the partial sums over K behind an output."""
+    """The same for one launch over `batch` matrices, with k_parts, the partial sums over K behind an output (0: one thread)."""
     out = [C.c_int32() for _ in range(5)]
     check(lib.sp_gemm_batched_config(_lib.DTYPES[dtype], m, n, k, batch, *[C.byref(o) for o in out]))
     return dict(zip(("m_tile", "n_tile", "k_tile", "threads", "k_parts"), (o.value for o in out)))

@@ -71,9 +71,20 @@ def test_f32_tile_choice_by_the_length_of_k(L, m, n, k, tile):
     assert [o.value for o in out[:2]] == [tile, tile]
 
 
+def test_odd_widths_of_the_shortest_k_take_one_thread_per_output(L):
+    """As far as that was measured to be faster than any tile; a batch like its members in f32."""
+    out = [C.c_int32() for _ in range(5)]
+    for dtype, m, n, k, each in ((2, 18043, 3, 16, True), (1, 375, 793, 16, True), (2, 20, 33, 8, True), (0, 25058, 6, 4, True), (0, 667, 134, 16, True),
+                                 (0, 810, 1377, 16, False), (2, 1405, 718, 24, False), (2, 270, 47, 48, False), (2, 376, 792, 16, False)):
+        for e in (1, 5):
+            assert L.lib.sp_gemm_batched_config(dtype, m, n, k, e, *[C.byref(o) for o in out]) == 0
+            if e == 1 or dtype == 0:
+                assert (out[4].value == 0) == each and (out[0].value == 0) == each, (dtype, m, n, k, e)
+
+
 def test_odd_widths_of_short_k_split_as_long_as_that_is_faster(L):
     out = [C.c_int32() for _ in range(5)]
-    for m, n, k, parts in ((375, 793, 16, 4), (1745, 163, 64, 4), (1650, 1102, 192, 1), (1304, 1979, 40, 1), (376, 792, 16, 1)):
+    for m, n, k, parts in ((375, 793, 40, 4), (1745, 163, 64, 4), (1650, 1102, 192, 1), (1304, 1979, 40, 1), (376, 792, 16, 1)):
         assert L.lib.sp_gemm_batched_config(2, m, n, k, 1, *[C.byref(o) for o in out]) == 0
         assert out[4].value == parts, (m, n, k)
 
@@ -107,7 +118,7 @@ def test_a_batch_adds_up_like_a_launch_per_member(L):
         dtype = rng.choice([0, 1, 2])
         m, n = (max(1, int(2 ** rng.uniform(0, 13)) // a * a) for a in (rng.choice([1, 16, 64]), rng.choice([1, 4, 64])))
         shapes.append((dtype, m, n, max(8, int(2 ** rng.uniform(3, 13)) // 8 * 8)))
-    kinds, alike = {1: 0, 4: 0}, {e: [] for e in (2, 4, 16, 33, 64, 65, 100, 300)}
+    kinds, alike = {0: 0, 1: 0, 4: 0}, {e: [] for e in (2, 4, 16, 33, 64, 65, 100, 300)}
     for dtype, m, n, k in shapes:
         one = config(dtype, m, n, k, 1)
         single = [C.c_int32() for _ in range(4)]
