@@ -3,8 +3,9 @@
 // A (M,K) and B (N,K) are both K-contiguous, so neither operand needs a transposing read: a
 // 32x32 MFMA fragment of either one is "32 rows x one 16-byte K-chunk per lane".
 //
-// Here the workgroup tiles (small and narrow outputs: gemm_wave.hip).  Two kernels: gemm_abt_w4_kernel (four waves, 16x16x32 MFMAs; large 16-bit shapes) and gemm_abt_kernel (eight or
-// four waves, 32x32 MFMAs; f32, small tiles, single-column outputs).
+// Here the workgroup tiles (small and narrow outputs: gemm_wave.hip) and the choice between all of them.  Two kernels:
+// gemm_abt_w4_kernel (four waves, 16x16x32 MFMAs; large 16-bit shapes) and gemm_abt_kernel (eight or four waves, 32x32 MFMAs; f32,
+// small tiles, single-column outputs).
 //
 // Data movement per workgroup and K-tile (128 bytes of K per row: 64 bf16/f16 or 32 f32):
 //   global --global_load_lds_dwordx4 (DMA, no registers)--> LDS (double buffered, XOR-swizzled
@@ -989,8 +990,9 @@ struct TileChoice {
 // Estimated time of the most loaded compute unit on a tile, in us, without the launch: n tiles one after the other, each nk
 // K-tiles of `tk` plus `overhead` (prologue, epilogue, padding of its stores), and never less than `latency` per K-tile (what a
 // lone workgroup per unit waits for its loads).  n is ceil(tiles / units) for 16-bit inputs; for f32, whose tiles hold a unit's
-// matrix pipes busy side by side, the mean of that and of tiles / units.  Fitted to every tile on some 330 shapes
-// (profiles/gemm_tiles.txt has them, with what each tile takes and which one the estimate picks); what matters is the order.
+// matrix pipes busy side by side, the mean of that and of tiles / units.  profiles/gemm_tiles.txt has what every tile takes on
+// 480 shapes and which one is picked (2 % behind the fastest on the mean); what matters is the order, a kernel that changes
+// asks for that table again.  f32 was fitted on 186 of them and checked on 110 others.
 // The f32 line is the second fit: the first had too little overhead for the large tiles and cost short K up to 1.6 times
 // (us, 256 / 128 / 64 wide tiles: 11200 x 1792 x 32 44 / 33 / 20, 2688 x 5760 x 64 31 / 25 / 23, 2112 x 1536 x 96 36 / 15 / 9.6;
 // 10688 x 768 x 3648, 824 / 467 / 485, keeps its 128).  16-bit rows that do not start on 128-byte lines cost every fetch a
