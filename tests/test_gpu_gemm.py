@@ -142,7 +142,7 @@ def test_split_k_and_odd_widths_are_exact(MM, dtype, m, n, kt):
 
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("e,m,n,kt", [(239, 64, 64, 1), (5, 16, 16, 7), (17, 64, 16, 9.5), (3, 132, 35, 30), (9, 84, 61, 8), (7, 212, 100, 7.5),
-                                      (70, 48, 33, 3), (2, 500, 331, 9)])
+                                      (70, 48, 33, 3), (2, 500, 331, 9), (9, 44, 35, 0.25), (2, 1000, 250, 0.5)])
 def test_batched_split_k_and_odd_widths_are_exact(MM, dtype, e, m, n, kt):
     """The tiles of a whole batch are numbered through, whatever a member has of them (one, a few, an odd number): integer
     operands give the exact products of every member, odd widths and partial K-tiles among them, with bias, ReLU and beta."""
@@ -158,6 +158,27 @@ def test_batched_split_k_and_odd_widths_are_exact(MM, dtype, e, m, n, kt):
     assert (host(MM.matmul_abt_batched(a, b)) == want).all()
     got = host(MM.matmul_abt_batched(a, b, c=dev(c0), beta=2.0, bias=dev(bias), relu=True))
     assert (got == np.maximum(want + 2 * c0 + bias, 0)).all()
+
+
+@pytest.mark.parametrize("dtypes,tile,places,e,m,n,k", [
+    (("f32",), (32, 32), 512, 1, 3278, 143, 104), (("f32",), (32, 32), 512, 3, 8156, 5, 64),       # one K-tile per wave; N of a few columns
+    (("f32",), (32, 32), 512, 40, 516, 36, 1000), (("f16", "bf16"), (32, 32), 512, 1, 863, 1159, 480),
+    (("f16", "bf16"), (32, 32), 512, 40, 516, 4, 104), (("f16", "bf16"), (64, 32), 256, 1, 4554, 194, 392),
+    (("f16", "bf16"), (64, 32), 256, 40, 819, 4, 104), (("f16", "bf16"), (64, 64), 256, 40, 624, 34, 480)])
+def test_one_stage_rings_are_exact(MM, dtypes, tile, places, e, m, n, k):
+    """Split-K launches with more tiles than the LDS rings leave places for run on one stage per wave: every such instance, on
+    shapes that take it (a whole and a partial last K-tile, K-tiles that do not divide among the waves)."""
+    for dtype in dtypes:
+        announce("gemm one-stage ring %s e=%d %dx%dx%d" % (dtype, e, m, n, k))
+        cfg = MM.matmul_config_batched(e, m, n, k, TORCH[dtype])
+        assert (cfg["m_tile"], cfg["n_tile"], cfg["k_parts"]) == tile + (4,) and -(-m // tile[0]) * -(-n // tile[1]) * e > places
+        rng = np.random.default_rng(m + n + k)
+        ai = rng.integers(-3, 4, size=(e, m, k)).astype(np.float32)
+        bi = rng.integers(-3, 4, size=(e, n, k)).astype(np.float32)
+        want = np.matmul(ai, bi.transpose(0, 2, 1)).astype(np.float64)          # exact: every sum is below 2^24
+        a, b = dev(ai, TORCH[dtype]), dev(bi, TORCH[dtype])
+        got = host(MM.matmul_abt_batched(a, b) if e > 1 else MM.matmul_abt(a[0], b[0]))
+        assert (got.reshape(want.shape) == want).all()
 
 
 def test_random_small_shapes_are_exact(MM):
