@@ -557,3 +557,89 @@ def test_batched(MM, dtype, e, m, n, k, shared):
     for i in (0, e - 1):
         one = host(MM.matmul_abt(dev(a[0 if shared == "a" else i], t), dev(b[0 if shared == "b" else i], t)))
         assert (many[i] == one).all()
+
+
+# f32 on the bf16 pipe: tile, shape; remainders of M, N, K, odd and even numbers of K-tiles, odd widths, one K-tile more than the ring
+PARTS = [(256, 16384, 1024, 512), (256, 15873, 1023, 36), (256, 16129, 2047, 44), (256, 16384, 1024, 528), (128, 12929, 578, 36),
+         (128, 12860, 513, 68), (128, 10497, 322, 268), (128, 4096, 1024, 512), (128, 3584, 1792, 272), (128, 4097, 4093, 1000)]
+
+
+def parts_config(MM, tile, m, n, k, members=1):
+    cfg = MM.matmul_config_batched(members, m, n, k)
+    assert (cfg["k_tile"], cfg["m_tile"]) == (16, tile)
+
+
+@pytest.mark.parametrize("tile,m,n,k", PARTS)
+def test_f32_in_three_parts(MM, tile, m, n, k):
+    """Against float64 the sums are no further off than a chain of f32 additions is (2-norm: 2^-24 sqrt(K / 2), with what the
+    products leave out and the last rounding, 1e-7, on top), for numbers of any size; and B = I gives A back to the last bit."""
+    announce("gemm f32 parts %d %dx%dx%d" % (tile, m, n, k))
+    parts_config(MM, tile, m, n, k)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(k)
+    a = torch.randn((m, k), generator=gen, device="cuda")
+    b = torch.randn((n, k), generator=gen, device="cuda") * torch.exp2(torch.randint(-40, 40, (n, 1), generator=gen, device="cuda").float())
+    want = a.double() @ b.double().T
+    got = MM.matmul_abt(a, b).double()
+    row = ((got - want).norm(dim=0) / want.norm(dim=0)).max().item()         # (by column of C: the rows of b differ in size)
+    assert row < 2.0 ** -24 * (k / 2) ** 0.5 + 1e-7
+    c = torch.randn((m, n), generator=gen, device="cuda")
+    bias = torch.randn((n,), generator=gen, device="cuda")
+    b = torch.randn((n, k), generator=gen, device="cuda")
+    want = torch.relu(0.5 * (a.double() @ b.double().T) - 2.0 * c.double() + bias.double())
+    got = MM.matmul_abt(a, b, c.clone(), 0.5, -2.0, bias=bias, relu=True).double()
+    assert ((got - want).norm() / want.norm()).item() < TOL["f32"]
+    one = torch.zeros((n, k), device="cuda")
+    one[torch.arange(n), torch.arange(n) % k] = 1.0
+    assert torch.equal(MM.matmul_abt(a, one), a[:, torch.arange(n, device="cuda") % k])
+
+
+@pytest.mark.parametrize("tile,m,n,k", [(256, 15873, 1023, 36), (128, 4096, 1024, 512)])
+def test_f32_in_three_parts_keeps_what_parts_cannot_hold(MM, tile, m, n, k):
+    """Infinities, NaN, values that round to an infinite bf16 and values whose lowest part is below the smallest bf16."""
+    announce("gemm f32 parts, special values %d %dx%dx%d" % (tile, m, n, k))
+    parts_config(MM, tile, m, n, k)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(7)
+    a = torch.randn((m, k), generator=gen, device="cuda")
+    b = torch.randn((n, k), generator=gen, device="cuda").abs() + 0.5
+    a[5, 3], a[5, 7] = float("inf"), 1.0
+    a[6, 1], a[6, 2] = float("inf"), float("-inf")
+    a[700, k - 1] = float("nan")
+    a[m - 1, 0] = float("-inf")
+    a[900] = 0.0
+    a[900, 4] = 3.4028234e38                                   # the largest f32: its bf16 is infinite
+    b[:, 4] = 0.75
+    a[901] *= 2.0 ** -120
+    a[902] *= 2.0 ** -140                                      # subnormal
+    got = MM.matmul_abt(a, b)
+    assert (got[5] == float("inf")).all() and got[6].isnan().all() and got[700].isnan().all() and (got[m - 1] == float("-inf")).all()
+    assert torch.equal(got[900], torch.full((n,), 3.4028234e38 * 0.75, device="cuda"))
+    rest = torch.ones(m, dtype=torch.bool, device="cuda")
+    rest[[5, 6, 700, m - 1]] = False
+    want = a.double() @ b.double().T
+    for rows in (rest, [901]):
+        assert ((got[rows].double() - want[rows]).norm() / want[rows].norm()).item() < TOL["f32"]
+    # (a sum of subnormal numbers is rounded to a multiple of 2^-149, and so are its terms)
+    assert (got[902].double() - want[902]).abs().max().item() <= 2.0 ** -149 * k
+
+
+def test_f32_in_three_parts_adds_a_batch_up_like_its_members(MM):
+    announce("gemm f32 parts, batch")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    m, n, k = 2560, 2047, 1036
+    a, b = torch.randn((3, m, k), generator=gen, device="cuda"), torch.randn((3, n, k), generator=gen, device="cuda")
+    parts_config(MM, 128, m, n, k)
+    parts_config(MM, 256, m, n, k, 3)
+    many = MM.matmul_abt_batched(a, b)
+    for i in range(3):
+        assert torch.equal(many[i], MM.matmul_abt(a[i], b[i]))
+
+
+@pytest.mark.parametrize("name", ["gemm_f32_parts_256x256", "gemm_f32_parts_256x256_ragged", "gemm_f32_parts_128x128", "gemm_f32_parts_128x128_ragged"])
+def test_every_instance_of_the_parts_kernel_is_named(name):
+    announce("kernel info " + name)
+    from ml import _lib
+    info = _lib.kernel_info(name)
+    assert info["threads_per_block"] == (512 if "256" in name else 256) and 0 < info["vgprs"] <= 256
