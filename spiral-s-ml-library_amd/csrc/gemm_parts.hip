@@ -21,6 +21,7 @@
 // waves have nobody to hide behind and take 1 us a K-tile, two side by side 0.6 each.
 // Against float64 the sums are closer than the f32 MFMAs' (K = 512 3.4e-7 / 4.0e-7, K = 4096 1.0e-6 / 1.15e-6 of the 2-norm).
 #include "gemm_tile.h"
+#include "parts.h"
 
 namespace sp {
 
@@ -30,7 +31,6 @@ __device__ __forceinline__ f32x4 load_quad(const unsigned char* base, unsigned l
     return *reinterpret_cast<const __attribute__((address_space(1))) f32x4*>((global_ptr)base + lane_offset);
 }
 
-constexpr unsigned TINY = (127u - 110u) << 24;     // 2^-110 as 2 |x|, in bits
 constexpr int PARTS_BK = 16;                       // f32 of K per stage
 constexpr int PART_ROW = PARTS_BK * 2;             // bytes of one part of a row
 
@@ -75,7 +75,7 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_parts_kernel(SP_GEMM_PREL
     }
     const bool k_tail = RAGGED && K % PARTS_BK != 0 && (nk - 1) * PARTS_BK + quad * 4 >= K;   // this lane's quad of the last K-tile is not there
     f32x4 ld[4];
-    unsigned least = 0xffffffffu;                  // the smallest 2 |x| - 1, as bits: zeros wrap to the largest
+    unsigned least = 0xffffffffu;                  // (parts.h)
     auto load = [&](int i, int kt) {
         const int at = kt < nk ? kt : nk - 1;      // (past the end: the last one again, into a stage that nobody reads)
         ld[i] = load_quad(src + (long)at * (PARTS_BK * 4), voff[i] - (RAGGED && k_tail && at == nk - 1 ? quad * 16 : 0));
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_parts_kernel(SP_GEMM_PREL
             if (RAGGED && k_tail && kt >= nk - 1) ld[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const unsigned w = (__float_as_uint(ld[i][e]) << 1) - 1u;
+                const unsigned w = parts_magnitude(ld[i][e]);
                 least = w < least ? w : least;
             }
             write_part(i, stage, 0);
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_parts_kernel(SP_GEMM_PREL
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) sum = __builtin_fmaf(acc[i][j][r], 0.f, sum);         // NaN if one of them is not finite
-    if (__syncthreads_or(sum != 0.f || least < TINY - 1u)) {
+    if (__syncthreads_or(sum != 0.f || parts_tiny(least))) {
         clear();
         const unsigned char *pa[TM], *pb[TN];
 #pragma unroll

@@ -217,18 +217,7 @@ __device__ __forceinline__ void head_row(const HeadOut& o, const float* src, lon
 // a short straight line instead of a chain of small blocks, each of which is a jump into code the instruction
 // cache has not seen yet.  Same formulas, same order of operations as head_row<4>.
 template <int HEAD>
-__device__ __forceinline__ void head_row4(const HeadOut& o, const float (&src)[4], long row, int N, int limit, float u,
-                                          int fill_end) {
-    float p[4];
-#pragma unroll
-    for (int n = 0; n < 4; ++n) p[n] = n < N ? src[n] : 0.f;
-    float* const policy_row = o.policy + row * o.stride;
-    if (o.logits != nullptr) {
-        float* logits_row = o.logits + row * o.stride;
-#pragma unroll
-        for (int n = 0; n < 4; ++n)
-            if (n < N) logits_row[n] = p[n];
-    }
+__device__ __forceinline__ void head_values4(float (&p)[4], int limit) {
     if constexpr (HEAD == SP_HEAD_SOFTMAX || HEAD == SP_HEAD_SOFTMAX_RM) {
         float m = -__builtin_inff();
 #pragma unroll
@@ -258,6 +247,38 @@ __device__ __forceinline__ void head_row4(const HeadOut& o, const float (&src)[4
 #pragma unroll
         for (int n = 0; n < 4; ++n) p[n] = s != 0.f ? p[n] * inv : (n < limit ? inv_len : 0.f);
     }
+}
+// Inverse-CDF sampling from them.
+__device__ __forceinline__ int head_pick4(const float (&p)[4], float u) {
+    float run = 0.f, m = -__builtin_inff();
+    float cdf[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+        run = run + p[n];
+        cdf[n] = run;
+        if (p[n] > 0.f) m = fmaxf(m, run);
+    }
+    const float thr = u * m;
+    int pick = INT_MAX_;
+#pragma unroll
+    for (int n = 3; n >= 0; --n)
+        if (p[n] > 0.f && cdf[n] >= thr) pick = n;
+    return pick;
+}
+template <int HEAD>
+__device__ __forceinline__ void head_row4(const HeadOut& o, const float (&src)[4], long row, int N, int limit, float u,
+                                          int fill_end) {
+    float p[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) p[n] = n < N ? src[n] : 0.f;
+    float* const policy_row = o.policy + row * o.stride;
+    if (o.logits != nullptr) {
+        float* logits_row = o.logits + row * o.stride;
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+            if (n < N) logits_row[n] = p[n];
+    }
+    head_values4<HEAD>(p, limit);
 #pragma unroll
     for (int n = 0; n < 4; ++n)
         if (n < N) policy_row[n] = p[n];
@@ -265,22 +286,7 @@ __device__ __forceinline__ void head_row4(const HeadOut& o, const float (&src)[4
         const int end = o.stride < fill_end ? o.stride : fill_end;      // (past fill_end the caller fills with whole waves)
         for (int c = N; c < end; ++c) policy_row[c] = 0.f;
     }
-    if (o.action != nullptr) {
-        float run = 0.f, m = -__builtin_inff();
-        float cdf[4];
-#pragma unroll
-        for (int n = 0; n < 4; ++n) {
-            run = run + p[n];
-            cdf[n] = run;
-            if (p[n] > 0.f) m = fmaxf(m, run);
-        }
-        const float thr = u * m;
-        int pick = INT_MAX_;
-#pragma unroll
-        for (int n = 3; n >= 0; --n)
-            if (p[n] > 0.f && cdf[n] >= thr) pick = n;
-        o.action[row] = pick;
-    }
+    if (o.action != nullptr) o.action[row] = head_pick4(p, u);
 }
 
 // The commonest shape of all, as short as it gets (every byte of a head is fetched cold, once per launch, at about a

@@ -21,12 +21,15 @@
 // with g = 0 run the head for their row of the first tile, the lanes with g = 1 for the second; the zeros behind the
 // valid columns of a masked head are written by the whole wave, 16 bytes per lane.
 #include "mlp_common.h"
+#include "parts.h"
+#include "gemm_dma.h"
 
 #pragma clang fp contract(off)
 
 namespace sp {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 en_bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int EN_ROWS = 32;       // batch rows per tile
 constexpr int EN_HIDDEN = 64;     // width of the hidden layer
@@ -211,6 +214,336 @@ __global__ __launch_bounds__(EN_THREADS) void mlp_ensemble_kernel(const Ensemble
     }
 }
 
+// The same on the bf16 matrix pipe, every f32 as three bf16 parts (parts.h): sixteen times the rate of the f32 MFMAs for the six
+// products of parts that count, and next to 16-bit MFMAs vector instructions hide.
+// Two waves per SIMD: wave w and w + 4 of a workgroup take the two halves of one member's hidden layer, in 12 KS registers as
+// parts.  A workgroup has four members and walks over tiles of 32 batch rows, a tile a round; the inputs of a round are split
+// once per workgroup, every wave its share, into LDS, in the order the fragments of v_mfma_f32_32x32x16_bf16 are read.  Under
+// the products of round n run the split of the inputs of round n + 1 and the second layer of round n - 1; in front of every
+// second round one wave of a pair, in turn, does the heads of rounds n - 4 and n - 3, next to the other's products, and behind
+// the barrier both store the rows of round n - 4.  Three buffers of inputs, so that the one barrier of a round can stand in its
+// middle: nobody waits at a round's ends.  Second layer and head are those of the kernel above, in f32.
+// What bounds it: 32 x 65536 rows of 128 inputs take 206 us traced, 65 rounds of 6.3 k cycles at 2.0 GHz; the matrix pipe is busy for
+// half of them (the clock with it alone busy would be 1.8), the rest is 280 vector instructions per wave and round, 40 % of
+// which the MFMAs do not hide, and what waves wait for LDS and each other.  (Taken back on the way: one wave per SIMD with both
+// halves 248 us, heads in front of a barrier at the round's end 240, zeros and probabilities of a row stored apart 257, fragments
+// two steps ahead instead of one 230, stores past the caches 228.)
+// Inputs or weights that parts cannot hold (parts.h; beyond 2^60 a sum of parts might overflow where the sum itself does not) send
+// a round, or all rounds of a member, through f32 MFMAs.
+typedef const __attribute__((address_space(1))) f32x4* global_f32x4;
+constexpr int EP_THREADS = 512;
+typedef unsigned u32x2_parts __attribute__((ext_vector_type(2)));
+
+template <int KS, int NO, bool ACTION>
+__global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const EnsembleArgs a) {
+    constexpr int BUFFER = KS * 3072, RAW_AT = 3 * BUFFER, W2_AT = RAW_AT + 8 * 6144, SUMS_AT = W2_AT + 4096, PROBS_AT = SUMS_AT + 16384, FLAGS_AT = PROBS_AT + 16384 / 2;
+    static_assert(KS == 2 || KS == 4 || KS == 8, "steps of 16 inputs, at most one for each wave to split");
+    // the barrier stands in front of this step (with two steps: behind them); a wave's share of the next inputs is split before
+    // it, and all of the second layer
+    constexpr int BARRIER = KS == 2 ? 2 : KS / 2, FEATURES = 16 / BARRIER, SPLIT = KS == 8 ? 1 : 0;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 31, g = lane >> 5;
+    const int half = wave >> 2, pair = wave & 3;
+    const int K0 = a.k0, N = a.n, NOUT = a.nout;
+    const long batch = a.batch;
+    const int tiles = (int)a.tiles;                    // (the launcher sees to it that they fit)
+    const bool active = (int)blockIdx.y * 4 + pair < a.members;
+    const int e = active ? (int)blockIdx.y * 4 + pair : a.members - 1;
+    const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+
+    auto load8 = [&](const float* row, int s, f32x4 (&v)[2]) {      // k = 16 s + 8 g .. + 7 of a row of x or W1
+        const int k = 16 * s + 8 * g;
+        const bool there = k < K0;                                  // (K0 is a multiple of 8)
+        const global_f32x4 at = (global_f32x4)(row + (there ? k : 0));
+        v[0] = at[0];
+        v[1] = at[1];
+        return there;
+    };
+    unsigned least = 0xffffffffu;
+    float most = 0.f;
+    auto track = [&](float x, float y) {
+        const unsigned wx = parts_magnitude(x), wy = parts_magnitude(y), w = wx < wy ? wx : wy;
+        least = w < least ? w : least;
+        most = fmaxf(fmaxf(most, fabsf(x)), fabsf(y));
+    };
+    auto out_of_range = [&]() {                                     // (NaN: a NaN either way)
+        const bool bad = __any(parts_tiny(least) || most > 0x1p60f);
+        least = 0xffffffffu;
+        most = 0.f;
+        return bad;
+    };
+
+    // ---- inputs: this wave's share of a round is step `wave` of its tile (with fewer steps than waves some do the same),
+    //      32 bytes a lane, by DMA into a ring of three ----
+    const int my_step = wave % KS;
+    const bool there = 16 * my_step + 8 * g < K0;      // (K0 is a multiple of 8)
+    const int stride = gridDim.x, mine = (tiles - (int)blockIdx.x + stride - 1) / stride;      // rounds: tiles blockIdx.x + n stride (at least one)
+    auto tile_at = [&](int n) { return (int)blockIdx.x + (n < mine ? n : 0) * stride; };
+    const unsigned raw_at = RAW_AT + wave * 6144;
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)lds);
+    auto fetch_share = [&](int n, unsigned slot) {
+        long row = (long)tile_at(n) * EN_ROWS + r;
+        row = row < batch ? row : batch - 1;
+        const unsigned char* const at = there ? (const unsigned char*)(a.x + row * K0 + 16 * my_step + 8 * g) : (const unsigned char*)kZeroChunk;
+        dma_to_lds_addr(at, lds0 + raw_at + slot * 2048);
+        dma_to_lds_addr(there ? at + 16 : at, lds0 + raw_at + slot * 2048 + 1024);
+    };
+    // one twelfth of splitting it: part i of numbers 2 d and 2 d + 1
+    f32x4 raw[2];
+    auto read_share = [&](unsigned slot) {
+        raw[0] = *reinterpret_cast<const f32x4*>(lds + raw_at + slot * 2048 + lane * 16);
+        raw[1] = *reinterpret_cast<const f32x4*>(lds + raw_at + slot * 2048 + 1024 + lane * 16);
+    };
+    u32x2_parts split_to[3];
+    float two[2];
+    auto split_slice = [&](unsigned buffer, int slice) {
+        const int d = slice / 3, i = slice % 3;
+        if (i == 0) {
+            two[0] = raw[d >> 1][2 * (d & 1)];
+            two[1] = raw[d >> 1][2 * (d & 1) + 1];
+            track(two[0], two[1]);
+        }
+        split_to[i][d & 1] = take_parts(two[0], two[1]);
+        if (i < 2) asm volatile("" : "+v"(two[0]), "+v"(two[1]));
+        if (slice % 6 == 5) {
+            unsigned char* const at = lds + buffer * BUFFER + my_step * 3072 + lane * 16 + (d >> 1) * 8;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) *reinterpret_cast<u32x2_parts*>(at + k * 1024) = split_to[k];
+        }
+    };
+    unsigned* const flags = reinterpret_cast<unsigned*>(lds + FLAGS_AT);     // [buffer][wave]: inputs that parts cannot hold
+    auto raise_flag = [&](unsigned buffer) {
+        const bool bad = out_of_range();
+        flags[buffer * 8 + wave] = bad;                // (every lane the same)
+    };
+    fetch_share(0, 0);
+    fetch_share(1, 1);
+    fetch_share(2, 2);
+
+    // ---- this half of the member's hidden layer, once ----
+    parts_u32x4 w1[KS][3];
+    {
+        const float* const w = a.w1 + ((long)e * EN_HIDDEN + 32 * half + r) * K0;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            f32x4 v[2];
+            if (!load8(w, s, v)) v[0] = v[1] = zero4;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) track(v[d >> 1][2 * (d & 1)], v[d >> 1][2 * (d & 1) + 1]);
+            split_parts(v, w1[s]);
+        }
+    }
+    const bool w_bad = out_of_range();
+    // W2[e][o][32 half + 8 a4 + 4 g ..] at (o * 4 + a4) * 2 + g of the wave's 512 bytes, rows past NOUT are zeros
+    f32x4* const w2 = reinterpret_cast<f32x4*>(lds + W2_AT + wave * 512);
+    if (lane < 32) {
+        const int o = lane >> 3, rest = lane & 7;
+        const f32x4 v = *(global_f32x4)(a.w2 + ((long)e * N + (o < NOUT ? o : 0)) * EN_HIDDEN + 32 * half + 4 * rest);
+        w2[lane] = o < NOUT ? v : zero4;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    read_share(0);
+#pragma unroll
+    for (int i = 0; i < 12; ++i) split_slice(0, i);
+    raise_flag(0);
+    __syncthreads();
+
+    // ---- heads of rounds n and, for the lanes with g = 1, n + 1: the chain costs the same for 64 lanes as for 32 ----
+    // sums: [round % 4][pair][half][output][row]
+    float* const sums = reinterpret_cast<float*>(lds + SUMS_AT) + pair * 256;
+    const int limit = a.mask_size > 0 ? a.mask_size : NOUT, s4 = N >> 2;
+    const bool quads = (N & 3) == 0;
+    float* const policy = a.policy + (long)e * batch * N;
+    f32x4* const probs = reinterpret_cast<f32x4*>(lds + PROBS_AT) + pair * 32;         // [round % 4][pair][row], the first four columns
+    auto heads = [&](int n, bool both) {
+        if (!active) return;
+        const int j = n + (both ? g : 0);
+        const float* const at = sums + (j & 3) * 1024 + r;
+        float p[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int o = 0; o < NO; ++o) p[o] = o < NOUT ? at[32 * o] + at[128 + 32 * o] : 0.f;
+        switch (a.head) {
+            case SP_HEAD_SOFTMAX: head_values4<SP_HEAD_SOFTMAX>(p, limit); break;
+            case SP_HEAD_REGRET_MATCHING: head_values4<SP_HEAD_REGRET_MATCHING>(p, limit); break;
+            case SP_HEAD_SOFTMAX_RM: head_values4<SP_HEAD_SOFTMAX_RM>(p, limit); break;
+            default: break;
+        }
+        if (quads) probs[(j & 3) * 128 + r] = f32x4{p[0], 1 < NOUT ? p[1] : 0.f, 2 < NOUT ? p[2] : 0.f, 3 < NOUT ? p[3] : 0.f};
+        const long row = ((long)blockIdx.x + (long)j * stride) * EN_ROWS + r;
+        if (g == 1 && !both || row >= batch) return;
+        if (!quads) {
+            float* const to = policy + row * N;
+#pragma unroll
+            for (int o = 0; o < 4; ++o)
+                if (o < NOUT) to[o] = p[o];
+            for (int c = NOUT; c < N; ++c) to[c] = 0.f;
+        }
+        if constexpr (ACTION) {
+            const long grow = (long)e * batch + row;
+            a.action[grow] = head_pick4(p, a.u != nullptr ? a.u[grow] : reference_row_uniform(a.ph, grow));
+        }
+    };
+    // Rows leave whole, 16 bytes per lane, in four stores from each wave of a pair for its 16 rows of a tile (lines that are written
+    // in two pieces leave the L2 in two).  Rows past the tile or the batch are the last one once more: every lane stores every time,
+    // so the counter of outstanding accesses runs at a known pace.
+    const bool rows_out = quads && active;
+    const int shift = (s4 & (s4 - 1)) == 0 ? 31 - __builtin_clz(s4) : -1;
+    auto store_quarter = [&](int n, int q) {
+        if (!rows_out) return;
+        int piece = lane + 64 * q;
+        asm volatile("" : "+v"(piece));                // (computed here: kept, the four of them are registers that are not there)
+        const int rr0 = shift >= 0 ? piece >> shift : piece / s4, c = piece - rr0 * s4;
+        const long tile0 = (long)tile_at(n) * EN_ROWS, left = batch - 1 - tile0;
+        const int first = 16 * half + (rr0 < 15 ? rr0 : 15), rr = first < left ? first : (int)left;
+        const f32x4 v = probs[(n & 3) * 128 + rr];
+        *reinterpret_cast<f32x4*>(policy + tile0 * N + (rr * N + 4 * c)) = c == 0 ? v : zero4;
+    };
+
+    f32x16 acc[2];
+    auto clear = [&](f32x16& c) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) c[i] = 0.f;
+    };
+    clear(acc[1]);
+    parts_u32x4 xf[2][3];
+    auto read_step = [&](unsigned buffer, int s, int i) {
+        xf[s & 1][i] = *reinterpret_cast<const parts_u32x4*>(lds + buffer * BUFFER + s * 3072 + i * 1024 + lane * 16);
+    };
+#pragma unroll
+    for (int i = 0; i < 3; ++i) read_step(0, 0, i);
+    unsigned now = 0, next = 1;                        // the buffers of this round's inputs and of the next one's
+    // W2 of G features at a time (four outputs of four features are registers that are not there)
+    constexpr int G = NO == 4 ? 2 : 4;
+    typedef float weights_of __attribute__((ext_vector_type(G)));
+    weights_of wv[NO];
+    auto second_weights = [&](int f) {                 // of features f .. f + G - 1 of the 16 that this lane holds
+#pragma unroll
+        for (int o = 0; o < NO; ++o) wv[o] = *reinterpret_cast<const weights_of*>((const float*)(w2 + (o * 4 + (f >> 2)) * 2 + g) + (f & 3));
+    };
+    second_weights(0);
+    // Round n: its products into acc[B]; the second layer of the round before it from acc[B ^ 1]; the inputs of the next.
+    auto work = [&](auto B_, int n) {
+        constexpr int B = decltype(B_)::value;
+        // The inputs of round n + 1 have landed: behind them came those of round n + 2 and, from round 4 on, four
+        // stores of each of the last two rounds (a head's store more, and the wait is for a little more).
+        if (rows_out && n >= 6) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+        if (SPLIT == 0) read_share(next);
+        if (B == 0 && n >= 4 && ((n >> 1) & 1) == half) heads(n - 4, true);
+        float s2[NO][2];
+#pragma unroll
+        for (int o = 0; o < NO; ++o) s2[o][0] = s2[o][1] = 0.f;
+        auto second = [&](int f) {
+            const float y = vmax(acc[B ^ 1][f], 0.f);
+#pragma unroll
+            for (int o = 0; o < NO; ++o) {
+                s2[o][f & 1] = __builtin_fmaf(wv[o][f % G], y, s2[o][f & 1]);
+                asm volatile("" : "+v"(s2[o][f & 1]));              // (here, and not where the sums are used)
+            }
+            if (f % G == G - 1) second_weights((f + 1) % 16);
+        };
+        auto put_sum = [&](int o, bool write) {
+            if (!write) {
+                s2[o][0] = s2[o][0] + s2[o][1];
+                s2[o][0] += __shfl_xor(s2[o][0], 32);
+            } else if (g == 0) {
+                sums[((n - 1) & 3) * 1024 + half * 128 + r + 32 * o] = s2[o][0];
+            }
+        };
+        auto barrier = [&]() {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xC07F);                     // lgkmcnt(0): loads and stores stay under way
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
+        const parts_u32x4 flag0 = *reinterpret_cast<const parts_u32x4*>(flags + now * 8), flag1 = *reinterpret_cast<const parts_u32x4*>(flags + now * 8 + 4);
+        // (the sums of the round before are there: its last MFMA ended a head, or a turn of the other wave, ago; what the compiler
+        //  cannot see is that they come from MFMAs)
+        asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[B ^ 1]));
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            constexpr int PW[6] = {2, 0, 1, 1, 0, 0}, PX[6] = {0, 2, 1, 0, 1, 0};
+            if (s == BARRIER) barrier();
+#pragma unroll
+            for (int m = 0; m < 6; ++m) {
+                if (s == 0 && m == 0)
+                    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(acc[B]) : "v"(w1[s][PW[m]]), "v"(xf[s & 1][PX[m]]));
+                else
+                    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc[B]) : "v"(w1[s][PW[m]]), "v"(xf[s & 1][PX[m]]));
+                // in the shadow of this MFMA:
+                if (m < 3 && s + 1 < KS) read_step(now, s + 1, m);
+                if (m < 3 && s + 1 == KS && BARRIER < KS) read_step(next, 0, m);
+                if (s < BARRIER)
+#pragma unroll
+                    for (int f = s * FEATURES + m * FEATURES / 6; f < s * FEATURES + (m + 1) * FEATURES / 6; ++f) second(f);
+                if (s + 1 == SPLIT && m == 4) read_share(next);
+                if (s == SPLIT || s == SPLIT + 1) {
+                    split_slice(next, (s - SPLIT) * 6 + m);
+                    if (s == SPLIT + 1 && m == 5) {
+                        raise_flag(next);
+                    }
+                }
+                if (s == 0 && m == 5) fetch_share(n + 3, now);
+                constexpr int APART = BARRIER < KS ? 6 * (KS - BARRIER) / 4 : 1;
+                if (s >= BARRIER && ((s - BARRIER) * 6 + m) % APART == 1 && n >= 4) store_quarter(n - 4, ((s - BARRIER) * 6 + m) / APART);
+                if (s == BARRIER && m < NO) put_sum(m, false);
+                if (s == BARRIER + 1 && m < NO) put_sum(m, true);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if constexpr (BARRIER + 1 >= KS) {
+#pragma unroll
+            for (int o = 0; o < NO; ++o) {
+                if (BARRIER >= KS) put_sum(o, false);
+                put_sum(o, true);
+            }
+        }
+        if constexpr (BARRIER >= KS) {
+            barrier();
+#pragma unroll
+            for (int i = 0; i < 3; ++i) read_step(next, 0, i);
+            if (n >= 4)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) store_quarter(n - 4, q);
+        }
+        if (w_bad || __any((flag0.x | flag0.y | flag0.z | flag0.w | flag1.x | flag1.y | flag1.z | flag1.w) != 0)) {
+            asm volatile("s_nop 15\n\ts_nop 15" : "+v"(acc[B]));
+            clear(acc[B]);
+            long row = (long)tile_at(n) * EN_ROWS + r;
+            row = row < batch ? row : batch - 1;
+            for (int s = 0; s < (K0 + 15) / 16; ++s) {
+                f32x4 xv[2], wv1[2];
+                if (!load8(a.x + row * K0, s, xv)) xv[0] = xv[1] = zero4;
+                if (!load8(a.w1 + ((long)e * EN_HIDDEN + 32 * half + r) * K0, s, wv1)) wv1[0] = wv1[1] = zero4;
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        asm volatile("s_nop 3\n\tv_mfma_f32_32x32x2_f32 %0, %1, %2, %0" : "+v"(acc[B]) : "v"(wv1[c][i]), "v"(xv[c][i]));
+            }
+        }
+        now = next;
+        next = next == 2 ? 0 : next + 1;
+    };
+    for (int n = 0;;) {                               // (one round more than there are: its products are not used)
+        work(std::integral_constant<int, 0>{}, n);
+        if (n++ == mine) break;
+        work(std::integral_constant<int, 1>{}, n);
+        if (n++ == mine) break;
+    }
+    // what the rounds did not get to: the last two (or one, if it has no partner), and with an odd last round the two before it
+    __syncthreads();
+    const int last = (mine - 1) & ~1;                // the even round of the last pair
+    if (half == 0) heads(last, last + 1 < mine);
+    else if (last >= 2 && last + 2 > mine) heads(last - 2, true);
+    __syncthreads();
+    for (int n = mine > 3 ? mine - 3 : 0; n < mine; ++n)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) store_quarter(n, q);
+}
+
 // ONE ensemble layer and its head: policy[e] = head(x . W[e]^T) for a head of at most 4 computed outputs, or
 // word[e][r] = (OR over j < 32 of (not (y[r][j] <= 0)) << j) mod modulo with y = x . W[e]^T -- the graphs of the
 // reference's other agents (game/nl_hu_holdem/model_cem.spi:84-100: matmul_ensemble_with_adjoint -> masked regret
@@ -332,6 +665,38 @@ static const void* pick_ensemble_kernel_kg(bool exact, bool action) {
     if (exact) return action ? (const void*)mlp_ensemble_kernel<KG, true, true> : (const void*)mlp_ensemble_kernel<KG, true, false>;
     return action ? (const void*)mlp_ensemble_kernel<KG, false, true> : (const void*)mlp_ensemble_kernel<KG, false, false>;
 }
+// Rounds per workgroup on the bf16 pipe: four members a workgroup, one workgroup per unit.
+static long ensemble_parts_blocks(long members, long tiles) {
+    const long blocks = device_cu_count() / ((members + 3) / 4);
+    return blocks < 1 ? 1 : blocks < tiles ? blocks : tiles;
+}
+// Which kernel takes two layers.  The one on the bf16 pipe does a round of four members in 3.5 us (128 inputs), the f32 one a
+// tile of one in 5.2 on each of a unit's four SIMDs; below three members the former leaves half of a workgroup idle, and where
+// the latter has one tile per wave it is through before two rounds are (us, f32 / bf16 pipe, 128 inputs: 2 x 65536 rows 33 / 37,
+// 5 x 6144 16.0 / 18.2; 4 x 6144 15.3 / 15.1, 9 x 6144 27.6 / 21.1, 3 x 65536 71 / 36, 5 x 65536 105 / 58, 9 x 65536 182 / 83,
+// 32 x 65536 346 / 230).
+static bool ensemble_takes_parts(long members, long batch) {
+    const long tiles = (batch + EN_ROWS - 1) / EN_ROWS, blocks = ensemble_parts_blocks(members, tiles);
+    const long each = (device_cu_count() + members - 1) / members;      // workgroups of a member in ensemble_launch
+    if (members < 3 || tiles > 2147480000l) return false;
+    return !(tiles <= 4 * each && tiles > blocks);
+}
+
+template <int KS>
+static int launch_ensemble_parts(EnsembleArgs& a, hipStream_t stream, const char* what) {
+    const bool action = a.action != nullptr;
+    const void* kernel = a.nout <= 3 ? (action ? (const void*)mlp_ensemble_parts_kernel<KS, 3, true> : (const void*)mlp_ensemble_parts_kernel<KS, 3, false>)
+                                     : (action ? (const void*)mlp_ensemble_parts_kernel<KS, 4, true> : (const void*)mlp_ensemble_parts_kernel<KS, 4, false>);
+    const int lds_bytes = 3 * KS * 3072 + 8 * 6144 + 4096 + 16384 + 8192 + 128;
+    const int rc = ensure_dynamic_lds(kernel, lds_bytes);
+    if (rc != SP_OK) return rc;
+    a.tiles = (a.batch + EN_ROWS - 1) / EN_ROWS;
+    const long groups = (a.members + 3) / 4, gx = ensemble_parts_blocks(a.members, a.tiles);
+    void* args[] = {(void*)&a};
+    const hipError_t err = hipLaunchKernel(kernel, dim3((unsigned)gx, (unsigned)groups), dim3(EP_THREADS), args, lds_bytes, stream);
+    if (err != hipSuccess) return fail(SP_ERR_DEVICE, "%s: launch failed: %s", what, hipGetErrorString(err));
+    return check_launch(what);
+}
 static const void* pick_ensemble_kernel(int kg, bool exact, bool action) {
     return kg == 4 ? pick_ensemble_kernel_kg<4>(exact, action) : kg == 8 ? pick_ensemble_kernel_kg<8>(exact, action)
                                                                          : pick_ensemble_kernel_kg<16>(exact, action);
@@ -409,6 +774,10 @@ extern "C" int sp_mlp_forward_ensemble(int dtype, const void* x, int32_t n_layer
     a.policy = policy_out; a.action = action_out; a.batch = batch; a.members = members; a.k0 = k0; a.n = n; a.nout = nout;
     a.head = head; a.mask_size = mask_size;
     const int kg = k0 <= 32 ? 4 : k0 <= 64 ? 8 : k0 <= 128 ? 16 : 32;
+    if (n_layers == 2 && ensemble_takes_parts(a.members, batch)) {
+        return kg == 4 ? launch_ensemble_parts<2>(a, (hipStream_t)stream, __func__) : kg == 8 ? launch_ensemble_parts<4>(a, (hipStream_t)stream, __func__)
+                                                                                               : launch_ensemble_parts<8>(a, (hipStream_t)stream, __func__);
+    }
     const void* kernel = n_layers == 2 ? pick_ensemble_kernel(kg, k0 == 8 * kg, action_out != nullptr)
                        : action_out != nullptr ? pick_layer_kernel<1>(kg, k0 == 8 * kg) : pick_layer_kernel<0>(kg, k0 == 8 * kg);
     return ensemble_launch(kernel, a, (hipStream_t)stream, __func__);
@@ -442,6 +811,10 @@ extern "C" int sp_ensemble_binarize(int dtype, const void* x, const void* weight
 
 namespace {
 struct MlpEnsembleKernelNames {
-    MlpEnsembleKernelNames() { register_kernel("mlp_forward_ensemble", (const void*)mlp_ensemble_kernel<16, true, false>, EN_THREADS); }
+    MlpEnsembleKernelNames() {
+        register_kernel("mlp_forward_ensemble", (const void*)mlp_ensemble_kernel<16, true, false>, EN_THREADS);
+        register_kernel("mlp_forward_ensemble_parts", (const void*)mlp_ensemble_parts_kernel<8, 3, false>, EP_THREADS);
+        register_kernel("mlp_forward_ensemble_parts_action", (const void*)mlp_ensemble_parts_kernel<8, 4, true>, EP_THREADS);
+    }
 } mlp_ensemble_kernel_names;
 }  // namespace

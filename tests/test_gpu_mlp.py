@@ -524,3 +524,81 @@ def test_ensemble_binarize(LY, members, batch, k0, n, modulo):
     node = host(primitives.binarize(y0, modulo)).view(np.uint32)
     sure0 = (np.abs(host(y0)[:, :32]) > 1e-4).all(axis=1)
     assert (node[sure0] == got[0][sure0]).all()
+
+
+# The ensemble on the bf16 pipe (three members and more): tiles of 32 rows per workgroup 1, 2, ... 8, a ragged last tile, widths of
+# a step of 16 and odd halves of one, rows of 4, 16, 20 and 64 columns, 1 to 4 outputs, a width that is no multiple of 4
+@pytest.mark.parametrize("members,batch,dims,head,mask,sample", [
+    (3, 31, [8, 64, 4], "softmax", 0, True), (4, 32 * 256 + 1, [16, 64, 16], "regret_matching", 2, False),
+    (5, 32 * 128 * 3, [24, 64, 20], "softmax", 3, False), (5, 32 * 128 * 4 - 17, [40, 64, 64], "softmax_regret_matching", 4, True),
+    (6, 32 * 128 * 5 + 9, [64, 64, 64], "regret_matching", 3, False), (7, 32 * 128 * 2 + 32, [72, 64, 6], "softmax", 1, True),
+    (4, 32 * 256 * 6 + 33, [128, 64, 8], "none", None, False), (9, 32 * 85 * 7 + 40, [120, 64, 64], "regret_matching", 4, False),
+    (9, 32 * 85 * 8, [128, 64, 64], "softmax", 3, True), (256, 200, [48, 64, 12], "regret_matching", 3, False)])
+def test_ensemble_in_three_parts(LY, members, batch, dims, head, mask, sample):
+    """Against float64: the hidden layer no further off than f32 sums are, so the f32 bar of the head holds row by row wherever the
+    head itself is not the quotient of two small numbers; exact zeros behind the mask; actions given the kernel's own policy."""
+    announce("ensemble parts members=%d batch=%d dims=%s head=%s mask=%s" % (members, batch, dims, head, mask))
+    if head == "none":
+        dims = dims[:2] + [4]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(batch)
+    x = torch.randn((batch, dims[0]), generator=gen, device="cuda")
+    w1 = torch.randn((members, 64, dims[0]), generator=gen, device="cuda") / dims[0] ** 0.5
+    w2 = torch.randn((members, dims[2], 64), generator=gen, device="cuda") / 8
+    u = 1 - torch.rand((members, batch), generator=gen, device="cuda") if sample else None
+    out = LY.mlp_forward_ensemble(x, (w1, w2), head, u, mask or 0)
+    policy, action = out if sample else (out, None)
+    cols = mask or dims[2]
+    assert (policy[:, :, cols:] == 0).all()
+    for e in range(members):
+        z = torch.relu(x.double() @ w1[e].double().T) @ w2[e, :cols].double().T
+        if head in ("softmax", "softmax_regret_matching"):
+            z = torch.softmax(z, 1)
+        got = policy[e, :, :cols].double()
+        if head == "regret_matching":
+            z = torch.relu(z)
+            total = z.sum(1, keepdim=True)
+            clear = (total > 0.01).squeeze(1)
+            assert clear.any()
+            z, got = (z / total)[clear], got[clear]
+        assert ((got - z).norm() / z.norm()).item() < 1e-5, e
+        if sample:
+            assert (host(action[e]) == orow.discrete_sampling(host(policy[e]), host(u[e]))).all(), e
+
+
+def test_ensemble_in_three_parts_keeps_what_parts_cannot_hold(LY):
+    """Members 0 and 1 of four on the bf16 pipe against the same two alone on the f32 kernel: inputs and weights with infinities, NaN,
+    values whose bf16 is infinite, values below 2^-110."""
+    announce("ensemble parts, special values")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    batch = 32 * 256 * 2
+    x = torch.randn((batch, 128), generator=gen, device="cuda")
+    w1 = torch.randn((4, 64, 128), generator=gen, device="cuda") / 11
+    w2 = torch.randn((4, 16, 64), generator=gen, device="cuda") / 8
+    x[3, 5] = float("inf")
+    x[40, 7] = float("-inf")
+    x[100, 0] = float("nan")
+    x[200] *= 2.0 ** -125
+    x[300] = 0.0
+    x[300, 9] = 3.4028234e38
+    x[batch - 1] *= 2.0 ** 90
+    for scale, poison in ((1.0, None), (1.0, float("inf")), (2.0 ** -118, None)):
+        w = w1.clone()
+        w[1] *= scale
+        if poison is not None:
+            w[1, 9, 3] = poison
+        four = LY.mlp_forward_ensemble(x, (w, w2), "softmax", mask_size=3)
+        two = LY.mlp_forward_ensemble(x, (w[:2].contiguous(), w2[:2].contiguous()), "softmax", mask_size=3)
+        a, b = four[:2].cpu(), two.cpu()
+        assert torch.equal(a.isnan(), b.isnan())
+        ok = ~b.isnan()
+        assert (a[ok] - b[ok]).abs().max().item() < 1e-5
+
+
+@pytest.mark.parametrize("name", ["mlp_forward_ensemble_parts", "mlp_forward_ensemble_parts_action"])
+def test_the_parts_ensemble_kernels_are_named(name):
+    announce("kernel info " + name)
+    from ml import _lib
+    info = _lib.kernel_info(name)
+    assert info["threads_per_block"] == 512 and 0 < info["vgprs"] <= 256
