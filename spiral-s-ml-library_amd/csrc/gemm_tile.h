@@ -159,8 +159,9 @@ __device__ __forceinline__ void store_accumulators(const GemmArgs& g, unsigned c
         if (g.relu) write_tile(std::false_type{}, std::true_type{}, stream_t{});
         else write_tile(std::false_type{}, std::false_type{}, stream_t{});
     } else {
-        if (g.relu) write_tile(std::false_type{}, std::true_type{}, through_t{});
-        else write_tile(std::false_type{}, std::false_type{}, through_t{});
+        typedef std::conditional_t<RAGGED, plain_t, through_t> other_t;      // (see where the policy is picked)
+        if (g.relu) write_tile(std::false_type{}, std::true_type{}, other_t{});
+        else write_tile(std::false_type{}, std::false_type{}, other_t{});
     }
 }
 

@@ -399,6 +399,29 @@ def test_streamed_and_written_through_outputs_are_exact_on_integers(MM, m, n, k)
     assert (host(c) == 2.0 * want - 3.0 * c0).all()
 
 
+@pytest.mark.parametrize("m,n,k", [(700, 63, 64), (1000, 272, 128), (1031, 257, 64), (5003, 1001, 72), (4100, 1040, 64), (3000, 3002, 136)])
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
+def test_ragged_outputs_are_exact_whatever_their_rows_start_on(MM, dtype, m, n, k):
+    """Tiles that do not divide the shape stream C where its rows start on 64 bytes and leave it to the L2 where they do not: both,
+    in each output type and with each epilogue option, on small integers (every partial sum is exact)."""
+    announce("gemm ragged store policies, %s %dx%dx%d" % (dtype, m, n, k))
+    t = TORCH[dtype]
+    a = ((np.arange(m * k, dtype=np.int64).reshape(m, k) * 7 + 3) % 5 - 2).astype(np.float32)
+    b = ((np.arange(n * k, dtype=np.int64).reshape(n, k) * 5 + 1) % 7 - 3).astype(np.float32)
+    want = a @ b.T
+    ad, bd = dev(a, t), dev(b, t)
+    bias = ((np.arange(n) * 5) % 201 - 100).astype(np.float32)
+    for out in {"f32", dtype}:
+        got = host(MM.matmul_abt(ad, bd, out_dtype=TORCH[out]).float())
+        assert (got == ogemm.round_to(want, out)).all()
+        got = host(MM.matmul_abt(ad, bd, bias=dev(bias), relu=True, out_dtype=TORCH[out]).float())
+        assert (got == ogemm.round_to(np.maximum(want + bias, 0.0).astype(np.float32), out)).all()
+    c0 = ((np.arange(m * n, dtype=np.int64).reshape(m, n) * 3) % 17 - 8).astype(np.float32)
+    c = dev(c0.copy())
+    MM.matmul_abt(ad, bd, c, 2.0, -3.0)
+    assert (host(c) == 2.0 * want - 3.0 * c0).all()
+
+
 @pytest.mark.parametrize("dtype,m,n,k", [("bf16", 2048, 2048, 2048), ("bf16", 4096, 4096, 4096), ("bf16", 65536, 256, 512),
                                          ("bf16", 65536, 1024, 512), ("bf16", 16384, 256, 256), ("f32", 2048, 2048, 512),
                                          ("f16", 1000, 1000, 1024)])
