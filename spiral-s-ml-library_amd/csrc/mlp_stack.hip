@@ -20,9 +20,16 @@
 // tile per SIMD.
 // Measured, that stack over 16384 rows (node by node / every layer through part_product, a draw per tile / this kernel, us):
 // one model 32.8 / 13.8 / 10.3, 16 members 206 / 87 / 68.8 (the matrix pipe alone: 41).
+//   PARTS: the same with the products in three bf16 parts (below), 144 MFMAs of 16 cycles for 16 rows instead of 192 of 32, and
+// 300 vector instructions more, which run beside them: 16 members of 16384 rows 70 -> 52.5, of 57344 223 -> 157.  Bound by the
+// vector ALU (1100 instructions, 4400 cycles a tile, of 6100 measured) and the 7 us in which a workgroup's sixteen waves start
+// together, with the same phases.  Sixteen waves because their norms and heads hide behind each other's products (eight: 63.6
+// and 186).  The sums are closer to float64 than the f32 pipe's (error of the probabilities 0.63 to 0.88 of that, 1.00 where it
+// is the exponential's).
 #include "mlp_common.h"
 #include "row_common.h"
 #include "gemm_dma.h"
+#include "parts.h"
 
 #pragma clang fp contract(off)
 
@@ -33,7 +40,9 @@ constexpr int ST_MAX_LAYERS = 8;
 constexpr int ST_MAX_WIDTH = 128;
 constexpr int ST_MAX_OUT = 64;
 constexpr int ST_MAX_THREADS = 512;
+constexpr int ST_PARTS_THREADS = 1024;
 constexpr int ST_BLOCK = 1024;         // bytes of a 16 x 16 block of weights
+constexpr int ST_PARTS_UNIT = 3072;    // 16 features and 32 of K as three parts
 constexpr int ST_SCRATCH = ST_ROWS * ST_MAX_OUT * 4;   // per wave: the logits on their way into rows
 constexpr int ST_LDS = 160 * 1024;
 
@@ -111,10 +120,83 @@ __device__ __forceinline__ void part_product(const unsigned char*& wp, const f32
     }
 }
 
-// HT: 16-wide tiles of the widest layer (4 or 8).  FULL: the input and every hidden layer have exactly that many.  REGRET:
+// ---- the products on the bf16 matrix pipe: both operands as three bf16 parts (parts.h), six of the nine products, each of
+// 32 of K in one v_mfma_f32_16x16x32_bf16.  Lane group q holds k = 32 j + 4 q + i and 32 j + 16 + 4 q + i, so that a layer's
+// results are here, too, the next one's operand.
+typedef __bf16 stack_bf16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ void stack_parts(f32x4 v, f32x4 w, parts_u32x4 (&p)[3]) {
+    const parts_f32x4 both[2] = {{v[0], v[1], v[2], v[3]}, {w[0], w[1], w[2], w[3]}};
+    split_parts(both, p);
+}
+__device__ __forceinline__ f32x4 parts_mfma(parts_u32x4 w, parts_u32x4 x, f32x4 y) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(stack_bf16x8, w), __builtin_bit_cast(stack_bf16x8, x), y, 0, 0, 0);
+}
+
+struct PartsRange {                     // whether parts hold all of the numbers seen (NaN: a NaN either way)
+    unsigned least = 0xffffffffu;
+    float most = 0.f;
+    __device__ __forceinline__ void take(f32x4 v) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const unsigned w = parts_magnitude(v[i]);
+            least = w < least ? w : least;
+            most = fmaxf(most, fabsf(v[i]));
+        }
+    }
+    __device__ __forceinline__ bool wide() const { return parts_tiny(least) || most > 0x1p60f; }
+};
+
+// A full layer, the weights of a tile of features and 32 of K read ahead of the products of the one before.
+__device__ __forceinline__ void parts_product(const unsigned char*& wp, const parts_u32x4 (&x)[2][3], f32x4 (&y)[4]) {
+    parts_u32x4 w[2][3];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) y[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s <= 8; ++s) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (s < 8) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) w[s & 1][i] = *reinterpret_cast<const parts_u32x4*>(wp + s * ST_PARTS_UNIT + i * 1024);
+        }
+        if (s > 0) {
+            const int j = (s - 1) >> 2, t = (s - 1) & 3, now = (s - 1) & 1;
+            y[t] = parts_mfma(w[now][2], x[j][0], y[t]);
+            y[t] = parts_mfma(w[now][0], x[j][2], y[t]);
+            y[t] = parts_mfma(w[now][1], x[j][1], y[t]);
+            y[t] = parts_mfma(w[now][1], x[j][0], y[t]);
+            y[t] = parts_mfma(w[now][0], x[j][1], y[t]);
+            y[t] = parts_mfma(w[now][0], x[j][0], y[t]);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    wp += 8 * ST_PARTS_UNIT;
+}
+
+// The product of rows that parts cannot hold, in f32 from the weights where they are, into the wave's scratch (a lane's own
+// 16 bytes of each tile of features).
+template <int HT>
+__device__ __forceinline__ void wide_product(const float* W, int K, int F, const f32x4 (&x)[HT], unsigned char* scratch, int r, int q) {
+    for (int t = 0; 16 * t < F; ++t) {
+        f32x4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < HT; ++j) {
+            const int row = 16 * t + r, col = 16 * j + 4 * q;
+            f32x4 w = {0.f, 0.f, 0.f, 0.f};
+            if (row < F && col < K) w = *reinterpret_cast<const f32x4*>(W + (long)row * K + col);
+            if (16 * j < K)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[j][i], y, 0, 0, 0);
+        }
+        *reinterpret_cast<f32x4*>(scratch + t * 1024 + (q * 16 + r) * 16) = y;
+    }
+}
+
+// HT: 16-wide tiles of the widest layer (4 or 8).  PARTS: products in bf16 parts (FULL, and as many outputs).  FULL: the input and every hidden layer have exactly that many.  REGRET:
 // regret matching instead of softmax as the head (of mask_size columns, either).
-template <int HT, bool REGRET, bool FULL>
-__global__ __launch_bounds__(ST_MAX_THREADS, HT == 4 ? 4 : 2) void mlp_stack_kernel(const StackArgs a) {
+template <int HT, bool REGRET, bool FULL, bool PARTS = false>
+__global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 ? 4 : 2) void mlp_stack_kernel(const StackArgs a) {
+    static_assert(!PARTS || HT == 4, "the scratch holds one product of 64 features");
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -141,11 +223,13 @@ __global__ __launch_bounds__(ST_MAX_THREADS, HT == 4 ? 4 : 2) void mlp_stack_ker
 
     // ---- the member's weights, once per workgroup ----
     const unsigned lds0 = (unsigned)(size_t)lds;
-    {
+    bool weights_wide = false;
+    auto weights_of = [&](int l) { return a.w[l] + (long)e * (l + 1 < layers ? (long)a.dims[l] * a.dims[l + 1] : a.out_stride); };
+    if constexpr (!PARTS) {
         unsigned dst = lds0;
         for (int l = 0; l < layers; ++l) {
             const int K = a.dims[l], F = a.dims[l + 1], kt = (K + 15) >> 4, nt = (F + 15) >> 4;
-            const float* W = a.w[l] + (long)e * (l + 1 < layers ? (long)F * K : a.out_stride);
+            const float* W = weights_of(l);
             const bool k_outer = FULL && (l + 1 < layers || nt == ST_MAX_OUT / 16);      // as full_product reads them
             const int inner = k_outer ? nt : kt;
             for (int b = wave; b < kt * nt; b += waves) {
@@ -157,6 +241,42 @@ __global__ __launch_bounds__(ST_MAX_THREADS, HT == 4 ? 4 : 2) void mlp_stack_ker
             dst += kt * nt * ST_BLOCK;
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    } else {
+        // units wave, wave + waves, ... of the whole stack, two of them in flight
+        const int units = 8 * layers;
+        PartsRange range;
+        for (int n0 = wave; n0 < units; n0 += 2 * waves) {
+            f32x4 v[2][2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int n = n0 + i * waves < units ? n0 + i * waves : n0, l = n >> 3, K = a.dims[l];
+                const int row = 16 * (n & 3) + r, col = 32 * ((n >> 2) & 1) + 4 * q;
+                const float* const at = weights_of(l) + (long)row * K + col;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    v[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    if (row < a.dims[l + 1] && col + 16 * h < K) v[i][h] = *reinterpret_cast<const f32x4*>(at + 16 * h);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                if (i == 1 && n0 + waves >= units) break;
+                parts_u32x4 p[3];
+                range.take(v[i][0]);
+                range.take(v[i][1]);
+                stack_parts(v[i][0], v[i][1], p);
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    *reinterpret_cast<parts_u32x4*>(lds + (n0 + i * waves) * ST_PARTS_UNIT + k * 1024 + lane * 16) = p[k];
+            }
+        }
+        int* const flags = reinterpret_cast<int*>(lds + a.w_bytes);       // (the scratch, not in use yet)
+        flags[wave] = __any(range.wide());                                // every lane the same
+        __syncthreads();
+        int any = 0;
+        for (int w = 0; w < waves; ++w) any |= flags[w];
+        weights_wide = __builtin_amdgcn_readfirstlane(any) != 0;
         __syncthreads();
     }
 #pragma unroll
@@ -180,10 +300,31 @@ __global__ __launch_bounds__(ST_MAX_THREADS, HT == 4 ? 4 : 2) void mlp_stack_ker
         const unsigned char* wp = lds + lane * 16;
         f32x4 xn[HT];
         load_x(tile + stride < a.tiles ? tile + stride : tile, xn);
+        // rows with numbers that parts cannot hold get the f32 product: the others' sums are theirs alone either way
+        auto product_of_parts = [&](int l, f32x4 (&y)[HT]) {
+          if constexpr (PARTS) {
+            PartsRange range;
+            parts_u32x4 xp[2][3];
+#pragma unroll
+            for (int j = 0; j < HT; ++j) range.take(x[j]);
+            const unsigned long long lanes = __ballot(range.wide() || weights_wide);
+            if (lanes != 0) wide_product<HT>(weights_of(l), a.dims[l], a.dims[l + 1], x, scratch, r, q);
+            stack_parts(x[0], x[1], xp[0]);
+            stack_parts(x[2], x[3], xp[1]);
+            parts_product(wp, xp, y);
+            if (lanes != 0) {
+                const bool mine = (((lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) >> r) & 1) != 0;
+#pragma unroll
+                for (int t = 0; t < HT; ++t)
+                    if (mine && 16 * t < a.dims[l + 1]) y[t] = *reinterpret_cast<const f32x4*>(scratch + t * 1024 + lane * 16);
+            }
+          }
+        };
         for (int l = 0; l + 1 < layers; ++l) {
             const int nt = a.dims[l + 1] >> 4;
             f32x4 y[HT];
-            if constexpr (FULL) full_product<HT, HT>(wp, x, y);
+            if constexpr (PARTS) product_of_parts(l, y);
+            else if constexpr (FULL) full_product<HT, HT>(wp, x, y);
             else part_product<HT, HT>(wp, x, y, (a.dims[l] + 15) >> 4, nt);
             const int act = a.acts[l];
             if (act & SP_STACK_LN_L2) {       // local_ln_l2 (ml/primitives.spi:701-703)
@@ -212,7 +353,8 @@ __global__ __launch_bounds__(ST_MAX_THREADS, HT == 4 ? 4 : 2) void mlp_stack_ker
         }
         f32x4 logits[ST_MAX_OUT / 16];
         const int nt = (a.dims[layers] + 15) >> 4;
-        if (FULL && nt == ST_MAX_OUT / 16) full_product<HT, ST_MAX_OUT / 16>(wp, x, logits);
+        if constexpr (PARTS) product_of_parts(layers - 1, logits);
+        else if (FULL && nt == ST_MAX_OUT / 16) full_product<HT, ST_MAX_OUT / 16>(wp, x, logits);
         else part_product<HT, ST_MAX_OUT / 16>(wp, x, logits, (a.dims[layers - 1] + 15) >> 4, nt);
 
         // ---- logits into rows: quad c of row r at slot c ^ r of its 256 bytes ----
@@ -294,9 +436,9 @@ __global__ __launch_bounds__(ST_MAX_THREADS, HT == 4 ? 4 : 2) void mlp_stack_ker
 
 using namespace sp;
 
-template <int HT, bool FULL>
+template <int HT, bool FULL, bool PARTS = false>
 static const void* pick_stack_kernel(bool regret) {
-    return regret ? (const void*)mlp_stack_kernel<HT, true, FULL> : (const void*)mlp_stack_kernel<HT, false, FULL>;
+    return regret ? (const void*)mlp_stack_kernel<HT, true, FULL, PARTS> : (const void*)mlp_stack_kernel<HT, false, FULL, PARTS>;
 }
 
 // Bytes of LDS the weights take; computed: the outputs that a mask leaves.
@@ -372,27 +514,41 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
     a.mask_size = masked ? mask_size : n;
     a.dims[n_layers] = a.mask_size;
     a.out_stride = (long)n * dims[n_layers - 1];
-    const long w_bytes = stack_weight_bytes(n_layers, dims, a.mask_size);
+    long w_bytes = stack_weight_bytes(n_layers, dims, a.mask_size);
     rc = require_gfx950(__func__);
     if (rc != SP_OK) return rc;
     a.x = (const float*)x; a.u = u; a.policy = policy_out; a.action = action_out;
-    a.n_layers = n_layers; a.n = n; a.w_bytes = (int)w_bytes; a.batch = (int)batch;
+    a.n_layers = n_layers; a.n = n; a.batch = (int)batch;
     a.tiles = (int)((batch + ST_ROWS - 1) / ST_ROWS);
+    const int ht = widest <= 64 ? 4 : 8;
+    bool full = true;
+    for (int l = 0; l < n_layers; ++l) full = full && (dims[l] + 15) / 16 == ht;
+    // Full 64 wide stacks in bf16 parts, sixteen waves in one workgroup per unit, from a tile for every wave of every unit up (one
+    // layer: two, its product is less of the work, and three quarters of the units at work).  Splitting the weights takes a few us
+    // a workgroup: with more members than units each has two tiles a wave at least (64-64-64-64, 300 members of 240 rows 31 / 34,
+    // 6000 of 16 129 / 239, but 512 of 1000 141 / 107).  Us, f32 / parts, 64-64-64-64: 30000 rows 13.4 / 17.9, 65536 21.4 / 18.4,
+    // 131072 37.1 / 29.2, 16 members of 16384 74.5 / 55.3, of 57344 223 / 157; 64-64-64: 30000 rows 10.6 / 15.2, 65536 16.5 /
+    // 15.8, 131072 27.6 / 23.8; 64-64: 65536 rows 11.9 / 12.3, 131072 19.0 / 18.4, 4 members of 50000 33.0 / 28.0.
+    constexpr int PARTS_WAVES = ST_PARTS_THREADS / 64;
+    const long cus = device_cu_count();
+    const long w_parts = (long)n_layers * 8 * ST_PARTS_UNIT;
+    const bool parts = full && ht == 4 && (a.mask_size + 15) / 16 == 4 && w_parts + PARTS_WAVES * ST_SCRATCH <= ST_LDS &&
+                       (long)a.tiles * members >= (n_layers > 1 ? 1 : 2) * PARTS_WAVES * cus &&
+                       (members > cus ? a.tiles >= 2 * PARTS_WAVES : n_layers > 1 || cus / members * members * 4 >= 3 * cus);
+    if (parts) w_bytes = w_parts;
+    a.w_bytes = (int)w_bytes;
     // Four waves a workgroup while that is one tile per SIMD; beyond it eight, so that one wave's norms and head run beside
     // another's products, and as many workgroups per unit as the LDS holds (at most two).
-    const long cus = device_cu_count();
-    const int waves = (long)a.tiles * members > 4 * cus && w_bytes + 8 * ST_SCRATCH <= ST_LDS ? 8 : 4;
+    const int waves = parts ? PARTS_WAVES : (long)a.tiles * members > 4 * cus && w_bytes + 8 * ST_SCRATCH <= ST_LDS ? 8 : 4;
     const int lds_bytes = (int)w_bytes + waves * ST_SCRATCH;
     const int resident = 2 * lds_bytes <= ST_LDS ? 2 : 1;
-    long gx = (cus * resident + members - 1) / members;
+    long gx = parts ? (cus < members ? 1 : cus / members) : (cus * resident + members - 1) / members;      // (parts: one round of workgroups)
     const long most = (a.tiles + waves - 1) / waves;
     if (gx > most) gx = most;
     const long each = (a.tiles + gx * waves - 1) / (gx * waves);      // tiles per wave: no more workgroups than give that
     gx = (a.tiles + each * waves - 1) / (each * waves);
-    const int ht = widest <= 64 ? 4 : 8;
-    bool full = true;
-    for (int l = 0; l < n_layers; ++l) full = full && (dims[l] + 15) / 16 == ht;
-    const void* kernel = ht == 4 ? (full ? pick_stack_kernel<4, true>(regret) : pick_stack_kernel<4, false>(regret))
+    const void* kernel = parts ? pick_stack_kernel<4, true, true>(regret)
+                       : ht == 4 ? (full ? pick_stack_kernel<4, true>(regret) : pick_stack_kernel<4, false>(regret))
                                  : (full ? pick_stack_kernel<8, true>(regret) : pick_stack_kernel<8, false>(regret));
     rc = ensure_dynamic_lds(kernel, ST_LDS);
     if (rc != SP_OK) return rc;
@@ -407,6 +563,8 @@ struct MlpStackKernelNames {
     MlpStackKernelNames() {
         register_kernel("stack_forward_f32", (const void*)mlp_stack_kernel<4, false, true>, ST_MAX_THREADS);
         register_kernel("stack_forward_f32_regret", (const void*)mlp_stack_kernel<4, true, true>, ST_MAX_THREADS);
+        register_kernel("stack_forward_f32_parts", (const void*)mlp_stack_kernel<4, false, true, true>, ST_PARTS_THREADS);
+        register_kernel("stack_forward_f32_parts_regret", (const void*)mlp_stack_kernel<4, true, true, true>, ST_PARTS_THREADS);
         register_kernel("stack_forward_f32_part", (const void*)mlp_stack_kernel<4, false, false>, ST_MAX_THREADS);
         register_kernel("stack_forward_f32_part_regret", (const void*)mlp_stack_kernel<4, true, false>, ST_MAX_THREADS);
         register_kernel("stack_forward_f32_128", (const void*)mlp_stack_kernel<8, false, true>, ST_MAX_THREADS);

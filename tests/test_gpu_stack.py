@@ -140,3 +140,53 @@ def test_rows_of_nan_and_infinity_stay_their_own(S):
     rest = [r for r in range(100) if r not in (17, 40, 99)]
     assert torch.equal(mixed[:, rest], clean[:, rest]) and torch.equal(mixed_picks[:, rest], picks[:, rest])
     assert bool(policy[:, [17, 40, 99]].isnan().all()) and bool((action[:, [17, 40, 99]] == 2147483647).all())
+
+
+# ---- full 64 wide stacks of enough rows: the products as three bf16 parts ----
+@pytest.mark.parametrize("members,rows,widths,acts,head,mask", [
+    (1, 65521, (64, 64, 64), "ln+relu", "ROW_SOFTMAX", 0),                              # the fewest tiles, the last of one row
+    (1, 131057, (52, 64), "", "ROW_REGRET_MATCHING", 0),                                # one layer, a part of a K-block
+    (5, 30011, (64, 64, 64, 60), "tanh", "ROW_MASKED_SOFTMAX", 49),                     # workgroups that do not divide the units; masked
+    (200, 330, (56, 64, 64), "ln+sigmoid", "ROW_SOFTMAX", 0),                           # a workgroup a member
+    (300, 500, (64, 64, 64), "relu", "ROW_SOFTMAX", 0)])                                # more members than units, the fewest tiles
+def test_parts(S, members, rows, widths, acts, head, mask):
+    announce("stack in parts: %d x %d rows %s %s" % (members, rows, widths, head))
+    rng = np.random.default_rng(rows)
+    x, ws = make(rng, members, rows, widths)
+    check(S, x, ws, [acts] * (len(widths) - 2), getattr(S, head), mask, uniforms(rng, members * rows), None)
+
+
+@pytest.mark.parametrize("what", ["rows", "weights"])
+def test_numbers_that_parts_cannot_hold(S, what):
+    """Infinities, numbers below 2^-110 and above 2^60, in some rows of the input or in a member's weights: such rows as the f32 kernel
+    gives them alone (few rows take that one) -- the same bits where every layer's inputs are out of range, as here in all rows
+    but 18 (whose second layer is in parts: the bound of this module) -- and the other rows as they are without them."""
+    announce("stack in parts, %s out of range" % what)
+    rng = np.random.default_rng(3)
+    x, ws = make(rng, 2, 40000, (64, 64, 64))
+    acts = ["relu"]
+    clean, _ = forward(S, x, ws, acts, S.ROW_SOFTMAX, sample=False)
+    if what == "rows":
+        odd = [17, 18, 5000, 39999]
+        x[17, 3], x[18, 60], x[5000], x[39999, 0] = float("inf"), 1e-36, 1e-35, 3e30
+        policy, _ = forward(S, x, ws, acts, S.ROW_SOFTMAX, sample=False)
+        alone, _ = forward(S, x[odd].contiguous(), ws, acts, S.ROW_SOFTMAX, sample=False)
+        assert torch.equal(policy[:, odd].isnan(), alone.isnan()) and bool(alone[:, 0].isnan().all()) and not bool(alone[:, 1:].isnan().any())
+        assert torch.equal(policy[:, [5000, 39999]], alone[:, 2:])
+        assert float((policy[:, 18] - alone[:, 1]).norm() / alone[:, 1].norm()) < 1e-5
+        rest = torch.ones(40000, dtype=torch.bool, device="cuda")
+        rest[odd] = False
+        assert torch.equal(policy[:, rest], clean[:, rest])
+    else:
+        ws[0][1, 5, 7], ws[1][1, 63, 0] = 1e-37, float("-inf")
+        policy, _ = forward(S, x, ws, acts, S.ROW_SOFTMAX, sample=False)
+        alone, _ = forward(S, x[:300].contiguous(), ws, acts, S.ROW_SOFTMAX, sample=False)
+        assert torch.equal(policy[1, :300].isnan(), alone[1].isnan()) and torch.equal(policy[1, :300].nan_to_num(), alone[1].nan_to_num())
+        assert torch.equal(policy[0], clean[0])
+
+
+@pytest.mark.parametrize("name", ["stack_forward_f32_parts", "stack_forward_f32_parts_regret"])
+def test_the_instances_in_parts_are_named(S, name):
+    announce("kernel info " + name)
+    info = S.kernel_info(name)
+    assert info["threads_per_block"] == 1024 and 0 < info["vgprs"] <= 128
