@@ -21,9 +21,9 @@
 // Measured, that stack over 16384 rows (node by node / every layer through part_product, a draw per tile / this kernel, us):
 // one model 32.8 / 13.8 / 10.3, 16 members 206 / 87 / 68.8 (the matrix pipe alone: 41).
 //   PARTS: the same with the products in three bf16 parts (below), 144 MFMAs of 16 cycles for 16 rows instead of 192 of 32, and
-// 300 vector instructions more, which run beside them: 16 members of 16384 rows 70 -> 52.5, of 57344 223 -> 157.  Bound by the
-// vector ALU (1100 instructions, 4400 cycles a tile, of 6100 measured) and the 7 us in which a workgroup's sixteen waves start
-// together, with the same phases.  Sixteen waves because their norms and heads hide behind each other's products (eight: 63.6
+// 400 vector instructions more, in part beside them: 16 members of 16384 rows 70 -> 52.5, of 57344 223 -> 157.  Bound by the
+// vector ALU (1122 instructions, 4490 cycles a tile, of 6100 in the long run) and the 7 us in which a workgroup's sixteen waves
+// start together, with the same phases; a raised priority for waves in their products changed nothing.  Sixteen waves because their norms and heads hide behind each other's products (eight: 63.6
 // and 186).  The sums are closer to float64 than the f32 pipe's (error of the probabilities 0.63 to 0.88 of that, 1.00 where it
 // is the exponential's).
 #include "mlp_common.h"
