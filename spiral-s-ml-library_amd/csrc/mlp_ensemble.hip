@@ -674,12 +674,14 @@ static long ensemble_parts_blocks(long members, long tiles) {
 // tile of one in 5.2 on each of a unit's four SIMDs; below three members the former leaves half of a workgroup idle, and where
 // the latter has one tile per wave it is through before two rounds are (us, f32 / bf16 pipe, 128 inputs: 2 x 65536 rows 33 / 37,
 // 5 x 6144 16.0 / 18.2; 4 x 6144 15.3 / 15.1, 9 x 6144 27.6 / 21.1, 3 x 65536 71 / 36, 5 x 65536 105 / 58, 9 x 65536 182 / 83,
-// 32 x 65536 346 / 230).
-static bool ensemble_takes_parts(long members, long batch) {
+// 32 x 65536 346 / 230).  Up to 64 inputs, half or a quarter of the products, it is ahead from five tiles for each of the f32
+// kernel's waves (32 inputs: 32 x 256 6.5 / 8.7, 8 x 8192 11.5 / 12.6, 4 x 32768 16.8 / 17.2; 16 x 12288 21.7 / 21.4, 32 x 8192
+// 26.0 / 24.7, 32 x 65536 167 / 145).
+static bool ensemble_takes_parts(long members, long batch, int k0) {
     const long tiles = (batch + EN_ROWS - 1) / EN_ROWS, blocks = ensemble_parts_blocks(members, tiles);
     const long each = (device_cu_count() + members - 1) / members;      // workgroups of a member in ensemble_launch
     if (members < 3 || tiles > 2147480000l) return false;
-    return !(tiles <= 4 * each && tiles > blocks);
+    return k0 <= 64 ? tiles > 4 * 4 * each : !(tiles <= 4 * each && tiles > blocks);
 }
 
 template <int KS>
@@ -774,7 +776,7 @@ extern "C" int sp_mlp_forward_ensemble(int dtype, const void* x, int32_t n_layer
     a.policy = policy_out; a.action = action_out; a.batch = batch; a.members = members; a.k0 = k0; a.n = n; a.nout = nout;
     a.head = head; a.mask_size = mask_size;
     const int kg = k0 <= 32 ? 4 : k0 <= 64 ? 8 : k0 <= 128 ? 16 : 32;
-    if (n_layers == 2 && ensemble_takes_parts(a.members, batch)) {
+    if (n_layers == 2 && ensemble_takes_parts(a.members, batch, k0)) {
         return kg == 4 ? launch_ensemble_parts<2>(a, (hipStream_t)stream, __func__) : kg == 8 ? launch_ensemble_parts<4>(a, (hipStream_t)stream, __func__)
                                                                                                : launch_ensemble_parts<8>(a, (hipStream_t)stream, __func__);
     }

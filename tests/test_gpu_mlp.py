@@ -533,7 +533,9 @@ def test_ensemble_binarize(LY, members, batch, k0, n, modulo):
     (5, 32 * 128 * 3, [24, 64, 20], "softmax", 3, False), (5, 32 * 128 * 4 - 17, [40, 64, 64], "softmax_regret_matching", 4, True),
     (6, 32 * 128 * 5 + 9, [64, 64, 64], "regret_matching", 3, False), (7, 32 * 128 * 2 + 32, [72, 64, 6], "softmax", 1, True),
     (4, 32 * 256 * 6 + 33, [128, 64, 8], "none", None, False), (9, 32 * 85 * 7 + 40, [120, 64, 64], "regret_matching", 4, False),
-    (9, 32 * 85 * 8, [128, 64, 64], "softmax", 3, True), (256, 200, [48, 64, 12], "regret_matching", 3, False)])
+    (9, 32 * 85 * 8, [128, 64, 64], "softmax", 3, True), (256, 200, [48, 64, 12], "regret_matching", 3, False),
+    (4, 32 * 1024 + 1, [16, 64, 16], "regret_matching", 2, False), (7, 32 * 600 - 5, [24, 64, 20], "softmax", 3, True),      # up to 64 inputs:
+    (6, 32 * 690 + 9, [64, 64, 64], "regret_matching", 3, False), (300, 32 * 17 + 1, [40, 64, 12], "softmax", 4, True)])    # from five tiles a wave
 def test_ensemble_in_three_parts(LY, members, batch, dims, head, mask, sample):
     """Against float64: the hidden layer no further off than f32 sums are, so the f32 bar of the head holds row by row wherever the
     head itself is not the quotient of two small numbers; exact zeros behind the mask; actions given the kernel's own policy."""
