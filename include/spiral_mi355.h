@@ -103,10 +103,7 @@ int sp_clock_sample(uint64_t* out, void* stream);
  * variant tests/matmul/test3_kernel.spi:148.
  *
  *   A (M,K), B (N,K), C (M,N) row-major.  dtype_in in {SP_F32, SP_F16, SP_BF16} is the storage
- *   type of A and B; products are exact and accumulation is f32 (MFMA).  (Large f32 shapes: every number as three
- *   bf16 parts, of whose nine products the three below 2^-24 of the whole are left out; closer to the exact sum than f32
- *   MFMAs are.  A tile that holds numbers the parts cannot -- infinities, magnitudes below 2^-110 or that round to an infinite
- *   bf16 -- runs on f32 MFMAs as a whole.)  dtype_out is the storage
+ *   type of A and B; products are exact and accumulation is f32 (MFMA).  dtype_out is the storage
  *   type of C (SP_F32, or the same 16-bit type as the input).  bias (N,) f32 may be NULL.
  *   alpha must be non-zero (kernel.spi:49).  beta == 0 means C is never read, so NaNs in the
  *   old C do not propagate (kernel.spi:152-154).
@@ -125,8 +122,7 @@ int sp_gemm_abt(int dtype_in, int dtype_out, const void* A, const void* B, void*
  * weight tensor, stride_b = out * in.  The tile is chosen for the whole batch, so many small members
  * fill the chip.  bias (N,) is shared by all members.
  * f32: every member's C is bit-identical to sp_gemm_abt on that member (the shape of one member alone decides the order
- * in which K is added up; the exception are tiles with numbers that parts cannot hold, see above, as the batch may be cut into
- * other tiles).  16-bit inputs: equal to the rounding of the sums; a large batch may add up K in another order.
+ * in which K is added up).  16-bit inputs: equal to the rounding of the sums; a large batch may add up K in another order.
  */
 int sp_gemm_abt_batched(int dtype_in, int dtype_out, const void* A, const void* B, void* C, const float* bias,
                         int64_t M, int64_t N, int64_t K, int64_t batch, int64_t stride_a, int64_t stride_b,
@@ -134,7 +130,7 @@ int sp_gemm_abt_batched(int dtype_in, int dtype_out, const void* A, const void* 
 
 /* Which tile configuration sp_gemm_abt picks for a shape (the counterpart of
  * `matmul_config_tf32`, ml/matmul/run.spi:8-19).  Writes block tile sizes and the workgroup size; tile_m == 0 means one thread
- * per output (odd widths of the shortest K), tile_k == 16 that f32 runs on the bf16 matrix pipe. */
+ * per output (odd widths of the shortest K). */
 int sp_gemm_config(int dtype_in, int64_t M, int64_t N, int64_t K,
                    int32_t* tile_m, int32_t* tile_n, int32_t* tile_k, int32_t* threads);
 

@@ -3,7 +3,7 @@
 // A (M,K) and B (N,K) are both K-contiguous, so neither operand needs a transposing read: a
 // 32x32 MFMA fragment of either one is "32 rows x one 16-byte K-chunk per lane".
 //
-// Here the workgroup tiles (large f32: gemm_parts.hip; small and narrow outputs: gemm_wave.hip) and the choice between all of them.  Two kernels:
+// Here the workgroup tiles (small and narrow outputs: gemm_wave.hip) and the choice between all of them.  Two kernels:
 // gemm_abt_w4_kernel (four waves, 16x16x32 MFMAs; large 16-bit shapes) and gemm_abt_kernel (eight or four waves, 32x32 MFMAs; f32,
 // small tiles, single-column outputs).
 //
@@ -15,11 +15,30 @@
 //   16-byte chunk each lane fetches.
 //
 // Semantics follow matmul_tf32_template (ml/matmul/kernel.spi:25-240) with a_trans=false,
-// b_trans=true; the f32 path multiplies in full f32 (v_mfma_f32_32x32x2_f32, or parts that add up to it: gemm_parts.hip),
-// not TF32.
-#include "gemm_tile.h"
+// b_trans=true; the f32 path multiplies in full f32 (v_mfma_f32_32x32x2_f32), not TF32.
+#include "gemm_common.h"
 
 namespace sp {
+
+// Map the linear workgroup id to an output tile.  Workgroups are dealt round-robin to the 8 XCDs
+// (each with a private L2), so id % 8 selects the XCD; each XCD gets a contiguous range of the
+// tile sequence, and the sequence walks the tile grid in column-major groups of GROUP_M tile rows
+// so that an XCD's concurrent tiles share A and B panels.
+__device__ __forceinline__ void tile_of_block(int pid, int tiles_m, int tiles_n, int GROUP_M, int& tm, int& tn) {
+    constexpr int XCDS = 8;
+    const int n = tiles_m * tiles_n;
+    const int xcd = pid % XCDS;
+    const int idx = pid / XCDS;
+    const int base = n / XCDS, rem = n % XCDS;
+    const int t = xcd * base + (xcd < rem ? xcd : rem) + idx;
+    const int group_size = GROUP_M * tiles_n;
+    const int g = t / group_size;
+    const int first_m = g * GROUP_M;
+    const int gsz = (tiles_m - first_m) < GROUP_M ? (tiles_m - first_m) : GROUP_M;
+    const int in_group = t % group_size;
+    tm = first_m + in_group % gsz;
+    tn = in_group / gsz;
+}
 
 // RAGGED: M, N and K need not be multiples of the tile (K a multiple of 16 bytes).  Rows past the end are fetched as
 // copies of the last row and the chunks of the last K-tile that lie past the end of a row as zeros, so every load stays
@@ -322,9 +341,126 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_abt_kernel(SP_GEMM_PRELOADED
     first_three_steps();
     mma(fa[1], fb[1]);
 
-    static_assert(NW * strip_bytes(WTN) <= 2 * STAGE_BYTES, "epilogue staging must fit the tile buffers");
+    // ---- epilogue: each wave transposes its accumulators through a private LDS strip of 32 rows x
+    //      up to 64 columns, so that C is written (and, for beta != 0, read) as whole row segments:
+    //      16 bytes per lane, up to 256 contiguous bytes per row ----
+    constexpr int SW = WTN < 64 ? WTN : 64;        // columns per strip
+    constexpr int SF = SW / 32;                    // fragments per strip
+    constexpr int EPI_STRIDE = SW * 4 + 16;        // bytes; the pad keeps the 16-byte column writes conflict free
+    constexpr int LPR = SW / 4;                    // lanes per output row
+    constexpr int RPP = 64 / LPR;                  // rows per pass
+    static_assert(NW * 32 * EPI_STRIDE <= 2 * STAGE_BYTES, "epilogue staging must fit the tile buffers");
     __syncthreads();                               // every wave is done reading the tile buffers
-    store_accumulators<OT, WTM, WTN, RAGGED>(g, Cb, acc, lds + wave * strip_bytes(WTN), m0 + wm * WTM, n0 + wn * WTN, lane);
+    unsigned char* stg = lds + wave * (32 * EPI_STRIDE);
+    const int er = lane / LPR, ec = (lane % LPR) * 4;
+    const float alpha = g.alpha, beta = g.beta;
+    const long row_step = (long)RPP * g.N;
+    // The options are compile-time inside the loops: a branch per output row would split them into blocks of one
+    // LDS read -> one store each, with every latency exposed.
+    auto write_tile = [&](auto BETA_, auto RELU_, auto POLICY_) {
+        constexpr bool HAS_BETA = decltype(BETA_)::value, RELU = decltype(RELU_)::value;
+        constexpr int POLICY = decltype(POLICY_)::value;
+        auto finish = [&](f32x4 v, const f32x4& old, const f32x4& bias) {
+            v = v * alpha;
+            if constexpr (HAS_BETA) v += beta * old;
+            v += bias;
+            if constexpr (RELU) { v.x = fmaxf(v.x, 0.f); v.y = fmaxf(v.y, 0.f); v.z = fmaxf(v.z, 0.f); v.w = fmaxf(v.w, 0.f); }
+            return v;
+        };
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int js = 0; js < TN / SF; ++js) {
+                const long col = n0 + wn * WTN + js * SW + ec;
+                const bool col_ok = !RAGGED || col + 3 < g.N;          // all four columns of this lane
+                f32x4 bias4 = {0.f, 0.f, 0.f, 0.f};
+                if (g.bias && col_ok) bias4 = *reinterpret_cast<const f32x4*>(g.bias + col);
+#pragma unroll
+                for (int jj = 0; jj < SF; ++jj)
+#pragma unroll
+                    for (int gq = 0; gq < 4; ++gq) {
+                        const f32x16& c16 = acc[i][js * SF + jj];
+                        f32x4 v = {c16[4 * gq], c16[4 * gq + 1], c16[4 * gq + 2], c16[4 * gq + 3]};
+                        *reinterpret_cast<f32x4*>(stg + frag_row * EPI_STRIDE + (jj * 32 + gq * 8 + frag_half * 4) * 4) = v;
+                    }
+                const long row_first = m0 + wm * WTM + i * 32 + er;
+                long idx = row_first * g.N + col;     // advanced by RPP rows per pass
+                // one 4-column piece: what C held there, and the store
+                constexpr int AT32 = RAGGED ? 4 : 16, AT16 = RAGGED ? 2 : 8;      // ragged rows begin at any element
+                auto read_old = [&](long at) {
+                    if constexpr (OT == SP_F32) {
+                        return load_aligned<AT32, f32x4>((const float*)Cb + at);
+                    } else {
+                        const u32x2 o = load_aligned<AT16, u32x2>((const unsigned short*)Cb + at);
+                        return f32x4{half_bits_to_f32<OT>(o.x & 0xffffu), half_bits_to_f32<OT>(o.x >> 16),
+                                     half_bits_to_f32<OT>(o.y & 0xffffu), half_bits_to_f32<OT>(o.y >> 16)};
+                    }
+                };
+                auto write = [&](long at, const f32x4& r) {
+                    if constexpr (OT == SP_F32) {
+                        store_c<POLICY, AT32>((float*)Cb + at, r);
+                    } else {
+                        u32x2 o;
+                        o.x = pack_halves<OT>(r.x, r.y);
+                        o.y = pack_halves<OT>(r.z, r.w);
+                        store_c<POLICY, AT16>((unsigned short*)Cb + at, o);
+                    }
+                };
+                constexpr int PASSES = 32 / RPP;
+                if constexpr (RAGGED) {
+                    // The masks split every pass into blocks of its own, so nothing may wait inside them: all of LDS (and
+                    // of the old C) is read first, then everything is stored (63 x 223 x 24 f32 with beta: one read, one
+                    // store per pass 7.4 us, this form 4.4).
+                    f32x4 v[PASSES], old[PASSES];
+                    const long rows_left = g.M - row_first;
+#pragma unroll
+                    for (int p = 0; p < PASSES; ++p) {
+                        v[p] = *reinterpret_cast<const f32x4*>(stg + (p * RPP + er) * EPI_STRIDE + ec * 4);
+                        if constexpr (HAS_BETA) {
+                            old[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+                            if (col_ok && p * RPP < rows_left) old[p] = read_old(idx + p * row_step);
+                        }
+                    }
+                    const bool row_end = g.N % 4 != 0 && n0 + wn * WTN + js * SW < g.N && g.N < n0 + wn * WTN + (js + 1) * SW;
+                    if (row_end) {                       // the last one to three columns of this strip's 32 rows
+                        const int first = (int)(g.N / 4 * 4 - (n0 + wn * WTN + js * SW)), count = (int)(g.N % 4);
+                        const long row = m0 + wm * WTM + i * 32 + (lane & 31);
+                        for (int e = lane >> 5; e < count && row < g.M; e += 2) {
+                            const long c = n0 + wn * WTN + js * SW + first + e;
+                            const float sum = *reinterpret_cast<const float*>(stg + (lane & 31) * EPI_STRIDE + (first + e) * 4);
+                            store_element(Cb, OT, row * g.N + c, sum * alpha, HAS_BETA ? beta : 0.f, g.bias ? g.bias[c] : 0.f, RELU);
+                        }
+                    }
+#pragma unroll
+                    for (int p = 0; p < PASSES; ++p)
+                        if (col_ok && p * RPP < rows_left)
+                            write(idx + p * row_step, finish(v[p], HAS_BETA ? old[p] : f32x4{0.f, 0.f, 0.f, 0.f}, bias4));
+                } else {
+#pragma unroll
+                    for (int p = 0; p < PASSES; ++p, idx += row_step) {
+                        const f32x4 v = *reinterpret_cast<const f32x4*>(stg + (p * RPP + er) * EPI_STRIDE + ec * 4);
+                        f32x4 old = {0.f, 0.f, 0.f, 0.f};
+                        if constexpr (HAS_BETA) old = read_old(idx);
+                        write(idx, finish(v, old, bias4));
+                    }
+                }
+            }
+        }
+    };
+    typedef std::integral_constant<int, ST_PLAIN> plain_t;
+    typedef std::integral_constant<int, ST_THROUGH> through_t;
+    typedef std::integral_constant<int, ST_STREAM> stream_t;
+    if (beta != 0.f) {
+        if (g.relu) write_tile(std::true_type{}, std::true_type{}, plain_t{});
+        else write_tile(std::true_type{}, std::false_type{}, plain_t{});
+    } else if (g.store_policy == ST_STREAM) {
+        if (g.relu) write_tile(std::false_type{}, std::true_type{}, stream_t{});
+        else write_tile(std::false_type{}, std::false_type{}, stream_t{});
+    } else {
+        typedef std::conditional_t<RAGGED, plain_t, through_t> other_t;      // (see where the policy is picked)
+        if (g.relu) write_tile(std::false_type{}, std::true_type{}, other_t{});
+        else write_tile(std::false_type{}, std::false_type{}, other_t{});
+    }
 }
 
 // ---- 256 x 256 x 64 tiles on FOUR waves (one per SIMD), 16x16x32 MFMAs: the kernel for large 16-bit GEMMs ----
@@ -842,8 +978,8 @@ static int choose_cfg(int dtype_in, long M, long N, long K, long batch, long cus
     return smallest;
 }
 
-// The tile a GEMM runs on: a workgroup tile of kTileCfgs (cfg 0..2), of gemm_parts.hip (cfg 3), a split-K tile of gemm_wave.hip
-// (cfg -1) or none, one thread per output (cfg -2).
+// The tile a GEMM runs on: a workgroup tile of kTileCfgs (cfg 0..2), a split-K tile of gemm_wave.hip (cfg -1) or none, one
+// thread per output (cfg -2).
 // `ragged`: the tile does not divide M, N and K -- rows clamped in the loader, zeros for the missing part of the last
 // K-tile, a masked epilogue.
 struct TileChoice {
@@ -875,14 +1011,7 @@ static const TileCost kCostCrossing[] = {{0, 256, 256, 1.5f, 14.f, 0.f}, {1, 128
                                          {-1, 64, 64, 0.27f, 1.5f, 0.f}, {-1, 64, 32, 0.19f, 0.8f, 0.f}, {-1, 32, 32, 0.11f, 0.5f, 0.f},
                                          {-1, 16, 16, 0.055f, 0.3f, 0.f}};
 
-// f32 on the bf16 pipe (gemm_parts.hip), in K-tiles of 16, taken in place of a workgroup tile where the estimate has it 10 %
-// ahead, n the full rounds.  Fitted on 680 shapes whose f32 tile is a workgroup tile: the pick is 0.6 % behind the fastest of the
-// three on the geometric mean (21 % at the worst, 564 x 5668 x 1544, 100 us in f32, 83 on 128 wide parts) and never more than 1 %
-// behind the f32 tile; short K and small outputs stay there (us, f32 / parts: 1008 x 560 x 88 6.7 / 13.4, 24592 x 352 x 24 12.7 / 19).
-// profiles/gemm_parts.txt has what it gives, and the errors.
-static const TileCost kCostParts[] = {{3, 256, 256, 1.63f, 15.8f, 1.55f}, {3, 128, 128, 0.59f, 4.1f, 0.92f}};
-
-enum TileKind { TILE_ANY, TILE_WORKGROUP, TILE_SPLIT, TILE_PARTS };
+enum TileKind { TILE_ANY, TILE_WORKGROUP, TILE_SPLIT };
 
 static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, long cus, TileKind kind) {
     const int es = dtype_in == SP_F32 ? 4 : 2, bk = ROW_BYTES / es;
@@ -896,12 +1025,6 @@ static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, lo
     // 3000 tiles of 16 x 16 up: 1134 x 583 x 24 4.4 / 4.2, 1650 x 1102 x 192 5.8 / 7.7).
     const double small = (double)((M + 15) / 16) * (double)((N + 15) / 16);
     const bool may_split = kind == TILE_SPLIT || nk >= 7 || (batch <= 64 && small <= (N % 4 ? 2048 : 64));
-    auto estimate = [&](const TileCost& c, double tiles, long k_tiles) {
-        const float rounds = (float)((tiles + cus - 1) / cus >= 1e9 ? 1e9 : (double)(long)((tiles + cus - 1) / cus));
-        const float n = dtype_in == SP_F32 && c.cfg != 3 && tiles > cus ? 0.5f * (rounds + (float)(tiles / cus)) : rounds;
-        const float per_k = n * c.tk > c.latency ? n * c.tk : c.latency;
-        return n * c.overhead + (float)k_tiles * per_k;
-    };
     const TileCost* best = nullptr;
     float best_us = 0.f;
     auto consider = [&](const TileCost& c) {
@@ -912,31 +1035,20 @@ static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, lo
         const double tiles = of_member * (double)batch;
         if (c.cfg != 0 && !launch_holds(of_member, 256)) return;
         if (c.cfg < 0 && tiles >= 4294967296.0) return;     // the split form numbers the tiles of a whole batch in 32 bits
-        const float us = estimate(c, tiles, nk);
+        const float rounds = (float)((tiles + cus - 1) / cus >= 1e9 ? 1e9 : (double)(long)((tiles + cus - 1) / cus));
+        const float n = dtype_in == SP_F32 && tiles > cus ? 0.5f * (rounds + (float)(tiles / cus)) : rounds;
+        const float per_k = n * c.tk > c.latency ? n * c.tk : c.latency;
+        const float us = n * c.overhead + (float)nk * per_k;
         if (best == nullptr || us < best_us) {
             best = &c;
             best_us = us;
         }
     };
-    if (kind == TILE_PARTS) {}
-    else if (dtype_in == SP_F32) for (const TileCost& c : kCostF32) consider(c);
+    if (dtype_in == SP_F32) for (const TileCost& c : kCostF32) consider(c);
     else if (K % bk == 0) for (const TileCost& c : kCostLines) consider(c);
     else for (const TileCost& c : kCostCrossing) consider(c);
-    const bool workgroup = best != nullptr && best->cfg >= 0;
-    if (dtype_in == SP_F32 && (kind == TILE_PARTS || (kind == TILE_ANY && workgroup)) && K * es <= kWaveMaxRowBytes) {
-        for (const TileCost& c : kCostParts) {
-            const double of_member = (double)((M + c.bm - 1) / c.bm) * (double)((N + c.bn - 1) / c.bn);
-            if (!launch_holds(of_member, c.bm * 2)) continue;
-            const float us = estimate(c, of_member * (double)batch, (K + 15) / 16);
-            if (best == nullptr || us < (best->cfg == 3 ? best_us : best_us / 1.1f)) {
-                best = &c;
-                best_us = us;
-            }
-        }
-    }
     if (best == nullptr) return best_tile(dtype_in, M, N, K, batch, cus, TILE_WORKGROUP);   // (a split form that cannot be numbered)
     if (best->cfg < 0) return {-1, best->bm, best->bn, 256, true, best_us};
-    if (best->cfg == 3) return {3, best->bm, best->bn, 2 * best->bm, M % best->bm != 0 || N % best->bn != 0 || K % 16 != 0, best_us};
     const TileCfg& t = kTileCfgs[best->cfg];
     const bool ragged = M % t.bm != 0 || N % t.bn != 0 || K % bk != 0;
     const int threads = best->cfg == 0 && !ragged && use_four_waves(dtype_in, N, K) ? 256 : t.wm * t.wn * 64;
@@ -953,7 +1065,7 @@ static bool one_thread_each(int dtype_in, long M, long N, long K) {
 }
 
 // The members of a batch are to add up like a plain launch of each.  The split-K tiles all add an output's products in one
-// order, the workgroup tiles of f32 in another and those of gemm_parts.hip in a third, so the shape of ONE member decides between the kinds and the batch
+// order and the workgroup tiles of f32 in another, so the shape of ONE member decides between the kinds and the batch
 // between the tiles of that kind.  Always for f32, whose batched and member-by-member runs are bit-identical; it costs most
 // where small whole tiles come in large numbers (us, workgroup tiles / split K: 300 x (128 x 128 x 224) 28.8 / 31.7,
 // 37 x (960 x 384 x 320) 78 / 104, 300 x (64 x 64 x 64) 4.8 / 7.8).  For 16-bit inputs, whose 256 wide tiles have MFMAs and
@@ -962,8 +1074,7 @@ static TileChoice choose_tile(int dtype_in, long M, long N, long K, long batch, 
     const TileChoice each = {-2, 0, 0, 256, true, 4e-6f * (float)M * (float)N * (float)batch};
     const TileChoice member = one_thread_each(dtype_in, M, N, K) ? each : best_tile(dtype_in, M, N, K, 1, cus, TILE_ANY);
     if (batch == 1) return member;
-    const TileChoice alike = member.cfg == -2 ? each : best_tile(dtype_in, M, N, K, batch, cus,
-                                                                        member.cfg < 0 ? TILE_SPLIT : member.cfg == 3 ? TILE_PARTS : TILE_WORKGROUP);
+    const TileChoice alike = member.cfg == -2 ? each : best_tile(dtype_in, M, N, K, batch, cus, member.cfg < 0 ? TILE_SPLIT : TILE_WORKGROUP);
     if (dtype_in == SP_F32) return alike;
     const TileChoice any = best_tile(dtype_in, M, N, K, batch, cus, TILE_ANY);
     return alike.us <= 1.25f * any.us ? alike : any;
@@ -1159,7 +1270,7 @@ static int gemm_config(const char* fn, int dtype_in, int64_t M, int64_t N, int64
     const TileChoice t = choose_tile(dtype_in, M, N, K, batch, device_cu_count());
     *tile_m = t.bm;
     *tile_n = t.bn;
-    *tile_k = t.cfg == 3 ? 16 : dtype_in == SP_F32 ? 32 : 64;
+    *tile_k = dtype_in == SP_F32 ? 32 : 64;
     *threads = t.threads;
     *k_parts = t.cfg == -1 ? 4 : t.cfg == -2 ? 0 : 1;
     return SP_OK;
@@ -1225,7 +1336,6 @@ static int gemm_entry(const char* fn, int dtype_in, int dtype_out, const void* A
             g.tiles_n = (int)((N + t.bn - 1) / t.bn);
         }
         if (cfg == -1) return launch_gemm_wave(dtype_in, t.bm, t.bn, cus, g, s);
-        if (cfg == 3) return launch_gemm_parts(t.bm, g, s);
     }
     switch (dtype_in) {
         case SP_F32: return launch_dtype<SP_F32, SP_F32>(cfg, g, s);

@@ -130,86 +130,6 @@ __device__ __forceinline__ void store_element(unsigned char* C, int out_dtype, l
     }
 }
 
-// The tile of this workgroup in the kernels that split K over their waves.  Workgroups are dealt round-robin to the 8 XCDs: each
-// XCD walks a contiguous range of the tiles of the whole batch, along the longer side of a member's tile grid last, so that the
-// panel its neighbours share stays in its L2.  (With ranges within every member, members of one to seven tiles all began on the
-// first XCDs: bf16 71 x (112 x 48 x 952) 25.2 us, numbered through 7.4; f32 103 x (64 x 64 x 448) 16.6 / 7.8; the same tiles
-// without a batch unchanged.)
-__device__ __forceinline__ void wave_tile_of_block(int tiles_m, int tiles_n, int batch, int bm, int bn, unsigned& member, long& m0, long& n0) {
-    const unsigned tiles = (unsigned)tiles_m * (unsigned)tiles_n, all = tiles * (unsigned)batch;
-    const unsigned block = blockIdx.y * tiles + blockIdx.x, xcd = block & 7u;
-    unsigned t = xcd * (all / 8u) + (xcd < (all & 7u) ? xcd : (all & 7u)) + (block >> 3);
-    member = 0;
-    if (batch > 1) {
-        member = t / tiles;
-        t -= member * tiles;
-    }
-    const bool m_last = tiles_m >= tiles_n;
-    const unsigned inner = m_last ? (unsigned)tiles_n : (unsigned)tiles_m;
-    const unsigned hi = t / inner, lo = t - hi * inner;
-    m0 = (long)(m_last ? hi : lo) * bm;
-    n0 = (long)(m_last ? lo : hi) * bn;
-}
-
-// One quad of registers of a kernel whose outputs are scattered over its lanes: C[row][col .. col + 3] at any alignment, the last
-// one to three columns of a row element by element.  All that is read is requested before any of it is waited for.  OT16: the
-// type of an output that is not f32.
-template <int OT16>
-__device__ __forceinline__ void put_quad(const GemmArgs& g, unsigned char* Cb, long row, long col, f32x4 v) {
-    const bool half = g.out_dtype != SP_F32;
-    if (row >= g.M || col >= g.N) return;
-    const long idx = row * g.N + col;
-    const bool whole = col + 3 < g.N;
-    float* c32 = (float*)Cb + idx;
-    unsigned short* c16 = (unsigned short*)Cb + idx;
-    f32x4 old = {0.f, 0.f, 0.f, 0.f}, bias = {0.f, 0.f, 0.f, 0.f};
-    unsigned h[4] = {0, 0, 0, 0};
-    if (whole) {
-        if (g.beta != 0.f) {
-            if (half) {
-                const u32x2 o = *reinterpret_cast<const u32x2_unaligned*>(c16);
-                h[0] = o.x & 0xffffu; h[1] = o.x >> 16; h[2] = o.y & 0xffffu; h[3] = o.y >> 16;
-            } else {
-                old = *reinterpret_cast<const f32x4_unaligned*>(c32);
-            }
-        }
-        if (g.bias) bias = *reinterpret_cast<const f32x4*>(g.bias + col);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 3; ++e)
-            if (col + e < g.N) {
-                if (g.beta != 0.f) {
-                    if (half) h[e] = c16[e];
-                    else old[e] = c32[e];
-                }
-                if (g.bias) bias[e] = g.bias[col + e];
-            }
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        v[e] *= g.alpha;
-        if (g.beta != 0.f) v[e] += g.beta * (half ? half_bits_to_f32<OT16>(h[e]) : old[e]);
-        v[e] += bias[e];
-        if (g.relu) v[e] = fmaxf(v[e], 0.f);
-    }
-    if (half) {
-        const u32x2 o = {pack_halves<OT16>(v[0], v[1]), pack_halves<OT16>(v[2], v[3])};
-        if (whole) {
-            *reinterpret_cast<u32x2_unaligned*>(c16) = o;
-        } else {
-#pragma unroll
-            for (int e = 0; e < 3; ++e)
-                if (col + e < g.N) c16[e] = (unsigned short)(e < 2 ? o.x >> (16 * e) : o.y);
-        }
-    } else if (whole) {
-        *reinterpret_cast<f32x4_unaligned*>(c32) = v;
-    } else {
-#pragma unroll
-        for (int e = 0; e < 3; ++e)
-            if (col + e < g.N) c32[e] = v[e];
-    }
-}
-
 // One wave-wide DMA: every lane copies 16 bytes from global memory (uniform base + per-lane
 // 32-bit offset) to LDS byte m0 + 16 * lane.  Completion is tracked by vmcnt; the instruction is
 // issued from inline assembly so that the tile in flight does not make the compiler wait before
@@ -233,8 +153,5 @@ __device__ __forceinline__ const unsigned char* uniform_ptr(const unsigned char*
 // than 2^32 tiles in the batch; cus: the compute units of the device.
 int launch_gemm_wave(int dtype_in, int tile_m, int tile_n, long cus, const GemmArgs& g, hipStream_t stream);
 constexpr long kWaveMaxRowBytes = 1l << 25;
-
-// f32 on the bf16 matrix pipe (gemm_parts.hip): tiles 256 or 128 wide, the same limit on rows.
-int launch_gemm_parts(int tile, const GemmArgs& g, hipStream_t stream);
 
 }  // namespace sp

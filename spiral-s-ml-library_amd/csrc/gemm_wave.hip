@@ -48,9 +48,21 @@ __global__ __launch_bounds__(256) void gemm_wave_kernel(const void* A_first, con
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    unsigned member;
-    long m0, n0;
-    wave_tile_of_block(tiles_m, tiles_n, batch, 16 * TM, 16 * TN, member, m0, n0);
+    // workgroups are dealt round-robin to the 8 XCDs: each XCD walks a contiguous range of the tiles of the whole batch,
+    // along the longer side of a member's tile grid last, so that the panel its neighbours share stays in its L2.  (With
+    // ranges within every member, members of one to seven tiles all began on the first XCDs: bf16 71 x (112 x 48 x 952)
+    // 25.2 us, numbered through 7.4; f32 103 x (64 x 64 x 448) 16.6 / 7.8; the same tiles without a batch unchanged.)
+    const unsigned tiles = (unsigned)tiles_m * (unsigned)tiles_n, all = tiles * (unsigned)batch;
+    const unsigned block = blockIdx.y * tiles + blockIdx.x, xcd = block & 7u;
+    unsigned t = xcd * (all / 8u) + (xcd < (all & 7u) ? xcd : (all & 7u)) + (block >> 3), member = 0;
+    if (batch > 1) {
+        member = t / tiles;
+        t -= member * tiles;
+    }
+    const bool m_last = tiles_m >= tiles_n;
+    const unsigned inner = m_last ? (unsigned)tiles_n : (unsigned)tiles_m;
+    const unsigned hi = t / inner, lo = t - hi * inner;
+    const long m0 = (long)(m_last ? hi : lo) * (16 * TM), n0 = (long)(m_last ? lo : hi) * (16 * TN);
 
     const long row_bytes = (long)K * ES;
     const unsigned char* pA = uniform_ptr((const unsigned char*)A_first + (long)member * stride_a + m0 * row_bytes);
@@ -131,8 +143,64 @@ __global__ __launch_bounds__(256) void gemm_wave_kernel(const void* A_first, con
                 for (int jn = 0; jn < TN; ++jn) acc[i][jn] = mma<DT>(fb[ks][jn], fa[ks][i], acc[i][jn]);
     }
 
+    // One quad of registers: C[row][col .. col + 3], the last one to three columns of a row element by element.  All
+    // that is read is requested before any of it is waited for.
     constexpr int OT16 = DT == SP_BF16 ? SP_BF16 : SP_F16;
     unsigned char* const Cb = (unsigned char*)g.C + (long)member * g.stride_c;
+    const bool half = g.out_dtype != SP_F32;
+    auto put = [&](long row, long col, f32x4 v) {
+        if (row >= M || col >= N) return;
+        const long idx = row * N + col;
+        const bool whole = col + 3 < N;
+        float* c32 = (float*)Cb + idx;
+        unsigned short* c16 = (unsigned short*)Cb + idx;
+        f32x4 old = {0.f, 0.f, 0.f, 0.f}, bias = {0.f, 0.f, 0.f, 0.f};
+        unsigned h[4] = {0, 0, 0, 0};
+        if (whole) {
+            if (g.beta != 0.f) {
+                if (half) {
+                    const u32x2 o = *reinterpret_cast<const u32x2_unaligned*>(c16);
+                    h[0] = o.x & 0xffffu; h[1] = o.x >> 16; h[2] = o.y & 0xffffu; h[3] = o.y >> 16;
+                } else {
+                    old = *reinterpret_cast<const f32x4_unaligned*>(c32);
+                }
+            }
+            if (g.bias) bias = *reinterpret_cast<const f32x4*>(g.bias + col);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (col + e < N) {
+                    if (g.beta != 0.f) {
+                        if (half) h[e] = c16[e];
+                        else old[e] = c32[e];
+                    }
+                    if (g.bias) bias[e] = g.bias[col + e];
+                }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] *= g.alpha;
+            if (g.beta != 0.f) v[e] += g.beta * (half ? half_bits_to_f32<OT16>(h[e]) : old[e]);
+            v[e] += bias[e];
+            if (g.relu) v[e] = fmaxf(v[e], 0.f);
+        }
+        if (half) {
+            const u32x2 o = {pack_halves<OT16>(v[0], v[1]), pack_halves<OT16>(v[2], v[3])};
+            if (whole) {
+                *reinterpret_cast<u32x2_unaligned*>(c16) = o;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    if (col + e < N) c16[e] = (unsigned short)(e < 2 ? o.x >> (16 * e) : o.y);
+            }
+        } else if (whole) {
+            *reinterpret_cast<f32x4_unaligned*>(c32) = v;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (col + e < N) c32[e] = v[e];
+        }
+    };
     // partial tiles: fragment f of wave w at (f * 4 + w) * 1 KiB; fragment f is then finished by wave f % 4.
     // The registers of lane l of a 16 x 16 fragment: row l % 16, columns 4 (l / 16) ...
     __syncthreads();                                    // the rings are not read any more
@@ -149,7 +217,7 @@ __global__ __launch_bounds__(256) void gemm_wave_kernel(const void* A_first, con
             const int f = i * TN + jn;
             if (f % 4 != wave) continue;
             const f32x4* p = part + f * 4 * 64 + lane;
-            put_quad<OT16>(g, Cb, m0 + 16 * i + fi, n0 + 16 * jn + 4 * fq, (p[0] + p[64]) + (p[128] + p[192]));
+            put(m0 + 16 * i + fi, n0 + 16 * jn + 4 * fq, (p[0] + p[64]) + (p[128] + p[192]));
         }
 }
 

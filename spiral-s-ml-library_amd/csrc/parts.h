@@ -1,4 +1,8 @@
-// A f32 as the sum of three bf16 numbers, for products on the bf16 matrix pipe (what is left out and why: gemm_parts.hip).
+// A f32 as the sum of three bf16 numbers, for products on the bf16 matrix pipe.
+//
+// Every f32 is the exact sum of three bf16 numbers, x = h + m + l: h is x rounded to bf16, m what is left rounded to bf16, l
+// the rest (8 significant bits each and two signs: 24 bits and more).  A product of two f32 is then nine products of bf16, of
+// which the three smallest (m l, l m, l l) are below 2^-24 of it, of either sign, and are left out.
 #pragma once
 #include "common.h"
 

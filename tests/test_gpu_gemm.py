@@ -582,24 +582,23 @@ def test_batched(MM, dtype, e, m, n, k, shared):
         assert (many[i] == one).all()
 
 
-# f32 on the bf16 pipe: tile, shape; remainders of M, N, K, odd and even numbers of K-tiles, odd widths, one K-tile more than the ring
-PARTS = [(256, 16384, 1024, 512), (256, 15873, 1023, 36), (256, 16129, 2047, 44), (256, 16384, 1024, 528), (128, 12929, 578, 36),
-         (128, 12860, 513, 68), (128, 10497, 322, 268), (128, 4096, 1024, 512), (128, 3584, 1792, 272), (128, 4097, 4093, 1000)]
+# f32 shapes of every size of tile: remainders of M, N, K, odd and even numbers of K-tiles, odd widths
+LARGE_F32 = [(16384, 1024, 512), (15873, 1023, 36), (16129, 2047, 44), (12929, 578, 36), (12860, 513, 68), (10497, 322, 268),
+             (4096, 1024, 512), (3584, 1792, 272), (4097, 4093, 1000), (700, 300, 64)]
 
 
-def parts_config(MM, tile, m, n, k, members=1):
-    cfg = MM.matmul_config_batched(members, m, n, k)
-    assert (cfg["k_tile"], cfg["m_tile"]) == (16, tile)
-
-
-@pytest.mark.parametrize("tile,m,n,k", PARTS)
-def test_f32_in_three_parts(MM, tile, m, n, k):
-    """Against float64 the sums are no further off than a chain of f32 additions is (2-norm: 2^-24 sqrt(K / 2), with what the
-    products leave out and the last rounding, 1e-7, on top), for numbers of any size; and B = I gives A back to the last bit."""
-    announce("gemm f32 parts %d %dx%dx%d" % (tile, m, n, k))
-    parts_config(MM, tile, m, n, k)
+def f32_gen(seed):
     gen = torch.Generator(device="cuda")
-    gen.manual_seed(k)
+    gen.manual_seed(seed)
+    return gen
+
+
+@pytest.mark.parametrize("m,n,k", LARGE_F32)
+def test_large_f32(MM, m, n, k):
+    """Against float64 the sums are no further off than a chain of f32 additions is (2-norm: 2^-24 sqrt(K / 2), and the last
+    rounding, 1e-7, on top), for numbers of any size; and B = I gives A back to the last bit."""
+    announce("gemm f32 %dx%dx%d" % (m, n, k))
+    gen = f32_gen(k)
     a = torch.randn((m, k), generator=gen, device="cuda")
     b = torch.randn((n, k), generator=gen, device="cuda") * torch.exp2(torch.randint(-40, 40, (n, 1), generator=gen, device="cuda").float())
     want = a.double() @ b.double().T
@@ -617,52 +616,72 @@ def test_f32_in_three_parts(MM, tile, m, n, k):
     assert torch.equal(MM.matmul_abt(a, one), a[:, torch.arange(n, device="cuda") % k])
 
 
-@pytest.mark.parametrize("tile,m,n,k", [(256, 15873, 1023, 36), (128, 4096, 1024, 512)])
-def test_f32_in_three_parts_keeps_what_parts_cannot_hold(MM, tile, m, n, k):
-    """Infinities, NaN, values that round to an infinite bf16 and values whose lowest part is below the smallest bf16."""
-    announce("gemm f32 parts, special values %d %dx%dx%d" % (tile, m, n, k))
-    parts_config(MM, tile, m, n, k)
-    gen = torch.Generator(device="cuda")
-    gen.manual_seed(7)
-    a = torch.randn((m, k), generator=gen, device="cuda")
-    b = torch.randn((n, k), generator=gen, device="cuda").abs() + 0.5
+@pytest.mark.parametrize("m,n,k", LARGE_F32)
+def test_f32_products_round_no_more_often_than_there_are_terms(MM, m, n, k):
+    """A product with a diagonal matrix is the correctly rounded product of two numbers, and a row of t non-zero elements is off
+    by at most t roundings of its partial sums, none of which is above the sum of the magnitudes: t 2^-24 of that."""
+    announce("gemm f32 sparse %dx%dx%d" % (m, n, k))
+    gen = f32_gen(m)
+    b = torch.randn((n, k), generator=gen, device="cuda")
+    for terms in (1, 2, 4):
+        at = torch.rand((m, k), generator=gen, device="cuda").topk(terms).indices
+        a = torch.zeros((m, k), device="cuda").scatter_(1, at, torch.randn((m, terms), generator=gen, device="cuda"))
+        got, want = MM.matmul_abt(a, b), a.double() @ b.double().T
+        if terms == 1:
+            assert torch.equal(got, want.float())
+        assert ((got.double() - want).abs() <= terms * 2.0 ** -24 * (a.double().abs() @ b.double().abs().T)).all()
+
+
+SPECIAL = [5, 6, 700, 800, 900, 901, 902, -1]
+
+
+def special_rows(a, k):
+    """The rows SPECIAL of a with infinities, NaN, the largest f32 (its bf16 is infinite), tiny and subnormal numbers."""
+    a = a.clone()
     a[5, 3], a[5, 7] = float("inf"), 1.0
     a[6, 1], a[6, 2] = float("inf"), float("-inf")
     a[700, k - 1] = float("nan")
-    a[m - 1, 0] = float("-inf")
+    a[-1, 0] = float("-inf")
     a[900] = 0.0
-    a[900, 4] = 3.4028234e38                                   # the largest f32: its bf16 is infinite
+    a[900, 4] = 3.4028234e38
+    a[901] *= 2.0 ** -90
+    a[902] *= 2.0 ** -140
+    a[800, ::2] *= 2.0 ** -105
+    return a
+
+
+@pytest.mark.parametrize("m,n,k", [(15873, 1023, 36), (4096, 1024, 512), (1000, 300, 64)])
+def test_f32_rows_of_special_values_stay_their_own(MM, m, n, k):
+    """An output depends on its row of A and its row of B alone, to the last bit: infinities, NaN and tiny numbers in other rows
+    change nothing.  A row scaled by a power of two gives the scaled sums."""
+    announce("gemm f32, special values %dx%dx%d" % (m, n, k))
+    gen = f32_gen(7)
+    clean = torch.randn((m, k), generator=gen, device="cuda")
+    a = special_rows(clean, k)
+    b = torch.randn((n, k), generator=gen, device="cuda").abs() + 0.5
     b[:, 4] = 0.75
-    a[901] *= 2.0 ** -120
-    a[902] *= 2.0 ** -140                                      # subnormal
-    got = MM.matmul_abt(a, b)
-    assert (got[5] == float("inf")).all() and got[6].isnan().all() and got[700].isnan().all() and (got[m - 1] == float("-inf")).all()
+    got, plain = MM.matmul_abt(a, b), MM.matmul_abt(clean, b)
+    assert (got[5] == float("inf")).all() and got[6].isnan().all() and got[700].isnan().all() and (got[-1] == float("-inf")).all()
     assert torch.equal(got[900], torch.full((n,), 3.4028234e38 * 0.75, device="cuda"))
     rest = torch.ones(m, dtype=torch.bool, device="cuda")
-    rest[[5, 6, 700, m - 1]] = False
-    want = a.double() @ b.double().T
-    for rows in (rest, [901]):
-        assert ((got[rows].double() - want[rows]).norm() / want[rows].norm()).item() < TOL["f32"]
+    rest[SPECIAL] = False
+    assert torch.equal(got[rest], plain[rest])
+    assert torch.equal(got[901], plain[901] * 2.0 ** -90)
+    want = a[[800, 902]].double() @ b.double().T
+    assert ((got[800].double() - want[0]).norm() / want[0].norm()).item() < 2.0 ** -24 * (k / 2) ** 0.5 + 1e-7
     # (a sum of subnormal numbers is rounded to a multiple of 2^-149, and so are its terms)
-    assert (got[902].double() - want[902]).abs().max().item() <= 2.0 ** -149 * k
+    assert (got[902].double() - want[1]).abs().max().item() <= 2.0 ** -149 * k
 
 
-def test_f32_in_three_parts_adds_a_batch_up_like_its_members(MM):
-    announce("gemm f32 parts, batch")
-    gen = torch.Generator(device="cuda")
-    gen.manual_seed(3)
+def test_f32_adds_a_batch_up_like_its_members(MM):
+    """Also where the batch and a member alone take tiles of different sizes, and whatever the numbers are."""
+    announce("gemm f32, batch")
+    gen = f32_gen(3)
     m, n, k = 2560, 2047, 1036
     a, b = torch.randn((3, m, k), generator=gen, device="cuda"), torch.randn((3, n, k), generator=gen, device="cuda")
-    parts_config(MM, 128, m, n, k)
-    parts_config(MM, 256, m, n, k, 3)
+    a[1] = special_rows(a[1], k)
     many = MM.matmul_abt_batched(a, b)
     for i in range(3):
-        assert torch.equal(many[i], MM.matmul_abt(a[i], b[i]))
-
-
-@pytest.mark.parametrize("name", ["gemm_f32_parts_256x256", "gemm_f32_parts_256x256_ragged", "gemm_f32_parts_128x128", "gemm_f32_parts_128x128_ragged"])
-def test_every_instance_of_the_parts_kernel_is_named(name):
-    announce("kernel info " + name)
-    from ml import _lib
-    info = _lib.kernel_info(name)
-    assert info["threads_per_block"] == (512 if "256" in name else 256) and 0 < info["vgprs"] <= 256
+        one = MM.matmul_abt(a[i], b[i])
+        assert torch.equal(many[i].view(torch.int32), one.view(torch.int32)) or (
+            torch.equal(many[i].isnan(), one.isnan()) and torch.equal(many[i].nan_to_num(), one.nan_to_num()))
