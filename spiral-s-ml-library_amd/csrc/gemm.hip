@@ -457,9 +457,14 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_abt_kernel(SP_GEMM_PRELOADED
         if (g.relu) write_tile(std::false_type{}, std::true_type{}, stream_t{});
         else write_tile(std::false_type{}, std::false_type{}, stream_t{});
     } else {
-        typedef std::conditional_t<RAGGED, plain_t, through_t> other_t;      // (see where the policy is picked)
-        if (g.relu) write_tile(std::false_type{}, std::true_type{}, other_t{});
-        else write_tile(std::false_type{}, std::false_type{}, other_t{});
+        if constexpr (RAGGED)
+            if (g.store_policy == ST_PLAIN) {
+                if (g.relu) write_tile(std::false_type{}, std::true_type{}, plain_t{});
+                else write_tile(std::false_type{}, std::false_type{}, plain_t{});
+                return;
+            }
+        if (g.relu) write_tile(std::false_type{}, std::true_type{}, through_t{});
+        else write_tile(std::false_type{}, std::false_type{}, through_t{});
     }
 }
 
@@ -1325,13 +1330,18 @@ static int gemm_entry(const char* fn, int dtype_in, int dtype_out, const void* A
         cfg = t.cfg;
         if (cfg != -2) {
             g.ragged = t.ragged;
-            // Tiles that do not divide the shape: rows on 64 bytes are streamed (what a tile writes of a line is whole sectors, and
-            // nobody else's), others left to the L2, which puts the ends of rows and tiles together before they go to memory --
-            // written through or streamed they go as pieces.  580 shapes, times as fast as written through (geometric mean /
-            // worst): bf16 rows off 64 bytes, plain 1.15 / 0.95, streamed 1.06 / 0.56; on 64 bytes, plain 1.06 / 0.81, streamed
-            // 1.12 / 0.92; f32, whose products take longer, 1.01 / 0.95 and 1.04 / 0.98 (51579 x 62 x 232 bf16 14.9 -> 8.7 us,
-            // 24658 x 2426 x 624 167 -> 111, 13152 x 2608 x 224 53 -> 38).  Where a tile divides the shape the rule above stands.
-            if (t.ragged) g.store_policy = N * es_out % 64 == 0 ? ST_STREAM : ST_PLAIN;
+            // Tiles that do not divide the shape, where there is more to gain than a reader behind loses: rows on 64 bytes are
+            // streamed (what a tile writes of a line is whole sectors, and nobody else's), others left to the L2, which puts the
+            // ends of rows and tiles together before they go to memory -- written through or streamed they go as pieces.
+            // Times as fast as written through, alone and with a kernel behind that reads C, geometric mean (worst): 16-bit inputs
+            // on tiles of 128 and more 1.20 (1.02) and 1.15 (1.01), 51 shapes; outputs of 40 MiB up 1.21 (1.11) and 1.20 (0.98),
+            // f32 inputs 1.04 (0.99) and 1.04 (0.99), 40 shapes; 16-bit inputs with K from 448 up 1.06 (1.01) and 1.03 (0.97), 25
+            // shapes (runs of one form differ by up to 4 %).  The rest a reader finds in the caches if it was written through,
+            // and stays so: alone 1.05, but with a reader 0.99 (0.94) (16309 x 205 x 56 7.8 -> 6.1 us, and 13.9 -> 14.8;
+            // 10674 x 386 x 40 f32 12.3 -> 11.3, and 19.8 -> 21.1).  Where a tile divides the shape the rule above stands.
+            const bool wide = dtype_in != SP_F32 && (t.bm >= 128 || K >= 448);
+            if (t.ragged && (wide || (double)M * (double)N * (double)es_out * (double)batch >= 40.0 * (1 << 20)))
+                g.store_policy = N * es_out % 64 == 0 ? ST_STREAM : ST_PLAIN;
             g.tiles_m = (int)((M + t.bm - 1) / t.bm);
             g.tiles_n = (int)((N + t.bn - 1) / t.bn);
         }

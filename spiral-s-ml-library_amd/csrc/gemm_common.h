@@ -28,7 +28,7 @@ struct GemmArgs {
     int group_m;   // tile rows per group of the block -> tile walk (4: an XCD's 32 concurrent tiles form a 4 x 8 patch)
     int ragged;    // M or N is not a multiple of the tile: tiles_m / tiles_n are rounded up
     int k_rotate;  // workgroup t starts its K loop at K-tile (t * k_rotate) % nk and wraps around (0: everyone at 0)
-    int store_policy;   // of the stores of C when beta == 0: ST_THROUGH or ST_STREAM, ragged tiles ST_PLAIN or ST_STREAM (with beta != 0 C is read here: ST_PLAIN)
+    int store_policy;   // of the stores of C when beta == 0: ST_THROUGH or ST_STREAM, of ragged tiles also ST_PLAIN (with beta != 0 C is read here: ST_PLAIN)
     int phase_groups;   // persistent four-wave kernel: workgroup w starts ((w / 8) % phase_groups) * phase_skew
     int phase_skew;     // sleeps of ~2048 cycles late (0 / 1 groups: everybody at once)
 };

@@ -399,11 +399,13 @@ def test_streamed_and_written_through_outputs_are_exact_on_integers(MM, m, n, k)
     assert (host(c) == 2.0 * want - 3.0 * c0).all()
 
 
-@pytest.mark.parametrize("m,n,k", [(700, 63, 64), (1000, 272, 128), (1031, 257, 64), (5003, 1001, 72), (4100, 1040, 64), (3000, 3002, 136)])
+@pytest.mark.parametrize("m,n,k", [(700, 63, 64), (1000, 272, 128), (1031, 257, 64), (5003, 1001, 72), (4100, 1040, 64), (3000, 3002, 136),
+                                   (3600, 3002, 64), (3600, 3008, 64), (1031, 257, 448), (1031, 256, 448)])
 @pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
 def test_ragged_outputs_are_exact_whatever_their_rows_start_on(MM, dtype, m, n, k):
-    """Tiles that do not divide the shape stream C where its rows start on 64 bytes and leave it to the L2 where they do not: both,
-    in each output type and with each epilogue option, on small integers (every partial sum is exact)."""
+    """Tiles that do not divide the shape write C through or, large outputs, large tiles and long K, stream it where its rows start
+    on 64 bytes and leave it to the L2 where they do not: all three, in each output type and with each epilogue option, on small
+    integers (every partial sum is exact)."""
     announce("gemm ragged store policies, %s %dx%dx%d" % (dtype, m, n, k))
     t = TORCH[dtype]
     a = ((np.arange(m * k, dtype=np.int64).reshape(m, k) * 7 + 3) % 5 - 2).astype(np.float32)
