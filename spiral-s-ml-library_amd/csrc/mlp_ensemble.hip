@@ -29,7 +29,6 @@
 namespace sp {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __bf16 en_bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int EN_ROWS = 32;       // batch rows per tile
 constexpr int EN_HIDDEN = 64;     // width of the hidden layer
@@ -214,7 +213,7 @@ __global__ __launch_bounds__(EN_THREADS) void mlp_ensemble_kernel(const Ensemble
     }
 }
 
-// The same on the bf16 matrix pipe, every f32 as three bf16 parts (parts.h): sixteen times the rate of the f32 MFMAs for the six
+// The same on the bf16 matrix pipe, every f32 as three bf16 parts (parts.h): sixteen times the rate of the f32 MFMAs for the eight
 // products of parts that count, and next to 16-bit MFMAs vector instructions hide.
 // Two waves per SIMD: wave w and w + 4 of a workgroup take the two halves of one member's hidden layer, in 12 KS registers as
 // parts.  A workgroup has four members and walks over tiles of 32 batch rows, a tile a round; the inputs of a round are split
@@ -223,13 +222,14 @@ __global__ __launch_bounds__(EN_THREADS) void mlp_ensemble_kernel(const Ensemble
 // second round one wave of a pair, in turn, does the heads of rounds n - 4 and n - 3, next to the other's products, and behind
 // the barrier both store the rows of round n - 4.  Three buffers of inputs, so that the one barrier of a round can stand in its
 // middle: nobody waits at a round's ends.  Second layer and head are those of the kernel above, in f32.
-// What bounds it: 32 x 65536 rows of 128 inputs take 206 us traced, 65 rounds of 6.3 k cycles at 2.0 GHz; the matrix pipe is busy for
-// half of them (the clock with it alone busy would be 1.8), the rest is 280 vector instructions per wave and round, 40 % of
-// which the MFMAs do not hide, and what waves wait for LDS and each other.  (Taken back on the way: one wave per SIMD with both
-// halves 248 us, heads in front of a barrier at the round's end 240, zeros and probabilities of a row stored apart 257, fragments
-// two steps ahead instead of one 230, stores past the caches 228.)
-// Inputs or weights that parts cannot hold (parts.h; beyond 2^60 a sum of parts might overflow where the sum itself does not) send
-// a round, or all rounds of a member, through f32 MFMAs.
+// A round has three sums: `large` of the products h h, which come from zero for each step of 16 inputs and are added by the vector
+// ALU (three MFMAs later), and `small` of the other seven; both in `done` at its end.
+// What bounds it: 32 x 65536 rows of 128 inputs take 260 us (f32 MFMAs 335 to 360), 65 rounds of 8 k cycles; the matrix pipe is
+// busy for 4.1 k of a round, the rest is 450 vector instructions per wave and round that the MFMAs hide in part, and what waves
+// wait for LDS and each other.  (Six products in one sum, without the additions, took 210 us and lost bits, see parts.h.  Taken
+// back on the way there: one wave per SIMD with both halves 248 us, heads in front of a barrier at the round's end 240, zeros and
+// probabilities of a row stored apart 257, fragments two steps ahead instead of one 230, stores past the caches 228.)
+// Inputs or weights that parts cannot hold (parts.h) send a round, or all rounds of a member, through f32 MFMAs.
 typedef const __attribute__((address_space(1))) f32x4* global_f32x4;
 constexpr int EP_THREADS = 512;
 typedef unsigned u32x2_parts __attribute__((ext_vector_type(2)));
@@ -261,19 +261,6 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
         v[1] = at[1];
         return there;
     };
-    unsigned least = 0xffffffffu;
-    float most = 0.f;
-    auto track = [&](float x, float y) {
-        const unsigned wx = parts_magnitude(x), wy = parts_magnitude(y), w = wx < wy ? wx : wy;
-        least = w < least ? w : least;
-        most = fmaxf(fmaxf(most, fabsf(x)), fabsf(y));
-    };
-    auto out_of_range = [&]() {                                     // (NaN: a NaN either way)
-        const bool bad = __any(parts_tiny(least) || most > 0x1p60f);
-        least = 0xffffffffu;
-        most = 0.f;
-        return bad;
-    };
 
     // ---- inputs: this wave's share of a round is step `wave` of its tile (with fewer steps than waves some do the same),
     //      32 bytes a lane, by DMA into a ring of three ----
@@ -297,13 +284,15 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
         raw[1] = *reinterpret_cast<const f32x4*>(lds + raw_at + slot * 2048 + 1024 + lane * 16);
     };
     u32x2_parts split_to[3];
-    float two[2];
+    float two[2], most = 0.f;
     auto split_slice = [&](unsigned buffer, int slice) {
         const int d = slice / 3, i = slice % 3;
         if (i == 0) {
             two[0] = raw[d >> 1][2 * (d & 1)];
             two[1] = raw[d >> 1][2 * (d & 1) + 1];
-            track(two[0], two[1]);
+            most = parts_most(most, two[0], two[1]);
+            two[0] *= PARTS_X_SCALE;
+            two[1] *= PARTS_X_SCALE;
         }
         split_to[i][d & 1] = take_parts(two[0], two[1]);
         if (i < 2) asm volatile("" : "+v"(two[0]), "+v"(two[1]));
@@ -313,10 +302,11 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
             for (int k = 0; k < 3; ++k) *reinterpret_cast<u32x2_parts*>(at + k * 1024) = split_to[k];
         }
     };
-    unsigned* const flags = reinterpret_cast<unsigned*>(lds + FLAGS_AT);     // [buffer][wave]: inputs that parts cannot hold
+    unsigned* const flags = reinterpret_cast<unsigned*>(lds + FLAGS_AT);     // [buffer][wave]: bit r: inputs of row r that parts cannot hold
     auto raise_flag = [&](unsigned buffer) {
-        const bool bad = out_of_range();
-        flags[buffer * 8 + wave] = bad;                // (every lane the same)
+        const unsigned long long bad = __ballot(most > PARTS_MOST);
+        flags[buffer * 8 + wave] = (unsigned)(bad | bad >> 32);        // (every lane the same)
+        most = 0.f;
     };
     fetch_share(0, 0);
     fetch_share(1, 1);
@@ -324,6 +314,7 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
 
     // ---- this half of the member's hidden layer, once ----
     parts_u32x4 w1[KS][3];
+    PartsWeights range;
     {
         const float* const w = a.w1 + ((long)e * EN_HIDDEN + 32 * half + r) * K0;
 #pragma unroll
@@ -331,11 +322,11 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
             f32x4 v[2];
             if (!load8(w, s, v)) v[0] = v[1] = zero4;
 #pragma unroll
-            for (int d = 0; d < 4; ++d) track(v[d >> 1][2 * (d & 1)], v[d >> 1][2 * (d & 1) + 1]);
-            split_parts(v, w1[s]);
+            for (int k = 0; k < 8; ++k) range.take(v[k >> 2][k & 3]);
+            split_parts(v, PARTS_W_SCALE, w1[s]);
         }
     }
-    const bool w_bad = out_of_range();
+    const bool w_bad = __any(range.wide());
     // W2[e][o][32 half + 8 a4 + 4 g ..] at (o * 4 + a4) * 2 + g of the wave's 512 bytes, rows past NOUT are zeros
     f32x4* const w2 = reinterpret_cast<f32x4*>(lds + W2_AT + wave * 512);
     if (lane < 32) {
@@ -401,12 +392,12 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
         *reinterpret_cast<f32x4*>(policy + tile0 * N + (rr * N + 4 * c)) = c == 0 ? v : zero4;
     };
 
-    f32x16 acc[2];
+    f32x16 done, large, small, these;                  // a round's results; the sums on their way there (parts.h)
     auto clear = [&](f32x16& c) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) c[i] = 0.f;
     };
-    clear(acc[1]);
+    clear(done);
     parts_u32x4 xf[2][3];
     auto read_step = [&](unsigned buffer, int s, int i) {
         xf[s & 1][i] = *reinterpret_cast<const parts_u32x4*>(lds + buffer * BUFFER + s * 3072 + i * 1024 + lane * 16);
@@ -423,20 +414,19 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
         for (int o = 0; o < NO; ++o) wv[o] = *reinterpret_cast<const weights_of*>((const float*)(w2 + (o * 4 + (f >> 2)) * 2 + g) + (f & 3));
     };
     second_weights(0);
-    // Round n: its products into acc[B]; the second layer of the round before it from acc[B ^ 1]; the inputs of the next.
-    auto work = [&](auto B_, int n) {
-        constexpr int B = decltype(B_)::value;
+    // Round n: its products; the second layer of the round before it from `done`; the inputs of the next.
+    auto work = [&](int n) {
         // The inputs of round n + 1 have landed: behind them came those of round n + 2 and, from round 4 on, four
         // stores of each of the last two rounds (a head's store more, and the wait is for a little more).
         if (rows_out && n >= 6) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
         else asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
         if (SPLIT == 0) read_share(next);
-        if (B == 0 && n >= 4 && ((n >> 1) & 1) == half) heads(n - 4, true);
+        if ((n & 1) == 0 && n >= 4 && ((n >> 1) & 1) == half) heads(n - 4, true);
         float s2[NO][2];
 #pragma unroll
         for (int o = 0; o < NO; ++o) s2[o][0] = s2[o][1] = 0.f;
         auto second = [&](int f) {
-            const float y = vmax(acc[B ^ 1][f], 0.f);
+            const float y = vmax(done[f], 0.f);
 #pragma unroll
             for (int o = 0; o < NO; ++o) {
                 s2[o][f & 1] = __builtin_fmaf(wv[o][f % G], y, s2[o][f & 1]);
@@ -458,36 +448,38 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
         };
-        const parts_u32x4 flag0 = *reinterpret_cast<const parts_u32x4*>(flags + now * 8), flag1 = *reinterpret_cast<const parts_u32x4*>(flags + now * 8 + 4);
-        // (the sums of the round before are there: its last MFMA ended a head, or a turn of the other wave, ago; what the compiler
-        //  cannot see is that they come from MFMAs)
-        asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[B ^ 1]));
+        parts_u32x4 flag[2];
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-            constexpr int PW[6] = {2, 0, 1, 1, 0, 0}, PX[6] = {0, 2, 1, 0, 1, 0};
             if (s == BARRIER) barrier();
 #pragma unroll
-            for (int m = 0; m < 6; ++m) {
-                if (s == 0 && m == 0)
-                    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(acc[B]) : "v"(w1[s][PW[m]]), "v"(xf[s & 1][PX[m]]));
-                else
-                    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc[B]) : "v"(w1[s][PW[m]]), "v"(xf[s & 1][PX[m]]));
+            for (int m = 0; m < 8; ++m) {
+                const parts_u32x4 w = w1[s][PARTS_W[m]], x = xf[s & 1][PARTS_X[m]];
+                if (m == 0 && s == 0) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(large) : "v"(w), "v"(x));
+                else if (m == 0) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(these) : "v"(w), "v"(x));
+                else if (m == 1 && s == 0) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(small) : "v"(w), "v"(x));
+                else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(small) : "v"(w), "v"(x));
                 // in the shadow of this MFMA:
                 if (m < 3 && s + 1 < KS) read_step(now, s + 1, m);
                 if (m < 3 && s + 1 == KS && BARRIER < KS) read_step(next, 0, m);
+                if (s > 0 && m >= 4) {                              // (three MFMAs behind the one that they come from)
+#pragma unroll
+                    for (int i = 4 * (m - 4); i < 4 * (m - 3); ++i) large[i] += these[i];
+                    asm volatile("" : "+v"(large));                 // (here, and not where the sums are used)
+                }
                 if (s < BARRIER)
 #pragma unroll
-                    for (int f = s * FEATURES + m * FEATURES / 6; f < s * FEATURES + (m + 1) * FEATURES / 6; ++f) second(f);
+                    for (int f = s * FEATURES + m * FEATURES / 8; f < s * FEATURES + (m + 1) * FEATURES / 8; ++f) second(f);
                 if (s + 1 == SPLIT && m == 4) read_share(next);
                 if (s == SPLIT || s == SPLIT + 1) {
-                    split_slice(next, (s - SPLIT) * 6 + m);
-                    if (s == SPLIT + 1 && m == 5) {
-                        raise_flag(next);
-                    }
+                    const int slice = (s - SPLIT) * 8 + m;
+                    if (slice < 12) split_slice(next, slice);
+                    else if (slice == 12) raise_flag(next);
                 }
                 if (s == 0 && m == 5) fetch_share(n + 3, now);
-                constexpr int APART = BARRIER < KS ? 6 * (KS - BARRIER) / 4 : 1;
-                if (s >= BARRIER && ((s - BARRIER) * 6 + m) % APART == 1 && n >= 4) store_quarter(n - 4, ((s - BARRIER) * 6 + m) / APART);
+                if (s + 1 == KS && m >= 4 && m < 6) flag[m - 4] = *reinterpret_cast<const parts_u32x4*>(flags + now * 8 + (m - 4) * 4);
+                constexpr int APART = BARRIER < KS ? 8 * (KS - BARRIER) / 4 : 1;
+                if (s >= BARRIER && ((s - BARRIER) * 8 + m) % APART == 1 && n >= 4) store_quarter(n - 4, ((s - BARRIER) * 8 + m) / APART);
                 if (s == BARRIER && m < NO) put_sum(m, false);
                 if (s == BARRIER + 1 && m < NO) put_sum(m, true);
                 __builtin_amdgcn_sched_barrier(0);
@@ -508,9 +500,14 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
 #pragma unroll
                 for (int q = 0; q < 4; ++q) store_quarter(n - 4, q);
         }
-        if (w_bad || __any((flag0.x | flag0.y | flag0.z | flag0.w | flag1.x | flag1.y | flag1.z | flag1.w) != 0)) {
-            asm volatile("s_nop 15\n\ts_nop 15" : "+v"(acc[B]));
-            clear(acc[B]);
+        // (what the compiler cannot see is that `small` comes from MFMAs: the last is eight passes)
+        asm volatile("s_nop 15\n\ts_nop 3" : "+v"(small));
+#pragma unroll
+        for (int i = 0; i < 16; ++i) done[i] = large[i] + small[i];
+        const parts_u32x4 both = flag[0] | flag[1];
+        const unsigned bad = both.x | both.y | both.z | both.w;
+        if (w_bad || __any(bad != 0)) {                             // a round with inputs that parts cannot hold
+            clear(these);
             long row = (long)tile_at(n) * EN_ROWS + r;
             row = row < batch ? row : batch - 1;
             for (int s = 0; s < (K0 + 15) / 16; ++s) {
@@ -521,18 +518,15 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
                 for (int c = 0; c < 2; ++c)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        asm volatile("s_nop 3\n\tv_mfma_f32_32x32x2_f32 %0, %1, %2, %0" : "+v"(acc[B]) : "v"(wv1[c][i]), "v"(xv[c][i]));
+                        asm volatile("s_nop 3\n\tv_mfma_f32_32x32x2_f32 %0, %1, %2, %0" : "+v"(these) : "v"(wv1[c][i]), "v"(xv[c][i]));
             }
+            asm volatile("s_nop 15\n\ts_nop 15" : "+v"(these));
+            done = these;
         }
         now = next;
         next = next == 2 ? 0 : next + 1;
     };
-    for (int n = 0;;) {                               // (one round more than there are: its products are not used)
-        work(std::integral_constant<int, 0>{}, n);
-        if (n++ == mine) break;
-        work(std::integral_constant<int, 1>{}, n);
-        if (n++ == mine) break;
-    }
+    for (int n = 0; n <= mine; ++n) work(n);          // (one round more than there are: its products are not used)
     // what the rounds did not get to: the last two (or one, if it has no partner), and with an odd last round the two before it
     __syncthreads();
     const int last = (mine - 1) & ~1;                // the even round of the last pair

@@ -20,12 +20,14 @@
 // tile per SIMD.
 // Measured, that stack over 16384 rows (node by node / every layer through part_product, a draw per tile / this kernel, us):
 // one model 32.8 / 13.8 / 10.3, 16 members 206 / 87 / 68.8 (the matrix pipe alone: 41).
-//   PARTS: the same with the products in three bf16 parts (below), 144 MFMAs of 16 cycles for 16 rows instead of 192 of 32, and
-// 400 vector instructions more, in part beside them: 16 members of 16384 rows 70 -> 52.5, of 57344 223 -> 157.  Bound by the
-// vector ALU (1122 instructions, 4490 cycles a tile, of 6100 in the long run) and the 7 us in which a workgroup's sixteen waves
-// start together, with the same phases; a raised priority for waves in their products changed nothing.  Sixteen waves because their norms and heads hide behind each other's products (eight: 63.6
-// and 186).  The sums are closer to float64 than the f32 pipe's (error of the probabilities 0.63 to 0.88 of that, 1.00 where it
-// is the exponential's).
+//   PARTS: the same with the products in three bf16 parts (parts.h), 192 MFMAs of 16 cycles for 16 rows instead of 192 of 32, and
+// 400 vector instructions more, in part beside them: 16 members of 16384 rows 68 -> 56 us, of 57344 228 -> 190.  Bound by the
+// vector ALU and the 7 us in which a workgroup's sixteen waves start together, with the same phases; a raised priority for waves
+// in their products changed nothing.  Sixteen waves because their norms and heads hide behind each other's products (with six
+// products instead of eight: sixteen waves 52.5 and 157, eight 63.6 and 186).  128 registers a lane are just enough: what the head,
+// the draws and the f32 product need of addresses is computed where it is used.  (Kept over the loop, they were up to 30 registers
+// in memory.)  The sums are closer to float64 than the f32 pipe's: error of the probabilities 0.41 to 1.00 of that, whatever
+// the inputs (N(0, 1), uniform, 0 and 1, relu, one to eight non-zero numbers a row).
 #include "mlp_common.h"
 #include "row_common.h"
 #include "gemm_dma.h"
@@ -120,38 +122,24 @@ __device__ __forceinline__ void part_product(const unsigned char*& wp, const f32
     }
 }
 
-// ---- the products on the bf16 matrix pipe: both operands as three bf16 parts (parts.h), six of the nine products, each of
+// ---- the products on the bf16 matrix pipe: both operands as three bf16 parts (parts.h), eight of the nine products, each of
 // 32 of K in one v_mfma_f32_16x16x32_bf16.  Lane group q holds k = 32 j + 4 q + i and 32 j + 16 + 4 q + i, so that a layer's
 // results are here, too, the next one's operand.
 typedef __bf16 stack_bf16x8 __attribute__((ext_vector_type(8)));
 
-__device__ __forceinline__ void stack_parts(f32x4 v, f32x4 w, parts_u32x4 (&p)[3]) {
+__device__ __forceinline__ void stack_parts(f32x4 v, f32x4 w, float scale, parts_u32x4 (&p)[3]) {
     const parts_f32x4 both[2] = {{v[0], v[1], v[2], v[3]}, {w[0], w[1], w[2], w[3]}};
-    split_parts(both, p);
+    split_parts(both, scale, p);
 }
 __device__ __forceinline__ f32x4 parts_mfma(parts_u32x4 w, parts_u32x4 x, f32x4 y) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(stack_bf16x8, w), __builtin_bit_cast(stack_bf16x8, x), y, 0, 0, 0);
 }
 
-struct PartsRange {                     // whether parts hold all of the numbers seen (NaN: a NaN either way)
-    unsigned least = 0xffffffffu;
-    float most = 0.f;
-    __device__ __forceinline__ void take(f32x4 v) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const unsigned w = parts_magnitude(v[i]);
-            least = w < least ? w : least;
-            most = fmaxf(most, fabsf(v[i]));
-        }
-    }
-    __device__ __forceinline__ bool wide() const { return parts_tiny(least) || most > 0x1p60f; }
-};
-
 // A full layer, the weights of a tile of features and 32 of K read ahead of the products of the one before.
 __device__ __forceinline__ void parts_product(const unsigned char*& wp, const parts_u32x4 (&x)[2][3], f32x4 (&y)[4]) {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     parts_u32x4 w[2][3];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) y[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 large = zero, small = zero;
 #pragma unroll
     for (int s = 0; s <= 8; ++s) {
         __builtin_amdgcn_sched_barrier(0);
@@ -160,13 +148,13 @@ __device__ __forceinline__ void parts_product(const unsigned char*& wp, const pa
             for (int i = 0; i < 3; ++i) w[s & 1][i] = *reinterpret_cast<const parts_u32x4*>(wp + s * ST_PARTS_UNIT + i * 1024);
         }
         if (s > 0) {
-            const int j = (s - 1) >> 2, t = (s - 1) & 3, now = (s - 1) & 1;
-            y[t] = parts_mfma(w[now][2], x[j][0], y[t]);
-            y[t] = parts_mfma(w[now][0], x[j][2], y[t]);
-            y[t] = parts_mfma(w[now][1], x[j][1], y[t]);
-            y[t] = parts_mfma(w[now][1], x[j][0], y[t]);
-            y[t] = parts_mfma(w[now][0], x[j][1], y[t]);
-            y[t] = parts_mfma(w[now][0], x[j][0], y[t]);
+            const int t = (s - 1) >> 1, j = (s - 1) & 1, now = (s - 1) & 1;
+            const f32x4 these = parts_mfma(w[now][0], x[j][0], zero);
+            if (j == 0) small = zero;
+#pragma unroll
+            for (int p = 1; p < 8; ++p) small = parts_mfma(w[now][PARTS_W[p]], x[j][PARTS_X[p]], small);
+            if (j == 0) large = these;
+            else y[t] = (large + these) + small;
         }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -243,15 +231,15 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     } else {
-        // units wave, wave + waves, ... of the whole stack, two of them in flight
+        // units (layer, tile of features, 32 of K) wave, wave + waves, ... of the whole stack, two of them in flight
         const int units = 8 * layers;
-        PartsRange range;
+        PartsWeights range;
         for (int n0 = wave; n0 < units; n0 += 2 * waves) {
             f32x4 v[2][2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int n = n0 + i * waves < units ? n0 + i * waves : n0, l = n >> 3, K = a.dims[l];
-                const int row = 16 * (n & 3) + r, col = 32 * ((n >> 2) & 1) + 4 * q;
+                const int row = 16 * ((n >> 1) & 3) + r, col = 32 * (n & 1) + 4 * q;
                 const float* const at = weights_of(l) + (long)row * K + col;
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -263,9 +251,9 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
             for (int i = 0; i < 2; ++i) {
                 if (i == 1 && n0 + waves >= units) break;
                 parts_u32x4 p[3];
-                range.take(v[i][0]);
-                range.take(v[i][1]);
-                stack_parts(v[i][0], v[i][1], p);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) range.take(v[i][k >> 2][k & 3]);
+                stack_parts(v[i][0], v[i][1], PARTS_W_SCALE, p);
 #pragma unroll
                 for (int k = 0; k < 3; ++k)
                     *reinterpret_cast<parts_u32x4*>(lds + (n0 + i * waves) * ST_PARTS_UNIT + k * 1024 + lane * 16) = p[k];
@@ -290,7 +278,9 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
     for (int turn = 0; tile < a.tiles; tile += stride, ++turn) {
         // The uniforms of four tiles at once, lane group q those of tile q from here: a draw is 250 vector instructions.
         if (a.action != nullptr && (turn & 3) == 0) {
-            const long at = (long)(tile + (long)q * stride) * ST_ROWS + r;
+            int rr = r, qq = q;
+            if constexpr (PARTS) asm volatile("" : "+v"(rr), "+v"(qq));      // (see wide_product)
+            const long at = (long)(tile + (long)qq * stride) * ST_ROWS + rr;
             const int row = at < a.batch ? (int)at : a.batch - 1;
             if (a.ph.philox_mode < 0) u4 = a.u[(long)e * a.batch + row];
             else if (a.ph.member_rows > 0) u4 = run_row_uniform<unsigned>(a.ph, row, a.ph.draw_offset + (unsigned long long)e * a.ph.member_draws);
@@ -303,14 +293,18 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
         // rows with numbers that parts cannot hold get the f32 product: the others' sums are theirs alone either way
         auto product_of_parts = [&](int l, f32x4 (&y)[HT]) {
           if constexpr (PARTS) {
-            PartsRange range;
+            float most = 0.f;
             parts_u32x4 xp[2][3];
 #pragma unroll
-            for (int j = 0; j < HT; ++j) range.take(x[j]);
-            const unsigned long long lanes = __ballot(range.wide() || weights_wide);
-            if (lanes != 0) wide_product<HT>(weights_of(l), a.dims[l], a.dims[l + 1], x, scratch, r, q);
-            stack_parts(x[0], x[1], xp[0]);
-            stack_parts(x[2], x[3], xp[1]);
+            for (int j = 0; j < HT; ++j) most = parts_most(parts_most(most, x[j][0], x[j][1]), x[j][2], x[j][3]);
+            const unsigned long long lanes = __ballot(most > PARTS_MOST || weights_wide);
+            if (lanes != 0) {
+                int row = r, group = q;
+                asm volatile("" : "+v"(row), "+v"(group));      // (addresses are computed here: kept, they are registers that are not there)
+                wide_product<HT>(weights_of(l), a.dims[l], a.dims[l + 1], x, scratch, row, group);
+            }
+            stack_parts(x[0], x[1], PARTS_X_SCALE, xp[0]);
+            stack_parts(x[2], x[3], PARTS_X_SCALE, xp[1]);
             parts_product(wp, xp, y);
             if (lanes != 0) {
                 const bool mine = (((lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) >> r) & 1) != 0;
@@ -373,13 +367,14 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
         // ---- the head and the sampling: lane l of 16 holds columns 4 l .. of its row, as in the row primitives ----
-        const int lq = r;                         // (lane % 16 again: here the column quad)
+        int lq = r, hq = q;                       // (lane % 16 again: here the column quad)
+        if constexpr (PARTS) asm volatile("" : "+v"(lq), "+v"(hq));      // (see wide_product)
         const int limit = a.mask_size;
         const int rows_here = a.batch - tile * ST_ROWS;
         float* const tile_policy = policy + (long)tile * (ST_ROWS * a.n);
 #pragma unroll
         for (int pass = 0; pass < 4; ++pass) {
-            const int rr = 4 * pass + q;
+            const int rr = 4 * pass + hq;
             f32x4 v = *reinterpret_cast<const f32x4*>(scratch + rr * 256 + ((lq ^ rr) & 15) * 16);
             // columns past the head's width, or its mask, enter as -inf (an exact 0 after the exponential) or 0
             if (limit < ST_MAX_OUT) {

@@ -598,6 +598,73 @@ def test_ensemble_in_three_parts_keeps_what_parts_cannot_hold(LY):
         assert (a[ok] - b[ok]).abs().max().item() < 1e-5
 
 
+def few(gen, m, k, terms):
+    at = torch.rand((m, k), generator=gen, device="cuda").topk(terms).indices
+    return torch.zeros((m, k), device="cuda").scatter_(1, at, torch.randn((m, terms), generator=gen, device="cuda"))
+
+
+PARTS_INPUTS = {
+    "normal": lambda gen, m, k: torch.randn((m, k), generator=gen, device="cuda"),
+    "uniform": lambda gen, m, k: torch.rand((m, k), generator=gen, device="cuda"),
+    "relu": lambda gen, m, k: torch.randn((m, k), generator=gen, device="cuda").relu(),
+    "features": lambda gen, m, k: (torch.rand((m, k), generator=gen, device="cuda") < 0.2).float(),
+    "lognormal": lambda gen, m, k: torch.randn((m, k), generator=gen, device="cuda") * torch.exp(2 * torch.randn((m, k), generator=gen, device="cuda")),
+    "eight": lambda gen, m, k: few(gen, m, k, 8), "two": lambda gen, m, k: few(gen, m, k, 2), "one": lambda gen, m, k: few(gen, m, k, 1)}
+
+
+def hidden_features(members):
+    """Second layers that pass features (11 e + 17 o) % 64, o < 4, of member e on as they are, and those features."""
+    features = [[(11 * e + 17 * o) % 64 for o in range(4)] for e in range(members)]
+    w2 = torch.zeros((members, 4, 64), device="cuda")
+    for e in range(members):
+        w2[e, torch.arange(4), torch.tensor(features[e])] = 1.0
+    return w2, features
+
+
+@pytest.mark.parametrize("inputs", sorted(PARTS_INPUTS))
+@pytest.mark.parametrize("k0", [16, 64, 120])
+def test_ensemble_in_three_parts_is_no_further_off_than_in_f32(LY, k0, inputs):
+    """Six members on the bf16 pipe against two of them alone, which f32 MFMAs take: the error of the hidden layer against float64
+    (2-norm) is no larger.  A single product is rounded once: to the nearest but for 3 in 1000, and those within 2^-7 of that."""
+    announce("ensemble parts error k0=%d %s" % (k0, inputs))
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(k0)
+    x = PARTS_INPUTS[inputs](gen, 65536, k0)
+    w1 = torch.randn((6, 64, k0), generator=gen, device="cuda") / k0 ** 0.5
+    w2, features = hidden_features(6)
+    parts = LY.mlp_forward_ensemble(x, (w1, w2), "none")[:2]
+    f32 = LY.mlp_forward_ensemble(x, (w1[:2].contiguous(), w2[:2].contiguous()), "none")
+    want = torch.stack([torch.relu(x.double() @ w1[e, features[e]].double().T) for e in range(2)])
+    assert (parts.double() - want).norm() <= 1.005 * (f32.double() - want).norm()
+    if inputs == "one":
+        assert (parts != want.float()).double().mean().item() < 3e-3
+        assert ((parts.double() - want).abs() <= 2.0 ** -24 * (1 + 2.0 ** -7) * want).all()
+
+
+@pytest.mark.parametrize("x_exp,w_exp", [(-60, 0), (-105, 50), (-126, 58), (-149, 58), (58, -93), (58, -110), (-70, -66)])
+def test_ensemble_in_three_parts_of_tiny_numbers(LY, x_exp, w_exp):
+    """Inputs down to the smallest subnormal and weights down to 2^-94 are held by their parts, smaller weights send their member
+    through f32 MFMAs: in every row as close as f32 sums are, also where the lowest parts are subnormal bf16 or (the last case)
+    the products subnormal f32, which are rounded to multiples of 2^-149."""
+    announce("ensemble parts, tiny numbers 2^%d 2^%d" % (x_exp, w_exp))
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(9)
+    k0 = 128
+    x = torch.randint(-2 ** 20, 2 ** 20, (65536, k0), generator=gen, device="cuda").float() * 2.0 ** (-20 if x_exp > -149 else 0)
+    x = (x.double() * 2.0 ** x_exp).float()
+    w1 = torch.randn((6, 64, k0), generator=gen, device="cuda")
+    w1[1] *= 2.0 ** w_exp
+    w1[2] = (w1[2].double() * 2.0 ** w_exp).float()
+    w2, features = hidden_features(6)
+    got = LY.mlp_forward_ensemble(x, (w1, w2), "none")
+    for e in (1, 2):
+        w = w1[e, features[e]].double()
+        want, scale = torch.relu(x.double() @ w.T), x.double().norm(dim=1, keepdim=True) * w.norm(dim=1)
+        off = (got[e].double() - want).abs()
+        assert (off <= 2.0 ** -24 * 16 * scale + 2.0 ** -149 * k0).all()
+        assert x_exp + w_exp < -120 or (off.norm() / want.norm()).item() < 2.0 ** -24 * (k0 / 2) ** 0.5 + 1e-7
+
+
 @pytest.mark.parametrize("name", ["mlp_forward_ensemble_parts", "mlp_forward_ensemble_parts_action"])
 def test_the_parts_ensemble_kernels_are_named(name):
     announce("kernel info " + name)

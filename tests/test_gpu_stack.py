@@ -185,6 +185,47 @@ def test_numbers_that_parts_cannot_hold(S, what):
         assert torch.equal(policy[0], clean[0])
 
 
+@pytest.mark.parametrize("inputs", ["normal", "uniform", "relu", "features", "eight", "two", "one"])
+@pytest.mark.parametrize("widths,acts", [((64, 64), []), ((56, 64, 64), ["relu"]), ((64, 64, 64, 64), ["tanh", "ln+relu"])])
+def test_parts_are_no_further_off_than_f32(S, widths, acts, inputs):
+    """All rows at once in parts against a sixteenth of them at a time, which f32 MFMAs take: the error of the probabilities against
+    float64 (2-norm) is no larger, whatever the inputs."""
+    announce("stack in parts, error %s %s" % (widths, inputs))
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(len(widths))
+    normal = lambda *shape: torch.randn(shape, generator=gen, device="cuda")
+    rows, k = 131072, widths[0]
+    if inputs in ("one", "two", "eight"):
+        terms = {"one": 1, "two": 2, "eight": 8}[inputs]
+        x = torch.zeros((rows, k), device="cuda").scatter_(1, normal(rows, k).topk(terms).indices, normal(rows, terms))
+    else:
+        x = {"normal": lambda: normal(rows, k), "uniform": lambda: normal(rows, k).abs().frac(), "relu": lambda: normal(rows, k).relu(),
+             "features": lambda: (normal(rows, k) > 0.84).float()}[inputs]()
+    ws = [normal(1, b, a) / a ** 0.5 for a, b in zip(widths[:-1], widths[1:])]
+    for head in (S.ROW_SOFTMAX, S.ROW_REGRET_MATCHING):
+        want = probabilities(x, ws, acts, head == S.ROW_REGRET_MATCHING, 0)
+        parts, _ = forward(S, x, ws, acts, head, sample=False)
+        f32 = torch.cat([forward(S, part.contiguous(), ws, acts, head, sample=False)[0] for part in x.chunk(16)], dim=1)
+        assert not torch.equal(parts, f32)
+        assert (parts.double() - want).norm() <= 1.005 * (f32.double() - want).norm()
+
+
+@pytest.mark.parametrize("x_exp,w_exp", [(-60, 0), (-105, 0), (-140, 58), (-70, -50), (58, -93), (58, -110)])
+def test_parts_of_tiny_numbers(S, x_exp, w_exp):
+    """A layer and regret matching, which does not see a common factor: inputs down to subnormal numbers are held by their parts,
+    and weights down to 2^-94 (smaller ones send their member through f32 MFMAs)."""
+    announce("stack in parts, tiny numbers 2^%d 2^%d" % (x_exp, w_exp))
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(11)
+    x = torch.randint(-511, 512, (131072, 64), generator=gen, device="cuda").double() * 2.0 ** (x_exp - 9)
+    w = torch.randn((1, 64, 64), generator=gen, device="cuda").double() * 2.0 ** w_exp
+    x, ws = x.float(), [w.float()]
+    got, _ = forward(S, x, ws, [], S.ROW_REGRET_MATCHING, sample=False)
+    want = probabilities(x, ws, [], True, 0)
+    assert (got.double() - want).norm() <= 4 * 2.0 ** -24 * want.norm()
+    assert ((got.double() - want).norm(dim=2) <= 32 * 2.0 ** -24 * want.norm(dim=2)).all()
+
+
 @pytest.mark.parametrize("name", ["stack_forward_f32_parts", "stack_forward_f32_parts_regret"])
 def test_the_instances_in_parts_are_named(S, name):
     announce("kernel info " + name)
