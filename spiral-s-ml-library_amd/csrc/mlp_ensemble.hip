@@ -229,7 +229,8 @@ __global__ __launch_bounds__(EN_THREADS) void mlp_ensemble_kernel(const Ensemble
 // wait for LDS and each other.  (Six products in one sum, without the additions, took 210 us and lost bits, see parts.h.  Taken
 // back on the way there: one wave per SIMD with both halves 248 us, heads in front of a barrier at the round's end 240, zeros and
 // probabilities of a row stored apart 257, fragments two steps ahead instead of one 230, stores past the caches 228.)
-// Inputs or weights that parts cannot hold (parts.h) send a round, or all rounds of a member, through f32 MFMAs.
+// Rows of inputs, or weights of a member, that parts cannot hold (parts.h) take f32 MFMAs: a round is multiplied twice then, and
+// the rows keep what is theirs, so a row's result depends on itself alone.
 typedef const __attribute__((address_space(1))) f32x4* global_f32x4;
 constexpr int EP_THREADS = 512;
 typedef unsigned u32x2_parts __attribute__((ext_vector_type(2)));
@@ -506,7 +507,7 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
         for (int i = 0; i < 16; ++i) done[i] = large[i] + small[i];
         const parts_u32x4 both = flag[0] | flag[1];
         const unsigned bad = both.x | both.y | both.z | both.w;
-        if (w_bad || __any(bad != 0)) {                             // a round with inputs that parts cannot hold
+        if (w_bad || __any(bad != 0)) {                             // rows that parts cannot hold, and no others, take their f32 sums
             clear(these);
             long row = (long)tile_at(n) * EN_ROWS + r;
             row = row < batch ? row : batch - 1;
@@ -521,7 +522,9 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
                         asm volatile("s_nop 3\n\tv_mfma_f32_32x32x2_f32 %0, %1, %2, %0" : "+v"(these) : "v"(wv1[c][i]), "v"(xv[c][i]));
             }
             asm volatile("s_nop 15\n\ts_nop 15" : "+v"(these));
-            done = these;
+            const bool mine = w_bad || ((bad >> r) & 1) != 0;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) done[i] = mine ? these[i] : done[i];
         }
         now = next;
         next = next == 2 ? 0 : next + 1;

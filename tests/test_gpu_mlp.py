@@ -665,6 +665,35 @@ def test_ensemble_in_three_parts_of_tiny_numbers(LY, x_exp, w_exp):
         assert x_exp + w_exp < -120 or (off.norm() / want.norm()).item() < 2.0 ** -24 * (k0 / 2) ** 0.5 + 1e-7
 
 
+@pytest.mark.parametrize("k0", [32, 64, 128])
+def test_ensemble_in_three_parts_keeps_rows_and_members_their_own(LY, k0):
+    """Rows with inputs that parts cannot hold, and a member with such weights, change nothing in other rows and members; and where
+    rows and members lie does not matter either: all to the last bit."""
+    announce("ensemble parts, rows and members of their own k0=%d" % k0)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(k0)
+    batch = 65536
+    x = torch.randn((batch, k0), generator=gen, device="cuda")
+    w1, w2 = torch.randn((6, 64, k0), generator=gen, device="cuda") / 8, torch.randn((6, 16, 64), generator=gen, device="cuda") / 8
+    w1[4, 60, 1] = 0.0
+    clean, _ = LY.mlp_forward_ensemble(x, (w1, w2), "softmax", torch.ones((6, batch), device="cuda"), mask_size=3)
+    odd = x.clone()
+    odd[3, 5], odd[40, 7], odd[100, 0], odd[20000] = float("inf"), float("-inf"), float("nan"), 1e20
+    odd[300], odd[batch - 1] = odd[300] * 2.0 ** -130, odd[batch - 1] * 2.0 ** 90
+    w = w1.clone()
+    w[1, 9, 3] = float("inf")
+    w[4, 60, 1] = 1e-35
+    policy = LY.mlp_forward_ensemble(odd, (w, w2), "softmax", mask_size=3)
+    rest = torch.ones(batch, dtype=torch.bool, device="cuda")
+    rest[[3, 40, 100, 300, 20000, batch - 1]] = False
+    for e in (0, 2, 3, 5):
+        assert torch.equal(policy[e, rest], clean[e, rest])
+    assert torch.allclose(policy[4, rest], clean[4, rest], rtol=0, atol=1e-5)
+    rows, members = torch.randperm(batch, generator=gen, device="cuda"), torch.randperm(6, generator=gen, device="cuda")
+    moved = LY.mlp_forward_ensemble(x[rows], (w1[members].contiguous(), w2[members].contiguous()), "softmax", mask_size=3)
+    assert torch.equal(moved, clean[members][:, rows])
+
+
 @pytest.mark.parametrize("name", ["mlp_forward_ensemble_parts", "mlp_forward_ensemble_parts_action"])
 def test_the_parts_ensemble_kernels_are_named(name):
     announce("kernel info " + name)
