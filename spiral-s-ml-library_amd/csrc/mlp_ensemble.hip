@@ -662,23 +662,34 @@ static const void* pick_ensemble_kernel_kg(bool exact, bool action) {
     if (exact) return action ? (const void*)mlp_ensemble_kernel<KG, true, true> : (const void*)mlp_ensemble_kernel<KG, true, false>;
     return action ? (const void*)mlp_ensemble_kernel<KG, false, true> : (const void*)mlp_ensemble_kernel<KG, false, false>;
 }
+// One workgroup (4 waves, one per SIMD) per compute unit while the members leave room for that: a wave then keeps its
+// member's weights for all its tiles.
+static long ensemble_blocks(long members, long tiles) {
+    const long gx = (device_cu_count() + members - 1) / members, most = (tiles + 3) / 4;
+    return gx < most ? gx : most;
+}
 // Rounds per workgroup on the bf16 pipe: four members a workgroup, one workgroup per unit.
 static long ensemble_parts_blocks(long members, long tiles) {
     const long blocks = device_cu_count() / ((members + 3) / 4);
     return blocks < 1 ? 1 : blocks < tiles ? blocks : tiles;
 }
-// Which kernel takes two layers.  The one on the bf16 pipe does a round of four members in 3.5 us (128 inputs), the f32 one a
-// tile of one in 5.2 on each of a unit's four SIMDs; below three members the former leaves half of a workgroup idle, and where
-// the latter has one tile per wave it is through before two rounds are (us, f32 / bf16 pipe, 128 inputs: 2 x 65536 rows 33 / 37,
-// 5 x 6144 16.0 / 18.2; 4 x 6144 15.3 / 15.1, 9 x 6144 27.6 / 21.1, 3 x 65536 71 / 36, 5 x 65536 105 / 58, 9 x 65536 182 / 83,
-// 32 x 65536 346 / 230).  Up to 64 inputs, half or a quarter of the products, it is ahead from five tiles for each of the f32
-// kernel's waves (32 inputs: 32 x 256 6.5 / 8.7, 8 x 8192 11.5 / 12.6, 4 x 32768 16.8 / 17.2; 16 x 12288 21.7 / 21.4, 32 x 8192
-// 26.0 / 24.7, 32 x 65536 167 / 145).
+// Which kernel takes two layers: the faster by what their rounds take.  The one on the bf16 pipe has rounds of a tile of four
+// members, a workgroup a unit, the f32 one of a tile on each of a unit's four SIMDs; either is a start and so much for each round
+// of the unit with the most.  Fitted on 350 calls of 2 to 1200 members, 16 to 131072 rows, with and without sampling, to 10 and
+// 17 % (ninety of a hundred); on 450 others none that it sends to the bf16 pipe is more than 1 % slower there than in f32, and it is 2 %
+// behind the faster one on the geometric mean.  (Us, f32 / bf16 pipe, taken first: 128 inputs, 17 x 32 rows 8.7 / 14.2,
+// 9 x 6144 26.2 / 22.3, 3 x 65536 70 / 42, 516 x 2048 259 / 191; 32 inputs, 1028 x 2048 191 / 248, 516 x 2048 117 / 122,
+// 5 x 65536 49 / 40, 33 x 8192 45 / 28.)  Below three members the bf16 pipe has half of its waves idle.
 static bool ensemble_takes_parts(long members, long batch, int k0) {
-    const long tiles = (batch + EN_ROWS - 1) / EN_ROWS, blocks = ensemble_parts_blocks(members, tiles);
-    const long each = (device_cu_count() + members - 1) / members;      // workgroups of a member in ensemble_launch
+    const long tiles = (batch + EN_ROWS - 1) / EN_ROWS, cus = device_cu_count();
     if (members < 3 || tiles > 2147480000l) return false;
-    return k0 <= 64 ? tiles > 4 * 4 * each : !(tiles <= 4 * each && tiles > blocks);
+    const long groups = (members + 3) / 4, blocks = ensemble_parts_blocks(members, tiles);
+    const long parts = (groups * blocks + cus - 1) / cus * ((tiles + blocks - 1) / blocks);
+    const long gx = ensemble_blocks(members, tiles);
+    const long f32 = (members * gx + cus - 1) / cus * ((tiles + 4 * gx - 1) / (4 * gx));
+    const float start[3][2] = {{6.2f, 3.7f}, {8.4f, 4.2f}, {11.5f, 6.1f}}, round[3][2] = {{2.f, 2.44f}, {2.45f, 3.55f}, {3.36f, 5.8f}};
+    const int k = k0 <= 32 ? 0 : k0 <= 64 ? 1 : 2;                       // 32, 64 or 128 inputs
+    return start[k][0] + round[k][0] * (float)parts < 0.9f * (start[k][1] + round[k][1] * (float)f32);
 }
 
 template <int KS>
@@ -711,17 +722,10 @@ static const void* pick_layer_kernel(int kg, bool exact) {
          : kg == 16 ? pick_layer_kernel_kg<16, MODE>(exact) : pick_layer_kernel_kg<32, MODE>(exact);
 }
 
-// One workgroup (4 waves, one per SIMD) per compute unit while the members leave room for that: a wave then keeps its
-// member's weights for all its tiles.
 static int ensemble_launch(const void* kernel, EnsembleArgs& a, hipStream_t stream, const char* what) {
     a.tiles = (a.batch + EN_ROWS - 1) / EN_ROWS;
-    const long cus = device_cu_count();
-    long gx = (cus + a.members - 1) / a.members;
-    const long most = (a.tiles + 3) / 4;
-    if (gx > most) gx = most;
-    if (gx < 1) gx = 1;
     void* args[] = {(void*)&a};
-    hipError_t err = hipLaunchKernel(kernel, dim3((unsigned)gx, (unsigned)a.members), dim3(EN_THREADS), args, 0, stream);
+    hipError_t err = hipLaunchKernel(kernel, dim3((unsigned)ensemble_blocks(a.members, a.tiles), (unsigned)a.members), dim3(EN_THREADS), args, 0, stream);
     if (err != hipSuccess) return fail(SP_ERR_DEVICE, "%s: launch failed: %s", what, hipGetErrorString(err));
     return check_launch(what);
 }

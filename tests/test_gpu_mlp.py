@@ -535,7 +535,10 @@ def test_ensemble_binarize(LY, members, batch, k0, n, modulo):
     (4, 32 * 256 * 6 + 33, [128, 64, 8], "none", None, False), (9, 32 * 85 * 7 + 40, [120, 64, 64], "regret_matching", 4, False),
     (9, 32 * 85 * 8, [128, 64, 64], "softmax", 3, True), (256, 200, [48, 64, 12], "regret_matching", 3, False),
     (4, 32 * 1024 + 1, [16, 64, 16], "regret_matching", 2, False), (7, 32 * 600 - 5, [24, 64, 20], "softmax", 3, True),      # up to 64 inputs:
-    (6, 32 * 690 + 9, [64, 64, 64], "regret_matching", 3, False), (300, 32 * 17 + 1, [40, 64, 12], "softmax", 4, True)])    # from five tiles a wave
+    (6, 32 * 690 + 9, [64, 64, 64], "regret_matching", 3, False), (300, 32 * 17 + 1, [40, 64, 12], "softmax", 4, True),    # from five tiles a wave
+    (768, 1, [128, 64, 64], "softmax", 3, True), (800, 31, [8, 64, 4], "softmax", 0, True), (1021, 64, [24, 64, 16], "regret_matching", 2, False),   # many members:
+    (900, 96, [104, 64, 20], "softmax", 3, False), (513, 129, [64, 64, 64], "softmax_regret_matching", 4, True),      # one to nine
+    (900, 160, [16, 64, 6], "softmax", 1, True), (777, 224, [120, 64, 8], "none", None, False), (900, 265, [32, 64, 64], "softmax", 3, True)])  # rounds
 def test_ensemble_in_three_parts(LY, members, batch, dims, head, mask, sample):
     """Against float64: the hidden layer no further off than f32 sums are, so the f32 bar of the head holds row by row wherever the
     head itself is not the quotient of two small numbers; exact zeros behind the mask; actions given the kernel's own policy."""
@@ -569,15 +572,16 @@ def test_ensemble_in_three_parts(LY, members, batch, dims, head, mask, sample):
 
 
 def test_ensemble_in_three_parts_keeps_what_parts_cannot_hold(LY):
-    """Members 0 and 1 of four on the bf16 pipe against the same two alone on the f32 kernel: inputs and weights with infinities, NaN,
-    values whose bf16 is infinite, values below 2^-110."""
+    """Members 0 and 1 of four on the bf16 pipe against the same two alone on the f32 kernel, hidden features as they are: inputs and
+    weights with infinities, NaN, values whose bf16 is infinite and values above 2^60, weights below 2^-94.  Infinities where the
+    f32 kernel has them, the rest to f32 sums of 128 terms, either of which is off by less than 16 roundings of the row's norm."""
     announce("ensemble parts, special values")
     gen = torch.Generator(device="cuda")
     gen.manual_seed(5)
-    batch = 32 * 256 * 2
+    batch = 65536
     x = torch.randn((batch, 128), generator=gen, device="cuda")
     w1 = torch.randn((4, 64, 128), generator=gen, device="cuda") / 11
-    w2 = torch.randn((4, 16, 64), generator=gen, device="cuda") / 8
+    w2, features = hidden_features(4)
     x[3, 5] = float("inf")
     x[40, 7] = float("-inf")
     x[100, 0] = float("nan")
@@ -585,17 +589,21 @@ def test_ensemble_in_three_parts_keeps_what_parts_cannot_hold(LY):
     x[300] = 0.0
     x[300, 9] = 3.4028234e38
     x[batch - 1] *= 2.0 ** 90
-    for scale, poison in ((1.0, None), (1.0, float("inf")), (2.0 ** -118, None)):
+    for scale, poison in ((1.0, None), (1.0, float("inf")), (2.0 ** -118, None), (2.0 ** 70, None)):
         w = w1.clone()
         w[1] *= scale
         if poison is not None:
-            w[1, 9, 3] = poison
-        four = LY.mlp_forward_ensemble(x, (w, w2), "softmax", mask_size=3)
-        two = LY.mlp_forward_ensemble(x, (w[:2].contiguous(), w2[:2].contiguous()), "softmax", mask_size=3)
-        a, b = four[:2].cpu(), two.cpu()
-        assert torch.equal(a.isnan(), b.isnan())
-        ok = ~b.isnan()
-        assert (a[ok] - b[ok]).abs().max().item() < 1e-5
+            w[1, features[1][2], 3] = poison
+        four = LY.mlp_forward_ensemble(x, (w, w2), "none")
+        two = LY.mlp_forward_ensemble(x, (w[:2].contiguous(), w2[:2].contiguous()), "none")
+        a, b = four[:2].double(), two.double()
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf())
+        for e in range(2):
+            norms = x.double().norm(dim=1, keepdim=True) * w[e, features[e]].double().norm(dim=1)
+            ok = b[e].isfinite() & norms.isfinite()
+            assert ok.sum().item() > (0.9 if poison is None else 0.3) * ok.numel()       # (a feature that is infinite makes all four NaN: 0 x inf)
+            assert ((a[e] - b[e]).abs()[ok] <= 32 * 2.0 ** -24 * norms[ok] + 128 * 2.0 ** -149).all()
+            assert (a[e][ok] != 0).any()
 
 
 def few(gen, m, k, terms):
