@@ -315,8 +315,9 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
 
     // ---- this half of the member's hidden layer, once ----
     parts_u32x4 w1[KS][3];
-    PartsWeights range;
-    {
+    bool w_bad, w_small = false;
+    for (;;) {
+        PartsWeights range;
         const float* const w = a.w1 + ((long)e * EN_HIDDEN + 32 * half + r) * K0;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
@@ -324,10 +325,13 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
             if (!load8(w, s, v)) v[0] = v[1] = zero4;
 #pragma unroll
             for (int k = 0; k < 8; ++k) range.take(v[k >> 2][k & 3]);
-            split_parts(v, PARTS_W_SCALE, w1[s]);
+            split_parts(v, w_small ? PARTS_W_SCALE_SMALL : PARTS_W_SCALE, w1[s]);
         }
+        const bool small = __any(range.small());
+        w_bad = __any(range.wide()) || (small && __any(range.large()));
+        if (!small || w_bad || w_small) break;
+        w_small = true;                                // (once more, with the other scale)
     }
-    const bool w_bad = __any(range.wide());
     // W2[e][o][32 half + 8 a4 + 4 g ..] at (o * 4 + a4) * 2 + g of the wave's 512 bytes, rows past NOUT are zeros
     f32x4* const w2 = reinterpret_cast<f32x4*>(lds + W2_AT + wave * 512);
     if (lane < 32) {
@@ -505,6 +509,10 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
         asm volatile("s_nop 15\n\ts_nop 3" : "+v"(small));
 #pragma unroll
         for (int i = 0; i < 16; ++i) done[i] = large[i] + small[i];
+        if (w_small) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) done[i] *= PARTS_UNSCALE_SMALL;
+        }
         const parts_u32x4 both = flag[0] | flag[1];
         const unsigned bad = both.x | both.y | both.z | both.w;
         if (w_bad || __any(bad != 0)) {                             // rows that parts cannot hold, and no others, take their f32 sums

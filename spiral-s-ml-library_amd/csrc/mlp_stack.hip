@@ -211,7 +211,7 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
 
     // ---- the member's weights, once per workgroup ----
     const unsigned lds0 = (unsigned)(size_t)lds;
-    bool weights_wide = false;
+    bool weights_wide = false, weights_small = false;
     auto weights_of = [&](int l) { return a.w[l] + (long)e * (l + 1 < layers ? (long)a.dims[l] * a.dims[l + 1] : a.out_stride); };
     if constexpr (!PARTS) {
         unsigned dst = lds0;
@@ -233,39 +233,44 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
     } else {
         // units (layer, tile of features, 32 of K) wave, wave + waves, ... of the whole stack, two of them in flight
         const int units = 8 * layers;
-        PartsWeights range;
-        for (int n0 = wave; n0 < units; n0 += 2 * waves) {
-            f32x4 v[2][2];
+        int* const flags = reinterpret_cast<int*>(lds + a.w_bytes);       // (the scratch, not in use yet)
+        for (;;) {
+            PartsWeights range;
+            for (int n0 = wave; n0 < units; n0 += 2 * waves) {
+                f32x4 v[2][2];
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int n = n0 + i * waves < units ? n0 + i * waves : n0, l = n >> 3, K = a.dims[l];
-                const int row = 16 * ((n >> 1) & 3) + r, col = 32 * (n & 1) + 4 * q;
-                const float* const at = weights_of(l) + (long)row * K + col;
+                for (int i = 0; i < 2; ++i) {
+                    const int n = n0 + i * waves < units ? n0 + i * waves : n0, l = n >> 3, K = a.dims[l];
+                    const int row = 16 * ((n >> 1) & 3) + r, col = 32 * (n & 1) + 4 * q;
+                    const float* const at = weights_of(l) + (long)row * K + col;
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    v[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
-                    if (row < a.dims[l + 1] && col + 16 * h < K) v[i][h] = *reinterpret_cast<const f32x4*>(at + 16 * h);
+                    for (int h = 0; h < 2; ++h) {
+                        v[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+                        if (row < a.dims[l + 1] && col + 16 * h < K) v[i][h] = *reinterpret_cast<const f32x4*>(at + 16 * h);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    if (i == 1 && n0 + waves >= units) break;
+                    parts_u32x4 p[3];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) range.take(v[i][k >> 2][k & 3]);
+                    stack_parts(v[i][0], v[i][1], weights_small ? PARTS_W_SCALE_SMALL : PARTS_W_SCALE, p);
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+                        *reinterpret_cast<parts_u32x4*>(lds + (n0 + i * waves) * ST_PARTS_UNIT + k * 1024 + lane * 16) = p[k];
                 }
             }
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                if (i == 1 && n0 + waves >= units) break;
-                parts_u32x4 p[3];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) range.take(v[i][k >> 2][k & 3]);
-                stack_parts(v[i][0], v[i][1], PARTS_W_SCALE, p);
-#pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    *reinterpret_cast<parts_u32x4*>(lds + (n0 + i * waves) * ST_PARTS_UNIT + k * 1024 + lane * 16) = p[k];
-            }
+            flags[wave] = (__any(range.small()) ? 1 : 0) | (__any(range.large()) ? 2 : 0) | (__any(range.wide()) ? 4 : 0);      // every lane the same
+            __syncthreads();
+            int any = 0;
+            for (int w = 0; w < waves; ++w) any |= flags[w];
+            any = __builtin_amdgcn_readfirstlane(any);
+            __syncthreads();
+            weights_wide = (any & 4) != 0 || (any & 3) == 3;
+            if ((any & 1) == 0 || weights_wide || weights_small) break;
+            weights_small = true;                      // (once more, with the other scale)
         }
-        int* const flags = reinterpret_cast<int*>(lds + a.w_bytes);       // (the scratch, not in use yet)
-        flags[wave] = __any(range.wide());                                // every lane the same
-        __syncthreads();
-        int any = 0;
-        for (int w = 0; w < waves; ++w) any |= flags[w];
-        weights_wide = __builtin_amdgcn_readfirstlane(any) != 0;
-        __syncthreads();
     }
 #pragma unroll
     for (int j = 0; j < HT; ++j) asm volatile("" : "+v"(x[j]));       // (the compiler's own wait for the first inputs: here, not in the loop)
@@ -306,6 +311,10 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
             stack_parts(x[0], x[1], PARTS_X_SCALE, xp[0]);
             stack_parts(x[2], x[3], PARTS_X_SCALE, xp[1]);
             parts_product(wp, xp, y);
+            if (weights_small) {
+#pragma unroll
+                for (int t = 0; t < HT; ++t) y[t] *= PARTS_UNSCALE_SMALL;
+            }
             if (lanes != 0) {
                 const bool mine = (((lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) >> r) & 1) != 0;
 #pragma unroll

@@ -25,14 +25,15 @@ typedef float parts_f32x4 __attribute__((ext_vector_type(4)));
 constexpr int PARTS_W[8] = {0, 2, 1, 2, 0, 1, 1, 0}, PARTS_X[8] = {0, 1, 2, 0, 2, 1, 0, 1};
 
 // l holds the last bit of a number as long as that is no smaller than the smallest bf16, 2^-133 (the pipe keeps subnormal numbers):
-// inputs are taken times 2^16, where every f32 is in range, and weights times 2^-16, where all from 2^-94 up are (the others
-// send a member through f32 MFMAs, and so do weights and rows of inputs above 2^60, whose sums might overflow in parts).
-constexpr float PARTS_X_SCALE = 0x1p16f, PARTS_W_SCALE = 0x1p-16f, PARTS_MOST = 0x1p60f;
+// inputs are taken times 2^16, where every f32 is in range, and weights times 2^-16, where all from 2^-94 up are.  If there are
+// smaller ones, the weights are taken times 2^16, too, and the sums times 2^-32.  Rows of inputs above 2^60, and weights above
+// that (with small ones among them, above 2^28), whose sums might overflow in parts, go through f32 MFMAs.
+constexpr float PARTS_X_SCALE = 0x1p16f, PARTS_W_SCALE = 0x1p-16f, PARTS_W_SCALE_SMALL = 0x1p16f, PARTS_UNSCALE_SMALL = 0x1p-32f, PARTS_MOST = 0x1p60f;
 // The smallest non-zero 2 |w|, in bits and less one (zeros wrap to the largest).
 constexpr unsigned PARTS_TINY = (127u - 94u) << 24;
 __device__ __forceinline__ unsigned parts_magnitude(float w) { return (__float_as_uint(w) << 1) - 1u; }
 
-struct PartsWeights {                     // whether parts hold all of the weights seen (NaN: a NaN either way)
+struct PartsWeights {                     // what the weights seen ask for (NaN: a NaN either way)
     unsigned least = 0xffffffffu;
     float most = 0.f;
     __device__ __forceinline__ void take(float w) {
@@ -40,7 +41,9 @@ struct PartsWeights {                     // whether parts hold all of the weigh
         least = m < least ? m : least;
         most = fmaxf(most, fabsf(w));
     }
-    __device__ __forceinline__ bool wide() const { return least < PARTS_TINY - 1u || most > PARTS_MOST; }
+    __device__ __forceinline__ bool small() const { return least < PARTS_TINY - 1u; }
+    __device__ __forceinline__ bool large() const { return most > 0x1p28f; }
+    __device__ __forceinline__ bool wide() const { return most > PARTS_MOST; }
 };
 
 // max(most, |x|, |y|), a NaN passed over.

@@ -649,7 +649,7 @@ def test_ensemble_in_three_parts_is_no_further_off_than_in_f32(LY, k0, inputs):
         assert ((parts.double() - want).abs() <= 2.0 ** -24 * (1 + 2.0 ** -7) * want).all()
 
 
-@pytest.mark.parametrize("x_exp,w_exp", [(-60, 0), (-105, 50), (-126, 58), (-149, 58), (58, -93), (58, -110), (-70, -66)])
+@pytest.mark.parametrize("x_exp,w_exp", [(-60, 0), (-105, 50), (-126, 58), (-149, 58), (58, -93), (58, -110), (40, -130), (-70, -66)])
 def test_ensemble_in_three_parts_of_tiny_numbers(LY, x_exp, w_exp):
     """Inputs down to the smallest subnormal and weights down to 2^-94 are held by their parts, smaller weights send their member
     through f32 MFMAs: in every row as close as f32 sums are, also where the lowest parts are subnormal bf16 or (the last case)

@@ -210,7 +210,7 @@ def test_parts_are_no_further_off_than_f32(S, widths, acts, inputs):
         assert (parts.double() - want).norm() <= 1.005 * (f32.double() - want).norm()
 
 
-@pytest.mark.parametrize("x_exp,w_exp", [(-60, 0), (-105, 0), (-140, 58), (-70, -50), (58, -93), (58, -110)])
+@pytest.mark.parametrize("x_exp,w_exp", [(-60, 0), (-105, 0), (-140, 58), (-70, -50), (58, -93), (58, -110), (40, -125)])
 def test_parts_of_tiny_numbers(S, x_exp, w_exp):
     """A layer and regret matching, which does not see a common factor: inputs down to subnormal numbers are held by their parts,
     and weights down to 2^-94 (smaller ones send their member through f32 MFMAs)."""
