@@ -527,37 +527,53 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
     const int ht = widest <= 64 ? 4 : 8;
     bool full = true;
     for (int l = 0; l < n_layers; ++l) full = full && (dims[l] + 15) / 16 == ht;
-    // Full 64 wide stacks in bf16 parts, sixteen waves in one workgroup per unit, from a tile for every wave of every unit up (one
-    // layer: two, its product is less of the work, and three quarters of the units at work).  Splitting the weights takes a few us
-    // a workgroup: with more members than units each has two tiles a wave at least (64-64-64-64, 300 members of 240 rows 31 / 34,
-    // 6000 of 16 129 / 239, but 512 of 1000 141 / 107).  Us, f32 / parts, 64-64-64-64: 30000 rows 13.4 / 17.9, 65536 21.4 / 18.4,
-    // 131072 37.1 / 29.2, 16 members of 16384 74.5 / 55.3, of 57344 223 / 157; 64-64-64: 30000 rows 10.6 / 15.2, 65536 16.5 /
-    // 15.8, 131072 27.6 / 23.8; 64-64: 65536 rows 11.9 / 12.3, 131072 19.0 / 18.4, 4 members of 50000 33.0 / 28.0.
-    constexpr int PARTS_WAVES = ST_PARTS_THREADS / 64;
-    const long cus = device_cu_count();
-    const long w_parts = (long)n_layers * 8 * ST_PARTS_UNIT;
-    const bool parts = full && ht == 4 && (a.mask_size + 15) / 16 == 4 && w_parts + PARTS_WAVES * ST_SCRATCH <= ST_LDS &&
-                       (long)a.tiles * members >= (n_layers > 1 ? 1 : 2) * PARTS_WAVES * cus &&
-                       (members > cus ? a.tiles >= 2 * PARTS_WAVES : n_layers > 1 || cus / members * members * 4 >= 3 * cus);
-    if (parts) w_bytes = w_parts;
-    a.w_bytes = (int)w_bytes;
+    // workgroups of a member, tiles of a wave (no more workgroups than give those), rounds of workgroups
+    struct Launch { long gx, each, rounds; };
+    const long cus = device_cu_count(), tiles = (long)a.tiles * members;
+    auto launch_of = [&](long gx, long waves, long at_once) {
+        const long most = (a.tiles + waves - 1) / waves;
+        if (gx > most) gx = most;
+        const long each = (a.tiles + gx * waves - 1) / (gx * waves);
+        gx = (a.tiles + each * waves - 1) / (each * waves);
+        return Launch{gx, each, (members * gx + at_once - 1) / at_once};
+    };
     // Four waves a workgroup while that is one tile per SIMD; beyond it eight, so that one wave's norms and head run beside
     // another's products, and as many workgroups per unit as the LDS holds (at most two).
-    const int waves = parts ? PARTS_WAVES : (long)a.tiles * members > 4 * cus && w_bytes + 8 * ST_SCRATCH <= ST_LDS ? 8 : 4;
-    const int lds_bytes = (int)w_bytes + waves * ST_SCRATCH;
+    int waves = tiles > 4 * cus && w_bytes + 8 * ST_SCRATCH <= ST_LDS ? 8 : 4;
+    int lds_bytes = (int)w_bytes + waves * ST_SCRATCH;
     const int resident = 2 * lds_bytes <= ST_LDS ? 2 : 1;
-    long gx = parts ? (cus < members ? 1 : cus / members) : (cus * resident + members - 1) / members;      // (parts: one round of workgroups)
-    const long most = (a.tiles + waves - 1) / waves;
-    if (gx > most) gx = most;
-    const long each = (a.tiles + gx * waves - 1) / (gx * waves);      // tiles per wave: no more workgroups than give that
-    gx = (a.tiles + each * waves - 1) / (each * waves);
+    Launch at = launch_of((cus * resident + members - 1) / members, waves, cus * resident);
+    // Full 64 wide stacks in bf16 parts, sixteen waves in one workgroup per unit, a member's, from a tile for every wave of every unit
+    // up (one layer: two, its product is less of the work).  Splitting the weights takes a few us a workgroup: with more members than
+    // units each has two tiles a wave at least.  A turn of the unit's sixteen waves takes 1.5 to 1.8 times one of eight in f32 (four
+    // layers less, their f32 weights leave room for one workgroup a unit); so either seven tenths of the turns of all rounds have a
+    // tile, or f32 has 2.2 times the turns, 2 if both have one round of workgroups (f32's last round gets by with less).  Of 800 calls
+    // of 1 to 600 members, one to four layers, with and without ln_l2, none that this takes is slower than in f32.  Us, f32 / parts,
+    // 64-64-64-64: 65536 rows 21.5 / 18.9, 131072 37.0 / 31.2, 16 members of 16384 70 / 57, of 57344 231 / 187, 512 of 1000 127 /
+    // 111; 64-64-64: 65536 rows 16.5 / 15.7, 131072 27.4 / 24.7, 200 members of 2000 96 / 74, but 300 of 762 54.7 / 62.5, 129 of 2000
+    // 71 / 73; 64-64: 131072 rows 18.7 / 17.7, 4 members of 50000 32.5 / 28.8.
+    constexpr int PARTS_WAVES = ST_PARTS_THREADS / 64;
+    const long w_parts = (long)n_layers * 8 * ST_PARTS_UNIT;
+    const Launch at_parts = launch_of(cus < members ? 1 : cus / members, PARTS_WAVES, cus);
+    const long turns = at_parts.rounds * at_parts.each, turns_f32 = at.rounds * at.each * (waves * resident / 8);
+    const bool parts = full && ht == 4 && (a.mask_size + 15) / 16 == 4 && w_parts + PARTS_WAVES * ST_SCRATCH <= ST_LDS &&
+                       tiles >= (n_layers > 1 ? 1 : 2) * PARTS_WAVES * cus && (members <= cus || a.tiles >= 2 * PARTS_WAVES) &&
+                       (n_layers == 4 || 10 * tiles >= 7 * turns * PARTS_WAVES * cus || 5 * turns_f32 >= 11 * turns ||
+                        (at.rounds == 1 && at_parts.rounds == 1 && turns_f32 >= 2 * turns));
+    if (parts) {
+        w_bytes = w_parts;
+        waves = PARTS_WAVES;
+        lds_bytes = (int)w_bytes + waves * ST_SCRATCH;
+        at = at_parts;
+    }
+    a.w_bytes = (int)w_bytes;
     const void* kernel = parts ? pick_stack_kernel<4, true, true>(regret)
                        : ht == 4 ? (full ? pick_stack_kernel<4, true>(regret) : pick_stack_kernel<4, false>(regret))
                                  : (full ? pick_stack_kernel<8, true>(regret) : pick_stack_kernel<8, false>(regret));
     rc = ensure_dynamic_lds(kernel, ST_LDS);
     if (rc != SP_OK) return rc;
     void* args[] = {(void*)&a};
-    const hipError_t err = hipLaunchKernel(kernel, dim3((unsigned)gx, (unsigned)members), dim3(64 * waves), args, lds_bytes, (hipStream_t)stream);
+    const hipError_t err = hipLaunchKernel(kernel, dim3((unsigned)at.gx, (unsigned)members), dim3(64 * waves), args, lds_bytes, (hipStream_t)stream);
     if (err != hipSuccess) return fail(SP_ERR_DEVICE, "sp_stack_forward_f32: launch failed: %s", hipGetErrorString(err));
     return check_launch(__func__);
 }

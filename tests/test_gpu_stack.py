@@ -148,7 +148,9 @@ def test_rows_of_nan_and_infinity_stay_their_own(S):
     (1, 131057, (52, 64), "", "ROW_REGRET_MATCHING", 0),                                # one layer, a part of a K-block
     (5, 30011, (64, 64, 64, 60), "tanh", "ROW_MASKED_SOFTMAX", 49),                     # workgroups that do not divide the units; masked
     (200, 330, (56, 64, 64), "ln+sigmoid", "ROW_SOFTMAX", 0),                           # a workgroup a member
-    (300, 500, (64, 64, 64), "relu", "ROW_SOFTMAX", 0)])                                # more members than units, the fewest tiles
+    (300, 500, (64, 64, 64), "relu", "ROW_SOFTMAX", 0),                                 # (f32: units idle)
+    (200, 500, (56, 64, 64), "ln+sigmoid", "ROW_SOFTMAX", 0), (450, 500, (64, 64, 64), "relu", "ROW_SOFTMAX", 0),    # more members than units, the fewest tiles
+    (300, 500, (64, 64, 64, 64, 64), "relu", "ROW_MASKED_REGRET_MATCHING", 50)])        # four layers
 def test_parts(S, members, rows, widths, acts, head, mask):
     announce("stack in parts: %d x %d rows %s %s" % (members, rows, widths, head))
     rng = np.random.default_rng(rows)
@@ -158,29 +160,43 @@ def test_parts(S, members, rows, widths, acts, head, mask):
 
 @pytest.mark.parametrize("what", ["rows", "weights"])
 def test_numbers_that_parts_cannot_hold(S, what):
-    """Infinities, numbers below 2^-110 and above 2^60, in some rows of the input or in a member's weights: such rows as the f32 kernel
-    gives them alone (few rows take that one) -- the same bits where every layer's inputs are out of range, as here in all rows
-    but 18 (whose second layer is in parts: the bound of this module) -- and the other rows as they are without them."""
+    """Infinities and numbers above 2^60 in some rows of the input or in a member's weights, and tiny numbers, under heads that make
+    them matter (regret matching does not see a row's scale): such rows as the f32 kernel gives them alone (few rows take that
+    one), the same bits where every layer's inputs are out of range, and the other rows as they are without them."""
     announce("stack in parts, %s out of range" % what)
     rng = np.random.default_rng(3)
-    x, ws = make(rng, 2, 40000, (64, 64, 64))
-    acts = ["relu"]
-    clean, _ = forward(S, x, ws, acts, S.ROW_SOFTMAX, sample=False)
+    rows = 32768
+    x, ws = make(rng, 2, rows, (64, 64, 64))
+    acts, head = ["relu"], S.ROW_REGRET_MATCHING
+    clean, _ = forward(S, x, ws, acts, head, sample=False)
     if what == "rows":
-        odd = [17, 18, 5000, 39999]
-        x[17, 3], x[18, 60], x[5000], x[39999, 0] = float("inf"), 1e-36, 1e-35, 3e30
-        policy, _ = forward(S, x, ws, acts, S.ROW_SOFTMAX, sample=False)
-        alone, _ = forward(S, x[odd].contiguous(), ws, acts, S.ROW_SOFTMAX, sample=False)
-        assert torch.equal(policy[:, odd].isnan(), alone.isnan()) and bool(alone[:, 0].isnan().all()) and not bool(alone[:, 1:].isnan().any())
-        assert torch.equal(policy[:, [5000, 39999]], alone[:, 2:])
-        assert float((policy[:, 18] - alone[:, 1]).norm() / alone[:, 1].norm()) < 1e-5
-        rest = torch.ones(40000, dtype=torch.bool, device="cuda")
+        odd = [17, 18, 40, 5000, rows - 1]
+        x[17, 3], x[18, 60], x[40, 0] = float("inf"), float("-inf"), float("nan")
+        x[5000] *= 2.0 ** -125
+        x[rows - 1] *= 2.0 ** 100
+        policy, _ = forward(S, x, ws, acts, head, sample=False)
+        alone, _ = forward(S, x[odd].contiguous(), ws, acts, head, sample=False)
+        assert torch.equal(policy[:, odd[:3]].isnan(), alone[:, :3].isnan())
+        assert torch.equal(policy[:, odd[4]], alone[:, 4])
+        assert float((policy[:, 5000] - clean[:, 5000]).norm() / clean[:, 5000].norm()) < 1e-6
+        rest = torch.ones(rows, dtype=torch.bool, device="cuda")
         rest[odd] = False
         assert torch.equal(policy[:, rest], clean[:, rest])
     else:
+        scaled = [w.clone() for w in ws]
+        scaled[0][1] *= 2.0 ** 70
+        scaled[1][1] *= 2.0 ** -115
+        policy, _ = forward(S, x, scaled, acts, head, sample=False)
+        alone, _ = forward(S, x[:300].contiguous(), scaled, acts, head, sample=False)
+        assert torch.equal(policy[1, :300], alone[1]) and torch.equal(policy[0], clean[0])
+        assert float((policy[1] - clean[1]).norm() / clean[1].norm()) < 1e-5
+        scaled[0][1], scaled[1][1] = ws[0][1] * 2.0 ** -115, ws[1][1] * 2.0 ** 20
+        policy, _ = forward(S, x, scaled, acts, head, sample=False)
+        assert torch.equal(policy[0], clean[0])
+        assert float((policy[1] - clean[1]).norm() / clean[1].norm()) < 1e-6
         ws[0][1, 5, 7], ws[1][1, 63, 0] = 1e-37, float("-inf")
-        policy, _ = forward(S, x, ws, acts, S.ROW_SOFTMAX, sample=False)
-        alone, _ = forward(S, x[:300].contiguous(), ws, acts, S.ROW_SOFTMAX, sample=False)
+        policy, _ = forward(S, x, ws, acts, head, sample=False)
+        alone, _ = forward(S, x[:300].contiguous(), ws, acts, head, sample=False)
         assert torch.equal(policy[1, :300].isnan(), alone[1].isnan()) and torch.equal(policy[1, :300].nan_to_num(), alone[1].nan_to_num())
         assert torch.equal(policy[0], clean[0])
 
