@@ -430,7 +430,10 @@ int sp_mlp_forward_packed(int dtype, const void* x, int32_t n_layers, const void
  * Replaces: `graph_run_host model {ensemble}` (ml/layers.spi:336-344, the interpreter of :194-240 run member by
  * member) for the graphs of the reference's CEM policies: game/leduc/model_cem.spi:55-63
  * (input -> matmul_ensemble_with_adjoint -> relu -> matmul_ensemble_with_adjoint -> masked_regret_matching') and
- * game/nl_hu_holdem/model_cem.spi:84-100 (input -> matmul_ensemble_with_adjoint -> masked_regret_matching'). */
+ * game/nl_hu_holdem/model_cem.spi:84-100 (input -> matmul_ensemble_with_adjoint -> masked_regret_matching').
+ * f32 throughout.  Two layers run on f32 MFMAs or, by members, batch and dims[0], with the products of the first layer as eight
+ * products of bf16 parts that add up in f32 (error against the exact sums no larger).  Within a launch a result depends on its
+ * row and its member alone; another number of members or rows may take the other kernel, and differ by roundings. */
 int sp_mlp_forward_ensemble(int dtype, const void* x, int32_t n_layers, const void* const* weights, const int32_t* dims,
                             int32_t members, const float* u, const sp_philox_t* philox, float* policy_out,
                             int32_t* action_out, int64_t batch, int32_t head, int32_t mask_size, void* stream);
@@ -443,7 +446,9 @@ int sp_mlp_forward_ensemble(int dtype, const void* x, int32_t n_layers, const vo
  * masked head only the valid columns) fit 144 KiB of LDS, else SP_ERR_UNSUPPORTED.  acts[l] (l < n_layers - 1): an sp_map_op,
  * plus SP_STACK_LN_L2 for ln_l2 in front of it.  head_op: SP_ROW_SOFTMAX, SP_ROW_MASKED_SOFTMAX, SP_ROW_REGRET_MATCHING or
  * SP_ROW_MASKED_REGRET_MATCHING, with the results of sp_row_sample on the logits.  u, philox, policy_out, action_out as for
- * sp_mlp_forward_ensemble; members x batch below 2^31.
+ * sp_mlp_forward_ensemble; members x batch below 2^31.  f32 throughout; stacks whose layers are all 64 wide (the first and the
+ * last from 49) and that have many rows multiply in bf16 parts, as described there: within a launch a result depends on its row
+ * and its member alone, another number of rows or members may differ by roundings.
  * Replaces: the node-by-node run (ml/layers.spi:194-240, 336-344) of the graphs of ml/layers.spi:564-665. */
 #define SP_STACK_LN_L2 0x100
 /* Whether a call of these sizes and this head is taken: SP_OK, or the error it would be refused with.  A host query. */

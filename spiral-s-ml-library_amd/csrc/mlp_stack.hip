@@ -161,7 +161,8 @@ __device__ __forceinline__ void parts_product(const unsigned char*& wp, const pa
     wp += 8 * ST_PARTS_UNIT;
 }
 
-// The product of rows that parts cannot hold, in f32 from the weights where they are, into the wave's scratch (a lane's own
+// The product of rows that parts cannot hold (16 members of 16384 rows with one in every tile 95 us, without 68, f32 75, host
+// included), in f32 from the weights where they are, into the wave's scratch (a lane's own
 // 16 bytes of each tile of features).
 template <int HT>
 __device__ __forceinline__ void wide_product(const float* W, int K, int F, const f32x4 (&x)[HT], unsigned char* scratch, int r, int q) {

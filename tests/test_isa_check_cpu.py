@@ -4,6 +4,7 @@ it as data."""
 import glob
 import importlib.util
 import os
+import re
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PKG = os.path.join(ROOT, "spiral-s-ml-library_amd")
@@ -101,3 +102,17 @@ def test_built_kernels_are_clean():
     mod = _module()
     for path in glob.glob(os.path.join(PKG, "build", "*-gfx950.s")):
         assert mod.scan_file(path) == [], path
+
+
+def test_built_kernels_keep_their_registers():
+    """The kernels in bf16 parts run at the edge of the register file: none of their instances may spill vector registers to memory
+    (assembly the last build kept; nothing to look at where none was built)."""
+    seen = 0
+    for name in ("mlp_stack", "mlp_ensemble"):
+        for path in glob.glob(os.path.join(PKG, "build", name + "-hip-*-gfx950.s")):
+            with open(path) as f:
+                text = f.read()
+            for kernel, scratch in re.findall(r"\.name: +(_Z\S+)\n(?:.*\n)*?.*\.private_segment_fixed_size: (\d+)", text[text.index(".amdgpu_metadata"):]):
+                seen += 1
+                assert int(scratch) == 0, (kernel, scratch)
+    assert seen == 0 or seen >= 20
