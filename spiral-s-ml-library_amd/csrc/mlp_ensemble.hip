@@ -224,8 +224,8 @@ __global__ __launch_bounds__(EN_THREADS) void mlp_ensemble_kernel(const Ensemble
 // middle: nobody waits at a round's ends.  Second layer and head are those of the kernel above, in f32.
 // A round has three sums: `large` of the products h h, which come from zero for each step of 16 inputs and are added by the vector
 // ALU (three MFMAs later), and `small` of the other seven; both in `done` at its end.
-// What bounds it: 32 x 65536 rows of 128 inputs take 260 us (f32 MFMAs 335 to 360), 65 rounds of 8 k cycles; the matrix pipe is
-// busy for 4.1 k of a round, the rest is 450 vector instructions per wave and round that the MFMAs hide in part, and what waves
+// What bounds it: 32 x 65536 rows of 128 inputs take 250 to 260 us (f32 MFMAs 335 to 360), 65 rounds of 6.8 k cycles at 1.75 GHz; the matrix pipe is
+// busy for 4.1 k of a round, beside it 410 vector instructions per wave and round, in part, and what waves
 // wait for LDS and each other.  (Six products in one sum, without the additions, took 210 us and lost bits, see parts.h.  Taken
 // back on the way there: one wave per SIMD with both halves 248 us, heads in front of a barrier at the round's end 240, zeros and
 // probabilities of a row stored apart 257, fragments two steps ahead instead of one 230, stores past the caches 228.)
