@@ -129,7 +129,8 @@ def mlp_forward_ensemble(x, weights, head="regret_matching", u=None, mask_size=0
     ml/layers.spi:468-479); head and mask_size as for mlp_forward, with at most 4 computed outputs (out, or mask_size).
     u: (E, batch) uniforms or rng: a Philox stream over the E * batch stacked rows (member_rows = batch) for an action
     per member and row; without either only the policy (E, batch, out) is computed -- the graphs of the reference's CEM
-    policies, game/leduc/model_cem.spi:55-63 and game/nl_hu_holdem/model_cem.spi:84-100."""
+    policies, game/leduc/model_cem.spi:55-63 and game/nl_hu_holdem/model_cem.spi:84-100.  Within a call a result depends on
+    its row and its member alone; another number of rows or members may take another kernel and differ by roundings."""
     n = len(weights)
     if n not in (1, 2):
         raise ValueError("one weight tensor (E, out, in), or two: (E, 64, in) and (E, out, 64)")

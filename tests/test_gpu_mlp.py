@@ -526,7 +526,7 @@ def test_ensemble_binarize(LY, members, batch, k0, n, modulo):
     assert (node[sure0] == got[0][sure0]).all()
 
 
-# The ensemble on the bf16 pipe (three members and more): tiles of 32 rows per workgroup 1, 2, ... 8, a ragged last tile, widths of
+# The ensemble on the bf16 pipe, and calls on the other side of its rule: rounds of 1, 2, ... 9 tiles of 32 rows, a ragged last tile, widths of
 # a step of 16 and odd halves of one, rows of 4, 16, 20 and 64 columns, 1 to 4 outputs, a width that is no multiple of 4
 @pytest.mark.parametrize("members,batch,dims,head,mask,sample", [
     (3, 31, [8, 64, 4], "softmax", 0, True), (4, 32 * 256 + 1, [16, 64, 16], "regret_matching", 2, False),
@@ -534,11 +534,11 @@ def test_ensemble_binarize(LY, members, batch, k0, n, modulo):
     (6, 32 * 128 * 5 + 9, [64, 64, 64], "regret_matching", 3, False), (7, 32 * 128 * 2 + 32, [72, 64, 6], "softmax", 1, True),
     (4, 32 * 256 * 6 + 33, [128, 64, 8], "none", None, False), (9, 32 * 85 * 7 + 40, [120, 64, 64], "regret_matching", 4, False),
     (9, 32 * 85 * 8, [128, 64, 64], "softmax", 3, True), (256, 200, [48, 64, 12], "regret_matching", 3, False),
-    (4, 32 * 1024 + 1, [16, 64, 16], "regret_matching", 2, False), (7, 32 * 600 - 5, [24, 64, 20], "softmax", 3, True),      # up to 64 inputs:
-    (6, 32 * 690 + 9, [64, 64, 64], "regret_matching", 3, False), (300, 32 * 17 + 1, [40, 64, 12], "softmax", 4, True),    # from five tiles a wave
-    (768, 1, [128, 64, 64], "softmax", 3, True), (800, 31, [8, 64, 4], "softmax", 0, True), (1021, 64, [24, 64, 16], "regret_matching", 2, False),   # many members:
-    (900, 96, [104, 64, 20], "softmax", 3, False), (513, 129, [64, 64, 64], "softmax_regret_matching", 4, True),      # one to nine
-    (900, 160, [16, 64, 6], "softmax", 1, True), (777, 224, [120, 64, 8], "none", None, False), (900, 265, [32, 64, 64], "softmax", 3, True)])  # rounds
+    (4, 32 * 1024 + 1, [16, 64, 16], "regret_matching", 2, False), (7, 32 * 600 - 5, [24, 64, 20], "softmax", 3, True),
+    (6, 32 * 690 + 9, [64, 64, 64], "regret_matching", 3, False), (300, 32 * 17 + 1, [40, 64, 12], "softmax", 4, True),
+    (768, 1, [128, 64, 64], "softmax", 3, True), (800, 31, [8, 64, 4], "softmax", 0, True), (1021, 64, [24, 64, 16], "regret_matching", 2, False),
+    (900, 96, [104, 64, 20], "softmax", 3, False), (513, 129, [64, 64, 64], "softmax_regret_matching", 4, True),
+    (900, 160, [16, 64, 6], "softmax", 1, True), (777, 224, [120, 64, 8], "none", None, False), (900, 265, [32, 64, 64], "softmax", 3, True)])
 def test_ensemble_in_three_parts(LY, members, batch, dims, head, mask, sample):
     """Against float64: the hidden layer no further off than f32 sums are, so the f32 bar of the head holds row by row wherever the
     head itself is not the quotient of two small numbers; exact zeros behind the mask; actions given the kernel's own policy."""

@@ -147,9 +147,10 @@ def test_rows_of_nan_and_infinity_stay_their_own(S):
     (1, 65521, (64, 64, 64), "ln+relu", "ROW_SOFTMAX", 0),                              # the fewest tiles, the last of one row
     (1, 131057, (52, 64), "", "ROW_REGRET_MATCHING", 0),                                # one layer, a part of a K-block
     (5, 30011, (64, 64, 64, 60), "tanh", "ROW_MASKED_SOFTMAX", 49),                     # workgroups that do not divide the units; masked
-    (200, 330, (56, 64, 64), "ln+sigmoid", "ROW_SOFTMAX", 0),                           # a workgroup a member
+    (200, 330, (56, 64, 64), "ln+sigmoid", "ROW_SOFTMAX", 0),                           # (f32: half of the turns without a tile)
     (300, 500, (64, 64, 64), "relu", "ROW_SOFTMAX", 0),                                 # (f32: units idle)
-    (200, 500, (56, 64, 64), "ln+sigmoid", "ROW_SOFTMAX", 0), (450, 500, (64, 64, 64), "relu", "ROW_SOFTMAX", 0),    # more members than units, the fewest tiles
+    (200, 500, (56, 64, 64), "ln+sigmoid", "ROW_SOFTMAX", 0),                           # a workgroup a member
+    (450, 500, (64, 64, 64), "relu", "ROW_SOFTMAX", 0),                                 # more members than units, the fewest tiles
     (300, 500, (64, 64, 64, 64, 64), "relu", "ROW_MASKED_REGRET_MATCHING", 50)])        # four layers
 def test_parts(S, members, rows, widths, acts, head, mask):
     announce("stack in parts: %d x %d rows %s %s" % (members, rows, widths, head))
