@@ -1,26 +1,23 @@
-// Fused dense-stack forward for gfx950.
+// Fused dense-stack forward for gfx950: stacks of 256-wide hidden layers under a narrow head, on row-major weights, and the
+// entry point of all 16-bit stacks (other hidden widths and wider heads: mlp_any.hip).
 //
-// A workgroup is 4 waves; every wave owns 16 batch rows and pushes them through ALL layers, so
-// activations never leave the wave's registers: the f32 accumulator fragment of one layer,
-// after bias / ReLU / rounding to 16 bits, is bit-for-bit the MFMA operand fragment of the next
-// layer.  (v_mfma_f32_16x16x32_{f16,bf16}: a lane ends up with 4 consecutive rows of the first
-// operand.  The weight rows are therefore fed in the order 32 u + 8 (i / 4) + i % 4 for an even
-// output tile and + 4 for the odd tile next to it, so that the two quads a lane holds in a pair
-// of tiles are the 8 consecutive columns 32 u + 8 q .. + 7: exactly the K-values lane group q
-// feeds to the next layer's MFMA.)
+// mlp_h256_kernel, more than 64 rows per compute unit: every wave owns 16 batch rows and pushes them through ALL layers, so
+// activations never leave the wave's registers: the f32 accumulator fragment of one layer, after bias / ReLU / rounding to 16
+// bits, is bit-for-bit the MFMA operand fragment of the next layer.  (v_mfma_f32_16x16x32_{f16,bf16}: a lane ends up with 4
+// consecutive rows of the first operand.  The weight rows are therefore fed in the order 32 u + 8 (i / 4) + i % 4 for an even
+// output tile and + 4 for the odd tile next to it, so that the two quads a lane holds in a pair of tiles are the 8 consecutive
+// columns 32 u + 8 q .. + 7: exactly the K-values lane group q feeds to the next layer's MFMA.)
 //
-// Weights are the shared operand.  All layers' weight matrices are cut into chunks of 64 K-columns
-// and streamed as one flat sequence through a ring of 4 LDS stages by global_load_lds DMA, three
-// chunks ahead of the MFMAs (also across layer boundaries); one barrier per chunk.  Inside a
-// stage a chunk is stored as 128-byte rows (one weight row each) whose eight 16-byte pieces are
-// XOR-swizzled with swz(row) = 2 * ((row >> 3) & 3) + ((row >> 1) & 1): a DMA instruction then fetches 8 whole 128-byte lines (8
-// adjacent lanes per line), and the ds_read_b128 operand fetches of the 16 rows of a tile are
+// Weights are the shared operand.  All layers' weight matrices are cut into chunks of 64 K-columns and streamed as one flat
+// sequence through a ring of 4 LDS stages by global_load_lds DMA, three chunks ahead of the MFMAs (also across layer
+// boundaries); one barrier per chunk.  Inside a stage a chunk is stored as 128-byte rows (one weight row each) whose eight
+// 16-byte pieces are XOR-swizzled with swz(row) = 2 * ((row >> 3) & 3) + ((row >> 1) & 1): a DMA instruction then fetches 8
+// whole 128-byte lines (8 adjacent lanes per line), and the ds_read_b128 operand fetches of the 16 rows of a tile are
 // bank-conflict free.
 //
 // The head (softmax / regret matching / sampling) runs on the last layer's f32 outputs.
 //
-// Stacks of 256-wide hidden layers with a narrow head and at most 64 rows per compute unit take another
-// route (mlp_split_kernel, described where it is defined): there a wave owns 64 OUTPUT FEATURES of all
+// mlp_split_kernel, at most 64 rows per compute unit (described where it is defined): a wave owns 64 OUTPUT FEATURES of all
 // 64 rows of the workgroup and the activations are exchanged through LDS.
 //
 // Semantics follow the graph interpreter of ml/layers.spi:194-240 (BlockMatmul = x . w^T with w
@@ -31,250 +28,15 @@
 
 namespace sp {
 
-
-// NW waves per workgroup, 16 batch rows per wave.
-template <int DT, int NW>
-__global__ __launch_bounds__(NW * 64) void mlp_forward_kernel(const MlpArgs a) {
-    constexpr int MLP_THREADS = NW * 64;
-    constexpr int MLP_ROWS = NW * 16;
-    constexpr int MLP_DMA_PER_WAVE = MLP_DMA_PER_CHUNK / NW;
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int j = lane & 15;       // batch row inside the wave's 16-row tile; weight row inside a 16-row tile
-    const int q = lane >> 4;       // which 8 of the 32 K-values of an MFMA step this lane feeds
-    const long row = (long)blockIdx.x * MLP_ROWS + wave * 16 + j;
-    const bool row_ok = row < a.batch;
-    const unsigned lds_base = (unsigned)(size_t)lds;
-    const unsigned dummy_dst = lds_base + MLP_STAGES * MLP_STAGE_BYTES;
-
-    // ---- weight chunk pipeline: chunk = (layer, 64-column slab c) ----
-    int pf_layer = 0, pf_c = 0;    // next chunk to fetch
-    int pf_stage = 0;
-    auto fetch_next_chunk = [&]() {
-        const bool live = pf_layer < a.n_layers;
-        const int layer = live ? pf_layer : 0;
-        const int K = a.dims[layer], N = a.dims[layer + 1];
-        const unsigned char* W = (const unsigned char*)a.w[layer];
-        const int n_instr = live ? (N + 7) / 8 : 0;            // 8 weight rows (128 bytes each) per instruction
-#pragma unroll
-        for (int m = 0; m < MLP_DMA_PER_WAVE; ++m) {
-            const int ii = wave + NW * m;
-            if (ii < n_instr) {
-                int n = ii * 8 + (lane >> 3);
-                const int piece = (lane & 7) ^ mlp_swz(n);        // the K piece that belongs in LDS slot lane & 7
-                n = n < N ? n : N - 1;                             // rows past N: any valid row, never used
-                int k = pf_c * 64 + piece * 8;
-                k = k <= K - 8 ? k : K - 8;                        // pieces past K: multiplied by zero activations
-                mlp_dma(W, (unsigned)((n * K + k) * 2), lds_base + pf_stage * MLP_STAGE_BYTES + ii * 1024);
-            } else {
-                mlp_dma((const unsigned char*)a.w[0], 0u, dummy_dst);  // keeps the per-chunk DMA count fixed
-            }
-        }
-        if (live) {
-            ++pf_c;
-            if (pf_c * 64 >= K) { pf_c = 0; ++pf_layer; }
-        }
-        pf_stage = (pf_stage + 1) & (MLP_STAGES - 1);
-    };
-    fetch_next_chunk();
-    fetch_next_chunk();
-    fetch_next_chunk();
-
-    // ---- the wave's input rows as MFMA operand fragments: for step s (32 K-values) lane (j, q)
-    //      holds x[row][32 s + 8 q .. + 7] ----
-    u32x4 act[MLP_MAX_DIM / 32];
-    {
-        const int K0 = a.dims[0];
-        const unsigned char* xr = (const unsigned char*)a.x + row * K0 * 2;
-#pragma unroll
-        for (int s = 0; s < MLP_MAX_DIM / 32; ++s) {
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if (row_ok && 32 * s + 8 * q < K0) v = *reinterpret_cast<const u32x4*>(xr + (32 * s + 8 * q) * 2);
-            act[s] = v;
-        }
-    }
-
-    f32x4 acc[MLP_MAX_DIM / 16];
-    int stage = 0;
-    // LDS byte offset of this lane's 16-byte weight piece for the first tile of a chunk: lane j feeds
-    // weight row n0 = 8 (j / 4) + j % 4 of the 32-row group, K piece 4 sp + q (sp = which 32-wide step
-    // of the chunk).  Tile t adds (t / 2) * 32 + (t % 2) * 4 rows, which leaves swz() unchanged.
-    const int n0 = 8 * (j >> 2) + (j & 3);
-    unsigned frag_off[2];
-#pragma unroll
-    for (int sp = 0; sp < 2; ++sp) frag_off[sp] = (unsigned)(n0 * 128 + (((4 * sp + q) ^ mlp_swz(n0)) << 4));
-    auto tile_off = [](int t) { return ((t >> 1) * 32 + (t & 1) * 4) * 128; };
-    auto tile_col = [&](int t) { return 32 * (t >> 1) + 4 * (t & 1) + 8 * q; };  // first of this lane's 4 columns
-    // per-wave f32 staging of the last layer's outputs; it reuses the first weight stage once every
-    // wave is done with the weights
-    float* head_rows = reinterpret_cast<float*>(lds) + wave * 16 * MLP_MAX_OUT;
-    static_assert(NW * 16 * MLP_MAX_OUT * 4 <= MLP_STAGE_BYTES, "head staging must fit one weight stage");
-
-    for (int layer = 0; layer < a.n_layers; ++layer) {
-        const int K = a.dims[layer], N = a.dims[layer + 1];
-        const int nt = 2 * ((N + 31) / 32);   // output tiles come in pairs covering 32 columns
-        const bool last = layer + 1 == a.n_layers;
-#pragma unroll
-        for (int t = 0; t < MLP_MAX_DIM / 16; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-#pragma unroll
-        for (int c = 0; c < MLP_MAX_DIM / 64; ++c) {
-            if (c * 64 < K) {
-                // the two newer chunks may still be in flight; everything older has landed
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * MLP_DMA_PER_WAVE) : "memory");
-                __syncthreads();
-                fetch_next_chunk();   // into the stage every wave finished reading before this barrier
-                const unsigned char* st = lds + stage * MLP_STAGE_BYTES;
-                // Output tiles are walked in groups of 4 (64 columns) with one uniform branch per
-                // group, so that the 8 or 16 LDS reads and the MFMAs of a group form one straight
-                // line the scheduler can overlap.  A partly filled last group multiplies whatever
-                // the stage holds past row N; those columns are never used.
-                const bool two_steps = c * 64 + 32 < K;
-                auto mma = [&](int t, int sp, const u32x4& w) {
-                    // weights are the first operand: the result fragment is (n, batch row)
-                    if constexpr (DT == SP_F16)
-                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            __builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, act[2 * c + sp]), acc[t], 0, 0, 0);
-                    else
-                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            __builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, act[2 * c + sp]), acc[t], 0, 0, 0);
-                };
-                auto read = [&](int t, int sp) {
-                    return *reinterpret_cast<const u32x4*>(st + frag_off[sp] + tile_off(t));
-                };
-                if (nt == MLP_MAX_DIM / 16 && two_steps) {
-                    // full-width chunk: 8 groups of (4 tiles, one 32-wide step), software pipelined by
-                    // hand: the weight pieces of group g + 2 are requested before the MFMAs of group g
-                    // (with one wave per SIMD nothing else hides the LDS latency)
-                    u32x4 w[3][4];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) w[0][t] = read(t, 0);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) w[1][t] = read(t, 1);
-#pragma unroll
-                    for (int g = 0; g < 8; ++g) {
-                        if (g + 2 < 8) {
-#pragma unroll
-                            for (int t = 0; t < 4; ++t) w[(g + 2) % 3][t] = read(((g + 2) >> 1) * 4 + t, (g + 2) & 1);
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                        for (int t = 0; t < 4; ++t) mma((g >> 1) * 4 + t, g & 1, w[g % 3][t]);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                } else {
-#pragma unroll
-                    for (int g4 = 0; g4 < MLP_MAX_DIM / 64; ++g4) {
-                        if (g4 * 4 < nt) {
-                            u32x4 w0[4], w1[4];
-#pragma unroll
-                            for (int t = 0; t < 4; ++t) w0[t] = read(g4 * 4 + t, 0);
-                            if (two_steps) {
-#pragma unroll
-                                for (int t = 0; t < 4; ++t) w1[t] = read(g4 * 4 + t, 1);
-                            }
-#pragma unroll
-                            for (int t = 0; t < 4; ++t) mma(g4 * 4 + t, 0, w0[t]);
-                            if (two_steps) {
-#pragma unroll
-                                for (int t = 0; t < 4; ++t) mma(g4 * 4 + t, 1, w1[t]);
-                            }
-                        }
-                    }
-                }
-                stage = (stage + 1) & (MLP_STAGES - 1);
-            }
-        }
-
-        // ---- layer epilogue: in tile t lane (j, q) holds columns tile_col(t) + 0..3 of batch row j;
-        //      tiles 2 s and 2 s + 1 together give it columns 32 s + 8 q .. + 7 ----
-        const float* bias = a.b[layer];
-#pragma unroll
-        for (int t = 0; t < MLP_MAX_DIM / 16; ++t) {
-            if (t < nt && bias != nullptr) {
-                const int n = tile_col(t);
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (n + r < N) acc[t][r] += bias[n + r];
-            }
-        }
-        if (!last) {
-#pragma unroll
-            for (int s = 0; s < MLP_MAX_DIM / 32; ++s) {
-                u32x4 v = {0u, 0u, 0u, 0u};
-                if (32 * s < N) {
-                    const f32x4 lo = acc[2 * s], hi = acc[2 * s + 1];
-                    v.x = relu_pack2<DT>(lo[0], lo[1]);
-                    v.y = relu_pack2<DT>(lo[2], lo[3]);
-                    v.z = relu_pack2<DT>(hi[0], hi[1]);
-                    v.w = relu_pack2<DT>(hi[2], hi[3]);
-                }
-                act[s] = v;
-            }
-        } else {
-            __syncthreads();   // all waves have read their last weight chunk: the stage can be reused
-#pragma unroll
-            for (int t = 0; t < MLP_MAX_OUT / 16; ++t) {
-                if (t < nt) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) head_rows[j * MLP_MAX_OUT + tile_col(t) + r] = acc[t][r];
-                }
-            }
-        }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // drain the dummy DMAs before the LDS is released
-
-    // ---- head: lanes 0..15 of every wave own one batch row each (the staging is wave private) ----
-    const int N = a.dims[a.n_layers];
-    const int limit = a.mask_size > 0 ? a.mask_size : N;
-    float past = 0.f;
-    if (lane < 16 && row_ok) {
-        float* p = head_rows + lane * MLP_MAX_OUT;   // this row's outputs
-        const float u = a.ph.philox_mode >= 0 ? reference_row_uniform(a.ph, row) : a.action != nullptr ? a.u[row] : 1.f;
-        // narrow heads run in registers, at the smallest width that holds them: the head is a chain of this lane's own (batch
-        // 64, us, always 64 columns / these widths: 64-64-64-10 14.9 / 10.0, 64-96-96-16 16.7 / 11.8, 128-64-24 14.1 / 10.2)
-        if (N <= 8) head_row<8>(head_out(a), p, row, N, limit, u, N, &past);
-        else if (N <= 16) head_row<16>(head_out(a), p, row, N, limit, u);
-        else if (N <= 32) head_row<32>(head_out(a), p, row, N, limit, u);
-        else head_row<MLP_MAX_OUT>(head_out(a), p, row, N, limit, u);
-    }
-    if (a.out_stride > N) {
-        // a masked head computed for its valid columns only (N < 8): the wave fills the rest of its 16 policy rows, 16 bytes
-        // per lane where rows are whole pieces, the columns in front of the first whole piece by the row's own lane
-        const int stride = a.out_stride, s4 = stride >> 2, c0 = stride % 4 == 0 ? (N + 3) >> 2 : s4 + 1;
-        if (lane < 16 && row_ok)
-            for (int c = N; c < stride && c < 4 * c0; ++c) a.policy[row * stride + c] = past;
-        if (c0 < s4) {
-            const long first = (long)blockIdx.x * MLP_ROWS + wave * 16;
-            int r = lane / s4, c = lane - r * s4;
-            const int dr = 64 / s4, dc = 64 - dr * s4;
-            for (int idx = lane; idx < 16 * s4; idx += 64) {      // (16 s4 is a multiple of 16: the lanes of the rows stay in)
-                const float v = __shfl(past, r);
-                if (c >= c0 && first + r < a.batch) *reinterpret_cast<float4*>(a.policy + (first + r) * stride + 4 * c) = make_float4(v, v, v, v);
-                r += dr;
-                c += dc;
-                if (c >= s4) {
-                    c -= s4;
-                    ++r;
-                }
-            }
-        }
-    }
-}
-
-
 // ---- stacks whose hidden layers are all 256 wide ------------------------------------------------
-// Same data flow as mlp_forward_kernel (16 batch rows per wave, activations in registers, weights
-// streamed through the LDS ring three chunks ahead), with the hidden width a compile-time 256 and
+// 16 batch rows per wave, activations in registers, weights streamed through the LDS ring three chunks ahead, the hidden width a compile-time 256 and
 // NO data-dependent control flow around the register arrays: every 256-row chunk has the same
 // shape, all per-lane DMA offsets are computed once, a chunk costs a wave no vector instructions
 // besides its 32 MFMAs and 32 LDS reads, and the DMA instructions are issued one by one between
 // the MFMA groups.  The first layer always runs C0 whole chunks (1 for K0 <= 64, else 4; K-pieces
-// past K0 re-read the last valid piece and meet zero activations), the last layer (at most 64
+// past K0 re-read the last valid piece and meet zero activations), the last layer (at most 16
 // outputs) travels as ONE chunk holding its four 64-column slabs at 64-row spacing and always
-// computes 4 tiles (rows past the outputs are stale but finite-or-not they only reach unused columns).
+// computes 2 tiles (rows past the outputs are stale but finite-or-not they only reach unused columns).
 template <int DT, int NW, int C0>
 __global__ __launch_bounds__(NW * 64) void mlp_h256_kernel(const MlpArgs a) {
     constexpr int H = 256;
@@ -460,7 +222,7 @@ __global__ __launch_bounds__(NW * 64) void mlp_h256_kernel(const MlpArgs a) {
     };
     // KIND 0..3: chunk KIND of a layer, i.e. K-columns 64 KIND .. + 63 for all 16 output tiles (chunk 0
     // starts the accumulators from zero); KIND 4: the last layer, whose chunk holds the K-columns
-    // 64 s .. + 63 of all its (at most 64) outputs in slab s = g / 2 and accumulates into tiles 0..3.
+    // 64 s .. + 63 of all its (at most 16) outputs in slab s = g / 2 and accumulates into tiles 0 and 1.
     // FIRST: the chunk behind first_sync (no earlier fetch is waiting for its last DMA instructions).
     auto run_chunk = [&](auto KIND_, auto FIRST_) {
         constexpr int kind = decltype(KIND_)::value;
@@ -485,7 +247,7 @@ __global__ __launch_bounds__(NW * 64) void mlp_h256_kernel(const MlpArgs a) {
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
+            for (int t = 0; t < (last ? 2 : 4); ++t) {
                 if constexpr (last) {
                     acc[t] = mfma(g == 0 ? zero4 : acc[t], w[g % RING][t], act[g]);
                 } else {
@@ -558,7 +320,7 @@ __global__ __launch_bounds__(NW * 64) void mlp_h256_kernel(const MlpArgs a) {
         next_activations((const float*)table_ptr(tab_b, layer));
     }
 
-    // ---- last layer: 256 -> NOUT <= 64, one chunk, 4 tiles ----
+    // ---- last layer: 256 -> NOUT <= 16, one chunk, 2 tiles ----
     run_chunk(IC<4>{}, IC<0>{});
     // the dummy DMAs (they land in their own KiB) must be done before the LDS is released; they are
     // long done, and waiting here rather than at the end keeps the outputs' stores out of the wait
@@ -583,7 +345,7 @@ __global__ __launch_bounds__(NW * 64) void mlp_h256_kernel(const MlpArgs a) {
         __syncthreads();                                    // every wave has read its last weights: reuse stage 0
         float* head_rows = reinterpret_cast<float*>(lds) + wave * 16 * MLP_MAX_OUT;
 #pragma unroll
-        for (int t = 0; t < MLP_MAX_OUT / 16; ++t) {
+        for (int t = 0; t < 2; ++t) {
             f32x4 v = acc[t];
             if (bias != nullptr) {
 #pragma unroll
@@ -593,7 +355,7 @@ __global__ __launch_bounds__(NW * 64) void mlp_h256_kernel(const MlpArgs a) {
             *reinterpret_cast<f32x4*>(head_rows + j * MLP_MAX_OUT + tile_col(t)) = v;
         }
         // lanes 0..15 of every wave own one batch row each (the staging is wave private)
-        if (lane < 16 && row_ok) head_row<MLP_MAX_OUT>(out, head_rows + lane * MLP_MAX_OUT, row, NOUT, limit, u_row);
+        if (lane < 16 && row_ok) head_row<16>(out, head_rows + lane * MLP_MAX_OUT, row, NOUT, limit, u_row);
     }
 }
 
@@ -975,15 +737,6 @@ __global__ __launch_bounds__(256) void mlp_split_kernel(const void* x_first, con
     }
 }
 
-namespace {
-struct MlpKernelNames {
-    MlpKernelNames() {
-        register_kernel("mlp_forward", (const void*)mlp_forward_kernel<SP_F16, 4>, 256);
-        register_kernel("mlp_forward_wide", (const void*)mlp_forward_kernel<SP_F16, 8>, 512);
-    }
-} mlp_kernel_names;
-}  // namespace
-
 }  // namespace sp
 
 using namespace sp;
@@ -1046,28 +799,25 @@ extern "C" int sp_mlp_forward(int dtype, const void* x, int32_t n_layers, const 
     a.x = x; a.n_layers = n_layers; a.u = u; a.policy = policy_out; a.action = action_out; a.logits = logits_out;
     a.batch = batch; a.head = head; a.mask_size = mask_size; a.k0 = dims[0]; a.nout = dims[n_layers];
     a.out_stride = dims[n_layers];
-    // 4 waves (64 rows) per workgroup while such workgroups fit the compute units in one round: every
-    // wave reads all weights from LDS, so 8 waves on a unit are LDS-bandwidth bound (2048 cycles per
-    // 32 KiB chunk) where 4 are not; beyond one round, 8 waves (128 rows) halve the rounds
+    // more than 64 rows per compute unit: 8 waves (128 rows) per workgroup halve the rounds
     const int cus = device_cu_count();
     const bool wide = (batch + 63) / 64 > cus;
-    const int nw = wide ? 8 : 4;
-    bool h256 = n_layers >= 2;   // all hidden layers 256 wide: the lean kernel
+    bool h256 = n_layers >= 3;   // two and more hidden layers, all 256 wide
     for (int i = 1; i < n_layers; ++i) h256 = h256 && dims[i] == 256;
     // A masked head gives probability zero to the columns past the mask whatever their logits are: when the logits
     // themselves are not asked for, the last layer is computed for the valid columns only (the first rows of its
     // weight matrix) and the head fills the rest of each policy row with zeros.  A 64-wide layer with 3 valid
-    // columns, the shape the reference's 16-byte row primitives force on a 3-action game, then runs on the
-    // narrow-head kernels.
-    if (h256 && head != SP_HEAD_NONE && logits_out == nullptr && mask_size > 0 && mask_size <= 16 &&
-        mask_size < dims[n_layers])
-        a.nout = mask_size;
-    // The same in the kernel of the other hidden widths, whose head walks its outputs column by column in one lane (bf16
-    // 128-64-64 masked to 3, regret matching and a sample, 64 rows: 14.4 us with all 64 columns, 9.3 so).  Seven at most, so that the
-    // head has a column past the mask of its own: what the rest of the row is filled with.
-    if (!h256 && head != SP_HEAD_NONE && logits_out == nullptr && mask_size > 0 && mask_size <= 7 && mask_size < dims[n_layers])
-        a.dims[n_layers] = mask_size;
-    if (h256 && mlp_resident_takes(n_layers, dims, a.nout) &&
+    // columns, the shape the reference's 16-byte row primitives force on a 3-action game, then is a narrow head.
+    if (head != SP_HEAD_NONE && logits_out == nullptr && mask_size > 0) a.nout = mask_size;
+    // Other hidden widths, heads of more than 16 outputs, a single hidden layer: mlp_any.hip.  Of stacks with 256-wide layers those two
+    // kinds, too (bf16, us, the kernels here / there: 64-256-64 64 rows 11.4 / 7.4, 40000 32.2 / 16.1, 400000 194 / 92; 64-256-10 10.9 /
+    // 6.5, 23.3 / 12.0, 137 / 65; 128-256-256-256-24 17.0 / 12.0, 44 / 33, 271 / 225), while up to 16 outputs behind two of them stay
+    // (32-256-256-256-3 64 rows 8.0 / 10.7, 40000 20.2 / 24.2; 256-256-256-256-256-6 12.8 / 15.7, 35 / 48).
+    if (!h256 || a.nout > 16) {
+        a.dims[n_layers] = a.nout;
+        return mlp_any_launch(dtype, a, (hipStream_t)stream, __func__);
+    }
+    if (mlp_resident_takes(n_layers, dims, a.nout) &&
         (batch + 63) / 64 >= (long)(mlp_pipe_takes(n_layers, dims, a.nout) ? SP_MLP_PIPE_MIN_TILES_ROWMAJOR
                                                                            : SP_MLP_RESIDENT_MIN_TILES_ROWMAJOR) * cus) {
         // many tiles per compute unit: the kernel that loads the weights once and keeps them in registers
@@ -1081,30 +831,21 @@ extern "C" int sp_mlp_forward(int dtype, const void* x, int32_t n_layers, const 
         }
         return mlp_resident_launch(dtype, false, n_layers, r, (hipStream_t)stream, __func__);
     }
+    // at most one 64-row workgroup per compute unit: hidden layers split by output features
+    const bool split = !wide;
     const void* kernel;
     int lds_bytes = MLP_STAGES * MLP_STAGE_BYTES + 1024;   // weight ring + the dummy DMA target
-    int rows_per_block = nw * 16;
-    int threads = nw * 64;
-    // at most one 64-row workgroup per compute unit and a narrow head: hidden layers split by output features
-    const bool split = h256 && n_layers >= 3 && !wide && a.nout <= 16;
+    int rows_per_block = 128, threads = 512;
     if (split) {
         const int ks0 = dims[0] <= 32 ? 1 : dims[0] <= 64 ? 2 : 8;
         kernel = pick_split_kernel(dtype, ks0);
         lds_bytes = SPLIT_LDS_BYTES;
         rows_per_block = SPLIT_ROWS;
         threads = 256;
-    } else if (h256) {
-        const bool small_k = dims[0] <= 64;
-        if (dtype == SP_F16)
-            kernel = wide ? (small_k ? (const void*)mlp_h256_kernel<SP_F16, 8, 1> : (const void*)mlp_h256_kernel<SP_F16, 8, 4>)
-                          : (small_k ? (const void*)mlp_h256_kernel<SP_F16, 4, 1> : (const void*)mlp_h256_kernel<SP_F16, 4, 4>);
-        else
-            kernel = wide ? (small_k ? (const void*)mlp_h256_kernel<SP_BF16, 8, 1> : (const void*)mlp_h256_kernel<SP_BF16, 8, 4>)
-                          : (small_k ? (const void*)mlp_h256_kernel<SP_BF16, 4, 1> : (const void*)mlp_h256_kernel<SP_BF16, 4, 4>);
-    } else if (dtype == SP_F16) {
-        kernel = wide ? (const void*)mlp_forward_kernel<SP_F16, 8> : (const void*)mlp_forward_kernel<SP_F16, 4>;
     } else {
-        kernel = wide ? (const void*)mlp_forward_kernel<SP_BF16, 8> : (const void*)mlp_forward_kernel<SP_BF16, 4>;
+        const bool small_k = dims[0] <= 64;
+        if (dtype == SP_F16) kernel = small_k ? (const void*)mlp_h256_kernel<SP_F16, 8, 1> : (const void*)mlp_h256_kernel<SP_F16, 8, 4>;
+        else kernel = small_k ? (const void*)mlp_h256_kernel<SP_BF16, 8, 1> : (const void*)mlp_h256_kernel<SP_BF16, 8, 4>;
     }
     rc = ensure_dynamic_lds(kernel, lds_bytes);
     if (rc != SP_OK) return rc;

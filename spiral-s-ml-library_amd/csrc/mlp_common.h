@@ -19,7 +19,6 @@ constexpr int MLP_MAX_DIM = 256;       // widest layer input / hidden width
 constexpr int MLP_MAX_OUT = 64;        // widest head
 constexpr int MLP_STAGES = 4;
 constexpr int MLP_STAGE_BYTES = MLP_MAX_DIM * 128;   // 256 weight rows x 64 K-columns x 2 bytes
-constexpr int MLP_DMA_PER_CHUNK = MLP_MAX_DIM / 8;         // 1 KiB DMA instructions per full chunk
 constexpr int INT_MAX_ = 2147483647;
 
 struct MlpArgs {
@@ -87,6 +86,9 @@ int mlp_pipe_launch(int dtype, bool packed, MlpResidentArgs a, hipStream_t strea
 #define SP_MLP_PIPE_MIN_TILES_ROWMAJOR 5
 #endif
 
+// Stacks of any hidden width and head (mlp_any.hip): `a` complete but for k0 and nout, dims[n_layers] the computed outputs.
+int mlp_any_launch(int dtype, const MlpArgs& a, hipStream_t stream, const char* what);
+
 // The Philox stream of a head that draws its own uniforms: the sampling node of the layer graph works on rows of
 // `cols` = the last layer's full width, which the reference's row primitives need to be a multiple of 4.
 inline int mlp_set_philox(PhiloxStream& ph, const sp_philox_t* philox, int64_t batch, int cols, const char* fn) {
@@ -141,10 +143,9 @@ __device__ __forceinline__ HeadOut head_out(const MlpArgs& a) {
     return HeadOut{a.policy, a.action, a.logits, a.head, a.out_stride};
 }
 
-// `past` (N < MAXN only): receives what a column past the mask gets -- 0, or NaN where the row's sum is NaN.
 template <int MAXN>
 __device__ __forceinline__ void head_row(const HeadOut& o, const float* src, long row, int N, int limit, float u,
-                                         int fill_end = 1 << 30, float* past = nullptr) {
+                                         int fill_end = 1 << 30) {
     float p[MAXN];
 #pragma unroll
     for (int n = 0; n < MAXN; ++n) p[n] = n < N ? src[n] : 0.f;
@@ -184,7 +185,6 @@ __device__ __forceinline__ void head_row(const HeadOut& o, const float* src, lon
 #pragma unroll
         for (int n = 0; n < MAXN; ++n) p[n] = s != 0.f ? p[n] * inv : (n < limit ? inv_len : 0.f);
     }
-    if (past != nullptr) *past = p[MAXN - 1];
 #pragma unroll
     for (int n = 0; n < MAXN; ++n)
         if (n < N) o.policy[row * o.stride + n] = p[n];

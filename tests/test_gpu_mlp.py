@@ -170,6 +170,31 @@ def test_head_widths_of_other_stacks(LY, dims, head, mask):
     check(LY, x, ws, u, "f16", head, mask)
 
 
+@pytest.mark.parametrize("dims,mask,batch,with_bias", [
+    ([16, 3], 0, 1, True), ([16, 32, 4], 0, 17, False),                   # one layer; waves without a tile of their own
+    ([144, 96, 5], 0, 16, True), ([256, 128, 96, 64], 60, 33, False),     # K that ends in mid-step; inputs on both planes; a wide mask
+    ([48, 32, 32, 32, 32, 32, 32, 32, 33], 0, 50, True),                  # eight layers
+    ([80, 192, 192, 24], 0, 100, True), ([256, 224, 256, 256, 64], 0, 65, False),      # sixteen waves; more units than slots
+    ([64, 160, 64, 16], 0, "16+1", True), ([64, 128, 7], 0, "32+1", False), ([64, 64, 192, 2], 0, "64", True),    # 32 and 64 rows a workgroup
+    ([256, 64, 128, 9], 0, "64+1", True), ([48, 96, 3], 0, "64+33", True), ([16, 3], 0, "65", False),     # rows shared out
+    ([128, 160, 64], 5, "64+1", False), ([64, 256, 40], 0, "64+1", True), ([64, 32, 12], 2, "66", False),
+    ([64, 192, 192, 192, 3], 0, "128+1", True), ([128, 128, 128, 128, 128, 128, 20], 0, "128+40", False),     # and weights that do not fit
+    ([256, 224, 256, 256, 64], 0, "129", False)])
+def test_stacks_of_any_width_at_the_edges_of_their_kernels(LY, dims, mask, batch, with_bias):
+    """Widths and batches around every rule of the kernels for any hidden width; batches as "rows per compute unit + rows"."""
+    announce("mlp any width %s mask=%d batch=%s bias=%s" % (dims, mask, batch, with_bias))
+    if isinstance(batch, str):
+        per_cu, _, more = batch.partition("+")
+        batch = int(per_cu) * torch.cuda.get_device_properties(0).multi_processor_count + int(more or 0)
+    rng = np.random.default_rng(sum(dims))
+    dtype = "bf16" if len(dims) % 2 else "f16"
+    x, ws, u = make_problem(rng, batch, dims, dtype)
+    biases = [rng.standard_normal(o).astype(np.float32) * 0.1 for o in dims[1:]] if with_bias else None
+    if biases is not None and len(biases) > 1:
+        biases[0] = None
+    check(LY, x, ws, u, dtype, "softmax", mask, biases)
+
+
 @pytest.mark.parametrize("dims,head,mask,batch,dtype", [([128, 64, 64], "regret_matching", 3, 64, "bf16"),
                                                         ([48, 96, 128, 10], "softmax", 4, 37, "f16"),      # rows of no whole pieces
                                                         ([16, 32, 12], "softmax_regret_matching", 7, 130, "bf16"),
