@@ -20,6 +20,7 @@
 // tile per SIMD.
 // Measured, that stack over 16384 rows (node by node / every layer through part_product, a draw per tile / this kernel, us):
 // one model 32.8 / 13.8 / 10.3, 16 members 206 / 87 / 68.8 (the matrix pipe alone: 41).
+//   Few rows: stack_features_kernel, below.
 //   PARTS: the same with the products in three bf16 parts (parts.h), 192 MFMAs of 16 cycles for 16 rows instead of 192 of 32, and
 // 400 vector instructions more, in part beside them: 16 members of 16384 rows 68 -> 56 us, of 57344 228 -> 190.  Bound by the
 // vector ALU and the 7 us in which a workgroup's sixteen waves start together, with the same phases; a raised priority for waves
@@ -56,6 +57,7 @@ struct StackArgs {
     const float* w[ST_MAX_LAYERS];     // (members, dims[l + 1], dims[l])
     int dims[ST_MAX_LAYERS + 1];       // the last one: the computed outputs (a mask leaves only its own)
     int acts[ST_MAX_LAYERS];           // sp_map_op, plus SP_STACK_LN_L2
+    unsigned per_kt[ST_MAX_LAYERS];    // of kt = 16 wide blocks of a layer's inputs: b / kt is b * per_kt >> 16 for b <= 64
     int n_layers, n, mask_size;        // n: output width; mask_size: the valid columns of the head
     int w_bytes;                       // weights in LDS
     int batch, tiles;
@@ -100,24 +102,50 @@ __device__ __forceinline__ void full_product(const unsigned char*& wp, const f32
     wp += KT * NT * ST_BLOCK;
 }
 
-// The same for kt <= KT blocks of K and nt <= NT tiles of features, feature tiles outermost, the weights one block ahead
-// (behind the last block of the stack lies the scratch: read, not used).
+// The same for kt <= KT blocks of K and nt <= NT tiles of features: groups of four tiles as above (their sums are four chains, which the
+// matrix pipe takes in turn), the tiles behind the last whole group one after the other, the weights one block ahead (behind the last
+// block of the stack lies the scratch: read, not used).
 template <int KT, int NT>
 __device__ __forceinline__ void part_product(const unsigned char*& wp, const f32x4 (&x)[KT], f32x4 (&y)[NT], int kt, int nt) {
-    f32x4 w = *reinterpret_cast<const f32x4*>(wp);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        y[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (t < nt) {
+    for (int g = 0; g < NT; g += 4) {
+        if (g + 4 <= nt) {
+            f32x4 w[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                y[g + t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                w[t] = *reinterpret_cast<const f32x4*>(wp + t * ST_BLOCK);
+            }
 #pragma unroll
             for (int j = 0; j < KT; ++j)
                 if (j < kt) {
-                    wp += ST_BLOCK;
-                    const f32x4 next = *reinterpret_cast<const f32x4*>(wp);
+                    wp += 4 * ST_BLOCK;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) y[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[j][i], y[t], 0, 0, 0);
-                    w = next;
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) {
+                            y[g + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][i], x[j][i], y[g + t], 0, 0, 0);
+                            if (i == 3) w[t] = *reinterpret_cast<const f32x4*>(wp + t * ST_BLOCK);      // (the next block's, in time for its first use)
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
+        } else {
+            f32x4 w = *reinterpret_cast<const f32x4*>(wp);
+#pragma unroll
+            for (int t = g; t < g + 4; ++t) {
+                y[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (t < nt) {
+#pragma unroll
+                    for (int j = 0; j < KT; ++j)
+                        if (j < kt) {
+                            wp += ST_BLOCK;
+                            const f32x4 next = *reinterpret_cast<const f32x4*>(wp);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) y[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[j][i], y[t], 0, 0, 0);
+                            w = next;
+                        }
+                }
+            }
         }
     }
 }
@@ -181,6 +209,54 @@ __device__ __forceinline__ void wide_product(const float* W, int K, int F, const
     }
 }
 
+// The head of a row in 16 lanes, lane lq with columns 4 lq .. in v (used up): softmax or regret matching of its first `limit` columns.
+template <bool REGRET>
+__device__ __forceinline__ void stack_head(f32x4& v, int lq, int limit, float (&p)[4]) {
+    // columns past the head's width, or its mask, enter as -inf (an exact 0 after the exponential) or 0
+    if (limit < ST_MAX_OUT) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (4 * lq + k >= limit) v[k] = -__builtin_inff();
+    }
+    if constexpr (REGRET) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) p[k] = 4 * lq + k < limit ? fmaxf(v[k], 0.f) : 0.f;
+        const float s = group_reduce<16>(sum4(p), [](float m, float n) { return m + n; });
+        const float inv_len = 1.f / (float)limit;
+        const RowDivisor over_s(s);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) p[k] = 4 * lq + k < limit ? (s != 0.f ? over_s(p[k]) : inv_len) : 0.f;
+    } else {
+        const float m = group_max<16>(vmax(vmax(v[0], v[1]), vmax(v[2], v[3])));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) p[k] = fast_exp(v[k] - m);
+        const float s = group_reduce<16>(sum4(p), [](float m, float n) { return m + n; });
+        const float inv = 1.f / s;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) p[k] = p[k] * inv;
+    }
+}
+
+// local_discrete_sampling (ml/primitives.spi:782-798) of such a row.
+__device__ __forceinline__ int stack_pick(const float (&p)[4], int lq, float u) {
+    const float incl = group_inclusive_scan<16>(sum4(p), lq);
+    float run = dpp_move<0x138>(incl);
+    if (lq == 0) run = 0.f;
+    float c[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        run = run + p[k];
+        c[k] = run;
+    }
+    const float m = group_max<16>(sum4(p) > 0.f ? c[3] : -__builtin_inff());
+    const float thr = u * m;
+    int pick = 2147483647;
+#pragma unroll
+    for (int k = 3; k >= 0; --k)
+        if (p[k] > 0.f && c[k] >= thr) pick = 4 * lq + k;
+    return group_reduce<16>(pick, [](int m, int n) { return m < n ? m : n; });
+}
+
 // HT: 16-wide tiles of the widest layer (4 or 8).  PARTS: products in bf16 parts (FULL, and as many outputs).  FULL: the input and every hidden layer have exactly that many.  REGRET:
 // regret matching instead of softmax as the head (of mask_size columns, either).
 template <int HT, bool REGRET, bool FULL, bool PARTS = false>
@@ -198,18 +274,41 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
     auto load_x = [&](int tile, f32x4 (&x)[HT]) {
         int row = tile * ST_ROWS + r;
         row = row < a.batch ? row : a.batch - 1;
-        const float* xr = a.x + (long)row * k0;
+        const float* xr = a.x + (long)row * k0 + 4 * q;
+        // (a load that only some lanes take part in is waited for where the others go on: at most the last one is of that kind.
+        // 108-64-32, 48 rows: 5 k cycles for the inputs with every load of that kind.)
+        if (!PARTS && k0 < 16) {
+#pragma unroll
+            for (int j = 0; j < HT; ++j) x[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (4 * q < k0) x[0] = *reinterpret_cast<const f32x4*>(xr);
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < HT; ++j) {
-            x[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            const int col = 16 * j + 4 * q;
-            if (j < kt0 && col < k0) x[j] = *reinterpret_cast<const f32x4*>(xr + col);
+            if (!PARTS && 16 * j + 16 <= k0) {
+                x[j] = *reinterpret_cast<const f32x4*>(xr + 16 * j);
+            } else {
+                x[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (j < kt0 && 16 * j + 4 * q < k0) x[j] = *reinterpret_cast<const f32x4*>(xr + 16 * j);
+            }
         }
     };
     int tile = blockIdx.x * waves + wave;
     f32x4 x[HT];
     load_x(tile < a.tiles ? tile : 0, x);
 
+    const int stride = gridDim.x * waves;
+    // The uniforms of four tiles at once, lane group q those of tile q from here: a draw is 250 vector instructions.
+    auto draw = [&](int tile) {
+        int rr = r, qq = q;
+        if constexpr (PARTS) asm volatile("" : "+v"(rr), "+v"(qq));      // (see wide_product)
+        const long at = (long)(tile + (long)qq * stride) * ST_ROWS + rr;
+        const int row = at < a.batch ? (int)at : a.batch - 1;
+        if (a.ph.philox_mode < 0) return a.u[(long)e * a.batch + row];
+        if (a.ph.member_rows > 0) return run_row_uniform<unsigned>(a.ph, row, a.ph.draw_offset + (unsigned long long)e * a.ph.member_draws);
+        return run_row_uniform<unsigned>(a.ph, (unsigned)e * a.batch + row, a.ph.draw_offset);
+    };
+    float u4 = 1.f;
     // ---- the member's weights, once per workgroup ----
     const unsigned lds0 = (unsigned)(size_t)lds;
     bool weights_wide = false, weights_small = false;
@@ -219,18 +318,34 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
         for (int l = 0; l < layers; ++l) {
             const int K = a.dims[l], F = a.dims[l + 1], kt = (K + 15) >> 4, nt = (F + 15) >> 4;
             const float* W = weights_of(l);
-            const bool k_outer = FULL && (l + 1 < layers || nt == ST_MAX_OUT / 16);      // as full_product reads them
-            const int inner = k_outer ? nt : kt;
+            // in the order the products read them: full_product's tiles in one group, part_product's in fours and then one by one
+            const bool full = FULL && (l + 1 < layers || nt == ST_MAX_OUT / 16);
+            const unsigned mine = (unsigned)(r * K + 4 * q) * 4;
+            const int whole = full ? nt : nt & ~3, log_group = full && nt == 8 ? 3 : 2;       // tiles in groups (of 8 or 4)
+            const unsigned per_kt = a.per_kt[l];
             for (int b = wave; b < kt * nt; b += waves) {
-                const int hi = b / inner, lo = b - hi * inner;
-                const int row = 16 * (k_outer ? lo : hi) + r, col = 16 * (k_outer ? hi : lo) + 4 * q;
-                const unsigned char* at = (const unsigned char*)(W + (long)row * K + col);
-                dma_to_lds_addr(row < F && col < K ? at : (const unsigned char*)kZeroChunk, __builtin_amdgcn_readfirstlane(dst + b * ST_BLOCK));
+                int tile, block;
+                if (b < kt * whole) {
+                    const int turn = b >> log_group, group = (int)((unsigned)turn * per_kt >> 16);
+                    tile = (group << log_group) + (b & ((1 << log_group) - 1));
+                    block = turn - group * kt;
+                } else {
+                    const int over = b - kt * whole, t = (int)((unsigned)over * per_kt >> 16);
+                    tile = whole + t;
+                    block = over - t * kt;
+                }
+                const int row = 16 * tile, col = 16 * block;
+                const unsigned to = __builtin_amdgcn_readfirstlane(dst + b * ST_BLOCK);
+                const unsigned char* const at = (const unsigned char*)(W + row * K + col);
+                if (row + 16 <= F && col + 16 <= K) mlp_dma(at, mine, to);
+                else dma_to_lds_addr(row + r < F && col + 4 * q < K ? at + mine : (const unsigned char*)kZeroChunk, to);
             }
             dst += kt * nt * ST_BLOCK;
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
+        if (tile >= a.tiles) {                           // (a wave with rows: in front of its first products)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+        }
     } else {
         // units (layer, tile of features, 32 of K) wave, wave + waves, ... of the whole stack, two of them in flight
         const int units = 8 * layers;
@@ -276,23 +391,17 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
 #pragma unroll
     for (int j = 0; j < HT; ++j) asm volatile("" : "+v"(x[j]));       // (the compiler's own wait for the first inputs: here, not in the loop)
     unsigned char* const scratch = lds + a.w_bytes + wave * ST_SCRATCH;
-    const int stride = gridDim.x * waves;
 
     float* const policy = a.policy + (long)e * a.batch * a.n;
     int* const action = a.action + (long)e * a.batch;       // (only used where a.action is not null)
-    float u4 = 1.f;
     for (int turn = 0; tile < a.tiles; tile += stride, ++turn) {
-        // The uniforms of four tiles at once, lane group q those of tile q from here: a draw is 250 vector instructions.
-        if (a.action != nullptr && (turn & 3) == 0) {
-            int rr = r, qq = q;
-            if constexpr (PARTS) asm volatile("" : "+v"(rr), "+v"(qq));      // (see wide_product)
-            const long at = (long)(tile + (long)qq * stride) * ST_ROWS + rr;
-            const int row = at < a.batch ? (int)at : a.batch - 1;
-            if (a.ph.philox_mode < 0) u4 = a.u[(long)e * a.batch + row];
-            else if (a.ph.member_rows > 0) u4 = run_row_uniform<unsigned>(a.ph, row, a.ph.draw_offset + (unsigned long long)e * a.ph.member_draws);
-            else u4 = run_row_uniform<unsigned>(a.ph, (unsigned)e * a.batch + row, a.ph.draw_offset);
+        if (a.action != nullptr && (turn & 3) == 0) u4 = draw(tile);
+        if constexpr (!PARTS) {
+            if (turn == 0) {                             // the draw runs while the weights are on their way
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+            }
         }
-
         const unsigned char* wp = lds + lane * 16;
         f32x4 xn[HT];
         load_x(tile + stride < a.tiles ? tile + stride : tile, xn);
@@ -386,54 +495,239 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
         for (int pass = 0; pass < 4; ++pass) {
             const int rr = 4 * pass + hq;
             f32x4 v = *reinterpret_cast<const f32x4*>(scratch + rr * 256 + ((lq ^ rr) & 15) * 16);
-            // columns past the head's width, or its mask, enter as -inf (an exact 0 after the exponential) or 0
-            if (limit < ST_MAX_OUT) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (4 * lq + k >= limit) v[k] = NEG_INF;
-            }
             float p[4];
-            if constexpr (REGRET) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k) p[k] = 4 * lq + k < limit ? fmaxf(v[k], 0.f) : 0.f;
-                const float s = group_reduce<16>(sum4(p), [](float m, float n) { return m + n; });
-                const float inv_len = 1.f / (float)limit;
-                const RowDivisor over_s(s);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) p[k] = 4 * lq + k < limit ? (s != 0.f ? over_s(p[k]) : inv_len) : 0.f;
-            } else {
-                const float m = group_max<16>(vmax(vmax(v[0], v[1]), vmax(v[2], v[3])));
-#pragma unroll
-                for (int k = 0; k < 4; ++k) p[k] = fast_exp(v[k] - m);
-                const float s = group_reduce<16>(sum4(p), [](float m, float n) { return m + n; });
-                const float inv = 1.f / s;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) p[k] = p[k] * inv;
-            }
+            stack_head<REGRET>(v, lq, limit, p);
             const bool row_ok = rr < rows_here;
             if (row_ok && 4 * lq < a.n)
                 store16_through(reinterpret_cast<f32x4*>(tile_policy + rr * a.n + 4 * lq), f32x4{p[0], p[1], p[2], p[3]});
-            if (a.action != nullptr) {            // local_discrete_sampling (ml/primitives.spi:782-798)
-                const float incl = group_inclusive_scan<16>(sum4(p), lq);
-                float run = dpp_move<0x138>(incl);
-                if (lq == 0) run = 0.f;
-                float c[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    run = run + p[k];
-                    c[k] = run;
-                }
-                const float m = group_max<16>(sum4(p) > 0.f ? c[3] : NEG_INF);
-                const float thr = __shfl(u4, rr + 16 * (turn & 3)) * m;
-                int pick = 2147483647;
-#pragma unroll
-                for (int k = 3; k >= 0; --k)
-                    if (p[k] > 0.f && c[k] >= thr) pick = 4 * lq + k;
-                pick = group_reduce<16>(pick, [](int m, int n) { return m < n ? m : n; });
+            if (a.action != nullptr) {
+                const int pick = stack_pick(p, lq, __shfl(u4, rr + 16 * (turn & 3)));
                 if (row_ok && lq == 0) action[tile * ST_ROWS + rr] = pick;
             }
         }
         __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// ---- few rows: the waves of a workgroup share a layer's features ------------------------------------------------------------------
+// Where there is a tile of 16 rows per unit or two, latency is all there is: the chain of loads, products and barriers behind a row,
+// and the instructions themselves, which a launch fetches cold at about a byte a cycle.  A workgroup takes R x 16 rows of one member;
+// wave w computes the tiles w, w + waves, ... of 16 features of every layer, each in one rolled loop over units of 32 K-values whose
+// weights it streams through a ring of its own, and the activations cross LDS (a barrier a layer; one more where rows are normalised,
+// by the waves of the row tiles).  Inputs, uniforms and as many weights as the ring holds are asked for at once; the draws run
+// meanwhile.  Every sum, norm and head has the operations and the order of the kernel above.
+// LDS: [two buffers of activations][uniforms][a wave's ring].  A buffer is `planes` planes of 64 columns; row r of a plane is 256 bytes,
+// its 16-byte piece p in slot p ^ (r & 15), and so are the rows of logits.  A unit is 16 rows of 128 bytes, piece p of row i in slot
+// p ^ 2 ((i >> 1) & 3): no bank conflicts in either (16 lanes of a ds_read_b128: rows 0-3 and 12-15 of one lane group with rows 4-11
+// of the next).
+constexpr int SF_UNIT = 2048, SF_UNIFORMS = 2048, SF_MAX_THREADS = 512, SF_SLOTS = 16;
+
+template <int R, bool REGRET>
+__global__ __launch_bounds__(SF_MAX_THREADS) void stack_features_kernel(const float* x_first, const float* w0_first, const float* w1_first,
+                                                                        const float* w2_first, unsigned long long widths, int batch, unsigned counts,
+                                                                        int slots, unsigned acts, const StackArgs a) {
+    constexpr int PLANE = R * ST_ROWS * 256;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int e = blockIdx.y;
+    const int NL = (int)(counts & 15u), N = (int)(counts >> 4 & 0xffu), waves = (int)(counts >> 12 & 15u), planes = (int)(counts >> 16 & 3u), n = (int)(counts >> 18);
+    const int acts_bytes = planes * PLANE;
+    const int row0 = blockIdx.x * (ST_ROWS * R);
+    const unsigned lds0 = (unsigned)(size_t)lds;
+    const float NEG_INF = -__builtin_inff();
+    auto width = [&](int l) { return (int)((unsigned)(widths >> (8 * l)) & 0xffu) << 2; };
+    auto outputs_of = [&](int l) { return l + 1 < NL ? width(l + 1) : N; };
+    const int K0 = width(0);
+
+    // ---- inputs: four rows of a plane per instruction, zeros past the batch and past K0 ----
+#pragma unroll 1
+    for (int b = wave; b < (K0 > 64 ? 8 * R : 4 * R); b += waves) {
+        const int plane = b >= 4 * R ? 1 : 0, row = 4 * (b - plane * 4 * R) + (lane >> 4);
+        const int col = 4 * (16 * plane + ((lane & 15) ^ (row & 15)));
+        const bool inside = row0 + row < batch && col < K0;
+        const unsigned char* at = (const unsigned char*)(x_first + (long)(row0 + row) * K0 + col);
+        dma_to_lds_addr(inside ? at : (const unsigned char*)kZeroChunk, lds0 + b * 1024);
+    }
+    // the head's rows: with one row tile four waves take four rows each, else wave w the rows of tile w
+    const int head_tile = R == 1 ? 0 : wave;
+    const bool head_wave = R == 1 ? wave < 4 : wave < R;
+    const int my_row = row0 + ST_ROWS * head_tile + r;
+    const bool explicit_u = a.action != nullptr && a.ph.philox_mode < 0;
+    if (explicit_u && head_wave) {
+        const float* at = a.u + (long)e * batch + (my_row < batch ? my_row : batch - 1);
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(at), "s"(lds0 + 2 * acts_bytes + wave * 256) : "memory", "m0");
+    }
+
+    // ---- the stream of this wave's weights ----
+    const int ring_bytes = slots * SF_UNIT, ring_at = 2 * acts_bytes + SF_UNIFORMS + wave * ring_bytes;
+    const int r8 = lane >> 3, piece = (lane & 7) ^ (((r8 >> 1) & 3) << 1);
+    int f_layer = 0, f_tile = wave, f_k = 0, f_slot = 0, issued = 0;
+    auto member_of = [&](int l) { return (long)e * (width(l) * (l + 1 < NL ? width(l + 1) : n)); };
+    const float* f_base = w0_first + member_of(0);
+    auto next_unit = [&]() {                            // (layer, tile) to fetch from, past the layers that have none for this wave
+        while (f_layer < NL && 16 * f_tile >= outputs_of(f_layer)) {
+            ++f_layer;
+            f_tile = wave;
+            f_base = (f_layer == 1 ? w1_first : f_layer == 2 ? w2_first : a.w[f_layer & (ST_MAX_LAYERS - 1)]) + member_of(f_layer);
+        }
+    };
+    next_unit();
+    auto issue_unit = [&]() {
+        const int K = width(f_layer), F = outputs_of(f_layer);
+        const int k = f_k + 4 * piece, row = 16 * f_tile + r8;
+        const unsigned char* at = (const unsigned char*)(f_base + (long)row * K + k);
+        const bool k_inside = k < K;
+        dma_to_lds_addr(k_inside && row < F ? at : (const unsigned char*)kZeroChunk, lds0 + ring_at + f_slot);
+        dma_to_lds_addr(k_inside && row + 8 < F ? at + 32l * K : (const unsigned char*)kZeroChunk, lds0 + ring_at + f_slot + 1024);
+        f_slot = f_slot + SF_UNIT == ring_bytes ? 0 : f_slot + SF_UNIT;
+        ++issued;
+        f_k += 32;
+        if (f_k >= K) {
+            f_k = 0;
+            f_tile += waves;
+            next_unit();
+        }
+    };
+    int x_at[4], w_at[2];                               // the 16 wide blocks of a plane, and of a unit
+#pragma unroll
+    for (int b = 0; b < 4; ++b) x_at[b] = r * 256 + (((4 * b + q) ^ r) << 4);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) w_at[b] = ring_at + r * 128 + (((4 * b + q) ^ (((r >> 1) & 3) << 1)) << 4);
+    // all slots but two: those behind the units being multiplied are filled next, under their products
+#pragma unroll 1
+    for (int s = 2; s < slots && f_layer < NL; ++s) issue_unit();
+    float uniform = 1.f;
+    if (a.action != nullptr && head_wave && a.ph.philox_mode >= 0) {
+        const int row = my_row < batch ? my_row : batch - 1;
+        if (a.ph.member_rows > 0) uniform = run_row_uniform<unsigned>(a.ph, row, a.ph.draw_offset + (unsigned long long)e * a.ph.member_draws);
+        else uniform = run_row_uniform<unsigned>(a.ph, (unsigned)e * batch + row, a.ph.draw_offset);
+    }
+    // the oldest loads first: at most `young` units that were asked for later may be outstanding
+    auto wait_units = [&](int young) {
+        if (young >= 12) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+        else if (young >= 6) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+        else if (young >= 3) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+        else if (young >= 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    };
+    wait_units(issued);                                 // this wave's inputs have landed
+    asm volatile("s_barrier" ::: "memory");
+
+    int buffer = 0, c_slot = 0, consumed = 0;
+#pragma unroll 1
+    for (int layer = 0; layer < NL; ++layer) {
+        const int K = width(layer), F = outputs_of(layer);
+        const unsigned act = acts >> (4 * layer) & 15u;
+        const int map = (int)(act & 3u);              // of the last layer: none
+        auto mapped = [&](f32x4& y) {
+            if (map == SP_MAP_RELU) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y[i] = fmaxf(y[i], 0.f);
+            } else if (map != SP_MAP_COPY) {
+#pragma unroll 1
+                for (int i = 0; i < 4; ++i) {            // (rolled: one copy of the function)
+                    float v = y[0];
+                    if (map == SP_MAP_TANH) v = tanhf(v);
+                    else v = 1.f / (1.f + expf(-v));
+                    y = f32x4{y[1], y[2], y[3], v};
+                }
+            }
+        };
+        const int to = acts_bytes - buffer;             // the other buffer
+#pragma unroll 1
+        for (int t = wave; 16 * t < F; t += waves) {
+            f32x4 y[R];
+#pragma unroll
+            for (int rt = 0; rt < R; ++rt) y[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int k = 0; k < K; k += 64) {
+                const int units = k + 32 < K ? 2 : 1;
+                wait_units(issued - consumed - units);
+                const unsigned char* const acts_at = lds + buffer + (k >> 6) * PLANE;
+                f32x4 x[4][R], w[4];
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    if (b < 2 || units == 2) {
+                        w[b] = *reinterpret_cast<const f32x4*>(lds + w_at[b & 1] + c_slot);
+                        if (b & 1) c_slot = c_slot + SF_UNIT == ring_bytes ? 0 : c_slot + SF_UNIT;
+#pragma unroll
+                        for (int rt = 0; rt < R; ++rt) x[b][rt] = *reinterpret_cast<const f32x4*>(acts_at + x_at[b] + rt * 4096);
+                    }
+                consumed += units;
+                for (int u = 0; u < units && f_layer < NL; ++u) issue_unit();      // into the slots of the units before these
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    if (k + 16 * b < K)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+#pragma unroll
+                            for (int rt = 0; rt < R; ++rt) y[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[b][i], x[b][rt][i], y[rt], 0, 0, 0);
+            }
+            // lane (r, q): features 16 t + 4 q .. + 3 of batch row r
+            const int at = to + (t >> 2) * PLANE + r * 256 + (((4 * (t & 3) + q) ^ r) << 4);
+#pragma unroll
+            for (int rt = 0; rt < R; ++rt) {
+                if (!(act & 8u)) mapped(y[rt]);
+                *reinterpret_cast<f32x4*>(lds + at + rt * 4096) = y[rt];
+            }
+        }
+        buffer = to;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (act & 8u) {                                  // local_ln_l2 (ml/primitives.spi:701-703) of the rows of tile `wave`
+            if (wave < R) {
+                unsigned char* const rows = lds + buffer + wave * 4096;
+                f32x4 y[ST_MAX_WIDTH / 16];
+                float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+                for (int t = 0; t < ST_MAX_WIDTH / 16; ++t)
+                    if (16 * t < F) y[t] = *reinterpret_cast<const f32x4*>(rows + (t >> 2) * PLANE + x_at[t & 3]);
+#pragma unroll
+                for (int t = 0; t < ST_MAX_WIDTH / 16; ++t)
+                    if (16 * t < F) {
+                        s0 = __builtin_fmaf(y[t][0], y[t][0], s0);
+                        s1 = __builtin_fmaf(y[t][1], y[t][1], s1);
+                        s0 = __builtin_fmaf(y[t][2], y[t][2], s0);
+                        s1 = __builtin_fmaf(y[t][3], y[t][3], s1);
+                    }
+                float s = s0 + s1;
+                s += __shfl_xor(s, 16);
+                s += __shfl_xor(s, 32);
+                const RowDivisor over_s(s);
+#pragma unroll
+                for (int t = 0; t < ST_MAX_WIDTH / 16; ++t)
+                    if (16 * t < F) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) y[t][i] = s != 0.f ? over_s(y[t][i]) : 0.f;
+                        mapped(y[t]);
+                        *reinterpret_cast<f32x4*>(rows + (t >> 2) * PLANE + x_at[t & 3]) = y[t];
+                    }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+    }
+    if (!head_wave) return;
+    if (explicit_u) uniform = *reinterpret_cast<const float*>(lds + 2 * acts_bytes + wave * 256 + lane * 4);
+
+    // ---- the head and the sampling, four rows at a time: lane l of 16 holds columns 4 l .. of its row, as in the row primitives ----
+    const int limit = a.mask_size;
+    const unsigned char* const logits = lds + buffer + head_tile * 4096;
+    float* const policy = a.policy + (long)e * batch * n;
+#pragma unroll 1
+    for (int pass = R == 1 ? wave : 0; pass < (R == 1 ? wave + 1 : 4); ++pass) {
+        const int rr = 4 * pass + q, row = row0 + ST_ROWS * head_tile + rr;
+        f32x4 v = *reinterpret_cast<const f32x4*>(logits + rr * 256 + ((r ^ rr) & 15) * 16);
+        float p[4];
+        stack_head<REGRET>(v, r, limit, p);
+        const bool row_ok = row < batch;
+        if (row_ok && 4 * r < n) store16_through(reinterpret_cast<f32x4*>(policy + (long)row * n + 4 * r), f32x4{p[0], p[1], p[2], p[3]});
+        if (a.action != nullptr) {
+            const int pick = stack_pick(p, r, __shfl(uniform, rr));
+            if (row_ok && r == 0) a.action[(long)e * batch + row] = pick;
+        }
     }
 }
 
@@ -509,6 +803,8 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
         }
         a.w[l] = (const float*)weights[l];
         a.dims[l] = dims[l];
+        const unsigned kt = (unsigned)(dims[l] + 15) / 16;
+        a.per_kt[l] = (65536 + kt - 1) / kt;
         if (dims[l] > widest) widest = dims[l];
     }
     a.ph.philox_mode = -1;
@@ -526,11 +822,45 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
     a.n_layers = n_layers; a.n = n; a.batch = (int)batch;
     a.tiles = (int)((batch + ST_ROWS - 1) / ST_ROWS);
     const int ht = widest <= 64 ? 4 : 8;
+    const long cus = device_cu_count(), tiles = (long)a.tiles * members;
+    {
+        // A tile of rows per unit at most: the waves share its features; two where layers are wider than 64, as they leave the other kernel
+        // one workgroup a unit.  Us of a captured launch, that kernel / so: 108-64-32 48 rows 9.7 / 6.9, 124-64-32 tanh 1680 rows 10.9 / 6.8,
+        // 4-16-4 48 rows 5.7 / 4.5, 64-64-64-64 ln_l2 relu 4096 rows 10.3 / 8.5, 128-128-64 48 rows x 4 13.6 / 7.2, 4096 rows 14.0 / 8.9;
+        // two tiles: 128-128-64 8192 rows 14.1 / 10.3, 128-96-64 12.6 / 10.0, 80-128-64 tanh 6656 rows 15.3 / 10.3, but 64-64-64-64
+        // 10.5 / 10.9, 100-16-32 7.7 / 7.8; four tiles 64-64-64-64 16384 rows 10.8 / 12.9.
+        const int rt = tiles <= cus ? 1 : tiles <= 2 * cus && widest > 64 ? 2 : 0;
+        if (rt > 0) {
+            unsigned long long widths = 0;
+            int most_tiles = (a.mask_size + 15) / 16, units = 0;
+            for (int l = 0; l < n_layers; ++l) {
+                widths |= (unsigned long long)(dims[l] / 4) << (8 * l);
+                if (l > 0 && dims[l] / 16 > most_tiles) most_tiles = dims[l] / 16;
+            }
+            const int waves = most_tiles < 4 ? 4 : most_tiles > 8 ? 8 : most_tiles;
+            for (int l = 0; l < n_layers; ++l) units += (dims[l] + 31) / 32 * (((l + 1 < n_layers ? dims[l + 1] : a.mask_size) + 15) / 16 + waves - 1) / waves;
+            const int planes = widest > 64 ? 2 : 1, ring_at = 2 * planes * rt * ST_ROWS * 256 + SF_UNIFORMS;
+            int slots = (ST_LDS - ring_at) / (waves * SF_UNIT);
+            slots = slots < SF_SLOTS ? slots : SF_SLOTS;
+            slots = units + 2 < slots ? units + 2 : slots;
+            unsigned counts = (unsigned)n_layers | (unsigned)a.mask_size << 4 | (unsigned)waves << 12 | (unsigned)planes << 16 | (unsigned)n << 18, acts_bits = 0;
+            for (int l = 0; l + 1 < n_layers; ++l) acts_bits |= (unsigned)((acts[l] & 3) | (acts[l] & SP_STACK_LN_L2 ? 8 : 0)) << (4 * l);
+            const void* kernel = rt == 1 ? (regret ? (const void*)stack_features_kernel<1, true> : (const void*)stack_features_kernel<1, false>)
+                                         : (regret ? (const void*)stack_features_kernel<2, true> : (const void*)stack_features_kernel<2, false>);
+            rc = ensure_dynamic_lds(kernel, ST_LDS);
+            if (rc != SP_OK) return rc;
+            const float *x_first = a.x, *w0 = a.w[0], *w1 = a.w[n_layers > 1 ? 1 : 0], *w2 = a.w[n_layers > 2 ? 2 : 0];
+            void* args[] = {(void*)&x_first, (void*)&w0, (void*)&w1, (void*)&w2, (void*)&widths, (void*)&a.batch, (void*)&counts, (void*)&slots, (void*)&acts_bits, (void*)&a};
+            const hipError_t err = hipLaunchKernel(kernel, dim3((unsigned)((a.tiles + rt - 1) / rt), (unsigned)members), dim3(64 * waves), args,
+                                                   ring_at + waves * slots * SF_UNIT, (hipStream_t)stream);
+            if (err != hipSuccess) return fail(SP_ERR_DEVICE, "sp_stack_forward_f32: launch failed: %s", hipGetErrorString(err));
+            return check_launch(__func__);
+        }
+    }
     bool full = true;
     for (int l = 0; l < n_layers; ++l) full = full && (dims[l] + 15) / 16 == ht;
     // workgroups of a member, tiles of a wave (no more workgroups than give those), rounds of workgroups
     struct Launch { long gx, each, rounds; };
-    const long cus = device_cu_count(), tiles = (long)a.tiles * members;
     auto launch_of = [&](long gx, long waves, long at_once) {
         const long most = (a.tiles + waves - 1) / waves;
         if (gx > most) gx = most;

@@ -111,6 +111,27 @@ def test_every_instance(S, rows, widths, head, mask):
           uniforms(rng, 3 * rows), None)
 
 
+@pytest.mark.parametrize("members,tiles_per_unit,short,widths,acts,head,mask", [
+    (1, 1, 5, (64, 64, 64, 64), "ln+relu", "ROW_SOFTMAX", 0), (1, 1, 0, (108, 64, 32), "tanh", "ROW_MASKED_SOFTMAX", 3),
+    (4, 1, 15, (4, 16, 4), "ln+copy", "ROW_REGRET_MATCHING", 0), (1, 2, 17, (116, 128, 96, 64), "ln+sigmoid", "ROW_SOFTMAX", 0),
+    (2, 2, 7, (80, 112, 20), "relu", "ROW_MASKED_REGRET_MATCHING", 17), (1, 2, 1, (36, 16, 128, 16, 16, 16, 16, 16, 48), "ln+relu", "ROW_SOFTMAX", 0)])
+def test_rows_of_few_are_those_of_many(S, members, tiles_per_unit, short, widths, acts, head, mask):
+    """Up to a tile of 16 rows per compute unit (two of wide layers) the waves share the features, beyond that the rows: a row's
+    result is the same bit for bit, at the last batch before the rule's line and, as part of a larger one, behind it."""
+    announce("stack, few rows %d x %d tiles per unit %s %s" % (members, tiles_per_unit, widths, head))
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    few = 16 * tiles_per_unit * cus // members - short
+    many = 16 * (2 * cus + 16)
+    rng = np.random.default_rng(few)
+    x, ws = make(rng, members, many, widths)
+    u = dev(uniforms(rng, members * many).reshape(members, many))
+    names = [acts] * (len(widths) - 2)
+    p, a = forward(S, x[:few].contiguous(), ws, names, getattr(S, head), mask, u[:, :few].contiguous())
+    want_p, want_a = forward(S, x, ws, names, getattr(S, head), mask, u)
+    assert torch.equal(p, want_p[:, :few]) and torch.equal(a, want_a[:, :few])
+    check(S, x[:few].contiguous(), ws, names, getattr(S, head), mask, host(u[:, :few].contiguous()).reshape(-1), None)
+
+
 @pytest.mark.parametrize("members,blocks,rows_per_block,widths", [(3, 24, 9101, (64, 64, 64)), (2, 7, 5, (128, 128, 16)), (1, 24, 13655, (32, 64, 8))])
 def test_uniforms_drawn_on_the_device(S, members, blocks, rows_per_block, widths):
     """A run per member (member_rows), later in the stream each, and one run over all members' rows."""
