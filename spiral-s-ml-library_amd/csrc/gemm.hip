@@ -344,7 +344,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_abt_kernel(SP_GEMM_PRELOADED
     // ---- epilogue: each wave transposes its accumulators through a private LDS strip of 32 rows x
     //      up to 64 columns, so that C is written (and, for beta != 0, read) as whole row segments:
     //      16 bytes per lane, up to 256 contiguous bytes per row ----
-    constexpr int SW = WTN < 64 ? WTN : 64;        // columns per strip
+    constexpr int SW = WTN % 64 == 0 ? 64 : 32;    // columns per strip
     constexpr int SF = SW / 32;                    // fragments per strip
     constexpr int EPI_STRIDE = SW * 4 + 16;        // bytes; the pad keeps the 16-byte column writes conflict free
     constexpr int LPR = SW / 4;                    // lanes per output row
@@ -947,7 +947,8 @@ __global__ __launch_bounds__(256) void gemm_abt_generic_kernel(const GemmArgs g)
 struct TileCfg {
     int bm, bn, wm, wn;
 };
-static const TileCfg kTileCfgs[] = {{256, 256, 2, 4}, {128, 128, 2, 2}, {64, 64, 2, 2}};
+// (the last two: 16-bit inputs, as ragged tiles, by the estimate)
+static const TileCfg kTileCfgs[] = {{256, 256, 2, 4}, {128, 128, 2, 2}, {64, 64, 2, 2}, {128, 64, 2, 2}, {128, 96, 4, 1}};
 constexpr int kNumCfgs = 3;
 
 // The four-wave kernel takes the 256 x 256 tiles of 16-bit GEMMs whose K is a whole number of K-tile pairs and whose
@@ -983,7 +984,7 @@ static int choose_cfg(int dtype_in, long M, long N, long K, long batch, long cus
     return smallest;
 }
 
-// The tile a GEMM runs on: a workgroup tile of kTileCfgs (cfg 0..2), a split-K tile of gemm_wave.hip (cfg -1) or none, one
+// The tile a GEMM runs on: a workgroup tile of kTileCfgs (cfg 0..4), a split-K tile of gemm_wave.hip (cfg -1) or none, one
 // thread per output (cfg -2).
 // `ragged`: the tile does not divide M, N and K -- rows clamped in the loader, zeros for the missing part of the last
 // K-tile, a masked epilogue.
@@ -1003,16 +1004,22 @@ struct TileChoice {
 // (us, 256 / 128 / 64 wide tiles: 11200 x 1792 x 32 44 / 33 / 20, 2688 x 5760 x 64 31 / 25 / 23, 2112 x 1536 x 96 36 / 15 / 9.6;
 // 10688 x 768 x 3648, 824 / 467 / 485, keeps its 128).  16-bit rows that do not start on 128-byte lines cost every fetch a
 // second line, hence two sets of numbers.
+// 128 x 64 and 128 x 96 tiles fill the units where 128 wide ones leave a last round nearly empty and 64 wide ones move twice the operands
+// (us, without / with them: f16 5001 x 1003 x 1000 27.1 / 21.6, bf16 2390 x 1252 x 5696 101 / 87, 14864 x 320 x 4800 64 / 42, 656 x 6992 x
+// 1152 29 / 22, 23732 x 234 x 56 12 / 8; 0.98 times the time on the geometric mean of 220 shapes of 0.4 GFLOP and more that no 128 tile
+// divides, 43 of which take them, the worst 1.08 times: 53584 x 16 x 272).  Fitted on those 220; also measured: 192 x 128, 128 x 192, 192 x
+// 192, 256 x 128, 256 x 192 and 96 x 128 tiles, which add less than a hundredth.
 struct TileCost {
     int cfg, bm, bn;
     float tk, overhead, latency;
 };
 static const TileCost kCostF32[] = {{0, 256, 256, 7.86f, 22.f, 0.f}, {1, 128, 128, 2.17f, 3.6f, 0.f}, {2, 64, 64, 0.556f, 0.52f, 0.f},
                                     {-1, 32, 32, 0.151f, 0.45f, 0.f}, {-1, 16, 16, 0.079f, 0.24f, 0.f}};
-static const TileCost kCostLines[] = {{0, 256, 256, 1.75f, 8.f, 0.f}, {1, 128, 128, 0.55f, 3.5f, 1.05f}, {2, 64, 64, 0.22f, 0.8f, 0.25f},
+static const TileCost kCostLines[] = {{0, 256, 256, 1.75f, 8.f, 0.f}, {1, 128, 128, 0.55f, 3.5f, 1.05f}, {2, 64, 64, 0.22f, 0.8f, 0.25f}, {3, 128, 64, 0.32f, 1.85f, 0.5f},
                                       {-1, 64, 64, 0.22f, 1.5f, 0.f}, {-1, 64, 32, 0.17f, 0.8f, 0.f}, {-1, 32, 32, 0.09f, 0.5f, 0.f},
                                       {-1, 16, 16, 0.05f, 0.3f, 0.f}};
 static const TileCost kCostCrossing[] = {{0, 256, 256, 1.5f, 14.f, 0.f}, {1, 128, 128, 0.65f, 4.f, 1.05f}, {2, 64, 64, 0.29f, 0.8f, 0.5f},
+                                         {3, 128, 64, 0.49f, 1.4f, 1.0f}, {4, 128, 96, 0.5f, 4.8f, 0.f},
                                          {-1, 64, 64, 0.27f, 1.5f, 0.f}, {-1, 64, 32, 0.19f, 0.8f, 0.f}, {-1, 32, 32, 0.11f, 0.5f, 0.f},
                                          {-1, 16, 16, 0.055f, 0.3f, 0.f}};
 
@@ -1033,7 +1040,7 @@ static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, lo
     const TileCost* best = nullptr;
     float best_us = 0.f;
     auto consider = [&](const TileCost& c) {
-        if (whole == 0 || whole == 1 ? c.cfg != whole : whole == 2 && (c.cfg == 0 || c.cfg == 1)) return;
+        if (whole == 0 || whole == 1 ? c.cfg != whole : whole == 2 && c.cfg >= 0 && c.cfg != 2) return;
         if (c.cfg < 0 ? kind == TILE_WORKGROUP : kind == TILE_SPLIT) return;
         if (c.cfg < 0 && (!may_split || K * es > kWaveMaxRowBytes || M > 2147483000l || N > 2147483000l)) return;
         const double of_member = (double)((M + c.bm - 1) / c.bm) * (double)((N + c.bn - 1) / c.bn);
@@ -1055,7 +1062,7 @@ static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, lo
     if (best == nullptr) return best_tile(dtype_in, M, N, K, batch, cus, TILE_WORKGROUP);   // (a split form that cannot be numbered)
     if (best->cfg < 0) return {-1, best->bm, best->bn, 256, true, best_us};
     const TileCfg& t = kTileCfgs[best->cfg];
-    const bool ragged = M % t.bm != 0 || N % t.bn != 0 || K % bk != 0;
+    const bool ragged = best->cfg >= kNumCfgs || M % t.bm != 0 || N % t.bn != 0 || K % bk != 0;
     const int threads = best->cfg == 0 && !ragged && use_four_waves(dtype_in, N, K) ? 256 : t.wm * t.wn * 64;
     return {best->cfg, t.bm, t.bn, threads, ragged, best_us};
 }
@@ -1219,6 +1226,10 @@ static int launch_dtype(int cfg, const GemmArgs& g, hipStream_t stream) {
             return launch_tiled<DT, OT, 256, 256, 2, 4>(g, stream);
         case 1: return launch_tiled<DT, OT, 128, 128, 2, 2>(g, stream);
         case 2: return launch_tiled<DT, OT, 64, 64, 2, 2>(g, stream);
+    }
+    if constexpr (DT != SP_F32) {
+        if (cfg == 3) return launch_tiled_stages<DT, OT, 128, 64, 2, 2, 2, 2, true>(g, stream);
+        if (cfg == 4) return launch_tiled_stages<DT, OT, 128, 96, 4, 1, 2, 2, true>(g, stream);
     }
     dim3 grid((unsigned)(((g.N + 15) / 16) * ((g.M + 15) / 16)), (unsigned)g.batch);
     hipLaunchKernelGGL(gemm_abt_generic_kernel<DT>, grid, dim3(256), 0, stream, g);

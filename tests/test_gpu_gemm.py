@@ -109,6 +109,35 @@ def test_ragged_m_and_n(MM, dtype, m, n, k):
     assert (got[pad:pad + m * n].reshape(m, n).astype(np.float64) == np.maximum(want + 2 * c0 + bias, 0)).all()
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("m,n,k,tile", [(8370, 332, 8, (128, 64)), (8449, 333, 8, (128, 64)), (6400, 449, 192, (128, 64)), (5612, 576, 192, (128, 64)),
+                                        (8817, 199, 400, (128, 96)), (6529, 280, 392, (128, 96)), (6656, 288, 392, (128, 96)), (5001, 1003, 1000, (128, 96))])
+def test_tiles_of_128_by_64_and_96_are_exact(MM, dtype, m, n, k, tile):
+    """16-bit inputs on the tiles between the 128 and 64 wide ones, at one row or column past a tile and at whole ones, with a partial last
+    K-tile: integer operands give the exact product in every output type, with bias + ReLU and beta, and nothing outside C is touched."""
+    announce("gemm tile %s %s %dx%dx%d" % (tile, dtype, m, n, k))
+    cfg = MM.matmul_config_tf32(False, True, m, n, k, TORCH[dtype])
+    assert (cfg["m_tile"], cfg["n_tile"]) == tile
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    w = (np.arange(k) // 64 % 3 + 1).astype(np.float32)            # a K-tile read twice, or from the wrong stage, shows
+    ai = rng.integers(-1, 2, size=(m, k)).astype(np.float32) * w
+    bi = rng.integers(-1, 2, size=(n, k)).astype(np.float32)
+    want = (dev(ai).double() @ dev(bi).double().T)
+    bias, c0 = dev(rng.integers(-5, 6, size=n).astype(np.float32)), dev(rng.integers(-4, 5, size=(m, n)).astype(np.float32))
+    a, b, pad = dev(ai, TORCH[dtype]), dev(bi, TORCH[dtype]), 64
+    for out in ("f32", dtype):
+        for beta, add in ((0.0, None), (0.0, bias), (2.0, bias)):
+            if out != "f32" and beta:
+                continue
+            buf = torch.full((pad + m * n + pad,), -77.0, dtype=TORCH[out], device="cuda")
+            c = buf[pad:pad + m * n].view(m, n)
+            c.copy_(c0)
+            MM.matmul_abt(a, b, c=c, bias=add, relu=add is not None, beta=beta)
+            exact = want + beta * c0.double() + (0.0 if add is None else add.double())
+            exact = exact.clamp(min=0) if add is not None else exact
+            assert torch.equal(c, exact.float().to(TORCH[out])) and (buf[:pad] == -77).all() and (buf[-pad:] == -77).all()
+
+
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("m,n,kt", [(1, 1, 1), (17, 3, 6), (31, 33, 6), (130, 31, 5.5), (5000, 5, 2), (16, 4096, 7), (33, 15, 7),
                                     (257, 16, 7.5), (250, 250, 8), (500, 331, 9), (1900, 241, 11), (331, 65, 27.5), (1, 9001, 13),
