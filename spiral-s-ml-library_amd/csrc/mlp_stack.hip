@@ -102,48 +102,45 @@ __device__ __forceinline__ void full_product(const unsigned char*& wp, const f32
     wp += KT * NT * ST_BLOCK;
 }
 
-// The same for kt <= KT blocks of K and nt <= NT tiles of features: groups of four tiles as above (their sums are four chains, which the
-// matrix pipe takes in turn), the tiles behind the last whole group one after the other, the weights one block ahead (behind the last
-// block of the stack lies the scratch: read, not used).
+// The same for kt <= KT blocks of K and nt <= NT tiles of features: groups of four tiles as above, then of two and of one (the sums of a
+// group are chains which the matrix pipe takes in turn), the weights one block ahead (behind the last block of the stack lies the
+// scratch: read, not used).
+template <int G, int KT, int NT>
+__device__ __forceinline__ void group_product(const unsigned char*& wp, const f32x4 (&x)[KT], f32x4 (&y)[NT], int t0, int kt) {
+    f32x4 w[G];
+#pragma unroll
+    for (int t = 0; t < G; ++t) {
+        y[t0 + t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        w[t] = *reinterpret_cast<const f32x4*>(wp + t * ST_BLOCK);
+    }
+#pragma unroll
+    for (int j = 0; j < KT; ++j)
+        if (j < kt) {
+            wp += G * ST_BLOCK;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int t = 0; t < G; ++t) {
+                    y[t0 + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][i], x[j][i], y[t0 + t], 0, 0, 0);
+                    if (i == 3) w[t] = *reinterpret_cast<const f32x4*>(wp + t * ST_BLOCK);      // (the next block's, in time for its first use)
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+}
 template <int KT, int NT>
 __device__ __forceinline__ void part_product(const unsigned char*& wp, const f32x4 (&x)[KT], f32x4 (&y)[NT], int kt, int nt) {
 #pragma unroll
     for (int g = 0; g < NT; g += 4) {
         if (g + 4 <= nt) {
-            f32x4 w[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                y[g + t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                w[t] = *reinterpret_cast<const f32x4*>(wp + t * ST_BLOCK);
-            }
-#pragma unroll
-            for (int j = 0; j < KT; ++j)
-                if (j < kt) {
-                    wp += 4 * ST_BLOCK;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int t = 0; t < 4; ++t) {
-                            y[g + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][i], x[j][i], y[g + t], 0, 0, 0);
-                            if (i == 3) w[t] = *reinterpret_cast<const f32x4*>(wp + t * ST_BLOCK);      // (the next block's, in time for its first use)
-                        }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+            group_product<4>(wp, x, y, g, kt);
         } else {
-            f32x4 w = *reinterpret_cast<const f32x4*>(wp);
 #pragma unroll
-            for (int t = g; t < g + 4; ++t) {
-                y[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                if (t < nt) {
-#pragma unroll
-                    for (int j = 0; j < KT; ++j)
-                        if (j < kt) {
-                            wp += ST_BLOCK;
-                            const f32x4 next = *reinterpret_cast<const f32x4*>(wp);
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) y[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[j][i], y[t], 0, 0, 0);
-                            w = next;
-                        }
+            for (int t = g; t < g + 4; ++t) y[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (g < nt) {
+                if (nt & 2) group_product<2>(wp, x, y, g, kt);
+                if (nt & 1) {
+                    if (nt & 2) group_product<1>(wp, x, y, g + 2, kt);
+                    else group_product<1>(wp, x, y, g, kt);
                 }
             }
         }
@@ -318,7 +315,7 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
         for (int l = 0; l < layers; ++l) {
             const int K = a.dims[l], F = a.dims[l + 1], kt = (K + 15) >> 4, nt = (F + 15) >> 4;
             const float* W = weights_of(l);
-            // in the order the products read them: full_product's tiles in one group, part_product's in fours and then one by one
+            // in the order the products read them: full_product's tiles in one group, part_product's in fours, two and one
             const bool full = FULL && (l + 1 < layers || nt == ST_MAX_OUT / 16);
             const unsigned mine = (unsigned)(r * K + 4 * q) * 4;
             const int whole = full ? nt : nt & ~3, log_group = full && nt == 8 ? 3 : 2;       // tiles in groups (of 8 or 4)
@@ -329,10 +326,10 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
                     const int turn = b >> log_group, group = (int)((unsigned)turn * per_kt >> 16);
                     tile = (group << log_group) + (b & ((1 << log_group) - 1));
                     block = turn - group * kt;
-                } else {
-                    const int over = b - kt * whole, t = (int)((unsigned)over * per_kt >> 16);
-                    tile = whole + t;
-                    block = over - t * kt;
+                } else {                                  // a group of two, if nt has one, and the last tile
+                    const int over = b - kt * whole, two = nt & 2;
+                    tile = over < kt * two ? whole + (over & 1) : whole + two;
+                    block = over < kt * two ? over >> 1 : over - kt * two;
                 }
                 const int row = 16 * tile, col = 16 * block;
                 const unsigned to = __builtin_amdgcn_readfirstlane(dst + b * ST_BLOCK);
