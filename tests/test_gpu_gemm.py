@@ -111,7 +111,7 @@ def test_ragged_m_and_n(MM, dtype, m, n, k):
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("m,n,k,tile", [(8370, 332, 8, (128, 64)), (8449, 333, 8, (128, 64)), (6400, 449, 192, (128, 64)), (5612, 576, 192, (128, 64)),
-                                        (8817, 199, 400, (128, 96)), (6529, 280, 392, (128, 96)), (6656, 288, 392, (128, 96)), (5001, 1003, 1000, (128, 96))])
+                                        (8193, 193, 456, (128, 96)), (6529, 280, 456, (128, 96)), (6656, 288, 456, (128, 96)), (5001, 1003, 1000, (128, 96))])
 def test_tiles_of_128_by_64_and_96_are_exact(MM, dtype, m, n, k, tile):
     """16-bit inputs on the tiles between the 128 and 64 wide ones, at one row or column past a tile and at whole ones, with a partial last
     K-tile: integer operands give the exact product in every output type, with bias + ReLU and beta, and nothing outside C is touched."""
