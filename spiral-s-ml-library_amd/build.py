@@ -17,6 +17,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libspiral_mi355.so")
+HOST_LIB = os.path.join(HERE, "spiral_host.so")      # the Python modules' way into the library (csrc/host.cpp)
 SOURCES = ["api.hip", "row_ops.hip", "elementwise.hip", "gemm.hip", "gemm_wave.hip", "mlp.hip", "mlp_any.hip", "mlp_packed.hip", "mlp_resident.hip", "mlp_pipe.hip", "mlp_ensemble.hip", "mlp_stack.hip"]
 # sources with MFMAs or wide stores in inline asm: their device assembly is kept and scanned (isa_check.py)
 ASM_MFMA_SOURCES = ["gemm.hip", "gemm_wave.hip", "mlp.hip", "mlp_any.hip", "mlp_packed.hip", "mlp_resident.hip", "mlp_pipe.hip", "mlp_ensemble.hip", "mlp_stack.hip", "row_ops.hip", "elementwise.hip"]
@@ -45,6 +46,19 @@ def _run(cmd):
     if p.returncode != 0:
         raise RuntimeError("command failed: %s\n%s" % (" ".join(cmd), out))
     return out
+
+
+def build_host():
+    """The CPython extension in front of the library, against this interpreter and this torch."""
+    import sysconfig
+    import torch
+    torch_dir = os.path.dirname(torch.__file__)
+    include = os.path.join(torch_dir, "include")
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wno-attributes",
+          "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-I" + os.path.join(ROOT, "include"),
+          "-isystem", include, "-isystem", os.path.join(include, "torch", "csrc", "api", "include"),
+          "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "host.cpp"), "-o", HOST_LIB,
+          "-L" + os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"])
 
 
 def device_asm(src):
@@ -93,8 +107,13 @@ def build(force=True, verbose=False):
                     os.remove(tmp)
         return o
 
-    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as ex:
-        objs = list(ex.map(compile_one, SOURCES))
+    with ThreadPoolExecutor(max_workers=8) as ex:
+        objs = ex.map(compile_one, SOURCES)
+        newest = max(os.path.getmtime(os.path.join(CSRC, "host.cpp")), os.path.getmtime(os.path.join(ROOT, "include", "spiral_mi355.h")))
+        host = None if not force and os.path.exists(HOST_LIB) and os.path.getmtime(HOST_LIB) > newest else ex.submit(build_host)
+        objs = list(objs)
+        if host is not None:
+            host.result()
     check_isa()
     _run([cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs)
     return LIB

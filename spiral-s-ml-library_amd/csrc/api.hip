@@ -68,7 +68,7 @@ int device_cu_count() {
 // itself is thread safe and idempotent, a second thread merely repeats it once).
 int ensure_dynamic_lds(const void* kernel, int lds_bytes) {
     struct Seen { const void* kernel; int device; };
-    static thread_local Seen seen[64];
+    static thread_local Seen seen[256];
     static thread_local int n_seen = 0;
     int dev = 0;
     (void)hipGetDevice(&dev);
@@ -76,7 +76,7 @@ int ensure_dynamic_lds(const void* kernel, int lds_bytes) {
         if (seen[i].kernel == kernel && seen[i].device == dev) return SP_OK;
     hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (e != hipSuccess) return fail(SP_ERR_DEVICE, "hipFuncSetAttribute(%d B LDS) failed: %s", lds_bytes, hipGetErrorString(e));
-    if (n_seen < 64) seen[n_seen++] = Seen{kernel, dev};
+    if (n_seen < 256) seen[n_seen++] = Seen{kernel, dev};
     return SP_OK;
 }
 

@@ -1,5 +1,8 @@
-"""ctypes binding of libspiral_mi355.so (declared in include/spiral_mi355.h)."""
+"""Binding of libspiral_mi355.so (declared in include/spiral_mi355.h): launches through the extension of csrc/host.cpp, everything
+else through ctypes."""
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
@@ -110,12 +113,17 @@ def load(path=LIB_PATH):
     return lib
 
 
-# Entry points that launch work; their last argument is the stream.
-LAUNCHES = frozenset(("sp_gemm_abt", "sp_gemm_abt_batched", "sp_row_ops", "sp_row_map_f32", "sp_row_map_i32",
-                      "sp_row_sample", "sp_philox_uniforms", "sp_row_get_prob", "sp_cem_resample", "sp_cem_resample_philox",
-                      "sp_row_reduce_f32", "sp_cem_update_mask",
-                      "sp_row_binarize", "sp_map_f32", "sp_reduce_sum", "sp_reduce", "sp_row_l1_normalize", "sp_reduce_sum_static", "sp_transpose_inner_b32", "sp_mlp_forward", "sp_mlp_pack_weights",
-                      "sp_mlp_forward_packed", "sp_mlp_forward_ensemble", "sp_ensemble_binarize", "sp_stack_forward_f32"))
+def _load_host():
+    path = os.path.join(os.path.dirname(_HERE), "spiral_host.so")
+    if not os.path.exists(path):
+        raise RuntimeError("%s is missing: build it with `python spiral-s-ml-library_amd/build.py`" % path)
+    loader = importlib.machinery.ExtensionFileLoader("spiral_host", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("spiral_host", path, loader=loader))
+    loader.exec_module(module)
+    return module
+
+
+_host = _load_host()
 
 
 class Tape:
@@ -134,42 +142,31 @@ class Tape:
                 check(rc)
 
 
-_tape = None
-
-
 def start_tape():
     """Every launch through `lib` from now until stop_tape() is also recorded."""
-    global _tape
-    _tape = Tape()
-    return _tape
+    tape = Tape()
+    _host.tape(tape.calls, tape.keep)
+    return tape
 
 
 def stop_tape():
-    global _tape
-    _tape = None
+    _host.tape(None, None)
 
 
 class _Library:
-    """The C-ABI library; launches pass through a thin wrapper that feeds the active tape, if any."""
+    """The C-ABI library; the entry points that launch work (their last argument is the stream) feed the active tape, if any."""
 
-    def __init__(self, cdll):
-        self._cdll = cdll
+    def __init__(self, path):
+        self._cdll = load(path)
+        self.__dict__.update(_host.bind(path))
 
     def __getattr__(self, name):
         fn = getattr(self._cdll, name)
-        if name in LAUNCHES:
-            raw = fn
-
-            def fn(*args):
-                rc = raw(*args)
-                if _tape is not None and rc == 0:
-                    _tape.calls.append((raw, args[:-1]))
-                return rc
         setattr(self, name, fn)     # looked up once
         return fn
 
 
-lib = _Library(load())
+lib = _Library(LIB_PATH)
 
 
 def check(rc):
@@ -184,28 +181,15 @@ def stream_ptr():
     """torch's current HIP stream as a hipStream_t.  The raw query skips the Stream object, which costs
     several microseconds per call: as much as a small kernel."""
     if _raw_stream is not None:
-        return C.c_void_p(_raw_stream(torch.cuda.current_device()))
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return _raw_stream(torch.cuda.current_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 DTYPES = {torch.float32: SP_F32, torch.float16: SP_F16, torch.bfloat16: SP_BF16}
 
 
-def ptr(t, dtype=None, name="tensor"):
-    """Device pointer of a contiguous ROCm tensor (None passes through as NULL)."""
-    if t is None:
-        return None
-    if not isinstance(t, torch.Tensor):
-        raise TypeError("%s must be a torch.Tensor" % name)
-    if not t.is_cuda:
-        raise ValueError("%s must live on the GPU (got %s)" % (name, t.device))
-    if not t.is_contiguous():
-        raise ValueError("%s must be contiguous (row-major, innermost stride 1)" % name)
-    if dtype is not None and t.dtype != dtype:
-        raise TypeError("%s must have dtype %s, got %s" % (name, dtype, t.dtype))
-    if _tape is not None:
-        _tape.keep.append(t)
-    return C.c_void_p(t.data_ptr())
+# ptr(t, dtype=None, name="tensor"): device pointer of a contiguous ROCm tensor, an integer (None passes through as NULL).
+ptr = _host.ptr
 
 
 def device_info():

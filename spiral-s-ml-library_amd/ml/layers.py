@@ -68,6 +68,9 @@ def pack_weights(weights, into=None):
     return into
 
 
+_WEIGHT_NAMES = ["weights[%d]" % i for i in range(8)]
+
+
 def mlp_forward(x, weights, biases=None, head="softmax_regret_matching", u=None, mask_size=0, want_logits=False,
                 policy_out=None, action_out=None, packed=None, rng=None):
     """policy, action[, logits] = fused forward of relu-MLP + head + discrete sampling.
@@ -101,19 +104,17 @@ def mlp_forward(x, weights, biases=None, head="softmax_regret_matching", u=None,
     logits = torch.empty((batch, dims[-1]), dtype=torch.float32, device=x.device) if want_logits else None
     bp = None
     if biases is not None:
-        bp = (C.c_void_p * n)(*[ptr(b, torch.float32, "biases[%d]" % i) if b is not None else None
-                                for i, b in enumerate(biases)])
-    dp = (C.c_int32 * (n + 1))(*dims)
+        bp = [ptr(b, torch.float32, "biases[%d]" % i) if b is not None else None for i, b in enumerate(biases)]
+        if len(bp) > n:
+            raise IndexError("more biases than layers")
     if packed is not None:
         check(lib.sp_mlp_forward_packed(_lib.DTYPES[x.dtype], ptr(x, name="x"), n, ptr(packed.buffer),
-                                        packed.buffer.numel(), bp, dp, ptr(u, torch.float32, "u"),
-                                        C.byref(rng) if rng is not None else None, ptr(policy, torch.float32, "policy_out"),
+                                        packed.buffer.numel(), bp, dims, ptr(u, torch.float32, "u"), rng, ptr(policy, torch.float32, "policy_out"),
                                         ptr(action, torch.int32, "action_out"), ptr(logits), batch, HEADS[head],
                                         mask_size, stream_ptr()))
     else:
-        wp = (C.c_void_p * n)(*[ptr(w, name="weights[%d]" % i) for i, w in enumerate(weights)])
-        check(lib.sp_mlp_forward(_lib.DTYPES[x.dtype], ptr(x, name="x"), n, wp, bp, dp, ptr(u, torch.float32, "u"),
-                                 C.byref(rng) if rng is not None else None, ptr(policy, torch.float32, "policy_out"), ptr(action, torch.int32, "action_out"),
+        wp = [ptr(w, None, _WEIGHT_NAMES[i & 7]) for i, w in enumerate(weights)]
+        check(lib.sp_mlp_forward(_lib.DTYPES[x.dtype], ptr(x, name="x"), n, wp, bp, dims, ptr(u, torch.float32, "u"), rng, ptr(policy, torch.float32, "policy_out"), ptr(action, torch.int32, "action_out"),
                                  ptr(logits), batch, HEADS[head], mask_size, stream_ptr()))
     out = (policy, action)
     return out + (logits,) if want_logits else out

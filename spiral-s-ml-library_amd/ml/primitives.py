@@ -119,7 +119,10 @@ def row_ops(logits, u=None, want=("rowmax", "rowsum", "probs", "cdf", "argmax", 
 
 def argmax(x):
     """row_reduce local_argmax (ml/primitives.spi:705-708, test2 :940); ties -> lowest index."""
-    return row_ops(x, want=("argmax",))["argmax"]
+    rows, cols = _rows_cols(x)
+    out = torch.empty(x.shape[:-1], dtype=torch.int32, device=x.device)
+    check(lib.sp_row_ops(ptr(x, torch.float32, "logits"), None, None, None, None, None, ptr(out), None, rows, cols, 0, stream_ptr()))
+    return out
 
 
 def philox(mode=_lib.PHILOX_BLOCK, seed=CONSTANT_SEED, threads_per_block=THREADS_PER_BLOCK,
@@ -142,19 +145,20 @@ def philox_uniforms(rng, rows, cols, out=None):
 def _sample(op, x, u=None, rng=None, mask_size=0, want_cdf=False, want_u=False, want_prob=False, probs_out=None,
             sample_out=None, want_probs=True):
     rows, cols = _rows_cols(x)
+    lead, dev = x.shape[:-1], x.device
     probs = probs_out
     if probs is None and want_probs:
         probs = torch.empty_like(x)
-    sample = torch.empty(x.shape[:-1], dtype=torch.int32, device=x.device) if sample_out is None else sample_out
+    sample = torch.empty(lead, dtype=torch.int32, device=dev) if sample_out is None else sample_out
     cdf = torch.empty_like(x) if want_cdf else None
-    u_out = torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device) if want_u else None
-    prob = torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device) if want_prob else None
+    u_out = torch.empty(lead, dtype=torch.float32, device=dev) if want_u else None
+    prob = torch.empty(lead, dtype=torch.float32, device=dev) if want_prob else None
     if (u is None) == (rng is None):
         raise ValueError("give exactly one of u (a tensor of uniforms in (0, 1]) and rng (a PhiloxConfig)")
-    if (probs is not None and probs.shape != x.shape) or sample.shape != x.shape[:-1]:
+    if (probs_out is not None and probs.shape != x.shape) or (sample_out is not None and sample.shape != lead):
         raise ValueError("the output tensors do not have the input's dimensions")
     check(lib.sp_row_sample(op, ptr(x, torch.float32, "x"), ptr(u, torch.float32, "u"),
-                            C.byref(rng) if rng is not None else None,
+                            rng,
                             ptr(probs, torch.float32, "probs") if probs is not None else None, ptr(cdf),
                             ptr(u_out), ptr(sample, torch.int32, "sample"), ptr(prob), rows, cols, mask_size,
                             stream_ptr()))
