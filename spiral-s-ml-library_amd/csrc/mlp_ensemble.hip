@@ -5,9 +5,9 @@
 // matmul_ensemble_with_adjoint (E, 64, 64) -> masked_regret_matching' 3), which the graph interpreter
 // (ml/layers.spi:194-240, 336-344) runs member by member, node by node.
 //
-// One wave per SIMD (four per workgroup, nothing shared between them: no LDS, no barrier).  A wave loads the weights
-// of its member once -- 128 registers for the first layer, 32 per computed output for the second -- and walks over
-// 32-row tiles of the batch.
+// One wave per SIMD (four per workgroup, which share nothing but the load of the first layer's weights).  A wave takes the
+// weights of its member into registers once -- 128 registers for the first layer, 32 per computed output for the second --
+// and walks over 32-row tiles of the batch.
 //   Layer 1 is v_mfma_f32_32x32x2_f32 with the WEIGHTS as the row operand, so a result tile is (features x batch rows)
 // and lane (r, g) -- r = lane % 32 the batch row, g = lane / 32 -- holds features 8 a + 4 g + b (a, b = 0..3) of row
 // r in register 4 a + b.  Both operands of an MFMA step take their two K-values from the lane halves g = 0, 1, and
@@ -46,8 +46,29 @@ struct EnsembleArgs {
     int members, k0, n, nout, head, mask_size;
     unsigned* words;              // (members, batch) hash words of the binarize head, or nullptr
     unsigned modulo;
+    unsigned per_piece;           // i / (k0 / 4) is i * per_piece >> 20 for i < 2048
     PhiloxStream ph;
 };
+
+// A member's first weight matrix, `rows` rows of K0 floats, into LDS for a workgroup of four waves: the loads in the order
+// of memory, whole lines at a time and once per workgroup.  Read straight into its registers by every wave, a lane a line,
+// the 32 KiB of 64 x 128 take 8 k cycles.  Microseconds of a captured launch, read straight / through LDS: 128-64-16, 8
+// members of 1792 rows 13.8 / 11.6; 96-64-16, 2 of 28448 21.1 / 19.2; a hash of 200-128, 16 of 10240 32.3 / 28.7; 64-32, 7 of
+// 5600 8.0 / 6.7.  Up to 32 inputs, a line or less a row, the barrier costs more: 16-64-64, 8 of 2016 6.3 / 6.7.
+// 16-byte piece p of row r lies at slot p ^ (r & (G - 1)) of the row, G the power of two in the pieces of a row, at most 16: lanes of
+// different rows then read different banks.
+constexpr bool ensemble_through_lds(int kg) { return kg > 4; }
+__device__ __forceinline__ int ensemble_swizzle(int pieces) {
+    const int g = pieces & -pieces;
+    return (g < 16 ? g : 16) - 1;
+}
+__device__ __forceinline__ void ensemble_weights_to_lds(const float* w, int rows, int K0, unsigned per_piece, unsigned lds0, int wave, int lane) {
+    const int pieces = K0 >> 2, mask = ensemble_swizzle(pieces);
+    for (int b = wave; 64 * b < rows * pieces; b += 4) {
+        const int i = 64 * b + lane, row = (int)((unsigned)i * per_piece >> 20), piece = (i - row * pieces) ^ (row & mask);
+        mlp_dma((const unsigned char*)w, (unsigned)((row < rows ? row * K0 + 4 * piece : 0) * 4), __builtin_amdgcn_readfirstlane(lds0 + b * 1024));
+    }
+}
 
 // KG: 8-wide groups of the input width the kernel is unrolled for; EXACT: K0 = 8 KG (else K0 < 8 KG and the groups
 // past K0 are zeros); ACTION: an action per row is wanted (a uniform per row, from a tensor or a Philox stream)
@@ -63,9 +84,12 @@ __global__ __launch_bounds__(EN_THREADS) void mlp_ensemble_kernel(const Ensemble
     const long batch = a.batch, tiles = a.tiles;
     const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
 
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     // ---- the member's weights, once ----
     f32x4 w1v[2][KG];             // [feature tile][j]: W1[e][32 t + r][8 j + 4 g .. + 3]
-    {
+    if constexpr (ensemble_through_lds(KG)) {
+        ensemble_weights_to_lds(a.w1 + (long)e * EN_HIDDEN * K0, EN_HIDDEN, K0, a.per_piece, (unsigned)(size_t)lds, wave, lane);
+    } else {
         const float* w1 = a.w1 + (long)e * EN_HIDDEN * K0;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -101,12 +125,28 @@ __global__ __launch_bounds__(EN_THREADS) void mlp_ensemble_kernel(const Ensemble
 
     const long stride = (long)gridDim.x * 4;
     long tile = (long)blockIdx.x * 4 + wave;
-    if (tile >= tiles) return;
+    if constexpr (!ensemble_through_lds(KG)) {
+        if (tile >= tiles) return;
+    }
     f32x4 xv[KG];
     {
-        const float* xr = x_row(tile);
+        const float* xr = x_row(ensemble_through_lds(KG) && tile >= tiles ? 0 : tile);
 #pragma unroll
         for (int j = 0; j < KG; ++j) xv[j] = load_piece(xr, j);
+    }
+    if constexpr (ensemble_through_lds(KG)) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tile >= tiles) return;
+        const int pieces = K0 >> 2, swizzle = r & ensemble_swizzle(pieces);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int j = 0; j < KG; ++j) {
+                const int jj = EXACT || j < groups ? j : 0;
+                const f32x4 v = *reinterpret_cast<const f32x4*>(lds + ((32 * t + r) * pieces + ((2 * jj + g) ^ swizzle)) * 16);
+                w1v[t][j] = EXACT || j < groups ? v : zero4;
+            }
     }
     const HeadOut out = HeadOut{a.policy, ACTION ? a.action : nullptr, nullptr, a.head, N};
     const int limit = a.mask_size > 0 ? a.mask_size : NOUT;
@@ -572,8 +612,11 @@ __global__ __launch_bounds__(EN_THREADS) void ensemble_layer_kernel(const Ensemb
     const long batch = a.batch, tiles = a.tiles;
     const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
 
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     f32x4 wv[KG];                                            // W[e][r][8 j + 4 g .. + 3], rows past NOUT are zeros
-    {
+    if constexpr (ensemble_through_lds(KG)) {
+        ensemble_weights_to_lds(a.w1 + (long)e * N * K0, NOUT, K0, a.per_piece, (unsigned)(size_t)lds, wave, lane);
+    } else {
         const float* w = a.w1 + ((long)e * N + (r < NOUT ? r : 0)) * K0 + 4 * g;
 #pragma unroll
         for (int j = 0; j < KG; ++j) {
@@ -590,12 +633,26 @@ __global__ __launch_bounds__(EN_THREADS) void ensemble_layer_kernel(const Ensemb
 
     const long stride = (long)gridDim.x * 4;
     long tile = (long)blockIdx.x * 4 + wave;
-    if (tile >= tiles) return;
+    if constexpr (!ensemble_through_lds(KG)) {
+        if (tile >= tiles) return;
+    }
     f32x4 xv[KG];
     {
-        const float* xr = x_row(tile);
+        const float* xr = x_row(ensemble_through_lds(KG) && tile >= tiles ? 0 : tile);
 #pragma unroll
         for (int j = 0; j < KG; ++j) xv[j] = load_piece(xr, j);
+    }
+    if constexpr (ensemble_through_lds(KG)) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tile >= tiles) return;
+        const int pieces = K0 >> 2, row = r < NOUT ? r : 0, swizzle = row & ensemble_swizzle(pieces);
+#pragma unroll
+        for (int j = 0; j < KG; ++j) {
+            const int jj = EXACT || j < groups ? j : 0;
+            const f32x4 v = *reinterpret_cast<const f32x4*>(lds + (row * pieces + ((2 * jj + g) ^ swizzle)) * 16);
+            wv[j] = (EXACT || j < groups) && r < NOUT ? v : zero4;
+        }
     }
     const HeadOut out = HeadOut{a.policy, MODE == 1 ? a.action : nullptr, nullptr, a.head, N};
     const int limit = a.mask_size > 0 ? a.mask_size : NOUT;
@@ -734,8 +791,11 @@ static const void* pick_layer_kernel(int kg, bool exact) {
 
 static int ensemble_launch(const void* kernel, EnsembleArgs& a, hipStream_t stream, const char* what) {
     a.tiles = (a.batch + EN_ROWS - 1) / EN_ROWS;
+    const int pieces = a.k0 / 4, rows = a.w2 != nullptr ? EN_HIDDEN : a.nout;
+    a.per_piece = ((1u << 20) + (unsigned)pieces - 1u) / (unsigned)pieces;
+    const int lds_bytes = a.k0 > 32 ? (rows * pieces + 63) / 64 * 1024 : 0;
     void* args[] = {(void*)&a};
-    hipError_t err = hipLaunchKernel(kernel, dim3((unsigned)ensemble_blocks(a.members, a.tiles), (unsigned)a.members), dim3(EN_THREADS), args, 0, stream);
+    hipError_t err = hipLaunchKernel(kernel, dim3((unsigned)ensemble_blocks(a.members, a.tiles), (unsigned)a.members), dim3(EN_THREADS), args, lds_bytes, stream);
     if (err != hipSuccess) return fail(SP_ERR_DEVICE, "%s: launch failed: %s", what, hipGetErrorString(err));
     return check_launch(what);
 }

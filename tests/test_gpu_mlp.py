@@ -493,6 +493,38 @@ def test_ensemble_rejects_what_it_does_not_take(LY):
     assert err.value.code == -2
 
 
+@pytest.mark.parametrize("k0", [32, 40, 56, 64, 72, 104, 120, 128, 136, 248, 256])
+def test_ensemble_weights_of_every_row_length(LY, k0):
+    """The first layer's weights come through LDS, in pieces whose row follows from a multiplication: weights that are one
+    in one column (feature, or output, i in column 5 i + 3 mod k0) hand that column of the inputs on, exactly."""
+    announce("ensemble weights k0=%d" % k0)
+    members, batch = 3, 33
+    x = (torch.randn((batch, k0), generator=torch.Generator().manual_seed(k0)) + 0.25).cuda()
+
+    def one_each(rows, e):
+        w = torch.zeros((rows, k0))
+        col = (5 * torch.arange(rows) + 3 + 7 * e) % k0
+        w[torch.arange(rows), col] = 1
+        return w, col
+
+    picked = [one_each(32, e) for e in range(members)]
+    got = LY.ensemble_binarize(x, torch.stack([w for w, _ in picked]).cuda(), 1 << 31).cpu()
+    for e, (_, col) in enumerate(picked):
+        want = orow.binarize(x.cpu()[:, col].numpy(), 1 << 31)
+        assert (host(got[e]).view(np.uint32) == want).all(), e
+    if k0 > 128:
+        return                     # (two layers: up to 128 inputs)
+    picked = [one_each(64, e) for e in range(members)]
+    w2 = torch.zeros((members, 4, 64))
+    feature = torch.tensor([0, 21, 42, 63])
+    w2[:, torch.arange(4), feature] = 1
+    got = LY.mlp_forward_ensemble(x, (torch.stack([w for w, _ in picked]).cuda(), w2.cuda()), "regret_matching").cpu()
+    for e, (_, col) in enumerate(picked):
+        y = x.cpu()[:, col[feature]].clamp(min=0).numpy()
+        want, _, _ = olayers.mlp_forward(y, [np.eye(4, dtype=np.float32)], None, HEAD_CODE["regret_matching"], None, None, None)
+        assert np.abs(got[e].numpy() - want).max() < 1e-6, e     # (a sum of four, a division: a few ulp of at most one)
+
+
 @pytest.mark.parametrize("members,batch,k0,n,head,mask,sample", [
     (4, 6144, 128, 64, "regret_matching", 3, None),     # the reference's hold'em CEM policy: one layer, 3 valid of 64 columns
     (6, 1000, 256, 64, "softmax", 4, "u"),              # the widest input, a ragged last tile, sampling
