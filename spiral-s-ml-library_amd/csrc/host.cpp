@@ -14,6 +14,8 @@
 #include <dlfcn.h>
 
 #include <exception>
+#include <memory>
+#include <new>
 #include <tuple>
 #include <type_traits>
 #include <utility>
@@ -26,9 +28,10 @@ PyObject* g_calls = nullptr;      // lists of the tape being recorded: (function
 PyObject* g_keep = nullptr;
 PyObject* g_void_p = nullptr;     // ctypes.c_void_p
 PyObject* g_byref = nullptr;      // the type of ctypes.byref(...)
+PyObject* g_cdata = nullptr;      // what ctypes arrays and structures are instances of
 
 // ---- arguments: what the caller's objects become; false with an exception set if they do not fit ----
-constexpr Py_ssize_t MOST = 16;   // elements of a host array given as a list or tuple
+constexpr Py_ssize_t MOST = 16;   // elements of a host array given as a list or tuple that need no allocation
 
 bool as_integer(PyObject* o, unsigned long long& v) {      // as ctypes: the low bits of any integer
     if (PyLong_Check(o)) {
@@ -94,7 +97,9 @@ struct Arg<T*> {
     typedef std::remove_const_t<T> Element;
     static constexpr bool HOST_ARRAY = std::is_pointer_v<Element> || std::is_same_v<T, const int32_t>;
     T* value = nullptr;
-    std::conditional_t<HOST_ARRAY, Element, char> elements[HOST_ARRAY ? MOST : 1];
+    typedef std::conditional_t<HOST_ARRAY, Element, char> Stored;
+    Stored few[HOST_ARRAY ? MOST : 1];
+    std::unique_ptr<Stored[]> many;
     Py_buffer buffer{};
     Arg() = default;
     Arg(const Arg&) = delete;
@@ -110,9 +115,14 @@ struct Arg<T*> {
         if constexpr (HOST_ARRAY) {
             if (PyTuple_Check(o) || PyList_Check(o)) {
                 const Py_ssize_t n = PySequence_Fast_GET_SIZE(o);
+                Stored* elements = few;
                 if (n > MOST) {
-                    PyErr_Format(PyExc_ValueError, "at most %zd elements, got %zd", MOST, n);
-                    return false;
+                    many.reset(new (std::nothrow) Stored[n]);
+                    elements = many.get();
+                    if (elements == nullptr) {
+                        PyErr_NoMemory();
+                        return false;
+                    }
                 }
                 for (Py_ssize_t i = 0; i < n; ++i) {
                     PyObject* e = PySequence_Fast_GET_ITEM(o, i);
@@ -143,7 +153,13 @@ struct Arg<T*> {
             Py_DECREF(target);
             return ok;
         }
-        return take_buffer(o);                             // ctypes arrays and structures
+        const int is_cdata = PyObject_IsInstance(o, g_cdata);   // ctypes arrays and structures; no other buffer, as with ctypes
+        if (is_cdata < 0) return false;
+        if (is_cdata == 0) {
+            PyErr_Format(PyExc_TypeError, "an address is None, an integer or an object of ctypes, not %s", Py_TYPE(o)->tp_name);
+            return false;
+        }
+        return take_buffer(o);
     }
 };
 
@@ -222,6 +238,9 @@ PyObject* bind(PyObject*, PyObject* path) {
         if (ref != nullptr) {
             g_byref = (PyObject*)Py_TYPE(ref);
             Py_INCREF(g_byref);
+            PyObject* const mro = Py_TYPE(any)->tp_mro;             // c_int, _SimpleCData, _CData, object
+            g_cdata = PyTuple_GET_ITEM(mro, PyTuple_GET_SIZE(mro) - 2);
+            Py_INCREF(g_cdata);
         }
         Py_XDECREF(ref);
         Py_XDECREF(any);

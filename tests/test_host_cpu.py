@@ -2,6 +2,7 @@
 the library sees the same values as through ctypes.  No launch: every call is refused by the library's own checks."""
 import ctypes as C
 
+import numpy as np
 import pytest
 import torch
 
@@ -33,11 +34,14 @@ def test_structures_and_numbers():
     for given in (ph, C.byref(ph)):
         assert refused(L.lib.sp_row_sample, L.ROW_SOFTMAX, P, None, given, None, None, None, P, None, 8, 64, 0, None)[0] == -5
     assert refused(L.lib.sp_map_f32, 1, P, P, -(1 << 40), None)[0] == -2                 # 64 bits arrive whole
-    for wrong in ((1, P, P, 4), (1, P, P, 4.5, None), (1, P, P, "4", None), (1, "P", P, 4, None), (1, object(), P, 4, None)):
+    for wrong in ((1, P, P, 4), (1, P, P, 4.5, None), (1, P, P, "4", None), (1, "P", P, 4, None), (1, object(), P, 4, None),
+                  (1, bytearray(8), P, 4, None), (1, np.zeros(2), P, 4, None), (1, torch.zeros(2), P, 4, None)):
         with pytest.raises(TypeError):
             L.lib.sp_map_f32(*wrong)
-    with pytest.raises(ValueError):
-        L.lib.sp_mlp_forward(1, P, 2, [P] * 17, None, [32] * 3, None, None, P, None, None, 16, 1, 0, None)
+    for layers in (8, 16, 17, 40):                           # more than a stack may have
+        assert refused(L.lib.sp_mlp_forward, 1, P, layers, [P] * layers, None, [32] * layers + [65], None, None, P, None, None, 16, 1, 0, None) == refused(
+            L.lib._cdll.sp_mlp_forward, 1, P, layers, (C.c_void_p * layers)(*[P] * layers), None, (C.c_int32 * (layers + 1))(*[32] * layers, 65), None, None, P,
+            None, None, 16, 1, 0, None)
 
 
 def test_pointers_of_tensors():
