@@ -4,7 +4,7 @@
 // Two kernels, by how much work there is: up to 64 rows per compute unit the first, beyond that the second (beyond 128 where the weights
 // exceed the LDS).  bf16, us of a captured launch, first / second: 64-128-128-4 4096 rows 5.5 / 8.1, 16384 6.4 / 8.3, 65536 21 / 8.7;
 // 192-96-64-64 masked to 3, 10061 rows 7.1 / 11.3; 64-192-192-192-4 16384 rows 10.2 / 19, 65536 35 / 20.
-//   mlp_features_kernel: a workgroup of four waves takes R x 16 rows through the stack.  The waves share out a layer's tiles of 16
+//   mlp_features_kernel: a workgroup of eight or sixteen waves takes R x 16 rows through the stack.  The waves share out a layer's tiles of 16
 // output features; each streams the weights of its own features through a ring in LDS that nobody else reads, so weights need no
 // barrier, and the activations cross LDS between layers (one barrier a layer, two buffers).  The last layer and the head of row
 // tile w are wave w's.  Everything comes in by DMA: inputs, uniforms and as many weights as the ring holds are asked for in the

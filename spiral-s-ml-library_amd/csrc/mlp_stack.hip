@@ -19,7 +19,7 @@
 // the uniforms of four tiles in one go, one reciprocal per norm.  16-row tiles because a batch of 16384 rows is then one
 // tile per SIMD.
 // Measured, that stack over 16384 rows (node by node / every layer through part_product, a draw per tile / this kernel, us):
-// one model 32.8 / 13.8 / 10.3, 16 members 206 / 87 / 68.8 (the matrix pipe alone: 41).
+// one model 32.8 / 13.8 / 9.9, 16 members 206 / 87 / 68.8 (the matrix pipe alone: 41).
 //   Few rows: stack_features_kernel, below.
 //   PARTS: the same with the products in three bf16 parts (parts.h), 192 MFMAs of 16 cycles for 16 rows instead of 192 of 32, and
 // 400 vector instructions more, in part beside them: 16 members of 16384 rows 68 -> 56 us, of 57344 228 -> 190.  Bound by the
