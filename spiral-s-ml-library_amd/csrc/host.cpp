@@ -1,8 +1,8 @@
 // The host path of a call: device pointers of tensors and launches of the C-ABI library without ctypes.
 //
 // A small kernel takes 2 to 4 us, and with ctypes a call took 6.5 to 10 us of host: about 0.7 us for the checks and the address of each
-// tensor in Python, and 2 us to convert the arguments.  Both are done here, with the same checks and messages; bind() makes a function
-// of every entry point that launches work, from its own declaration in spiral_mi355.h.  (us a call with the queue kept full, ctypes
+// tensor in Python, and 2 us to convert the arguments.  Both are done here; bind() makes a function of every entry point that launches
+// work, from its own declaration in spiral_mi355.h, and an argument has to be of the declared type.  (us a call with the queue kept full, ctypes
 // / here: a four-layer stack on packed weights 7.2 / 5.6, one on row-major weights 11.4 / 7.1, the CEM update 76 / 63, a GEMM of 16 x 16 x 296
 // 7.6 / 5.4, a sampled softmax of 32 rows with its outputs allocated 11.7 / 8.7.)  What is left is the runtime's launch, about 4 us.
 #define PY_SSIZE_T_CLEAN
@@ -12,6 +12,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <dlfcn.h>
+#include <string.h>
 
 #include <exception>
 #include <memory>
@@ -26,9 +27,13 @@ namespace {
 
 PyObject* g_calls = nullptr;      // lists of the tape being recorded: (function, arguments but the stream), tensors
 PyObject* g_keep = nullptr;
-PyObject* g_void_p = nullptr;     // ctypes.c_void_p
-PyObject* g_byref = nullptr;      // the type of ctypes.byref(...)
-PyObject* g_cdata = nullptr;      // what ctypes arrays and structures are instances of
+PyObject* g_void_p = nullptr;     // of ctypes: c_void_p, c_int32, Array, _Pointer, cast, the type of byref(...)
+PyObject* g_int32 = nullptr;
+PyObject* g_array = nullptr;
+PyObject* g_pointer = nullptr;
+PyObject* g_cast = nullptr;
+PyObject* g_byref = nullptr;
+PyObject* g_philox = nullptr;     // the ctypes structure that stands for sp_philox_t
 
 // ---- arguments: what the caller's objects become; false with an exception set if they do not fit ----
 constexpr Py_ssize_t MOST = 16;   // elements of a host array given as a list or tuple that need no allocation
@@ -51,8 +56,8 @@ bool as_address(PyObject* o, void*& p) {                   // None, an integer o
         return true;
     }
     if (PyLong_Check(o)) {
-        p = PyLong_AsVoidPtr(o);
-        return !(p == nullptr && PyErr_Occurred());
+        p = (void*)PyLong_AsUnsignedLongLongMask(o);      // as ctypes: the low bits
+        return true;
     }
     const int is_void_p = PyObject_IsInstance(o, g_void_p);
     if (is_void_p < 0) return false;
@@ -67,11 +72,72 @@ bool as_address(PyObject* o, void*& p) {                   // None, an integer o
     return ok;
 }
 
-template <typename T, typename = void>
+// The buffer behind an object of ctypes.
+struct Buffer {
+    Py_buffer view{};
+    Buffer() = default;
+    Buffer(const Buffer&) = delete;
+    ~Buffer() {
+        if (view.obj != nullptr) PyBuffer_Release(&view);
+    }
+    bool take(PyObject* o) { return PyObject_GetBuffer(o, &view, PyBUF_SIMPLE) == 0; }
+};
+
+bool refuse(PyObject* o, const char* what) {
+    PyErr_Format(PyExc_TypeError, "%s, not %s", what, Py_TYPE(o)->tp_name);
+    return false;
+}
+
+// Whether `o` is a ctypes array of `element`, or a ctypes pointer to it (`base`: ctypes.Array, ctypes._Pointer); -1 with an exception.
+int is_of(PyObject* o, PyObject* base, PyObject* element) {
+    const int is_base = PyObject_IsInstance(o, base);
+    if (is_base <= 0) return is_base;
+    PyObject* type = PyObject_GetAttrString((PyObject*)Py_TYPE(o), "_type_");
+    if (type == nullptr) return -1;
+    Py_DECREF(type);
+    return type == element;
+}
+
+// The address that a ctypes pointer object holds.
+bool pointed_to(PyObject* o, void*& p) {
+    Buffer own;
+    if (!own.take(o)) return false;
+    p = *(void**)own.view.buf;
+    return true;
+}
+
+// byref(x): x, if it is an instance of `type` and the reference is to its start; nullptr with an exception if not.
+PyObject* referred(PyObject* o, PyObject* type, const char* what) {
+    PyObject* target = PyObject_GetAttrString(o, "_obj");
+    if (target == nullptr) return nullptr;
+    Buffer own;
+    PyObject* at = nullptr;
+    const bool fits = PyObject_TypeCheck(target, (PyTypeObject*)type) != 0;
+    if (fits && own.take(target)) {
+        PyObject* address = PyObject_CallFunctionObjArgs(g_cast, o, g_void_p, nullptr);
+        at = address != nullptr ? PyObject_GetAttrString(address, "value") : nullptr;
+        Py_XDECREF(address);
+    }
+    const bool start = at != nullptr && at != Py_None && PyLong_AsVoidPtr(at) == own.view.buf;
+    Py_XDECREF(at);
+    if (!start) {
+        if (!PyErr_Occurred()) {
+            if (fits) PyErr_Format(PyExc_TypeError, "%s, not a reference with an offset", what);
+            else PyErr_Format(PyExc_TypeError, "%s, not a reference to %s", what, Py_TYPE(target)->tp_name);
+        }
+        Py_DECREF(target);
+        return nullptr;
+    }
+    return target;
+}
+
+// HOST_INTS: of an entry point whose const int32_t* are host arrays.  Those that take arrays of addresses take the widths of a stack
+// beside them; everywhere else a const int32_t* is device memory.
+template <typename T, bool HOST_INTS, typename = void>
 struct Arg;
 
-template <typename T>
-struct Arg<T, std::enable_if_t<std::is_integral_v<T>>> {
+template <typename T, bool HOST_INTS>
+struct Arg<T, HOST_INTS, std::enable_if_t<std::is_integral_v<T>>> {
     T value = 0;
     bool load(PyObject* o) {
         unsigned long long v = 0;
@@ -81,8 +147,8 @@ struct Arg<T, std::enable_if_t<std::is_integral_v<T>>> {
     }
 };
 
-template <typename T>
-struct Arg<T, std::enable_if_t<std::is_floating_point_v<T>>> {
+template <typename T, bool HOST_INTS>
+struct Arg<T, HOST_INTS, std::enable_if_t<std::is_floating_point_v<T>>> {
     T value = 0;
     bool load(PyObject* o) {
         const double v = PyFloat_AsDouble(o);
@@ -92,74 +158,124 @@ struct Arg<T, std::enable_if_t<std::is_floating_point_v<T>>> {
     }
 };
 
-template <typename T>
-struct Arg<T*> {
-    typedef std::remove_const_t<T> Element;
-    static constexpr bool HOST_ARRAY = std::is_pointer_v<Element> || std::is_same_v<T, const int32_t>;
+// Device memory: an address, or a ctypes pointer that holds one.
+template <typename T, bool HOST_INTS>
+struct Arg<T*, HOST_INTS, std::enable_if_t<!std::is_pointer_v<std::remove_const_t<T>> && !std::is_same_v<T, const sp_philox_t> &&
+                                           !(HOST_INTS && std::is_same_v<T, const int32_t>)>> {
     T* value = nullptr;
-    typedef std::conditional_t<HOST_ARRAY, Element, char> Stored;
-    Stored few[HOST_ARRAY ? MOST : 1];
-    std::unique_ptr<Stored[]> many;
-    Py_buffer buffer{};
-    Arg() = default;
-    Arg(const Arg&) = delete;
-    ~Arg() {
-        if (buffer.obj != nullptr) PyBuffer_Release(&buffer);
+    bool load(PyObject* o) {
+        void* p = nullptr;
+        if (o != Py_None && !PyLong_Check(o)) {
+            const int is_pointer = PyObject_IsInstance(o, g_pointer);
+            if (is_pointer < 0 || (is_pointer > 0 ? !pointed_to(o, p) : !as_address(o, p))) return false;
+        } else if (!as_address(o, p)) {
+            return false;
+        }
+        value = (T*)p;
+        return true;
     }
-    bool take_buffer(PyObject* o) {
-        if (PyObject_GetBuffer(o, &buffer, PyBUF_SIMPLE) != 0) return false;
-        value = (T*)buffer.buf;
+};
+
+// A host array of addresses or of 32-bit integers: a list, a tuple, or of ctypes an array of such elements, one of them by reference or a
+// pointer to them.  Elements are copied, zeros behind them, so that what reads further than was given -- a stack has eight layers at
+// most -- finds zeros; only longer arrays, and what a pointer points to, are read in place.
+template <typename T, bool HOST_INTS>
+struct Arg<T*, HOST_INTS, std::enable_if_t<std::is_pointer_v<std::remove_const_t<T>> || (HOST_INTS && std::is_same_v<T, const int32_t>)>> {
+    typedef std::remove_const_t<T> Element;
+    static constexpr bool ADDRESSES = std::is_pointer_v<Element>;
+    T* value = nullptr;
+    Element few[MOST] = {};
+    std::unique_ptr<Element[]> many;
+    Buffer buffer;
+
+    bool list(PyObject* o) {
+        const Py_ssize_t n = PySequence_Fast_GET_SIZE(o);
+        Element* elements = few;
+        if (n > MOST) {
+            many.reset(new (std::nothrow) Element[n]);
+            elements = many.get();
+            if (elements == nullptr) {
+                PyErr_NoMemory();
+                return false;
+            }
+        }
+        for (Py_ssize_t i = 0; i < n; ++i) {
+            PyObject* e = PySequence_Fast_GET_ITEM(o, i);
+            if constexpr (ADDRESSES) {
+                void* p = nullptr;
+                if (!as_address(e, p)) return false;
+                elements[i] = (Element)p;
+            } else {
+                unsigned long long v = 0;
+                if (!as_integer(e, v)) return false;
+                elements[i] = (Element)v;
+            }
+        }
+        value = elements;
+        return true;
+    }
+    bool memory(PyObject* o) {                             // of an array, or of one element
+        if (!buffer.take(o)) return false;
+        const size_t n = (size_t)buffer.view.len / sizeof(Element);
+        if (n <= (size_t)MOST) memcpy(few, buffer.view.buf, n * sizeof(Element));
+        value = n <= (size_t)MOST ? few : (T*)buffer.view.buf;
         return true;
     }
     bool load(PyObject* o) {
-        if constexpr (HOST_ARRAY) {
-            if (PyTuple_Check(o) || PyList_Check(o)) {
-                const Py_ssize_t n = PySequence_Fast_GET_SIZE(o);
-                Stored* elements = few;
-                if (n > MOST) {
-                    many.reset(new (std::nothrow) Stored[n]);
-                    elements = many.get();
-                    if (elements == nullptr) {
-                        PyErr_NoMemory();
-                        return false;
-                    }
-                }
-                for (Py_ssize_t i = 0; i < n; ++i) {
-                    PyObject* e = PySequence_Fast_GET_ITEM(o, i);
-                    if constexpr (std::is_pointer_v<Element>) {
-                        void* p = nullptr;
-                        if (!as_address(e, p)) return false;
-                        elements[i] = (Element)p;
-                    } else {
-                        unsigned long long v = 0;
-                        if (!as_integer(e, v)) return false;
-                        elements[i] = (Element)v;
-                    }
-                }
-                value = elements;
-                return true;
-            }
-        }
-        if (o == Py_None || PyLong_Check(o) || PyObject_IsInstance(o, g_void_p) == 1) {
+        if (PyTuple_Check(o) || PyList_Check(o)) return list(o);
+        if (o == Py_None) return true;
+        PyObject* const type = ADDRESSES ? g_void_p : g_int32;
+        const char* const what = ADDRESSES ? "an array of addresses is None, a list, a tuple or of c_void_p" : "an array of integers is None, a list, a tuple or of c_int32";
+        const int is_array = is_of(o, g_array, type);
+        if (is_array != 0) return is_array > 0 && memory(o);
+        const int is_pointer = is_of(o, g_pointer, type);
+        if (is_pointer != 0) {
             void* p = nullptr;
-            if (!as_address(o, p)) return false;
+            if (is_pointer < 0 || !pointed_to(o, p)) return false;
             value = (T*)p;
             return true;
         }
-        if ((PyObject*)Py_TYPE(o) == g_byref) {            // byref(x): the memory of x (no offset is given anywhere here)
-            PyObject* target = PyObject_GetAttrString(o, "_obj");
+        if ((PyObject*)Py_TYPE(o) == g_byref) {
+            PyObject* target = referred(o, type, what);
             if (target == nullptr) return false;
-            const bool ok = take_buffer(target);
+            const bool ok = memory(target);
             Py_DECREF(target);
             return ok;
         }
-        const int is_cdata = PyObject_IsInstance(o, g_cdata);   // ctypes arrays and structures; no other buffer, as with ctypes
-        if (is_cdata < 0) return false;
-        if (is_cdata == 0) {
-            PyErr_Format(PyExc_TypeError, "an address is None, an integer or an object of ctypes, not %s", Py_TYPE(o)->tp_name);
-            return false;
+        return refuse(o, what);
+    }
+};
+
+// The state of a random stream, a host structure: the structure, a reference or a ctypes pointer to it, or an array of them.
+template <bool HOST_INTS>
+struct Arg<const sp_philox_t*, HOST_INTS> {
+    const sp_philox_t* value = nullptr;
+    Buffer buffer;
+    bool memory(PyObject* o) {
+        if (!buffer.take(o)) return false;
+        if ((size_t)buffer.view.len < sizeof(sp_philox_t)) return refuse(o, "a random stream needs a whole PhiloxConfig");
+        value = (const sp_philox_t*)buffer.view.buf;
+        return true;
+    }
+    bool load(PyObject* o) {
+        if (o == Py_None) return true;
+        if (PyObject_TypeCheck(o, (PyTypeObject*)g_philox)) return memory(o);
+        const char* const what = "a random stream is None or a PhiloxConfig";
+        if ((PyObject*)Py_TYPE(o) == g_byref) {
+            PyObject* target = referred(o, g_philox, what);
+            if (target == nullptr) return false;
+            const bool ok = memory(target);
+            Py_DECREF(target);
+            return ok;
         }
-        return take_buffer(o);
+        const int is_array = is_of(o, g_array, g_philox);
+        if (is_array != 0) return is_array > 0 && memory(o);
+        const int is_pointer = is_of(o, g_pointer, g_philox);
+        if (is_pointer == 0) return refuse(o, what);
+        void* p = nullptr;
+        if (is_pointer < 0 || !pointed_to(o, p)) return false;
+        value = (const sp_philox_t*)p;
+        return true;
     }
 };
 
@@ -168,13 +284,14 @@ template <int ID, typename F>
 struct Entry;
 template <int ID, typename... A>
 struct Entry<ID, int(A...)> {
+    static constexpr bool HOST_INTS = ((std::is_pointer_v<A> && std::is_pointer_v<std::remove_const_t<std::remove_pointer_t<A>>>) || ...);
     static inline int (*fn)(A...) = nullptr;
     static inline PyObject* self = nullptr;
     static inline const char* name = nullptr;
 
     template <size_t... I>
     static PyObject* run(PyObject* const* given, std::index_sequence<I...>) {
-        std::tuple<Arg<A>...> args;
+        std::tuple<Arg<A, HOST_INTS>...> args;
         if (!(std::get<I>(args).load(given[I]) && ...)) return nullptr;
         int rc = 0;
         Py_BEGIN_ALLOW_THREADS
@@ -225,28 +342,27 @@ bool bind_one(void* library, PyObject* functions, const char* name, PyMethodDef&
     return PyDict_SetItemString(functions, name, E::self) == 0;
 }
 
-// bind(path): a dict of the functions behind the library at `path`, which the process keeps (one library per process).
-PyObject* bind(PyObject*, PyObject* path) {
-    const char* p = PyUnicode_AsUTF8(path);
+// bind(path, stream): a dict of the functions behind the library at `path`, which the process keeps (one library per process); `stream`: the
+// ctypes structure that stands for sp_philox_t.
+PyObject* bind(PyObject*, PyObject* const* given, Py_ssize_t n) {
+    if (n != 2 || !PyType_Check(given[1])) return PyErr_Format(PyExc_TypeError, "bind takes a path and a structure type");
+    const char* p = PyUnicode_AsUTF8(given[0]);
     if (p == nullptr) return nullptr;
     PyObject* ctypes = PyImport_ImportModule("ctypes");
     if (ctypes == nullptr) return nullptr;
-    if (g_void_p == nullptr) g_void_p = PyObject_GetAttrString(ctypes, "c_void_p");
-    if (g_void_p != nullptr && g_byref == nullptr) {
+    auto get = [&](PyObject*& to, const char* name) { return to != nullptr || (to = PyObject_GetAttrString(ctypes, name)) != nullptr; };
+    bool found = get(g_void_p, "c_void_p") && get(g_int32, "c_int32") && get(g_array, "Array") && get(g_pointer, "_Pointer") && get(g_cast, "cast");
+    if (found && g_byref == nullptr) {
         PyObject* any = PyObject_CallMethod(ctypes, "c_int", nullptr);
         PyObject* ref = any != nullptr ? PyObject_CallMethod(ctypes, "byref", "O", any) : nullptr;
-        if (ref != nullptr) {
-            g_byref = (PyObject*)Py_TYPE(ref);
-            Py_INCREF(g_byref);
-            PyObject* const mro = Py_TYPE(any)->tp_mro;             // c_int, _SimpleCData, _CData, object
-            g_cdata = PyTuple_GET_ITEM(mro, PyTuple_GET_SIZE(mro) - 2);
-            Py_INCREF(g_cdata);
-        }
+        if (ref != nullptr) g_byref = Py_NewRef((PyObject*)Py_TYPE(ref));
         Py_XDECREF(ref);
         Py_XDECREF(any);
+        found = g_byref != nullptr;
     }
     Py_DECREF(ctypes);
-    if (g_void_p == nullptr || g_byref == nullptr) return nullptr;
+    if (!found) return nullptr;
+    Py_XSETREF(g_philox, Py_NewRef(given[1]));
     void* library = dlopen(p, RTLD_NOW | RTLD_LOCAL);
     if (library == nullptr) return PyErr_Format(PyExc_RuntimeError, "%s", dlerror());
     PyObject* functions = PyDict_New();
@@ -325,7 +441,7 @@ PyObject* tape(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Py_RETURN_NONE;
 }
 
-PyMethodDef methods[] = {{"bind", bind, METH_O, nullptr},
+PyMethodDef methods[] = {{"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, nullptr},
                          {"ptr", (PyCFunction)(void (*)(void))ptr, METH_FASTCALL | METH_KEYWORDS, nullptr},
                          {"tape", (PyCFunction)(void (*)(void))tape, METH_FASTCALL, nullptr},
                          {nullptr, nullptr, 0, nullptr}};

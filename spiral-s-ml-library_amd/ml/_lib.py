@@ -158,7 +158,7 @@ class _Library:
 
     def __init__(self, path):
         self._cdll = load(path)
-        self.__dict__.update(_host.bind(path))
+        self.__dict__.update(_host.bind(path, PhiloxConfig))
 
     def __getattr__(self, name):
         fn = getattr(self._cdll, name)

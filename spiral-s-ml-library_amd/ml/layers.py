@@ -150,7 +150,7 @@ def mlp_forward_ensemble(x, weights, head="regret_matching", u=None, mask_size=0
     wp = (C.c_void_p * n)(*[ptr(w, name="weights[%d]" % i) for i, w in enumerate(weights)])
     dp = (C.c_int32 * (n + 1))(*dims)
     check(lib.sp_mlp_forward_ensemble(_lib.SP_F32, ptr(x, name="x"), n, wp, dp, members, ptr(u, torch.float32, "u"),
-                                      C.byref(rng) if rng is not None else None, ptr(policy, torch.float32, "policy_out"),
+                                      rng, ptr(policy, torch.float32, "policy_out"),
                                       ptr(action, torch.int32, "action_out"), batch, HEADS[head], mask_size, stream_ptr()))
     return (policy, action) if action is not None else policy
 
@@ -752,7 +752,7 @@ def _build_fused_run(model, plan, ls, static_weights=False):
     dp = (C.c_int32 * (n + 1))(*dims)
     # The head draws its uniforms inside the kernel, from the stream a run of the reference starts at its seed
     # (ml/layers.spi:339-344): no uniform tensor, no launch of its own, nothing carried over from run to run.
-    args = (_lib.DTYPES[x.dtype], ptr(x, name="x"), n, wp, None, dp, None, C.byref(rng),
+    args = (_lib.DTYPES[x.dtype], ptr(x, name="x"), n, wp, None, dp, None, rng,
             ptr(policy, torch.float32, "policy_out"), ptr(act, torch.int32, "action_out"), None, x.shape[0], HEADS[head],
             top.size)
     keep = (x, ws, probs, action, rng, policy, act)   # the views stay alive as long as the closure does
@@ -1072,7 +1072,7 @@ def _run_fused_stack(model, key, count, ls):
         ls.draws += draws
     check(lib.sp_stack_forward_f32(
         ptr(x, name="x"), n, (C.c_void_p * n)(*[ptr(t, name="weights[%d]" % i) for i, t in enumerate(ws)]), dims_c,
-        (C.c_int32 * n)(*acts), count, None, C.byref(rng) if rng is not None else None,
+        (C.c_int32 * n)(*acts), count, None, rng,
         ptr(outs[0], name="policy"), ptr(outs[1], name="action") if len(outs) == 2 else None, q * w, head_op, mask,
         stream_ptr()))
     if key is None:

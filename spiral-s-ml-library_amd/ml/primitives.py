@@ -138,7 +138,7 @@ def philox_uniforms(rng, rows, cols, out=None):
     """The uniform each of `rows` rows of width `cols` would draw from the reference's device stream `rng`."""
     if out is None:
         out = torch.empty((rows,), dtype=torch.float32, device="cuda")
-    check(lib.sp_philox_uniforms(C.byref(rng), ptr(out, torch.float32, "out"), rows, cols, stream_ptr()))
+    check(lib.sp_philox_uniforms(rng, ptr(out, torch.float32, "out"), rows, cols, stream_ptr()))
     return out
 
 

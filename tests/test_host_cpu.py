@@ -54,3 +54,85 @@ def test_pointers_of_tensors():
         torch.func.vmap(lambda t: L.ptr(t) or t)(torch.zeros(2, 3))
     with pytest.raises(TypeError):
         L.ptr()
+
+
+def bad_stream():
+    return L.PhiloxConfig(1, 0, 17, 256, 24, 0, 0, 0)        # no such mode: looked at behind widths and weights
+
+
+def stack(dims=(32, 64, 4), w=(P, P), rng=None, fn=None, biases=None, x=P):
+    """Status and message of a two-layer stack that the library's checks refuse at its random stream, if at nothing before."""
+    stream = bad_stream() if rng is None else rng
+    return refused(fn or L.lib.sp_mlp_forward, 1, x, 2, w, biases, dims, None, stream, P, P, None, 16, 1, 0, None)
+
+
+AT_THE_STREAM = (-5, "philox mode")
+
+
+def reaches(result, expected):
+    return result[0] == expected[0] and expected[1] in result[1]
+
+
+def test_elements_of_lists_arrive_as_addresses():
+    arrays = lambda *v: (C.c_void_p * len(v))(*v)
+    for make in (list, tuple, lambda v: arrays(*v)):
+        assert reaches(stack(w=make((P, P + 16))), AT_THE_STREAM)
+        assert reaches(stack(w=make((P, None))), (-1, "weights[1] is NULL"))
+        assert reaches(stack(w=make((P + 4, P))), (-3, "weights[0] is not 16-byte aligned"))
+        assert reaches(stack(w=make((P, P + 4))), (-3, "weights[1] is not 16-byte aligned"))
+        assert reaches(stack(w=make((P,))), (-1, "weights[1] is NULL"))                   # too short: nothing behind the last
+    for dims in ([32, 64], (32, 64), (C.c_int32 * 2)(32, 64)):
+        assert reaches(stack(dims=dims), (-2, "dims[2] must be positive"))
+    assert reaches(stack(w=[C.c_void_p(P), P], dims=(C.c_int32 * 40)(32, 64, 4)), AT_THE_STREAM)
+
+
+def test_pointers_of_ctypes_mean_what_they_point_to():
+    three, two, stream = (C.c_int32 * 3)(32, 64, 4), (C.c_void_p * 2)(P, P + 4), bad_stream()
+    for fn in (L.lib.sp_mlp_forward, L.lib._cdll.sp_mlp_forward):
+        ok = dict(fn=fn, dims=three, w=(C.c_void_p * 2)(P, P))
+        assert reaches(stack(**dict(ok, dims=C.cast(three, C.POINTER(C.c_int32)))), AT_THE_STREAM)
+        assert reaches(stack(**dict(ok, dims=C.POINTER(C.c_int32)())), (-1, "weights/dims is NULL"))
+        assert reaches(stack(**dict(ok, w=C.cast(two, C.POINTER(C.c_void_p)))), (-3, "weights[1]"))
+        assert reaches(stack(**dict(ok, rng=C.pointer(stream))), AT_THE_STREAM)
+        assert reaches(stack(**dict(ok, rng=C.byref(stream))), AT_THE_STREAM)
+        assert reaches(stack(**dict(ok, rng=stream)), AT_THE_STREAM)
+        assert reaches(stack(**dict(ok, rng=(L.PhiloxConfig * 2)(stream, stream))), AT_THE_STREAM)
+        assert reaches(stack(**dict(ok, x=C.cast(P + 8, C.POINTER(C.c_float)))), (-3, "x is not 16-byte aligned"))
+
+
+WRONG = (TypeError, C.ArgumentError)
+
+
+@pytest.mark.parametrize("rng", [1234, 0, C.c_void_p(P), C.c_int(5), C.byref(C.c_int(5)), C.pointer(C.c_int(5)), (C.c_int32 * 64)(), (1, 2), "seed",
+                                 L.DeviceInfo(), C.byref(bad_stream(), 8), (L.PhiloxConfig * 0)(), np.zeros(64), torch.zeros(64)])
+def test_a_random_stream_is_a_structure_of_its_type(rng):
+    """A seed given for the stream was read as the address of one."""
+    with pytest.raises(WRONG):
+        stack(rng=rng)
+    with pytest.raises(WRONG):
+        L.lib.sp_philox_uniforms(rng, P, 8, 8, None)
+
+
+@pytest.mark.parametrize("dims", [1234, C.c_void_p(P), (C.c_float * 3)(32, 64, 4), (C.c_int64 * 3)(32, 64, 4), (C.c_void_p * 3)(32, 64, 4), C.c_int64(5),
+                                  C.byref(C.c_float(1)), C.pointer(C.c_int64(5)), C.byref((C.c_int32 * 3)(32, 64, 4)), C.byref(C.c_int32(32), 4),
+                                  bad_stream(), np.zeros(3, np.int32), torch.zeros(3, dtype=torch.int32), [32.0, 64, 4], b"abcdefghijkl"])
+def test_widths_are_integers_of_32_bits(dims):
+    with pytest.raises(WRONG):
+        stack(dims=dims)
+
+
+@pytest.mark.parametrize("w", [P, C.c_void_p(P), (C.c_int64 * 2)(P, P), (C.c_int32 * 4)(), C.byref((C.c_void_p * 2)(P, P)), C.pointer(C.c_int64(P)),
+                               bad_stream(), np.zeros(2, np.int64), [P, 0.5], ["P", P], [(C.c_int32 * 4)(), P]])
+def test_weights_are_an_array_of_addresses(w):
+    with pytest.raises(WRONG):
+        stack(w=w)
+
+
+@pytest.mark.parametrize("x", [C.c_int(5), C.c_float(5), C.byref(C.c_int(5)), (C.c_float * 4)(), bad_stream(), [P], 1.5, np.zeros(4)])
+def test_device_memory_is_an_address(x):
+    """The memory of an object of the host is none that a kernel may read; nor is a list, for a const int32_t* of the device."""
+    with pytest.raises(WRONG):
+        stack(x=x)
+    with pytest.raises(WRONG):
+        L.lib.sp_row_map_i32(6, x, P, 8, 8, None)
+    assert refused(L.lib.sp_row_map_i32, 6, P + 4, P, 8, 8, None)[0] == -3
