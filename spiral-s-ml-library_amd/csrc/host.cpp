@@ -393,13 +393,13 @@ PyObject* ptr(PyObject*, PyObject* const* args, Py_ssize_t n, PyObject* keywords
         if (PyUnicode_CompareWithASCIIString(key, "name") == 0) name = args[n + i];
         else if (PyUnicode_CompareWithASCIIString(key, "dtype") == 0) dtype = args[n + i];
         else if (PyUnicode_CompareWithASCIIString(key, "t") == 0) t = args[n + i];
-        else return PyErr_Format(PyExc_TypeError, "ptr has no argument %U", key);
+        else return PyErr_Format(PyExc_TypeError, "ptr has no argument %S", key);
     }
     if (t == nullptr) return PyErr_Format(PyExc_TypeError, "ptr needs a tensor");
     if (t == Py_None) Py_RETURN_NONE;
     PyObject* const named = name;
     auto raise = [&](PyObject* type, const char* text) -> PyObject* {
-        if (named != nullptr) return PyErr_Format(type, "%U %s", named, text);
+        if (named != nullptr) return PyErr_Format(type, "%S %s", named, text);
         return PyErr_Format(type, "tensor %s", text);
     };
     try {
@@ -412,7 +412,7 @@ PyObject* ptr(PyObject*, PyObject* const* args, Py_ssize_t n, PyObject* keywords
             if (((THPDtype*)dtype)->scalar_type != x.scalar_type()) {
                 PyObject* got = PyObject_GetAttrString(t, "dtype");
                 if (got == nullptr) return nullptr;
-                if (named != nullptr) PyErr_Format(PyExc_TypeError, "%U must have dtype %S, got %S", named, dtype, got);
+                if (named != nullptr) PyErr_Format(PyExc_TypeError, "%S must have dtype %S, got %S", named, dtype, got);
                 else PyErr_Format(PyExc_TypeError, "tensor must have dtype %S, got %S", dtype, got);
                 Py_DECREF(got);
                 return nullptr;

@@ -136,3 +136,13 @@ def test_device_memory_is_an_address(x):
     with pytest.raises(WRONG):
         L.lib.sp_row_map_i32(6, x, P, 8, 8, None)
     assert refused(L.lib.sp_row_map_i32, 6, P + 4, P, 8, 8, None)[0] == -3
+
+
+@pytest.mark.parametrize("name", [None, 5, ("a", "b"), b"x"])
+def test_names_of_pointers_are_any_object(name):
+    for make in (lambda: L.ptr(3, None, name), lambda: L.ptr(3, name=name)):
+        with pytest.raises(TypeError) as err:
+            make()
+        assert str(err.value) == str(name) + " must be a torch.Tensor"
+    with pytest.raises(ValueError, match="must live on the GPU"):
+        L.ptr(torch.zeros(3), None, name)
