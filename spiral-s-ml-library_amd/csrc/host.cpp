@@ -131,6 +131,23 @@ PyObject* referred(PyObject* o, PyObject* type, const char* what) {
     return target;
 }
 
+// Scalars may come as objects of ctypes, of the parameter's own type.
+PyObject* g_scalars[5] = {};      // c_int32, c_int64, c_uint32, c_uint64, c_float
+const char* const SCALARS[5] = {"c_int32", "c_int64", "c_uint32", "c_uint64", "c_float"};
+template <typename T>
+PyObject* scalar_type() {
+    return g_scalars[std::is_floating_point_v<T> ? 4 : 2 * std::is_unsigned_v<T> + (sizeof(T) == 8)];
+}
+template <typename Take>
+bool unwrapped(PyObject* o, PyObject* type, const Take& take) {
+    if (!PyObject_TypeCheck(o, (PyTypeObject*)type)) return take(o);
+    PyObject* v = PyObject_GetAttrString(o, "value");
+    if (v == nullptr) return false;
+    const bool ok = take(v);
+    Py_DECREF(v);
+    return ok;
+}
+
 // HOST_INTS: of an entry point whose const int32_t* are host arrays.  Those that take arrays of addresses take the widths of a stack
 // beside them; everywhere else a const int32_t* is device memory.
 template <typename T, bool HOST_INTS, typename = void>
@@ -141,7 +158,7 @@ struct Arg<T, HOST_INTS, std::enable_if_t<std::is_integral_v<T>>> {
     T value = 0;
     bool load(PyObject* o) {
         unsigned long long v = 0;
-        if (!as_integer(o, v)) return false;
+        if (PyLong_Check(o) ? !as_integer(o, v) : !unwrapped(o, scalar_type<T>(), [&](PyObject* x) { return as_integer(x, v); })) return false;
         value = (T)v;
         return true;
     }
@@ -151,8 +168,12 @@ template <typename T, bool HOST_INTS>
 struct Arg<T, HOST_INTS, std::enable_if_t<std::is_floating_point_v<T>>> {
     T value = 0;
     bool load(PyObject* o) {
-        const double v = PyFloat_AsDouble(o);
-        if (v == -1.0 && PyErr_Occurred()) return false;
+        double v = 0;
+        auto number = [&](PyObject* x) {
+            v = PyFloat_AsDouble(x);
+            return !(v == -1.0 && PyErr_Occurred());
+        };
+        if (PyFloat_Check(o) ? !number(o) : !unwrapped(o, scalar_type<T>(), number)) return false;
         value = (T)v;
         return true;
     }
@@ -352,6 +373,7 @@ PyObject* bind(PyObject*, PyObject* const* given, Py_ssize_t n) {
     if (ctypes == nullptr) return nullptr;
     auto get = [&](PyObject*& to, const char* name) { return to != nullptr || (to = PyObject_GetAttrString(ctypes, name)) != nullptr; };
     bool found = get(g_void_p, "c_void_p") && get(g_int32, "c_int32") && get(g_array, "Array") && get(g_pointer, "_Pointer") && get(g_cast, "cast");
+    for (int i = 0; i < 5; ++i) found = found && get(g_scalars[i], SCALARS[i]);
     if (found && g_byref == nullptr) {
         PyObject* any = PyObject_CallMethod(ctypes, "c_int", nullptr);
         PyObject* ref = any != nullptr ? PyObject_CallMethod(ctypes, "byref", "O", any) : nullptr;

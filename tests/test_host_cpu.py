@@ -146,3 +146,22 @@ def test_names_of_pointers_are_any_object(name):
         assert str(err.value) == str(name) + " must be a torch.Tensor"
     with pytest.raises(ValueError, match="must live on the GPU"):
         L.ptr(torch.zeros(3), None, name)
+
+
+def test_scalars_may_be_of_ctypes():
+    """Of the parameter's own type, as through ctypes; every call is refused at a size or a misaligned address."""
+    for fn in (L.lib.sp_map_f32, L.lib._cdll.sp_map_f32):
+        assert refused(fn, C.c_int(1), P, P, C.c_int64(-(1 << 40)), None)[0] == -2
+        for wrong in ((C.c_int64(1), P, P, 4, None), (1, P, P, C.c_int32(4), None), (1, P, P, C.c_float(4), None)):
+            with pytest.raises(WRONG):
+                fn(*wrong)
+    for fn in (L.lib.sp_row_l1_normalize, L.lib._cdll.sp_row_l1_normalize):
+        got = [refused(fn, P + 4, P, 8, 8, t, None) for t in (C.c_float(0.5), 0.5, 1, True)]
+        assert got[0][0] == -3 and all(g == got[0] for g in got)
+        for wrong in (C.c_double(0.5), C.c_int(1), "1"):
+            with pytest.raises(WRONG):
+                fn(P + 4, P, 8, 8, wrong, None)
+    for fn in (L.lib.sp_row_binarize, L.lib._cdll.sp_row_binarize):
+        assert refused(fn, P, P, 8, 8, C.c_uint32(0), None)[0] == -5
+    for fn in (L.lib.sp_cem_resample_philox, L.lib._cdll.sp_cem_resample_philox):
+        assert refused(fn, P, P, C.c_uint64(1), C.c_uint64(2), P, 0, 8, 0.5, 0.5, None)[0] == -2
