@@ -300,6 +300,18 @@ struct Arg<const sp_philox_t*, HOST_INTS> {
     }
 };
 
+// What does not fit is reported as ctypes reports it; as a TypeError, too.
+PyObject* g_argument_error = nullptr;
+void refuse_argument(int number) {
+    if (!PyErr_ExceptionMatches(PyExc_TypeError)) return;
+    PyObject *type, *text, *trace;
+    PyErr_Fetch(&type, &text, &trace);
+    PyErr_Format(g_argument_error, "argument %d: %S", number, text != nullptr ? text : Py_None);
+    Py_XDECREF(type);
+    Py_XDECREF(text);
+    Py_XDECREF(trace);
+}
+
 // ---- one function per entry point ----
 template <int ID, typename F>
 struct Entry;
@@ -313,7 +325,10 @@ struct Entry<ID, int(A...)> {
     template <size_t... I>
     static PyObject* run(PyObject* const* given, std::index_sequence<I...>) {
         std::tuple<Arg<A, HOST_INTS>...> args;
-        if (!(std::get<I>(args).load(given[I]) && ...)) return nullptr;
+        if (int at = 0; !((++at, std::get<I>(args).load(given[I])) && ...)) {
+            refuse_argument(at);
+            return nullptr;
+        }
         int rc = 0;
         Py_BEGIN_ALLOW_THREADS
         rc = fn(std::get<I>(args).value...);
@@ -381,6 +396,14 @@ PyObject* bind(PyObject*, PyObject* const* given, Py_ssize_t n) {
         Py_XDECREF(ref);
         Py_XDECREF(any);
         found = g_byref != nullptr;
+    }
+    if (found && g_argument_error == nullptr) {
+        PyObject* of_ctypes = PyObject_GetAttrString(ctypes, "ArgumentError");
+        PyObject* bases = of_ctypes != nullptr ? PyTuple_Pack(2, of_ctypes, PyExc_TypeError) : nullptr;
+        g_argument_error = bases != nullptr ? PyErr_NewException("spiral_host.ArgumentError", bases, nullptr) : nullptr;
+        Py_XDECREF(bases);
+        Py_XDECREF(of_ctypes);
+        found = g_argument_error != nullptr;
     }
     Py_DECREF(ctypes);
     if (!found) return nullptr;

@@ -165,3 +165,15 @@ def test_scalars_may_be_of_ctypes():
         assert refused(fn, P, P, 8, 8, C.c_uint32(0), None)[0] == -5
     for fn in (L.lib.sp_cem_resample_philox, L.lib._cdll.sp_cem_resample_philox):
         assert refused(fn, P, P, C.c_uint64(1), C.c_uint64(2), P, 0, 8, 0.5, 0.5, None)[0] == -2
+
+
+def test_refused_arguments_raise_what_ctypes_raises():
+    for args, number in (((1, "P", P, 4, None), None), ((1, P, object(), 4, None), 3), ((1, P, P, 4.5, None), 4), ((C.c_float(1), P, P, 4, None), 1)):
+        with pytest.raises(C.ArgumentError) as err:
+            L.lib.sp_map_f32(*args)
+        assert isinstance(err.value, TypeError) and (number is None or str(err.value).startswith("argument %d: " % number))
+        if number is not None:
+            with pytest.raises(C.ArgumentError, match="argument %d: " % number):
+                L.lib._cdll.sp_map_f32(*args)
+    with pytest.raises(C.ArgumentError, match="argument 8: a random stream is None or a PhiloxConfig, not int"):
+        stack(rng=1234)
