@@ -313,22 +313,27 @@ void refuse_argument(int number) {
 }
 
 // ---- one function per entry point ----
-template <int ID, typename F>
+// What a function is bound to, in a capsule that the function object holds.
+struct Bound {
+    void* fn;
+    PyObject* function;           // the function object itself: what the tape records
+    const char* name;
+};
+
+template <typename F>
 struct Entry;
-template <int ID, typename... A>
-struct Entry<ID, int(A...)> {
+template <typename... A>
+struct Entry<int(A...)> {
     static constexpr bool HOST_INTS = ((std::is_pointer_v<A> && std::is_pointer_v<std::remove_const_t<std::remove_pointer_t<A>>>) || ...);
-    static inline int (*fn)(A...) = nullptr;
-    static inline PyObject* self = nullptr;
-    static inline const char* name = nullptr;
 
     template <size_t... I>
-    static PyObject* run(PyObject* const* given, std::index_sequence<I...>) {
+    static PyObject* run(const Bound& bound, PyObject* const* given, std::index_sequence<I...>) {
         std::tuple<Arg<A, HOST_INTS>...> args;
         if (int at = 0; !((++at, std::get<I>(args).load(given[I])) && ...)) {
             refuse_argument(at);
             return nullptr;
         }
+        int (*const fn)(A...) = (int (*)(A...))bound.fn;
         int rc = 0;
         Py_BEGIN_ALLOW_THREADS
         rc = fn(std::get<I>(args).value...);
@@ -340,7 +345,7 @@ struct Entry<ID, int(A...)> {
                 Py_INCREF(given[i]);
                 PyTuple_SET_ITEM(kept, i, given[i]);
             }
-            PyObject* call = PyTuple_Pack(2, self, kept);
+            PyObject* call = PyTuple_Pack(2, bound.function, kept);
             Py_DECREF(kept);
             if (call == nullptr) return nullptr;
             const int failed = PyList_Append(g_calls, call);
@@ -349,9 +354,11 @@ struct Entry<ID, int(A...)> {
         }
         return PyLong_FromLong(rc);
     }
-    static PyObject* call(PyObject*, PyObject* const* given, Py_ssize_t n) {
-        if (n != (Py_ssize_t)sizeof...(A)) return PyErr_Format(PyExc_TypeError, "%s takes %zu arguments (%zd given)", name, sizeof...(A), n);
-        return run(given, std::index_sequence_for<A...>{});
+    static PyObject* call(PyObject* capsule, PyObject* const* given, Py_ssize_t n) {
+        const Bound* const bound = (const Bound*)PyCapsule_GetPointer(capsule, nullptr);
+        if (bound == nullptr) return nullptr;
+        if (n != (Py_ssize_t)sizeof...(A)) return PyErr_Format(PyExc_TypeError, "%s takes %zu arguments (%zd given)", bound->name, sizeof...(A), n);
+        return run(*bound, given, std::index_sequence_for<A...>{});
     }
 };
 
@@ -362,24 +369,34 @@ struct Entry<ID, int(A...)> {
     X(sp_mlp_forward) X(sp_mlp_pack_weights) X(sp_mlp_forward_packed) X(sp_mlp_forward_ensemble) X(sp_ensemble_binarize)            \
     X(sp_stack_forward_f32)
 
-template <typename E>
-bool bind_one(void* library, PyObject* functions, const char* name, PyMethodDef& def) {
-    E::fn = (decltype(E::fn))dlsym(library, name);
-    if (E::fn == nullptr) {
+bool bind_one(void* library, PyObject* functions, const char* name, PyCFunction call, PyMethodDef& def) {
+    void* const fn = dlsym(library, name);
+    if (fn == nullptr) {
         PyErr_Format(PyExc_RuntimeError, "the library has no %s", name);
         return false;
     }
-    E::name = name;
-    if (E::self == nullptr) {
-        def = PyMethodDef{name, (PyCFunction)(void (*)(void))&E::call, METH_FASTCALL, nullptr};
-        E::self = PyCFunction_New(&def, nullptr);
-        if (E::self == nullptr) return false;
+    def = PyMethodDef{name, call, METH_FASTCALL, nullptr};
+    Bound* const bound = new (std::nothrow) Bound{fn, nullptr, name};
+    if (bound == nullptr) {
+        PyErr_NoMemory();
+        return false;
     }
-    return PyDict_SetItemString(functions, name, E::self) == 0;
+    PyObject* capsule = PyCapsule_New(bound, nullptr, [](PyObject* c) { delete (Bound*)PyCapsule_GetPointer(c, nullptr); });
+    if (capsule == nullptr) {
+        delete bound;
+        return false;
+    }
+    PyObject* function = PyCFunction_New(&def, capsule);
+    Py_DECREF(capsule);
+    if (function == nullptr) return false;
+    bound->function = function;                            // (borrowed: the function holds the capsule)
+    const int failed = PyDict_SetItemString(functions, name, function);
+    Py_DECREF(function);
+    return failed == 0;
 }
 
-// bind(path, stream): a dict of the functions behind the library at `path`, which the process keeps (one library per process); `stream`: the
-// ctypes structure that stands for sp_philox_t.
+// bind(path, stream): a dict of the functions behind the library at `path`, which the process keeps; `stream`: the ctypes structure
+// that stands for sp_philox_t.
 PyObject* bind(PyObject*, PyObject* const* given, Py_ssize_t n) {
     if (n != 2 || !PyType_Check(given[1])) return PyErr_Format(PyExc_TypeError, "bind takes a path and a structure type");
     const char* p = PyUnicode_AsUTF8(given[0]);
@@ -419,7 +436,7 @@ PyObject* bind(PyObject*, PyObject* const* given, Py_ssize_t n) {
 #undef SP_ID
     };
     static PyMethodDef defs[COUNT];
-#define SP_BIND(name) ok = ok && bind_one<Entry<ID_##name, std::remove_pointer_t<decltype(&::name)>>>(library, functions, #name, defs[ID_##name]);
+#define SP_BIND(name) ok = ok && bind_one(library, functions, #name, (PyCFunction)(void (*)(void))&Entry<std::remove_pointer_t<decltype(&::name)>>::call, defs[ID_##name]);
     SP_LAUNCHES(SP_BIND)
 #undef SP_BIND
     if (!ok) {

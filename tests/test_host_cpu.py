@@ -1,6 +1,7 @@
 """The extension between the Python modules and the C ABI (csrc/host.cpp): what it takes as an argument, what it refuses, and that
 the library sees the same values as through ctypes.  No launch: every call is refused by the library's own checks."""
 import ctypes as C
+import subprocess
 
 import numpy as np
 import pytest
@@ -177,3 +178,15 @@ def test_refused_arguments_raise_what_ctypes_raises():
                 L.lib._cdll.sp_map_f32(*args)
     with pytest.raises(C.ArgumentError, match="argument 8: a random stream is None or a PhiloxConfig, not int"):
         stack(rng=1234)
+
+
+def test_each_library_keeps_its_own_functions(tmp_path):
+    """Functions bound to a second library leave those of the first as they are."""
+    names = [n for n in L.SIGNATURES if L.SIGNATURES[n][1][-1:] == [L._P]]
+    (tmp_path / "other.c").write_text("".join("int %s() { return -42; }\n" % n for n in names))
+    other = str(tmp_path / "libother.so")
+    subprocess.run(["gcc", "-w", "-shared", "-fPIC", str(tmp_path / "other.c"), "-o", other], check=True)
+    refused_before = L.lib.sp_map_f32(1, P, P, -1, None)
+    functions = L._host.bind(other, L.PhiloxConfig)
+    assert refused_before == -2 and functions["sp_map_f32"](1, P, P, -1, None) == -42
+    assert L.lib.sp_map_f32(1, P, P, -1, None) == -2 and functions["sp_row_map_i32"](6, P, P, 8, 8, None) == -42
