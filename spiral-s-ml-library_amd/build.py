@@ -112,10 +112,10 @@ def build(force=True, verbose=False):
         newest = max(os.path.getmtime(os.path.join(CSRC, "host.cpp")), os.path.getmtime(os.path.join(ROOT, "include", "spiral_mi355.h")))
         host = None if not force and os.path.exists(HOST_LIB) and os.path.getmtime(HOST_LIB) > newest else ex.submit(build_host)
         objs = list(objs)
+        check_isa()
+        _run([cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs)
         if host is not None:
-            host.result()
-    check_isa()
-    _run([cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs)
+            host.result()         # (last: the C ABI needs neither g++ nor the headers of Python and torch)
     return LIB
 
 
