@@ -18,6 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libspiral_mi355.so")
 HOST_LIB = os.path.join(HERE, "spiral_host.so")      # the Python modules' way into the library (csrc/host.cpp)
+HOST_STAMP = os.path.join(OBJ, "spiral_host.txt")
 SOURCES = ["api.hip", "row_ops.hip", "elementwise.hip", "gemm.hip", "gemm_wave.hip", "mlp.hip", "mlp_any.hip", "mlp_packed.hip", "mlp_resident.hip", "mlp_pipe.hip", "mlp_ensemble.hip", "mlp_stack.hip"]
 # sources with MFMAs or wide stores in inline asm: their device assembly is kept and scanned (isa_check.py)
 ASM_MFMA_SOURCES = ["gemm.hip", "gemm_wave.hip", "mlp.hip", "mlp_any.hip", "mlp_packed.hip", "mlp_resident.hip", "mlp_pipe.hip", "mlp_ensemble.hip", "mlp_stack.hip", "row_ops.hip", "elementwise.hip"]
@@ -48,6 +49,20 @@ def _run(cmd):
     return out
 
 
+def host_stamp():
+    """What the extension is built against: another interpreter or torch needs another build."""
+    import torch
+    return "%s %s %d" % (sys.version, torch.__version__, int(torch._C._GLIBCXX_USE_CXX11_ABI))
+
+
+def host_is_built():
+    sources = (os.path.join(CSRC, "host.cpp"), os.path.join(ROOT, "include", "spiral_mi355.h"))
+    if not os.path.exists(HOST_LIB) or not os.path.exists(HOST_STAMP):
+        return False
+    with open(HOST_STAMP) as f:
+        return f.read() == host_stamp() and all(os.path.getmtime(HOST_LIB) > os.path.getmtime(s) for s in sources)
+
+
 def build_host():
     """The CPython extension in front of the library, against this interpreter and this torch."""
     import sysconfig
@@ -59,6 +74,8 @@ def build_host():
           "-isystem", include, "-isystem", os.path.join(include, "torch", "csrc", "api", "include"),
           "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "host.cpp"), "-o", HOST_LIB,
           "-L" + os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"])
+    with open(HOST_STAMP, "w") as f:
+        f.write(host_stamp())
 
 
 def device_asm(src):
@@ -109,13 +126,11 @@ def build(force=True, verbose=False):
 
     with ThreadPoolExecutor(max_workers=8) as ex:
         objs = ex.map(compile_one, SOURCES)
-        newest = max(os.path.getmtime(os.path.join(CSRC, "host.cpp")), os.path.getmtime(os.path.join(ROOT, "include", "spiral_mi355.h")))
-        host = None if not force and os.path.exists(HOST_LIB) and os.path.getmtime(HOST_LIB) > newest else ex.submit(build_host)
+        host = ex.submit(lambda: None if not force and host_is_built() else build_host())
         objs = list(objs)
         check_isa()
         _run([cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs)
-        if host is not None:
-            host.result()         # (last: the C ABI needs neither g++ nor the headers of Python and torch)
+        host.result()             # (last: the C ABI needs neither g++ nor the headers of Python and torch)
     return LIB
 
 

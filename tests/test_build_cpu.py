@@ -1,4 +1,4 @@
-"""The order of the build (build.py); nothing is compiled."""
+"""The order of the build and what makes it build the extension again (build.py); nothing is compiled."""
 import importlib.util
 import os
 
@@ -15,8 +15,9 @@ def B(monkeypatch, tmp_path):
     monkeypatch.setattr(mod, "OBJ", str(tmp_path))
     monkeypatch.setattr(mod, "LIB", str(tmp_path / "lib.so"))
     monkeypatch.setattr(mod, "HOST_LIB", str(tmp_path / "host.so"))
+    monkeypatch.setattr(mod, "HOST_STAMP", str(tmp_path / "host.txt"))
     monkeypatch.setattr(mod, "hipcc", lambda: "hipcc")
-    monkeypatch.setattr(mod, "commands", [], raising=False)
+    mod.commands = []
 
     def run(cmd):
         mod.commands.append(cmd)
@@ -35,3 +36,18 @@ def test_the_library_is_linked_where_the_extension_cannot_be_built(B):
     with pytest.raises(RuntimeError, match=r"g\+\+"):
         B.build(force=True)
     assert any("-shared" in c and c[c.index("-o") + 1] == B.LIB for c in B.commands)
+
+
+def test_another_interpreter_or_torch_builds_the_extension_again(B, monkeypatch):
+    built = lambda: sum(c[0] == "g++" for c in B.commands)
+    B.build(force=False)
+    assert built() == 1
+    B.build(force=False)
+    assert built() == 1
+    monkeypatch.setattr(B, "host_stamp", lambda: "another")
+    B.build(force=False)
+    assert built() == 2
+    B.build(force=False)
+    assert built() == 2
+    B.build(force=True)
+    assert built() == 3
