@@ -41,6 +41,19 @@ __device__ __forceinline__ f32x4 any_mfma(const u32x4& w, const u32x4& x, const 
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), c, 0, 0, 0);
 }
 
+// relu is max(0, x), a NaN becomes 0.  The matrix pipe's own NaNs have the sign set, whatever went in, and pack_relu2, which compares
+// rounded values as integers, makes them 0; one that a bias brings may have it clear, so sums with a bias pass an f32 maximum first.  (That
+// maximum for every sum costs 1 to 3 % without a bias: 64-192-192-192-4, 65536 rows.)  Stacks whose hidden layers are all 256 wide
+// (AN_ALL_256, in the layer count that a kernel is given) do without, as in the kernels that take the others of them: there a bias that is
+// a NaN stays one, and what a head of up to 16 outputs leaves past its mask are zeros, in a row of NaNs, too.
+constexpr unsigned AN_ALL_256 = 0x80;
+__device__ __forceinline__ float any_biased(float sum, float bias, bool all_256, bool last) {
+    float r;
+    asm("v_add_f32 %0, %1, %2" : "=v"(r) : "v"(sum), "v"(bias));       // (the sum first: of two NaNs it is the one that stays)
+    if (!all_256 && !last) asm("v_max_f32 %0, 0, %1" : "=v"(r) : "v"(r));
+    return r;
+}
+
 // The last layer's outputs as the matrix pipe leaves them when the weight rows of a pair of tiles are fed in the order 32 u + 8 (i / 4)
 // + i % 4 (even tile) and + 4 (odd tile): lane (j, q) holds columns 32 u + 8 q .. + 7 of batch row j.
 //   The head of those 16 rows, all 64 lanes at work: the formulas and the order of every sum are head_row's (mlp_common.h) -- sums
@@ -72,7 +85,7 @@ __device__ __forceinline__ float any_running_sum(const float (&p)[P][8], int n, 
 }
 
 template <int P>
-__device__ __forceinline__ void any_head(const HeadOut& o, const f32x4 (&v)[2 * P], long row, bool row_ok, int j, int q, int n, int limit, float uniform) {
+__device__ __forceinline__ void any_head(const HeadOut& o, const f32x4 (&v)[2 * P], long row, bool row_ok, int j, int q, int n, int limit, float uniform, bool all_256) {
     const float NEG_INF = -__builtin_inff();
     const int stride = o.stride;
     const bool whole = (stride & 3) == 0;
@@ -138,6 +151,13 @@ __device__ __forceinline__ void any_head(const HeadOut& o, const f32x4 (&v)[2 * 
             for (int k = 0; k < 8; ++k) p[u][k] = s != 0.f ? p[u][k] * inv : (32 * u + 8 * q + k < limit ? inv_len : 0.f);
         past = 0.f * inv;
     }
+    if (all_256 && n <= 16) {
+        past = 0.f;
+#pragma unroll
+        for (int u = 0; u < P; ++u)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) p[u][k] = 32 * u + 8 * q + k < n ? p[u][k] : 0.f;
+    }
     store_row(o.policy);
     if (o.action != nullptr) {
         float cdf[P][8];
@@ -171,7 +191,7 @@ __device__ __forceinline__ void any_head(const HeadOut& o, const f32x4 (&v)[2 * 
 
 // At most four outputs, all of them in every lane of a row: the same formulas.  store(out): the row's p and `past` behind it.
 template <typename Store>
-__device__ __forceinline__ void any_head4(const HeadOut& o, float (&p)[4], float& past, int n, int limit, const Store& store) {
+__device__ __forceinline__ void any_head4(const HeadOut& o, float (&p)[4], float& past, int n, int limit, bool all_256, const Store& store) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) p[k] = k < n ? p[k] : 0.f;
     past = 0.f;
@@ -207,6 +227,7 @@ __device__ __forceinline__ void any_head4(const HeadOut& o, float (&p)[4], float
         for (int k = 0; k < 4; ++k) p[k] = s != 0.f ? p[k] * inv : (k < limit ? inv_len : 0.f);
         past = 0.f * inv;
     }
+    if (all_256) past = 0.f;
     store(o.policy);
 }
 
@@ -233,7 +254,8 @@ __global__ __launch_bounds__(AN_FEATURES_THREADS) void mlp_features_kernel(const
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 15, q = lane >> 4;
-    const int NL = (int)(counts & 0xffu), N = (int)(counts >> 8 & 0xffu), waves = (int)(counts >> 16);
+    const bool all_256 = counts & AN_ALL_256;
+    const int NL = (int)(counts & 0x7fu), N = (int)(counts >> 8 & 0xffu), waves = (int)(counts >> 16);
     const long row0 = (long)blockIdx.x * (16 * R);
     const unsigned lds0 = (unsigned)(size_t)lds;
     const int K0 = any_width(widths, 0);
@@ -351,7 +373,7 @@ __global__ __launch_bounds__(AN_FEATURES_THREADS) void mlp_features_kernel(const
                     const int n = 16 * t + 4 * q + r;
                     const float b = bias[n < F ? n : F - 1];
 #pragma unroll
-                    for (int rt = 0; rt < R; ++rt) acc[rt][r] += b;
+                    for (int rt = 0; rt < R; ++rt) acc[rt][r] = any_biased(acc[rt][r], b, all_256, last);
                 }
             unsigned char* const to = lds + (buffer ^ L::ACTS) + j * 256;
             if (!last) {
@@ -377,7 +399,7 @@ __global__ __launch_bounds__(AN_FEATURES_THREADS) void mlp_features_kernel(const
     if (N <= 4) {
         const f32x4 v = outputs(0);
         float p[4] = {v[0], v[1], v[2], v[3]}, past;
-        any_head4(out, p, past, N, limit, [&](float* to) {      // the four lanes of a row share its pieces
+        any_head4(out, p, past, N, limit, all_256, [&](float* to) {      // the four lanes of a row share its pieces
             const int stride = out.stride;
             float* const at = to + my_row * stride;
             if (!row_ok) return;
@@ -393,10 +415,10 @@ __global__ __launch_bounds__(AN_FEATURES_THREADS) void mlp_features_kernel(const
         if (out.action != nullptr && row_ok && q == 0) out.action[my_row] = head_pick4(p, uniform);
     } else if (N <= 32) {
         const f32x4 v[2] = {outputs(2 * q), outputs(2 * q + 1)};
-        any_head<1>(out, v, my_row, row_ok, j, q, N, limit, uniform);
+        any_head<1>(out, v, my_row, row_ok, j, q, N, limit, uniform, all_256);
     } else {
         const f32x4 v[4] = {outputs(2 * q), outputs(2 * q + 1), outputs(8 + 2 * q), outputs(9 + 2 * q)};
-        any_head<2>(out, v, my_row, row_ok, j, q, N, limit, uniform);
+        any_head<2>(out, v, my_row, row_ok, j, q, N, limit, uniform, false);
     }
 }
 
@@ -415,7 +437,8 @@ __global__ __launch_bounds__(AN_THREADS, 2) void mlp_rows_kernel(unsigned long l
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 15, q = lane >> 4;
-    const int NL = (int)(counts & 0xffu);
+    const bool all_256 = HT == 16 && (counts & AN_ALL_256);
+    const int NL = (int)(counts & 0x7fu);
     const unsigned lds0 = (unsigned)(size_t)lds;
     const long tiles = (a.batch + AN_ROWS - 1) / AN_ROWS, step = (long)gridDim.x * AN_WAVES;
     const int r8 = lane >> 3;
@@ -577,8 +600,8 @@ __global__ __launch_bounds__(AN_THREADS, 2) void mlp_rows_kernel(unsigned long l
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
                             const float b = bias[32 * (t >> 1) + 4 * (t & 1) + 8 * q + r];
-                            acc[0][t][r] += b;
-                            acc[1][t][r] += b;
+                            acc[0][t][r] = any_biased(acc[0][t][r], b, all_256, false);
+                            acc[1][t][r] = any_biased(acc[1][t][r], b, all_256, false);
                         }
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt)
@@ -605,7 +628,7 @@ __global__ __launch_bounds__(AN_THREADS, 2) void mlp_rows_kernel(unsigned long l
                 if (bias != nullptr) p[k] += bias[k < N ? k : N - 1];
             }
             if (a.ph.philox_mode >= 0) uniform = reference_row_uniform(a.ph, my_row < a.batch ? my_row : 0);
-            any_head4(out, p, past, N, limit, [&](float* to) {
+            any_head4(out, p, past, N, limit, all_256, [&](float* to) {
                 // the 32 rows are one block: whole waves write it, 16 bytes or one column per lane (row r's p: lane r % 16 + 32 (r / 16))
                 const int stride = out.stride, piece = (stride & 3) == 0 ? 4 : 1, per_row = stride / piece;
                 int r = lane / per_row, c = lane - r * per_row;
@@ -652,9 +675,9 @@ __global__ __launch_bounds__(AN_THREADS, 2) void mlp_rows_kernel(unsigned long l
             }
             if (N <= 32) {
                 const f32x4 v[2] = {mine[0], mine[1]};
-                any_head<1>(out, v, row, ok, j, qh, N, limit, u);
+                any_head<1>(out, v, row, ok, j, qh, N, limit, u, all_256);
             } else {
-                any_head<2>(out, mine, row, ok, j, qh, N, limit, u);
+                any_head<2>(out, mine, row, ok, j, qh, N, limit, u, false);
             }
         }
     }
@@ -681,10 +704,14 @@ int mlp_any_launch(int dtype, const MlpArgs& a, hipStream_t stream, const char* 
         const long gk = (a.dims[l] + 63) / 64;
         group_bytes += gk * ((a.dims[l + 1] + 31) / 32) * AN_GROUP;
     }
-    unsigned counts = (unsigned)NL | (unsigned)N << 8;
     const long cus = device_cu_count();
     int widest = 32;
-    for (int l = 1; l < NL; ++l) widest = a.dims[l] > widest ? a.dims[l] : widest;
+    bool all_256 = NL > 1;
+    for (int l = 1; l < NL; ++l) {
+        widest = a.dims[l] > widest ? a.dims[l] : widest;
+        all_256 = all_256 && a.dims[l] == 256;
+    }
+    unsigned counts = (unsigned)NL | (all_256 ? AN_ALL_256 : 0u) | (unsigned)N << 8;
     const bool stream_weights = group_bytes > AN_LDS;
     if (a.batch > (stream_weights ? 128 : 64) * cus) {
         const void* kernel = dtype == SP_F16 ? pick_rows_kernel<SP_F16>(widest, stream_weights) : pick_rows_kernel<SP_BF16>(widest, stream_weights);

@@ -216,6 +216,60 @@ def test_masked_head_of_other_stacks_without_logits(LY, dims, head, mask, batch,
     assert torch.equal(policy_t.view(torch.int32), full_p.view(torch.int32)) and torch.equal(action, full_a)
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("dims,mask,rows_per_unit", [([128, 64, 64], 3, 0), ([64, 96, 160, 10], 0, 0), ([80, 192, 192, 24], 0, 0), ([64, 128, 64], 3, 65),
+                                                     ([64, 128, 40], 0, 65), ([48, 192, 64], 11, 65), ([128] * 7 + [20], 0, 129), ([64, 256, 128, 64], 3, 65)])
+def test_a_hidden_sum_that_is_no_number_becomes_zero(LY, dims, mask, rows_per_unit, dtype):
+    """relu is max(0, x) as in the reference.  Features with a NaN for a bias, of either sign, are zeros, as those with a bias far below
+    every sum are, bit for bit.  In a row with a NaN, of either sign, or inf - inf in every sum, the first hidden layer is zeros, hence the
+    outputs are without biases, and the head falls to the even distribution of the valid columns."""
+    announce("mlp hidden nan %s mask=%d %s" % (dims, mask, dtype))
+    batch = 50 if rows_per_unit == 0 else rows_per_unit * torch.cuda.get_device_properties(0).multi_processor_count
+    rng = np.random.default_rng(sum(dims))
+    t = TORCH[dtype]
+    x = rng.standard_normal((batch, dims[0])).astype(np.float32)
+    odd = [0, 7, batch // 2, batch - 1]
+    x[odd[0]], x[odd[1], 3], x[odd[2], 2:], x[odd[2], :2], x[odd[3]] = np.nan, -np.nan, 0, [np.inf, -np.inf], -np.nan
+    wd = [dev(rng.standard_normal((o, i)).astype(np.float32) / np.float32(np.sqrt(i)), t) for i, o in zip(dims[:-1], dims[1:])]
+    wd[0][:, :2] = wd[0][:, :2].abs() + 0.5                # (inf times the one minus inf times the other, in every feature)
+    bias = [rng.standard_normal(o).astype(np.float32) for o in dims[1:]]
+    none, low = [b.copy() for b in bias], [b.copy() for b in bias]
+    for l in range(len(dims) - 2):
+        off = rng.choice(dims[l + 1], 5, replace=False)
+        none[l][off], low[l][off] = [np.nan, -np.nan, np.nan, -np.nan, np.nan], -1e30
+    un = (1 - rng.random(batch)).astype(np.float32)
+    u, xd, valid = dev(un), dev(x, t), mask or dims[-1]
+    for head in ("softmax", "regret_matching", "softmax_regret_matching"):
+        got = LY.mlp_forward(xd, wd, [dev(b) for b in none], head, u, mask)
+        want = LY.mlp_forward(xd, wd, [dev(b) for b in low], head, u, mask)
+        assert all(torch.equal(g, w) for g, w in zip(got, want)) and torch.isfinite(got[0]).all()
+        for want_logits in (False, True):
+            policy, action = (host(o) for o in LY.mlp_forward(xd, wd, None, head, u, mask, want_logits)[:2])
+            assert np.isfinite(policy).all() and (action == orow.discrete_sampling(policy, un)).all()
+            assert np.abs(policy[odd, :valid] * valid - 1).max() < 1e-6 and (policy[odd, valid:] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("mask", [1, 3, 13, 16])
+def test_past_a_narrow_mask_are_zeros_behind_a_256_wide_layer(LY, mask, dtype):
+    """... whatever the valid columns are: in a row whose hidden sums are infinite those are NaN and there is no action."""
+    announce("mlp 64-256-64 nan rows mask=%d %s" % (mask, dtype))
+    rng = np.random.default_rng(mask)
+    t = TORCH[dtype]
+    wd = [dev(rng.standard_normal((o, i)).astype(np.float32) / np.float32(np.sqrt(i)), t) for i, o in ((64, 256), (256, 64))]
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    for batch in (20, 64 * units + 9):
+        x = rng.standard_normal((batch, 64)).astype(np.float32)
+        x[3, 0] = np.inf
+        x[batch - 2, 1] = -np.inf
+        u = dev((1 - rng.random(batch)).astype(np.float32))
+        policy, action = LY.mlp_forward(dev(x, t), wd, None, "softmax", u, mask)
+        policy, action = host(policy), host(action)
+        for row in (3, batch - 2):
+            assert np.isnan(policy[row, :mask]).all() and action[row] == 2147483647
+        assert (policy[:, mask:] == 0).all()
+
+
 @pytest.mark.parametrize("dims,head,mask,batch,dtype,with_bias", [
     ([32, 256, 256, 256, 3], "softmax_regret_matching", 0, 16384, "f16", False),     # the benchmark's policy network
     ([32, 256, 256, 256, 3], "softmax", 0, 1, "bf16", False),                        # a single row
