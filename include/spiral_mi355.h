@@ -380,6 +380,8 @@ typedef enum {
  * policy stays within a relative Frobenius error of 3e-3 for both types and so do f16 logits; the raw
  * logits_out of a BF16 stack (8 significant bits per hidden activation and layer) are only held to 1e-2.
  * Against an evaluation that rounds its activations the same way everything is within 2e-4.
+ * relu is max(0, x): a hidden sum that is a NaN becomes 0.  Where every hidden layer is 256 wide one that a bias brings (a NaN, or inf
+ * against an infinite sum) may stay a NaN; a masked head of at most 16 columns then still writes zeros past its mask.
  */
 int sp_mlp_forward(int dtype, const void* x, int32_t n_layers, const void* const* weights, const float* const* biases,
                    const int32_t* dims, const float* u, const sp_philox_t* philox, float* policy_out, int32_t* action_out,

@@ -47,11 +47,18 @@ __device__ __forceinline__ f32x4 any_mfma(const u32x4& w, const u32x4& x, const 
 // (AN_ALL_256, in the layer count that a kernel is given) do without, as in the kernels that take the others of them: there a bias that is
 // a NaN stays one, and what a head of up to 16 outputs leaves past its mask are zeros, in a row of NaNs, too.
 constexpr unsigned AN_ALL_256 = 0x80;
-__device__ __forceinline__ float any_biased(float sum, float bias, bool all_256, bool last) {
+__device__ __forceinline__ float any_biased(float sum, float bias) {
     float r;
     asm("v_add_f32 %0, %1, %2" : "=v"(r) : "v"(sum), "v"(bias));       // (the sum first: of two NaNs it is the one that stays)
-    if (!all_256 && !last) asm("v_max_f32 %0, 0, %1" : "=v"(r) : "v"(r));
     return r;
+}
+__device__ __forceinline__ void any_max0(f32x4& v) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        float m;
+        asm("v_max_f32 %0, 0, %1" : "=v"(m) : "v"(v[r]));
+        v[r] = m;
+    }
 }
 
 // The last layer's outputs as the matrix pipe leaves them when the weight rows of a pair of tiles are fed in the order 32 u + 8 (i / 4)
@@ -153,10 +160,10 @@ __device__ __forceinline__ void any_head(const HeadOut& o, const f32x4 (&v)[2 * 
     }
     if (all_256 && n <= 16) {
         past = 0.f;
+        int qz = q;
+        asm volatile("" : "+v"(qz));                    // (comparisons of its own: those above would be kept for it, two registers each)
 #pragma unroll
-        for (int u = 0; u < P; ++u)
-#pragma unroll
-            for (int k = 0; k < 8; ++k) p[u][k] = 32 * u + 8 * q + k < n ? p[u][k] : 0.f;
+        for (int k = 0; k < 8; ++k) p[0][k] = 8 * qz + k < n ? p[0][k] : 0.f;
     }
     store_row(o.policy);
     if (o.action != nullptr) {
@@ -367,14 +374,18 @@ __global__ __launch_bounds__(AN_FEATURES_THREADS) void mlp_features_kernel(const
             }
             // lane (j, q): features 16 t + 4 q .. + 3 of batch row j
             const float* const bias = a.b[layer];
-            if (bias != nullptr)
+            if (bias != nullptr) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int n = 16 * t + 4 * q + r;
                     const float b = bias[n < F ? n : F - 1];
 #pragma unroll
-                    for (int rt = 0; rt < R; ++rt) acc[rt][r] = any_biased(acc[rt][r], b, all_256, last);
+                    for (int rt = 0; rt < R; ++rt) acc[rt][r] = any_biased(acc[rt][r], b);
                 }
+                if (!last && !all_256)
+#pragma unroll
+                    for (int rt = 0; rt < R; ++rt) any_max0(acc[rt]);
+            }
             unsigned char* const to = lds + (buffer ^ L::ACTS) + j * 256;
             if (!last) {
                 const int at = (t >> 3) * L::PLANE + ((((2 * t & 15) + (q >> 1)) ^ j) << 4) + (q & 1) * 8;
@@ -593,16 +604,22 @@ __global__ __launch_bounds__(AN_THREADS, 2) void mlp_rows_kernel(unsigned long l
             f32x4 acc[2][HT];
             products(K, gn, acc, act, IC<4>{}, IC<HT>{});
             const float* bias = a.b[layer];
-            if (bias != nullptr)
+            if (bias != nullptr) {
 #pragma unroll
                 for (int t = 0; t < HT; ++t)
                     if (t < 2 * gn)
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
                             const float b = bias[32 * (t >> 1) + 4 * (t & 1) + 8 * q + r];
-                            acc[0][t][r] = any_biased(acc[0][t][r], b, all_256, false);
-                            acc[1][t][r] = any_biased(acc[1][t][r], b, all_256, false);
+                            acc[0][t][r] = any_biased(acc[0][t][r], b);
+                            acc[1][t][r] = any_biased(acc[1][t][r], b);
                         }
+                if (!all_256)
+#pragma unroll
+                    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                        for (int t = 0; t < HT; ++t) any_max0(acc[rt][t]);
+            }
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
