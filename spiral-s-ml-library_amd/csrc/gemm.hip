@@ -1007,9 +1007,11 @@ struct TileChoice {
 // 128 x 64 and 128 x 96 tiles fill the units where 128 wide ones leave a last round nearly empty and 64 wide ones move twice the operands
 // (us, without / with them: f16 5001 x 1003 x 1000 27.1 / 21.6, bf16 2390 x 1252 x 5696 101 / 87, 14864 x 320 x 4800 64 / 42, 656 x 6992 x
 // 1152 29 / 22, 23732 x 234 x 56 12 / 8; 0.98 times the time on the geometric mean of 220 shapes of 0.4 GFLOP and more that no 128 tile
-// divides, 42 of which take them, the worst 1.08 times: 53584 x 16 x 272).  Fitted on those 220, and three in a hundred put on top where rows
-// cross lines (2160 x 3248 x 160 10.7 / 11.3 without that); also measured: 192 x 128, 128 x 192, 192 x
-// 192, 256 x 128, 256 x 192 and 96 x 128 tiles, which add less than a hundredth.
+// divides, 42 of which take them).  Fitted on those 220, and three in a hundred put on top where rows cross lines (2160 x 3248 x 160 10.7 /
+// 11.3 without that).  A 128 x 96 workgroup alone on its unit waits 0.82 us for a K-tile: without that in its line it was taken for
+// 13040 x 96 x 5112 (105 us, now 67), 5168 x 224 x 5048 (61, 41), 1732 x 943 x 5784 (71, 54) and 24937 x 56 x 8088 (157, 125).  Where rows are
+// whole lines it is the fastest by 2 % on four of 117 shapes (0.999 on the mean) and stays out of that table.  Also measured: 192 x 128,
+// 128 x 192, 192 x 192, 256 x 128, 256 x 192 and 96 x 128 tiles, which add less than a hundredth.
 struct TileCost {
     int cfg, bm, bn;
     float tk, overhead, latency;
@@ -1020,7 +1022,7 @@ static const TileCost kCostLines[] = {{0, 256, 256, 1.75f, 8.f, 0.f}, {1, 128, 1
                                       {-1, 64, 64, 0.22f, 1.5f, 0.f}, {-1, 64, 32, 0.17f, 0.8f, 0.f}, {-1, 32, 32, 0.09f, 0.5f, 0.f},
                                       {-1, 16, 16, 0.05f, 0.3f, 0.f}};
 static const TileCost kCostCrossing[] = {{0, 256, 256, 1.5f, 14.f, 0.f}, {1, 128, 128, 0.65f, 4.f, 1.05f}, {2, 64, 64, 0.29f, 0.8f, 0.5f},
-                                         {3, 128, 64, 0.505f, 1.44f, 1.03f}, {4, 128, 96, 0.515f, 4.95f, 0.f},
+                                         {3, 128, 64, 0.505f, 1.44f, 1.03f}, {4, 128, 96, 0.515f, 4.5f, 0.82f},
                                          {-1, 64, 64, 0.27f, 1.5f, 0.f}, {-1, 64, 32, 0.19f, 0.8f, 0.f}, {-1, 32, 32, 0.11f, 0.5f, 0.f},
                                          {-1, 16, 16, 0.055f, 0.3f, 0.f}};
 

@@ -344,3 +344,12 @@ def test_stack_sizes_are_asked_without_a_call(L):
     assert takes(64, 16, members=70000) == -2 and takes(64, 16, batch=0) == -2 and takes(64, 16, members=2, batch=1 << 30) == -2
     assert takes(64, 16, head=3) == -5 and takes(64, 16, head=2, mask=17) == -5 and takes(*([64] * 10)) == -2
     assert L.lib.sp_stack_forward_takes(1, None, 1, 64, 1, 0) == -1
+
+
+@pytest.mark.parametrize("m,n,k", [(13040, 96, 5112), (5168, 224, 5048), (1732, 943, 5784), (24937, 56, 8088), (3584, 592, 2296), (16512, 96, 1000)])
+def test_long_k_of_one_round_is_not_left_to_lone_workgroups(L, m, n, k):
+    """16-bit shapes of at most one 128 x 96 tile per compute unit of 256, where nothing covers such a workgroup's loads."""
+    for dtype in (1, 2):
+        out = [C.c_int32() for _ in range(4)]
+        assert L.lib.sp_gemm_config(dtype, m, n, k, *[C.byref(o) for o in out]) == 0
+        assert (out[0].value, out[1].value) != (128, 96)
