@@ -1008,13 +1008,16 @@ struct TileChoice {
 // (us, without / with them: f16 5001 x 1003 x 1000 27.1 / 21.6, bf16 2390 x 1252 x 5696 101 / 87, 14864 x 320 x 4800 64 / 42, 656 x 6992 x
 // 1152 29 / 22, 23732 x 234 x 56 12 / 8; 0.98 times the time on the geometric mean of 220 shapes of 0.4 GFLOP and more that no 128 tile
 // divides, 42 of which take them).  Fitted on those 220, and three in a hundred put on top where rows cross lines (2160 x 3248 x 160 10.7 /
-// 11.3 without that).  A 128 x 96 workgroup alone on its unit waits 0.82 us for a K-tile: without that in its line it was taken for
-// 13040 x 96 x 5112 (105 us, now 67), 5168 x 224 x 5048 (61, 41), 1732 x 943 x 5784 (71, 54) and 24937 x 56 x 8088 (157, 125).  Where rows are
-// whole lines it is the fastest by 2 % on four of 117 shapes (0.999 on the mean) and stays out of that table.  Also measured: 192 x 128,
-// 128 x 192, 192 x 192, 256 x 128, 256 x 192 and 96 x 128 tiles, which add less than a hundredth.
+// 11.3 without that).  A 128 x 96 workgroup alone on its unit waits 0.82 us for a K-tile of long K: without that in its line it was taken
+// for 13040 x 96 x 5112 (105 us, now 67), 5168 x 224 x 5048 (61, 41), 1732 x 943 x 5784 (71, 54) and 24937 x 56 x 8088 (157, 125).  From 16
+// K-tiles on (us, this tile / the one taken otherwise: 6529 x 280 x 776 12.1 / 12.9, x 904 13.7 / 13.5, x 1032 17.1 / 14.5, x 1288 20.9 /
+// 17.1; 6656 x 288 x 520 9.4 / 11.1, x 904 12.2 / 13.6, x 1288 20.3 / 17.7).  Where rows are whole lines it is the fastest by 2 % on four
+// of 117 shapes (0.999 on the mean) and stays out of that table.  Also measured: 192 x 128, 128 x 192, 192 x 192, 256 x 128, 256 x 192 and
+// 96 x 128 tiles, which add less than a hundredth.
 struct TileCost {
     int cfg, bm, bn;
     float tk, overhead, latency;
+    int latency_from = 0;      // K-tiles from which on `latency` counts
 };
 static const TileCost kCostF32[] = {{0, 256, 256, 7.86f, 22.f, 0.f}, {1, 128, 128, 2.17f, 3.6f, 0.f}, {2, 64, 64, 0.556f, 0.52f, 0.f},
                                     {-1, 32, 32, 0.151f, 0.45f, 0.f}, {-1, 16, 16, 0.079f, 0.24f, 0.f}};
@@ -1022,7 +1025,7 @@ static const TileCost kCostLines[] = {{0, 256, 256, 1.75f, 8.f, 0.f}, {1, 128, 1
                                       {-1, 64, 64, 0.22f, 1.5f, 0.f}, {-1, 64, 32, 0.17f, 0.8f, 0.f}, {-1, 32, 32, 0.09f, 0.5f, 0.f},
                                       {-1, 16, 16, 0.05f, 0.3f, 0.f}};
 static const TileCost kCostCrossing[] = {{0, 256, 256, 1.5f, 14.f, 0.f}, {1, 128, 128, 0.65f, 4.f, 1.05f}, {2, 64, 64, 0.29f, 0.8f, 0.5f},
-                                         {3, 128, 64, 0.505f, 1.44f, 1.03f}, {4, 128, 96, 0.515f, 4.5f, 0.82f},
+                                         {3, 128, 64, 0.505f, 1.44f, 1.03f}, {4, 128, 96, 0.515f, 4.95f, 0.82f, 16},
                                          {-1, 64, 64, 0.27f, 1.5f, 0.f}, {-1, 64, 32, 0.19f, 0.8f, 0.f}, {-1, 32, 32, 0.11f, 0.5f, 0.f},
                                          {-1, 16, 16, 0.055f, 0.3f, 0.f}};
 
@@ -1052,7 +1055,7 @@ static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, lo
         if (c.cfg < 0 && tiles >= 4294967296.0) return;     // the split form numbers the tiles of a whole batch in 32 bits
         const float rounds = (float)((tiles + cus - 1) / cus >= 1e9 ? 1e9 : (double)(long)((tiles + cus - 1) / cus));
         const float n = dtype_in == SP_F32 && tiles > cus ? 0.5f * (rounds + (float)(tiles / cus)) : rounds;
-        const float per_k = n * c.tk > c.latency ? n * c.tk : c.latency;
+        const float per_k = n * c.tk > c.latency || nk < c.latency_from ? n * c.tk : c.latency;
         const float us = n * c.overhead + (float)nk * per_k;
         if (best == nullptr || us < best_us) {
             best = &c;
