@@ -128,7 +128,7 @@ int sp_gemm_abt_batched(int dtype_in, int dtype_out, const void* A, const void* 
                         int64_t M, int64_t N, int64_t K, int64_t batch, int64_t stride_a, int64_t stride_b,
                         int64_t stride_c, float alpha, float beta, uint32_t flags, void* stream);
 
-/* Which tile configuration sp_gemm_abt picks for a shape (the counterpart of
+/* Which tile configuration sp_gemm_abt picks for a shape with beta = 0 (the counterpart of
  * `matmul_config_tf32`, ml/matmul/run.spi:8-19).  Writes block tile sizes and the workgroup size; tile_m == 0 means one thread
  * per output (odd widths of the shortest K). */
 int sp_gemm_config(int dtype_in, int64_t M, int64_t N, int64_t K,

@@ -1031,7 +1031,7 @@ static const TileCost kCostCrossing[] = {{0, 256, 256, 1.5f, 14.f, 0.f}, {1, 128
 
 enum TileKind { TILE_ANY, TILE_WORKGROUP, TILE_SPLIT };
 
-static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, long cus, TileKind kind) {
+static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, long cus, TileKind kind, bool reads_c) {
     const int es = dtype_in == SP_F32 ? 4 : 2, bk = ROW_BYTES / es;
     const long nk = (K + bk - 1) / bk;
     // 16-bit shapes that a 256 or 128 tile divides: choose_cfg.  The rest, and f32, by the estimate.
@@ -1047,6 +1047,12 @@ static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, lo
     float best_us = 0.f;
     auto consider = [&](const TileCost& c) {
         if (whole == 0 || whole == 1 ? c.cfg != whole : whole == 2 && c.cfg >= 0 && c.cfg != 2) return;
+        // The 128 x 64 and 128 x 96 tiles where C is read: their waves read twice the rows one after the other, which three K-tiles do not
+        // pay for (us, 64 x 64 / so: 57049 x 37 x 88 6.8 / 7.7, 3692 x 2239 x 104 15.4 / 17.0, 9074 x 348 x 16 7.1 / 7.8, 880 x 4416 x 32 6.9 /
+        // 7.5; 18432 x 848 x 72 128 x 128 28.8 / 26.0), nor a tile that is half padding (55244 x 30 x 328 11.4 / 12.1).  Such a tile without
+        // reading C: only for odd widths, whose rows it leaves to the L2 (64068 x 14 x 144 10.2 / 8.3, 65504 x 30 x 240 17.4 / 10.7; 51392 x 16 x
+        // 120 6.1 / 6.5).
+        if (c.cfg >= kNumCfgs && ((reads_c && nk <= 3) || (2 * N <= c.bn && (reads_c || N % 4 == 0)))) return;
         if (c.cfg < 0 ? kind == TILE_WORKGROUP : kind == TILE_SPLIT) return;
         if (c.cfg < 0 && (!may_split || K * es > kWaveMaxRowBytes || M > 2147483000l || N > 2147483000l)) return;
         const double of_member = (double)((M + c.bm - 1) / c.bm) * (double)((N + c.bn - 1) / c.bn);
@@ -1065,7 +1071,7 @@ static TileChoice best_tile(int dtype_in, long M, long N, long K, long batch, lo
     if (dtype_in == SP_F32) for (const TileCost& c : kCostF32) consider(c);
     else if (K % bk == 0) for (const TileCost& c : kCostLines) consider(c);
     else for (const TileCost& c : kCostCrossing) consider(c);
-    if (best == nullptr) return best_tile(dtype_in, M, N, K, batch, cus, TILE_WORKGROUP);   // (a split form that cannot be numbered)
+    if (best == nullptr) return best_tile(dtype_in, M, N, K, batch, cus, TILE_WORKGROUP, reads_c);   // (a split form that cannot be numbered)
     if (best->cfg < 0) return {-1, best->bm, best->bn, 256, true, best_us};
     const TileCfg& t = kTileCfgs[best->cfg];
     const bool ragged = best->cfg >= kNumCfgs || M % t.bm != 0 || N % t.bn != 0 || K % bk != 0;
@@ -1088,13 +1094,13 @@ static bool one_thread_each(int dtype_in, long M, long N, long K) {
 // where small whole tiles come in large numbers (us, workgroup tiles / split K: 300 x (128 x 128 x 224) 28.8 / 31.7,
 // 37 x (960 x 384 x 320) 78 / 104, 300 x (64 x 64 x 64) 4.8 / 7.8).  For 16-bit inputs, whose 256 wide tiles have MFMAs and
 // K walks of their own anyway, as long as the other kind is not a quarter faster by the estimate.
-static TileChoice choose_tile(int dtype_in, long M, long N, long K, long batch, long cus) {
+static TileChoice choose_tile(int dtype_in, long M, long N, long K, long batch, long cus, bool reads_c) {
     const TileChoice each = {-2, 0, 0, 256, true, 4e-6f * (float)M * (float)N * (float)batch};
-    const TileChoice member = one_thread_each(dtype_in, M, N, K) ? each : best_tile(dtype_in, M, N, K, 1, cus, TILE_ANY);
+    const TileChoice member = one_thread_each(dtype_in, M, N, K) ? each : best_tile(dtype_in, M, N, K, 1, cus, TILE_ANY, reads_c);
     if (batch == 1) return member;
-    const TileChoice alike = member.cfg == -2 ? each : best_tile(dtype_in, M, N, K, batch, cus, member.cfg < 0 ? TILE_SPLIT : TILE_WORKGROUP);
+    const TileChoice alike = member.cfg == -2 ? each : best_tile(dtype_in, M, N, K, batch, cus, member.cfg < 0 ? TILE_SPLIT : TILE_WORKGROUP, reads_c);
     if (dtype_in == SP_F32) return alike;
-    const TileChoice any = best_tile(dtype_in, M, N, K, batch, cus, TILE_ANY);
+    const TileChoice any = best_tile(dtype_in, M, N, K, batch, cus, TILE_ANY, reads_c);
     return alike.us <= 1.25f * any.us ? alike : any;
 }
 
@@ -1289,7 +1295,7 @@ static int gemm_config(const char* fn, int dtype_in, int64_t M, int64_t N, int64
     int rc = validate_gemm(dtype_in, SP_F32, M, N, K);
     if (rc != SP_OK) return rc;
     if (batch < 1 || batch > 65535) return fail(SP_ERR_SHAPE, "%s: batch must be in [1, 65535], got %lld", fn, (long long)batch);
-    const TileChoice t = choose_tile(dtype_in, M, N, K, batch, device_cu_count());
+    const TileChoice t = choose_tile(dtype_in, M, N, K, batch, device_cu_count(), false);
     *tile_m = t.bm;
     *tile_n = t.bn;
     *tile_k = dtype_in == SP_F32 ? 32 : 64;
@@ -1343,7 +1349,7 @@ static int gemm_entry(const char* fn, int dtype_in, int dtype_out, const void* A
     int cfg = -2;                                         // one thread per output
     if (!(flags & SP_GEMM_FORCE_GENERIC)) {
         const long cus = device_cu_count();
-        const TileChoice t = choose_tile(dtype_in, M, N, K, batch, cus);
+        const TileChoice t = choose_tile(dtype_in, M, N, K, batch, cus, beta != 0.f);
         cfg = t.cfg;
         if (cfg != -2) {
             g.ragged = t.ragged;

@@ -353,3 +353,10 @@ def test_long_k_of_one_round_is_not_left_to_lone_workgroups(L, m, n, k):
         out = [C.c_int32() for _ in range(4)]
         assert L.lib.sp_gemm_config(dtype, m, n, k, *[C.byref(o) for o in out]) == 0
         assert (out[0].value, out[1].value) != (128, 96)
+
+
+@pytest.mark.parametrize("m,n,k", [(53584, 16, 272), (51392, 16, 120), (60000, 32, 200)])
+def test_tiles_that_are_half_padding_are_not_taken_for_whole_pieces(L, m, n, k):
+    out = [C.c_int32() for _ in range(4)]
+    assert L.lib.sp_gemm_config(1, m, n, k, *[C.byref(o) for o in out]) == 0
+    assert out[1].value <= 64 and (out[0].value, out[1].value) != (128, 64)

@@ -138,6 +138,17 @@ def test_tiles_of_128_by_64_and_96_are_exact(MM, dtype, m, n, k, tile):
             assert torch.equal(c, exact.float().to(TORCH[out])) and (buf[:pad] == -77).all() and (buf[-pad:] == -77).all()
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("m,n,k", [(8370, 332, 8), (8449, 333, 184), (8449, 333, 200), (51392, 16, 120), (55244, 30, 328), (58332, 9, 32)])
+def test_reading_c_may_change_the_tile_but_not_the_sums(MM, dtype, m, n, k):
+    """Where beta takes another tile than the same call without: C of zeros gives the bits of beta = 0."""
+    announce("gemm tile with and without C %s %dx%dx%d" % (dtype, m, n, k))
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, b = (torch.randn((r, k), generator=g, device="cuda").to(TORCH[dtype]) for r in (m, n))
+    want = MM.matmul_abt(a, b, c=torch.full((m, n), float("nan"), device="cuda"))
+    assert torch.equal(MM.matmul_abt(a, b, c=torch.zeros((m, n), device="cuda"), beta=1.0), want)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("m,n,kt", [(1, 1, 1), (17, 3, 6), (31, 33, 6), (130, 31, 5.5), (5000, 5, 2), (16, 4096, 7), (33, 15, 7),
                                     (257, 16, 7.5), (250, 250, 8), (500, 331, 9), (1900, 241, 11), (331, 65, 27.5), (1, 9001, 13),
