@@ -54,10 +54,12 @@ struct EnsembleArgs {
 // of memory, whole lines at a time and once per workgroup.  Read straight into its registers by every wave, a lane a line,
 // the 32 KiB of 64 x 128 take 8 k cycles.  Microseconds of a captured launch, read straight / through LDS: 128-64-16, 8
 // members of 1792 rows 13.8 / 11.6; 96-64-16, 2 of 28448 21.1 / 19.2; a hash of 200-128, 16 of 10240 32.3 / 28.7; 64-32, 7 of
-// 5600 8.0 / 6.7.  Up to 32 inputs, a line or less a row, the barrier costs more: 16-64-64, 8 of 2016 6.3 / 6.7.
+// 5600 8.0 / 6.7.  Up to 32 inputs, a line or less a row, the barrier costs more: 16-64-64, 8 of 2016 6.3 / 6.7.  So it does
+// for the four rows at most of a single layer under a head, up to 128 inputs: 64-64 masked to 2, 8 of 2128 4.8 / 5.6, 128-64 masked to 4,
+// 2 of 984 6.7 / 6.9, but 200-64 masked to 3, 2 of 984 10.7 / 10.3.
 // 16-byte piece p of row r lies at slot p ^ (r & (G - 1)) of the row, G the power of two in the pieces of a row, at most 16: lanes of
 // different rows then read different banks.
-constexpr bool ensemble_through_lds(int kg) { return kg > 4; }
+constexpr bool ensemble_through_lds(int kg, int most_rows) { return kg > (most_rows > EN_MAX_OUT ? 4 : 16); }
 __device__ __forceinline__ int ensemble_swizzle(int pieces) {
     const int g = pieces & -pieces;
     return (g < 16 ? g : 16) - 1;
@@ -74,6 +76,7 @@ __device__ __forceinline__ void ensemble_weights_to_lds(const float* w, int rows
 // past K0 are zeros); ACTION: an action per row is wanted (a uniform per row, from a tensor or a Philox stream)
 template <int KG, bool EXACT, bool ACTION>
 __global__ __launch_bounds__(EN_THREADS) void mlp_ensemble_kernel(const EnsembleArgs a) {
+    constexpr bool LDS = ensemble_through_lds(KG, EN_HIDDEN);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 31, g = lane >> 5;
@@ -87,7 +90,7 @@ __global__ __launch_bounds__(EN_THREADS) void mlp_ensemble_kernel(const Ensemble
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     // ---- the member's weights, once ----
     f32x4 w1v[2][KG];             // [feature tile][j]: W1[e][32 t + r][8 j + 4 g .. + 3]
-    if constexpr (ensemble_through_lds(KG)) {
+    if constexpr (LDS) {
         ensemble_weights_to_lds(a.w1 + (long)e * EN_HIDDEN * K0, EN_HIDDEN, K0, a.per_piece, (unsigned)(size_t)lds, wave, lane);
     } else {
         const float* w1 = a.w1 + (long)e * EN_HIDDEN * K0;
@@ -125,16 +128,16 @@ __global__ __launch_bounds__(EN_THREADS) void mlp_ensemble_kernel(const Ensemble
 
     const long stride = (long)gridDim.x * 4;
     long tile = (long)blockIdx.x * 4 + wave;
-    if constexpr (!ensemble_through_lds(KG)) {
+    if constexpr (!LDS) {
         if (tile >= tiles) return;
     }
     f32x4 xv[KG];
     {
-        const float* xr = x_row(ensemble_through_lds(KG) && tile >= tiles ? 0 : tile);
+        const float* xr = x_row(LDS && tile >= tiles ? 0 : tile);
 #pragma unroll
         for (int j = 0; j < KG; ++j) xv[j] = load_piece(xr, j);
     }
-    if constexpr (ensemble_through_lds(KG)) {
+    if constexpr (LDS) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (tile >= tiles) return;
@@ -602,6 +605,7 @@ __global__ __launch_bounds__(EP_THREADS, 2) void mlp_ensemble_parts_kernel(const
 // MODE 0: policy, 1: policy and action, 2: binarize.
 template <int KG, bool EXACT, int MODE>
 __global__ __launch_bounds__(EN_THREADS) void ensemble_layer_kernel(const EnsembleArgs a) {
+    constexpr bool LDS = ensemble_through_lds(KG, MODE == 2 ? 32 : EN_MAX_OUT);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 31, g = lane >> 5;
@@ -614,7 +618,7 @@ __global__ __launch_bounds__(EN_THREADS) void ensemble_layer_kernel(const Ensemb
 
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     f32x4 wv[KG];                                            // W[e][r][8 j + 4 g .. + 3], rows past NOUT are zeros
-    if constexpr (ensemble_through_lds(KG)) {
+    if constexpr (LDS) {
         ensemble_weights_to_lds(a.w1 + (long)e * N * K0, NOUT, K0, a.per_piece, (unsigned)(size_t)lds, wave, lane);
     } else {
         const float* w = a.w1 + ((long)e * N + (r < NOUT ? r : 0)) * K0 + 4 * g;
@@ -633,16 +637,16 @@ __global__ __launch_bounds__(EN_THREADS) void ensemble_layer_kernel(const Ensemb
 
     const long stride = (long)gridDim.x * 4;
     long tile = (long)blockIdx.x * 4 + wave;
-    if constexpr (!ensemble_through_lds(KG)) {
+    if constexpr (!LDS) {
         if (tile >= tiles) return;
     }
     f32x4 xv[KG];
     {
-        const float* xr = x_row(ensemble_through_lds(KG) && tile >= tiles ? 0 : tile);
+        const float* xr = x_row(LDS && tile >= tiles ? 0 : tile);
 #pragma unroll
         for (int j = 0; j < KG; ++j) xv[j] = load_piece(xr, j);
     }
-    if constexpr (ensemble_through_lds(KG)) {
+    if constexpr (LDS) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (tile >= tiles) return;
@@ -791,9 +795,9 @@ static const void* pick_layer_kernel(int kg, bool exact) {
 
 static int ensemble_launch(const void* kernel, EnsembleArgs& a, hipStream_t stream, const char* what) {
     a.tiles = (a.batch + EN_ROWS - 1) / EN_ROWS;
-    const int pieces = a.k0 / 4, rows = a.w2 != nullptr ? EN_HIDDEN : a.nout;
+    const int pieces = a.k0 / 4, rows = a.w2 != nullptr ? EN_HIDDEN : a.nout, most_rows = a.w2 != nullptr ? EN_HIDDEN : a.words != nullptr ? 32 : EN_MAX_OUT;
     a.per_piece = ((1u << 20) + (unsigned)pieces - 1u) / (unsigned)pieces;
-    const int lds_bytes = a.k0 > 32 ? (rows * pieces + 63) / 64 * 1024 : 0;
+    const int lds_bytes = ensemble_through_lds((a.k0 + 7) / 8, most_rows) ? (rows * pieces + 63) / 64 * 1024 : 0;
     void* args[] = {(void*)&a};
     hipError_t err = hipLaunchKernel(kernel, dim3((unsigned)ensemble_blocks(a.members, a.tiles), (unsigned)a.members), dim3(EN_THREADS), args, lds_bytes, stream);
     if (err != hipSuccess) return fail(SP_ERR_DEVICE, "%s: launch failed: %s", what, hipGetErrorString(err));

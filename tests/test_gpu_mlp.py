@@ -566,6 +566,10 @@ def test_ensemble_weights_of_every_row_length(LY, k0):
     for e, (_, col) in enumerate(picked):
         want = orow.binarize(x.cpu()[:, col].numpy(), 1 << 31)
         assert (host(got[e]).view(np.uint32) == want).all(), e
+    picked = [one_each(4, e) for e in range(members)]             # one layer under a head: four rows, straight or through LDS
+    got = LY.mlp_forward_ensemble(x, (torch.stack([w for w, _ in picked]).cuda(),), None)
+    for e, (_, col) in enumerate(picked):
+        assert torch.equal(got[e].cpu(), x.cpu()[:, col])
     if k0 > 128:
         return                     # (two layers: up to 128 inputs)
     picked = [one_each(64, e) for e in range(members)]
