@@ -1,7 +1,7 @@
 // Fused dense-stack forward for gfx950: stacks of 256-wide hidden layers under a narrow head, on row-major weights, and the
-// entry point of all 16-bit stacks (other hidden widths and wider heads: mlp_any.hip).
+// entry point of all 16-bit stacks (other hidden widths, wider heads and most single hidden layers: mlp_any.hip).
 //
-// mlp_h256_kernel, more than 64 rows per compute unit: every wave owns 16 batch rows and pushes them through ALL layers, so
+// mlp_h256_kernel, more than 64 rows per compute unit or a single hidden layer: every wave owns 16 batch rows and pushes them through ALL layers, so
 // activations never leave the wave's registers: the f32 accumulator fragment of one layer, after bias / ReLU / rounding to 16
 // bits, is bit-for-bit the MFMA operand fragment of the next layer.  (v_mfma_f32_16x16x32_{f16,bf16}: a lane ends up with 4
 // consecutive rows of the first operand.  The weight rows are therefore fed in the order 32 u + 8 (i / 4) + i % 4 for an even
@@ -17,7 +17,7 @@
 //
 // The head (softmax / regret matching / sampling) runs on the last layer's f32 outputs.
 //
-// mlp_split_kernel, at most 64 rows per compute unit (described where it is defined): a wave owns 64 OUTPUT FEATURES of all
+// mlp_split_kernel, at most 64 rows per compute unit of several hidden layers (described where it is defined): a wave owns 64 OUTPUT FEATURES of all
 // 64 rows of the workgroup and the activations are exchanged through LDS.
 //
 // Semantics follow the graph interpreter of ml/layers.spi:194-240 (BlockMatmul = x . w^T with w
@@ -741,6 +741,12 @@ __global__ __launch_bounds__(256) void mlp_split_kernel(const void* x_first, con
 
 using namespace sp;
 
+template <int DT>
+static const void* pick_h256_kernel(bool wide, bool small_k) {
+    if (wide) return small_k ? (const void*)mlp_h256_kernel<DT, 8, 1> : (const void*)mlp_h256_kernel<DT, 8, 4>;
+    return small_k ? (const void*)mlp_h256_kernel<DT, 4, 1> : (const void*)mlp_h256_kernel<DT, 4, 4>;
+}
+
 static const void* pick_split_kernel(int dtype, int ks0) {
     if (dtype == SP_F16) {
         if (ks0 == 1) return (const void*)mlp_split_kernel<SP_F16, 1>;
@@ -802,17 +808,23 @@ extern "C" int sp_mlp_forward(int dtype, const void* x, int32_t n_layers, const 
     // more than 64 rows per compute unit: 8 waves (128 rows) per workgroup halve the rounds
     const int cus = device_cu_count();
     const bool wide = (batch + 63) / 64 > cus;
-    bool h256 = n_layers >= 3;   // two and more hidden layers, all 256 wide
+    bool h256 = n_layers >= 2;   // all hidden layers 256 wide
     for (int i = 1; i < n_layers; ++i) h256 = h256 && dims[i] == 256;
     // A masked head gives probability zero to the columns past the mask whatever their logits are: when the logits
     // themselves are not asked for, the last layer is computed for the valid columns only (the first rows of its
     // weight matrix) and the head fills the rest of each policy row with zeros.  A 64-wide layer with 3 valid
     // columns, the shape the reference's 16-byte row primitives force on a 3-action game, then is a narrow head.
     if (head != SP_HEAD_NONE && logits_out == nullptr && mask_size > 0) a.nout = mask_size;
-    // Other hidden widths, heads of more than 16 outputs, a single hidden layer: mlp_any.hip.  Of stacks with 256-wide layers those two
-    // kinds, too (bf16, us, the kernels here / there: 64-256-64 64 rows 11.4 / 7.4, 40000 32.2 / 16.1, 400000 194 / 92; 64-256-10 10.9 /
-    // 6.5, 23.3 / 12.0, 137 / 65; 128-256-256-256-24 17.0 / 12.0, 44 / 33, 271 / 225), while up to 16 outputs behind two of them stay
-    // (32-256-256-256-3 64 rows 8.0 / 10.7, 40000 20.2 / 24.2; 256-256-256-256-256-6 12.8 / 15.7, 35 / 48).
+    // Other hidden widths and heads of more than 16 outputs: mlp_any.hip (bf16, us, the kernels here / there: 64-256-64 64 rows 11.4 / 7.4,
+    // 40000 32.2 / 16.1, 400000 194 / 92; 128-256-256-256-24 17.0 / 12.0, 44 / 33, 271 / 225; but 32-256-256-256-3 64 rows 8.0 / 10.7, 40000
+    // 20.2 / 24.2, 256-256-256-256-256-6 12.8 / 15.7, 35 / 48).  A single hidden layer stays here for up to eight outputs, whose head never
+    // leaves the registers (64-256-6 97 rows 5.2 / 6.4, 16384 5.4 / 7.7, 24000 5.5 / 11.6, 300000 42 / 46; 64-256-10 97 rows 11.4 / 6.6, 300000
+    // 107 / 48) -- for up to four only as far as a round of 128 rows a unit goes (32-256-4 24000 rows 5.2 / 7.4, 40000 8.6 / 7.6, 300000 36
+    // / 22), and not where half of the first layer's four chunks is padding and the units hold 64 rows at most (128-256-4 4096 rows 7.3 / 6.5,
+    // 24000 8.9 / 10.3; 256-256-4 4096 rows 7.1 / 7.7).
+    const bool one_hidden = n_layers == 2;
+    if (one_hidden)
+        h256 = h256 && a.nout <= 8 && (a.nout > 4 || (batch <= 128l * cus && (wide || dims[0] <= 64 || dims[0] > 128)));
     if (!h256 || a.nout > 16) {
         a.dims[n_layers] = a.nout;
         return mlp_any_launch(dtype, a, (hipStream_t)stream, __func__);
@@ -832,10 +844,10 @@ extern "C" int sp_mlp_forward(int dtype, const void* x, int32_t n_layers, const 
         return mlp_resident_launch(dtype, false, n_layers, r, (hipStream_t)stream, __func__);
     }
     // at most one 64-row workgroup per compute unit: hidden layers split by output features
-    const bool split = !wide;
+    const bool split = !wide && !one_hidden;
     const void* kernel;
     int lds_bytes = MLP_STAGES * MLP_STAGE_BYTES + 1024;   // weight ring + the dummy DMA target
-    int rows_per_block = 128, threads = 512;
+    int rows_per_block = wide ? 128 : 64, threads = 4 * rows_per_block;
     if (split) {
         const int ks0 = dims[0] <= 32 ? 1 : dims[0] <= 64 ? 2 : 8;
         kernel = pick_split_kernel(dtype, ks0);
@@ -843,9 +855,7 @@ extern "C" int sp_mlp_forward(int dtype, const void* x, int32_t n_layers, const 
         rows_per_block = SPLIT_ROWS;
         threads = 256;
     } else {
-        const bool small_k = dims[0] <= 64;
-        if (dtype == SP_F16) kernel = small_k ? (const void*)mlp_h256_kernel<SP_F16, 8, 1> : (const void*)mlp_h256_kernel<SP_F16, 8, 4>;
-        else kernel = small_k ? (const void*)mlp_h256_kernel<SP_BF16, 8, 1> : (const void*)mlp_h256_kernel<SP_BF16, 8, 4>;
+        kernel = dtype == SP_F16 ? pick_h256_kernel<SP_F16>(wide, dims[0] <= 64) : pick_h256_kernel<SP_BF16>(wide, dims[0] <= 64);
     }
     rc = ensure_dynamic_lds(kernel, lds_bytes);
     if (rc != SP_OK) return rc;

@@ -249,6 +249,31 @@ def test_a_hidden_sum_that_is_no_number_becomes_zero(LY, dims, mask, rows_per_un
             assert np.abs(policy[odd, :valid] * valid - 1).max() < 1e-6 and (policy[odd, valid:] == 0).all()
 
 
+@pytest.mark.parametrize("dims,mask,few,many", [([32, 256, 4], 0, "64", "128+1"), ([64, 256, 64], 4, "64+1", "129"), ([80, 256, 3], 0, "64", "64+1"),
+                                                ([128, 256, 2], 0, "128", "128+1"), ([256, 256, 4], 0, "64+1", "130"), ([16, 256, 8], 0, "64", "64+1"),
+                                                ([144, 256, 8], 5, "3", "140"), ([64, 256, 64], 8, "64", "200"), ([64, 256, 12], 9, "64", "129")])
+def test_a_single_hidden_layer_of_256_on_both_sides_of_its_lines(LY, dims, mask, few, many):
+    """Which kernel such a stack runs on goes by the outputs, the inputs and the rows per compute unit: the rows of a batch in front of a
+    line give the bits they give as part of one behind it, with and without biases, against the oracle."""
+    announce("mlp one hidden layer %s mask=%d rows %s / %s" % (dims, mask, few, many))
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    few, many = (int(r.partition("+")[0]) * units + int(r.partition("+")[2] or 0) for r in (few, many))
+    rng = np.random.default_rng(sum(dims) + few)
+    for dtype, with_bias in (("f16", True), ("bf16", False)):
+        x, ws, u = make_problem(rng, many, dims, dtype)
+        biases = [rng.standard_normal(o).astype(np.float32) for o in dims[1:]] if with_bias else None
+        t = TORCH[dtype]
+        xd, wd, ud = dev(x, t), [dev(w, t) for w in ws], dev(u)
+        bd = [dev(b) for b in biases] if with_bias else None
+        for head in ("softmax", "softmax_regret_matching"):
+            part = LY.mlp_forward(xd[:few].contiguous(), wd, bd, head, ud[:few].contiguous(), mask)
+            whole = LY.mlp_forward(xd, wd, bd, head, ud, mask)
+            assert all(torch.equal(p, w[:few]) for p, w in zip(part, whole))
+            assert (host(whole[1]) == orow.discrete_sampling(host(whole[0]), u)).all()
+        want, _, _ = olayers.mlp_forward(x, ws, biases, HEAD_CODE[head], u, dtype, mask or None)
+        assert ogemm.rel_frobenius(host(whole[0]), want) < 2e-4          # (the bound of the other stacks: order of sums, flipped roundings)
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("mask", [1, 3, 13, 16])
 def test_past_a_narrow_mask_are_zeros_behind_a_256_wide_layer(LY, mask, dtype):
