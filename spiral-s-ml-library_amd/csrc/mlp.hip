@@ -34,7 +34,7 @@ namespace sp {
 // shape, all per-lane DMA offsets are computed once, a chunk costs a wave no vector instructions
 // besides its 32 MFMAs and 32 LDS reads, and the DMA instructions are issued one by one between
 // the MFMA groups.  The first layer always runs C0 whole chunks (1 for K0 <= 64, else 4; K-pieces
-// past K0 re-read the last valid piece and meet zero activations), the last layer (at most 16
+// past K0 re-read the last valid piece and meet zero activations), the last layer (at most 32
 // outputs) travels as ONE chunk holding its four 64-column slabs at 64-row spacing and always
 // computes 2 tiles (rows past the outputs are stale but finite-or-not they only reach unused columns).
 template <int DT, int NW, int C0>
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(NW * 64) void mlp_h256_kernel(const MlpArgs a) {
     };
     // KIND 0..3: chunk KIND of a layer, i.e. K-columns 64 KIND .. + 63 for all 16 output tiles (chunk 0
     // starts the accumulators from zero); KIND 4: the last layer, whose chunk holds the K-columns
-    // 64 s .. + 63 of all its (at most 16) outputs in slab s = g / 2 and accumulates into tiles 0 and 1.
+    // 64 s .. + 63 of all its (at most 32) outputs in slab s = g / 2 and accumulates into tiles 0 and 1.
     // FIRST: the chunk behind first_sync (no earlier fetch is waiting for its last DMA instructions).
     auto run_chunk = [&](auto KIND_, auto FIRST_) {
         constexpr int kind = decltype(KIND_)::value;
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(NW * 64) void mlp_h256_kernel(const MlpArgs a) {
         next_activations((const float*)table_ptr(tab_b, layer));
     }
 
-    // ---- last layer: 256 -> NOUT <= 16, one chunk, 2 tiles ----
+    // ---- last layer: 256 -> NOUT <= 32, one chunk, 2 tiles ----
     run_chunk(IC<4>{}, IC<0>{});
     // the dummy DMAs (they land in their own KiB) must be done before the LDS is released; they are
     // long done, and waiting here rather than at the end keeps the outputs' stores out of the wait
@@ -355,7 +355,10 @@ __global__ __launch_bounds__(NW * 64) void mlp_h256_kernel(const MlpArgs a) {
             *reinterpret_cast<f32x4*>(head_rows + j * MLP_MAX_OUT + tile_col(t)) = v;
         }
         // lanes 0..15 of every wave own one batch row each (the staging is wave private)
-        if (lane < 16 && row_ok) head_row<16>(out, head_rows + lane * MLP_MAX_OUT, row, NOUT, limit, u_row);
+        if (lane < 16 && row_ok) {
+            if (NOUT <= 16) head_row<16>(out, head_rows + lane * MLP_MAX_OUT, row, NOUT, limit, u_row);
+            else head_row<32>(out, head_rows + lane * MLP_MAX_OUT, row, NOUT, limit, u_row);
+        }
     }
 }
 
@@ -825,7 +828,9 @@ extern "C" int sp_mlp_forward(int dtype, const void* x, int32_t n_layers, const 
     const bool one_hidden = n_layers == 2;
     if (one_hidden)
         h256 = h256 && a.nout <= 8 && (a.nout > 4 || (batch <= 128l * cus && (wide || dims[0] <= 64 || dims[0] > 128)));
-    if (!h256 || a.nout > 16) {
+    // up to 32 outputs: one round of 128 rows a unit against two of 64 (128-256-256-256-24 24620 rows 24.1 / 27.0)
+    const int most_out = wide && batch <= 128l * cus && a.nout == dims[n_layers] ? 32 : 16;
+    if (!h256 || a.nout > most_out) {
         a.dims[n_layers] = a.nout;
         return mlp_any_launch(dtype, a, (hipStream_t)stream, __func__);
     }

@@ -1,8 +1,8 @@
 // Fused forward of 16-bit stacks of any hidden width (multiples of 32 up to 256) under any head of up to 64 outputs: the stacks
 // that the kernels for 256 wide layers and narrow heads (mlp.hip, mlp_packed.hip, mlp_resident.hip, mlp_pipe.hip) do not take.
 //
-// Two kernels, by how much work there is: up to 64 rows per compute unit the first, beyond that the second (beyond 128 where the weights
-// exceed the LDS).  bf16, us of a captured launch, first / second: 64-128-128-4 4096 rows 5.5 / 8.1, 16384 6.4 / 8.3, 65536 21 / 8.7;
+// Three kernels, by how much work there is: up to 64 rows per compute unit the first, beyond that the second (beyond 128 where the weights
+// exceed the LDS; the third up to there).  bf16, us of a captured launch, first / second: 64-128-128-4 4096 rows 5.5 / 8.1, 16384 6.4 / 8.3, 65536 21 / 8.7;
 // 192-96-64-64 masked to 3, 10061 rows 7.1 / 11.3; 64-192-192-192-4 16384 rows 10.2 / 19, 65536 35 / 20.
 //   mlp_features_kernel: a workgroup of eight or sixteen waves takes R x 16 rows through the stack.  The waves share out a layer's tiles of 16
 // output features; each streams the weights of its own features through a ring in LDS that nobody else reads, so weights need no
@@ -12,6 +12,9 @@
 // there is.
 //   mlp_rows_kernel: all weights of the stack in LDS, loaded once per workgroup; a wave takes 32 rows at a time through the stack
 // with the activations in its registers, no barrier behind the first.  Weights that do not fit stream through a ring, for all waves alike.
+// Workgroups of four waves up to 128 rows per compute unit, so that twice as many units have one (us, eight waves / four: 256-256-16 24620
+// rows 20.0 / 16.6, 128-64-64 masked to 3 9.2 / 8.3, 64-192-24 11.0 / 10.1, 32-64-64-64-10 11.0 / 10.6).
+//   mlp_round_kernel: what does not fit, from 64 to 128 rows per compute unit under up to 32 outputs.
 //
 // Against one kernel of 16 rows a wave with all weights through a ring (us, before / now): 128-64-64 masked to 3, 64 rows 8.9 / 4.2;
 // 80-192-192-192-24, 115 rows 19.4 / 9.4; 80-128-128-128-64-4, 614 rows 16.3 / 7.5; 64-128-128-64, 4096 rows 17.5 / 7.6; 64-128-128-4,
@@ -440,10 +443,10 @@ __global__ __launch_bounds__(AN_FEATURES_THREADS) void mlp_features_kernel(const
 // Weights in LDS in groups of 32 rows x 64 of K (4 KiB): 128-byte rows, piece p of row r in slot p ^ mlp_swz(r).  All of the stack's, once;
 // or (STREAM), where they do not fit, a ring of four stages of one 64 wide step of K each, three steps ahead of the products and on
 // into the next rows, one barrier a step.  HT: 16-wide tiles of the widest hidden layer (8 or 16).
-constexpr int AN_GROUP = 4096, AN_ROWS = 32, AN_THREADS = 512, AN_WAVES = AN_THREADS / 64, AN_STAGE = 8 * AN_GROUP;
+constexpr int AN_GROUP = 4096, AN_ROWS = 32, AN_STAGE = 8 * AN_GROUP;
 
-template <int DT, int HT, bool STREAM>
-__global__ __launch_bounds__(AN_THREADS, 2) void mlp_rows_kernel(unsigned long long widths, unsigned counts, const MlpArgs a) {
+template <int DT, int HT, bool STREAM, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, WAVES / 4) void mlp_rows_kernel(unsigned long long widths, unsigned counts, const MlpArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -451,17 +454,17 @@ __global__ __launch_bounds__(AN_THREADS, 2) void mlp_rows_kernel(unsigned long l
     const bool all_256 = HT == 16 && (counts & AN_ALL_256);
     const int NL = (int)(counts & 0x7fu);
     const unsigned lds0 = (unsigned)(size_t)lds;
-    const long tiles = (a.batch + AN_ROWS - 1) / AN_ROWS, step = (long)gridDim.x * AN_WAVES;
+    const long tiles = (a.batch + AN_ROWS - 1) / AN_ROWS, step = (long)gridDim.x * WAVES;
     const int r8 = lane >> 3;
     int f_layer = 0, f_k = 0, f_stage = 0;                // the next step of K to fetch
-    long f_tile = (long)blockIdx.x * AN_WAVES;            // (of wave 0: the waves go through the same steps)
+    long f_tile = (long)blockIdx.x * WAVES;            // (of wave 0: the waves go through the same steps)
     // one 64 wide step of K of a layer, this wave's share of its 4 gn instructions; returns their number
     auto fetch_step = [&](unsigned at) {
         const int K = any_width(widths, f_layer), F = f_layer + 1 < NL ? any_width(widths, f_layer + 1) : (int)(counts >> 8);
         const unsigned char* const W = (const unsigned char*)a.w[f_layer];
         const int instructions = 4 * ((F + 31) >> 5);
         int count = 0;
-        for (int b = wave; b < instructions; b += AN_WAVES) {
+        for (int b = wave; b < instructions; b += WAVES) {
             const int r = 8 * b + r8;                     // instruction b fetches rows 8 b .. + 7
             int k = 64 * f_k + 8 * ((lane & 7) ^ mlp_swz(r));
             k = k <= K - 8 ? k : K - 8;                   // past K: meets zeros, or is not read
@@ -511,7 +514,9 @@ __global__ __launch_bounds__(AN_THREADS, 2) void mlp_rows_kernel(unsigned long l
     auto begin_step = [&]() {
         if constexpr (STREAM) {
             const int young = ahead[1] + ahead[2];        // what may be outstanding was asked for later
-            if (young >= 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+            if (young >= 16) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+            else if (young >= 12) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+            else if (young >= 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
             else if (young >= 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
             else if (young >= 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
             else if (young >= 2) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
@@ -590,7 +595,7 @@ __global__ __launch_bounds__(AN_THREADS, 2) void mlp_rows_kernel(unsigned long l
                 else if (32 * s < K0) x[rt][s] = *reinterpret_cast<const u32x4*>(q < 2 ? xr + 64 * s : (const unsigned char*)kZeroChunk);     // K ends in mid-step: zeros
         }
     };
-    for (long tile = (long)blockIdx.x * AN_WAVES + wave; STREAM ? tile - wave < tiles : tile < tiles; tile += step) {
+    for (long tile = (long)blockIdx.x * WAVES + wave; STREAM ? tile - wave < tiles : tile < tiles; tile += step) {
         int K0 = any_width(widths, 0), N = (int)(counts >> 8);
         asm volatile("" : "+s"(K0), "+s"(N));             // (or every comparison with them is kept over the loop)
         const long row0 = tile * AN_ROWS;
@@ -700,16 +705,259 @@ __global__ __launch_bounds__(AN_THREADS, 2) void mlp_rows_kernel(unsigned long l
     }
 }
 
+// ---- 65 to 128 rows per compute unit of stacks that do not fit the LDS: a round of workgroups of 128 rows -----------------------
+// Eight waves, 16 batch rows per wave: every wave pushes its rows through ALL layers with the activations in its registers, as in the
+// kernel of 256 wide layers (mlp.hip), whose weight stream -- chunks of 64 K-columns through a ring of four LDS stages, three
+// ahead, one barrier a chunk -- this is for any hidden width.  Two rounds of mlp_features_kernel, or four waves of 32 rows a unit, take longer
+// (us, this / mlp_features_kernel / mlp_rows_kernel, 24620 rows: 48-256-256-32-64 masked to 4 18.1 / 20.0 / 20.5, 64-256-256-128-6 18.0 / 22.3 /
+// 23.8, 128-192-192-192-4 18.7 / 19.7 / 20.3, 128-128-128-128-128-128-128-20 23.5 / 24.0 / 23.5); more than 32 computed outputs, whose head is a chain
+// of one lane's own here, do not gain (256-224-256-256-64 33.9 / 31.5 / 36.2).
+constexpr int AN_ROUND_WAVES = 8, AN_ROUND_ROWS = 16 * AN_ROUND_WAVES, AN_ROUND_OUT = 32;
+constexpr int AN_ROUND_LDS = MLP_STAGES * MLP_STAGE_BYTES + 1024;     // the ring, and what the loads that keep the count go to
+
+template <int DT>
+__global__ __launch_bounds__(AN_ROUND_WAVES * 64) void mlp_round_kernel(const MlpArgs a) {
+    constexpr int NW = AN_ROUND_WAVES, MLP_ROWS = AN_ROUND_ROWS;
+    constexpr int MLP_DMA_PER_WAVE = MLP_MAX_DIM / 8 / NW;         // of 1 KiB, in a full chunk
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15;       // batch row inside the wave's 16-row tile; weight row inside a 16-row tile
+    const int q = lane >> 4;       // which 8 of the 32 K-values of an MFMA step this lane feeds
+    const long row = (long)blockIdx.x * MLP_ROWS + wave * 16 + j;
+    const bool row_ok = row < a.batch;
+    const unsigned lds_base = (unsigned)(size_t)lds;
+    const unsigned dummy_dst = lds_base + MLP_STAGES * MLP_STAGE_BYTES;
+
+    // ---- weight chunk pipeline: chunk = (layer, 64-column slab c) ----
+    int pf_layer = 0, pf_c = 0;    // next chunk to fetch
+    int pf_stage = 0;
+    auto fetch_next_chunk = [&]() {
+        const bool live = pf_layer < a.n_layers;
+        const int layer = live ? pf_layer : 0;
+        const int K = a.dims[layer], N = a.dims[layer + 1];
+        const unsigned char* W = (const unsigned char*)a.w[layer];
+        const int n_instr = live ? (N + 7) / 8 : 0;            // 8 weight rows (128 bytes each) per instruction
+#pragma unroll
+        for (int m = 0; m < MLP_DMA_PER_WAVE; ++m) {
+            const int ii = wave + NW * m;
+            if (ii < n_instr) {
+                int n = ii * 8 + (lane >> 3);
+                const int piece = (lane & 7) ^ mlp_swz(n);        // the K piece that belongs in LDS slot lane & 7
+                n = n < N ? n : N - 1;                             // rows past N: any valid row, never used
+                int k = pf_c * 64 + piece * 8;
+                k = k <= K - 8 ? k : K - 8;                        // pieces past K: multiplied by zero activations
+                mlp_dma(W, (unsigned)((n * K + k) * 2), lds_base + pf_stage * MLP_STAGE_BYTES + ii * 1024);
+            } else {
+                mlp_dma((const unsigned char*)a.w[0], 0u, dummy_dst);  // keeps the per-chunk DMA count fixed
+            }
+        }
+        if (live) {
+            ++pf_c;
+            if (pf_c * 64 >= K) { pf_c = 0; ++pf_layer; }
+        }
+        pf_stage = (pf_stage + 1) & (MLP_STAGES - 1);
+    };
+    fetch_next_chunk();
+    fetch_next_chunk();
+    fetch_next_chunk();
+
+    // ---- the wave's input rows as MFMA operand fragments: for step s (32 K-values) lane (j, q)
+    //      holds x[row][32 s + 8 q .. + 7] ----
+    u32x4 act[MLP_MAX_DIM / 32];
+    {
+        const int K0 = a.dims[0];
+        const unsigned char* xr = (const unsigned char*)a.x + row * K0 * 2;
+#pragma unroll
+        for (int s = 0; s < MLP_MAX_DIM / 32; ++s) {
+            u32x4 v = {0u, 0u, 0u, 0u};
+            if (row_ok && 32 * s + 8 * q < K0) v = *reinterpret_cast<const u32x4*>(xr + (32 * s + 8 * q) * 2);
+            act[s] = v;
+        }
+    }
+
+    f32x4 acc[MLP_MAX_DIM / 16];
+    int stage = 0;
+    // LDS byte offset of this lane's 16-byte weight piece for the first tile of a chunk: lane j feeds
+    // weight row n0 = 8 (j / 4) + j % 4 of the 32-row group, K piece 4 sp + q (sp = which 32-wide step
+    // of the chunk).  Tile t adds (t / 2) * 32 + (t % 2) * 4 rows, which leaves swz() unchanged.
+    const int n0 = 8 * (j >> 2) + (j & 3);
+    unsigned frag_off[2];
+#pragma unroll
+    for (int sp = 0; sp < 2; ++sp) frag_off[sp] = (unsigned)(n0 * 128 + (((4 * sp + q) ^ mlp_swz(n0)) << 4));
+    auto tile_off = [](int t) { return ((t >> 1) * 32 + (t & 1) * 4) * 128; };
+    auto tile_col = [&](int t) { return 32 * (t >> 1) + 4 * (t & 1) + 8 * q; };  // first of this lane's 4 columns
+    // per-wave f32 staging of the last layer's outputs; it reuses the first weight stage once every
+    // wave is done with the weights
+    float* head_rows = reinterpret_cast<float*>(lds) + wave * 16 * MLP_MAX_OUT;
+    static_assert(NW * 16 * MLP_MAX_OUT * 4 <= MLP_STAGE_BYTES, "head staging must fit one weight stage");
+
+    for (int layer = 0; layer < a.n_layers; ++layer) {
+        const int K = a.dims[layer], N = a.dims[layer + 1];
+        const int nt = 2 * ((N + 31) / 32);   // output tiles come in pairs covering 32 columns
+        const bool last = layer + 1 == a.n_layers;
+#pragma unroll
+        for (int t = 0; t < MLP_MAX_DIM / 16; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+        for (int c = 0; c < MLP_MAX_DIM / 64; ++c) {
+            if (c * 64 < K) {
+                // the two newer chunks may still be in flight; everything older has landed
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * MLP_DMA_PER_WAVE) : "memory");
+                __syncthreads();
+                fetch_next_chunk();   // into the stage every wave finished reading before this barrier
+                const unsigned char* st = lds + stage * MLP_STAGE_BYTES;
+                // Output tiles are walked in groups of 4 (64 columns) with one uniform branch per
+                // group, so that the 8 or 16 LDS reads and the MFMAs of a group form one straight
+                // line the scheduler can overlap.  A partly filled last group multiplies whatever
+                // the stage holds past row N; those columns are never used.
+                const bool two_steps = c * 64 + 32 < K;
+                auto mma = [&](int t, int sp, const u32x4& w) {
+                    // weights are the first operand: the result fragment is (n, batch row)
+                    if constexpr (DT == SP_F16)
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            __builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, act[2 * c + sp]), acc[t], 0, 0, 0);
+                    else
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            __builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, act[2 * c + sp]), acc[t], 0, 0, 0);
+                };
+                auto read = [&](int t, int sp) {
+                    return *reinterpret_cast<const u32x4*>(st + frag_off[sp] + tile_off(t));
+                };
+                if (nt == MLP_MAX_DIM / 16 && two_steps) {
+                    // full-width chunk: 8 groups of (4 tiles, one 32-wide step), software pipelined by
+                    // hand: the weight pieces of group g + 2 are requested before the MFMAs of group g
+                    // (with one wave per SIMD nothing else hides the LDS latency)
+                    u32x4 w[3][4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) w[0][t] = read(t, 0);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) w[1][t] = read(t, 1);
+#pragma unroll
+                    for (int g = 0; g < 8; ++g) {
+                        if (g + 2 < 8) {
+#pragma unroll
+                            for (int t = 0; t < 4; ++t) w[(g + 2) % 3][t] = read(((g + 2) >> 1) * 4 + t, (g + 2) & 1);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) mma((g >> 1) * 4 + t, g & 1, w[g % 3][t]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                } else {
+#pragma unroll
+                    for (int g4 = 0; g4 < MLP_MAX_DIM / 64; ++g4) {
+                        if (g4 * 4 < nt) {
+                            u32x4 w0[4], w1[4];
+#pragma unroll
+                            for (int t = 0; t < 4; ++t) w0[t] = read(g4 * 4 + t, 0);
+                            if (two_steps) {
+#pragma unroll
+                                for (int t = 0; t < 4; ++t) w1[t] = read(g4 * 4 + t, 1);
+                            }
+#pragma unroll
+                            for (int t = 0; t < 4; ++t) mma(g4 * 4 + t, 0, w0[t]);
+                            if (two_steps) {
+#pragma unroll
+                                for (int t = 0; t < 4; ++t) mma(g4 * 4 + t, 1, w1[t]);
+                            }
+                        }
+                    }
+                }
+                stage = (stage + 1) & (MLP_STAGES - 1);
+            }
+        }
+
+        // ---- layer epilogue: in tile t lane (j, q) holds columns tile_col(t) + 0..3 of batch row j;
+        //      tiles 2 s and 2 s + 1 together give it columns 32 s + 8 q .. + 7 ----
+        const float* bias = a.b[layer];
+#pragma unroll
+        for (int t = 0; t < MLP_MAX_DIM / 16; ++t) {
+            if (t < nt && bias != nullptr) {
+                const int n = tile_col(t);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (n + r < N) acc[t][r] += bias[n + r];
+            }
+        }
+        if (!last) {
+#pragma unroll
+            for (int s = 0; s < MLP_MAX_DIM / 32; ++s) {
+                u32x4 v = {0u, 0u, 0u, 0u};
+                if (32 * s < N) {
+                    const f32x4 lo = acc[2 * s], hi = acc[2 * s + 1];
+                    v.x = relu_pack2<DT>(lo[0], lo[1]);
+                    v.y = relu_pack2<DT>(lo[2], lo[3]);
+                    v.z = relu_pack2<DT>(hi[0], hi[1]);
+                    v.w = relu_pack2<DT>(hi[2], hi[3]);
+                }
+                act[s] = v;
+            }
+        } else {
+            __syncthreads();   // all waves have read their last weight chunk: the stage can be reused
+#pragma unroll
+            for (int t = 0; t < AN_ROUND_OUT / 16; ++t) {
+                if (t < nt) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) head_rows[j * MLP_MAX_OUT + tile_col(t) + r] = acc[t][r];
+                }
+            }
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // drain the dummy DMAs before the LDS is released
+
+    // ---- head: lanes 0..15 of every wave own one batch row each (the staging is wave private) ----
+    const int N = a.dims[a.n_layers];
+    const int limit = a.mask_size > 0 ? a.mask_size : N;
+    float past = 0.f;
+    if (lane < 16 && row_ok) {
+        float* p = head_rows + lane * MLP_MAX_OUT;   // this row's outputs
+        const float u = a.ph.philox_mode >= 0 ? reference_row_uniform(a.ph, row) : a.action != nullptr ? a.u[row] : 1.f;
+        // narrow heads run in registers, at the smallest width that holds them: the head is a chain of this lane's own (batch
+        // 64, us, always 64 columns / these widths: 64-64-64-10 14.9 / 10.0, 64-96-96-16 16.7 / 11.8, 128-64-24 14.1 / 10.2)
+        if (N <= 8) head_row<8>(head_out(a), p, row, N, limit, u, N, &past);
+        else if (N <= 16) head_row<16>(head_out(a), p, row, N, limit, u);
+        else head_row<AN_ROUND_OUT>(head_out(a), p, row, N, limit, u);
+    }
+    if (a.out_stride > N) {
+        // a masked head computed for its valid columns only (N < 8): the wave fills the rest of its 16 policy rows, 16 bytes
+        // per lane where rows are whole pieces, the columns in front of the first whole piece by the row's own lane
+        const int stride = a.out_stride, s4 = stride >> 2, c0 = stride % 4 == 0 ? (N + 3) >> 2 : s4 + 1;
+        if (lane < 16 && row_ok)
+            for (int c = N; c < stride && c < 4 * c0; ++c) a.policy[row * stride + c] = past;
+        if (c0 < s4) {
+            const long first = (long)blockIdx.x * MLP_ROWS + wave * 16;
+            int r = lane / s4, c = lane - r * s4;
+            const int dr = 64 / s4, dc = 64 - dr * s4;
+            for (int idx = lane; idx < 16 * s4; idx += 64) {      // (16 s4 is a multiple of 16: the lanes of the rows stay in)
+                const float v = __shfl(past, r);
+                if (c >= c0 && first + r < a.batch) *reinterpret_cast<float4*>(a.policy + (first + r) * stride + 4 * c) = make_float4(v, v, v, v);
+                r += dr;
+                c += dc;
+                if (c >= s4) {
+                    c -= s4;
+                    ++r;
+                }
+            }
+        }
+    }
+}
+
 // ---- host -------------------------------------------------------------------------------------------------------------------------
 template <int DT>
 static const void* pick_features_kernel(int r) {
     return r == 1 ? (const void*)mlp_features_kernel<DT, 1> : r == 2 ? (const void*)mlp_features_kernel<DT, 2> : (const void*)mlp_features_kernel<DT, 4>;
 }
 
+template <int DT, int WAVES>
+static const void* pick_rows_kernel_waves(int widest, bool stream_weights) {
+    if (widest <= 128) return stream_weights ? (const void*)mlp_rows_kernel<DT, 8, true, WAVES> : (const void*)mlp_rows_kernel<DT, 8, false, WAVES>;
+    return stream_weights ? (const void*)mlp_rows_kernel<DT, 16, true, WAVES> : (const void*)mlp_rows_kernel<DT, 16, false, WAVES>;
+}
 template <int DT>
-static const void* pick_rows_kernel(int widest, bool stream_weights) {
-    if (widest <= 128) return stream_weights ? (const void*)mlp_rows_kernel<DT, 8, true> : (const void*)mlp_rows_kernel<DT, 8, false>;
-    return stream_weights ? (const void*)mlp_rows_kernel<DT, 16, true> : (const void*)mlp_rows_kernel<DT, 16, false>;
+static const void* pick_rows_kernel(int widest, bool stream_weights, int waves) {
+    return waves == 4 ? pick_rows_kernel_waves<DT, 4>(widest, stream_weights) : pick_rows_kernel_waves<DT, 8>(widest, stream_weights);
 }
 
 int mlp_any_launch(int dtype, const MlpArgs& a, hipStream_t stream, const char* what) {
@@ -730,11 +978,24 @@ int mlp_any_launch(int dtype, const MlpArgs& a, hipStream_t stream, const char* 
     }
     unsigned counts = (unsigned)NL | (all_256 ? AN_ALL_256 : 0u) | (unsigned)N << 8;
     const bool stream_weights = group_bytes > AN_LDS;
+    // of a masked head with at most seven valid columns only those are computed here, else all (what lies past them needs one of its own)
+    const int outputs = N <= 7 ? N : a.out_stride;
+    if (stream_weights && !all_256 && outputs <= AN_ROUND_OUT && a.batch > 64 * cus && a.batch <= AN_ROUND_ROWS * cus) {
+        const void* kernel = dtype == SP_F16 ? (const void*)mlp_round_kernel<SP_F16> : (const void*)mlp_round_kernel<SP_BF16>;
+        int rc = ensure_dynamic_lds(kernel, AN_ROUND_LDS);
+        if (rc != SP_OK) return rc;
+        MlpArgs whole = a;
+        whole.dims[NL] = outputs;
+        void* args[] = {(void*)&whole};
+        const hipError_t e = hipLaunchKernel(kernel, dim3((unsigned)((a.batch + AN_ROUND_ROWS - 1) / AN_ROUND_ROWS)), dim3(64 * AN_ROUND_WAVES), args, AN_ROUND_LDS, stream);
+        if (e != hipSuccess) return fail(SP_ERR_DEVICE, "%s: launch failed: %s", what, hipGetErrorString(e));
+        return check_launch(what);
+    }
     if (a.batch > (stream_weights ? 128 : 64) * cus) {
-        const void* kernel = dtype == SP_F16 ? pick_rows_kernel<SP_F16>(widest, stream_weights) : pick_rows_kernel<SP_BF16>(widest, stream_weights);
+        const long tiles = (a.batch + AN_ROWS - 1) / AN_ROWS, per_block = tiles <= 4 * cus ? 4 : 8;
+        const void* kernel = dtype == SP_F16 ? pick_rows_kernel<SP_F16>(widest, stream_weights, (int)per_block) : pick_rows_kernel<SP_BF16>(widest, stream_weights, (int)per_block);
         int rc = ensure_dynamic_lds(kernel, AN_LDS);
         if (rc != SP_OK) return rc;
-        const long tiles = (a.batch + AN_ROWS - 1) / AN_ROWS, per_block = AN_THREADS / 64;
         const long most = (tiles + per_block - 1) / per_block, blocks = most < cus ? most : cus;
         void* args[] = {(void*)&widths, (void*)&counts, (void*)&a};
         const hipError_t e = hipLaunchKernel(kernel, dim3((unsigned)blocks), dim3(64 * per_block), args, stream_weights ? 4 * AN_STAGE : (size_t)group_bytes, stream);
@@ -770,7 +1031,7 @@ namespace {
 struct MlpAnyKernelNames {
     MlpAnyKernelNames() {
         register_kernel("mlp_forward", (const void*)mlp_features_kernel<SP_F16, 1>, AN_FEATURES_THREADS);
-        register_kernel("mlp_forward_wide", (const void*)mlp_rows_kernel<SP_F16, 16, false>, AN_THREADS);
+        register_kernel("mlp_forward_wide", (const void*)mlp_rows_kernel<SP_F16, 16, false, 8>, 512);
     }
 } mlp_any_kernel_names;
 }  // namespace

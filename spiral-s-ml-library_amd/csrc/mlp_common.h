@@ -143,9 +143,10 @@ __device__ __forceinline__ HeadOut head_out(const MlpArgs& a) {
     return HeadOut{a.policy, a.action, a.logits, a.head, a.out_stride};
 }
 
+// `past` (N < MAXN only): receives what a column past the mask gets -- 0, or NaN where the row's sum is NaN.
 template <int MAXN>
 __device__ __forceinline__ void head_row(const HeadOut& o, const float* src, long row, int N, int limit, float u,
-                                         int fill_end = 1 << 30) {
+                                         int fill_end = 1 << 30, float* past = nullptr) {
     float p[MAXN];
 #pragma unroll
     for (int n = 0; n < MAXN; ++n) p[n] = n < N ? src[n] : 0.f;
@@ -185,6 +186,7 @@ __device__ __forceinline__ void head_row(const HeadOut& o, const float* src, lon
 #pragma unroll
         for (int n = 0; n < MAXN; ++n) p[n] = s != 0.f ? p[n] * inv : (n < limit ? inv_len : 0.f);
     }
+    if (past != nullptr) *past = p[MAXN - 1];
 #pragma unroll
     for (int n = 0; n < MAXN; ++n)
         if (n < N) o.policy[row * o.stride + n] = p[n];

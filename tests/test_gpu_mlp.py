@@ -274,6 +274,38 @@ def test_a_single_hidden_layer_of_256_on_both_sides_of_its_lines(LY, dims, mask,
         assert ogemm.rel_frobenius(host(whole[0]), want) < 2e-4          # (the bound of the other stacks: order of sums, flipped roundings)
 
 
+@pytest.mark.parametrize("dims,mask", [([48, 256, 256, 32, 64], 4), ([48, 256, 256, 32, 64], 9), ([64, 256, 224, 128, 6], 0), ([128, 192, 192, 192, 12], 5),
+                                       ([128, 256, 256, 32], 0), ([112, 256, 256, 256, 24], 17), ([128, 256, 256, 64], 20), ([128] * 7 + [30], 0),
+                                       ([256, 256, 16], 0), ([32, 64, 64, 64, 10], 0), ([128, 64, 64], 3)])
+def test_a_round_of_128_rows_per_unit(LY, dims, mask):
+    """Between 64 and 128 rows per compute unit other forms run than below and above: the rows of a batch just behind the first line and
+    just in front of the second give the bits they give as part of one behind it, a row of NaNs among them, with biases and without, and
+    nothing outside the policy is written."""
+    announce("mlp round of 128 rows %s mask=%d" % (dims, mask))
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    many = 128 * units + 77
+    rng = np.random.default_rng(sum(dims) + mask)
+    for dtype, with_bias, head in (("f16", True, "softmax"), ("bf16", False, "softmax_regret_matching")):
+        x, ws, u = make_problem(rng, many, dims, dtype)
+        x[5], x[17, 3] = np.nan, np.inf
+        t, n = TORCH[dtype], dims[-1]
+        xd, wd, ud = dev(x, t), [dev(w, t) for w in ws], dev(u)
+        biases = [rng.standard_normal(o).astype(np.float32) for o in dims[1:]] if with_bias else None
+        bd = [dev(b) for b in biases] if with_bias else None
+        whole = LY.mlp_forward(xd, wd, bd, head, ud, mask)
+        for rows in (64 * units, 64 * units + 1, 100 * units + 3, 128 * units):
+            buf = torch.full((64 + rows * n + 64,), -9.0, device="cuda")
+            policy = buf[64:64 + rows * n].view(rows, n)
+            _, action = LY.mlp_forward(xd[:rows].contiguous(), wd, bd, head, ud[:rows].contiguous(), mask, policy_out=policy)
+            assert torch.equal(policy.nan_to_num(7), whole[0][:rows].nan_to_num(7)) and torch.equal(action, whole[1][:rows])
+            assert (buf[:64] == -9).all() and (buf[-64:] == -9).all()
+        plain = np.ones(many, bool)
+        plain[[5, 17]] = False
+        want, _, _ = olayers.mlp_forward(x[plain], ws, biases, HEAD_CODE[head], u[plain], dtype, mask or None)
+        got = host(whole[0])[plain]
+        assert ogemm.rel_frobenius(got, want) < 2e-4 and (host(whole[1])[plain] == orow.discrete_sampling(got, u[plain])).all()
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("mask", [1, 3, 13, 16])
 def test_past_a_narrow_mask_are_zeros_behind_a_256_wide_layer(LY, mask, dtype):
