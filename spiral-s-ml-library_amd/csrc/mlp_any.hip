@@ -14,7 +14,7 @@
 // with the activations in its registers, no barrier behind the first.  Weights that do not fit stream through a ring, for all waves alike.
 // Workgroups of four waves up to 128 rows per compute unit, so that twice as many units have one (us, eight waves / four: 256-256-16 24620
 // rows 20.0 / 16.6, 128-64-64 masked to 3 9.2 / 8.3, 64-192-24 11.0 / 10.1, 32-64-64-64-10 11.0 / 10.6).
-//   mlp_round_kernel: what does not fit, from 64 to 128 rows per compute unit under up to 32 outputs.
+//   mlp_round_kernel: from 64 to 128 rows per compute unit what does not fit, under up to 32 outputs, and some short stacks.
 //
 // Against one kernel of 16 rows a wave with all weights through a ring (us, before / now): 128-64-64 masked to 3, 64 rows 8.9 / 4.2;
 // 80-192-192-192-24, 115 rows 19.4 / 9.4; 80-128-128-128-64-4, 614 rows 16.3 / 7.5; 64-128-128-64, 4096 rows 17.5 / 7.6; 64-128-128-4,
@@ -705,13 +705,15 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void mlp_rows_kernel(unsigne
     }
 }
 
-// ---- 65 to 128 rows per compute unit of stacks that do not fit the LDS: a round of workgroups of 128 rows -----------------------
+// ---- 65 to 128 rows per compute unit, mostly of stacks that do not fit the LDS: a round of workgroups of 128 rows -----------------------
 // Eight waves, 16 batch rows per wave: every wave pushes its rows through ALL layers with the activations in its registers, as in the
 // kernel of 256 wide layers (mlp.hip), whose weight stream -- chunks of 64 K-columns through a ring of four LDS stages, three
 // ahead, one barrier a chunk -- this is for any hidden width.  Two rounds of mlp_features_kernel, or four waves of 32 rows a unit, take longer
 // (us, this / mlp_features_kernel / mlp_rows_kernel, 24620 rows: 48-256-256-32-64 masked to 4 18.1 / 20.0 / 20.5, 64-256-256-128-6 18.0 / 22.3 /
 // 23.8, 128-192-192-192-4 18.7 / 19.7 / 20.3, 128-128-128-128-128-128-128-20 23.5 / 24.0 / 23.5); more than 32 computed outputs, whose head is a chain
-// of one lane's own here, do not gain (256-224-256-256-64 33.9 / 31.5 / 36.2).
+// of one lane's own here, do not gain (256-224-256-256-64 33.9 / 31.5 / 36.2).  So do, where weights fit, stacks of up to two hidden layers under
+// five to sixteen outputs, whose head is a large part (this / mlp_rows_kernel, 27000 rows: 128-192-10 10.8 / 12.0, 256-192-10 14.6 / 15.3, 32-64-64-10
+// 9.1 / 9.6; the other way 256-224-16 16.5 / 15.5, and with three hidden layers 192-96-96-96-6 15.4 / 13.8).
 constexpr int AN_ROUND_WAVES = 8, AN_ROUND_ROWS = 16 * AN_ROUND_WAVES, AN_ROUND_OUT = 32;
 constexpr int AN_ROUND_LDS = MLP_STAGES * MLP_STAGE_BYTES + 1024;     // the ring, and what the loads that keep the count go to
 
@@ -980,7 +982,8 @@ int mlp_any_launch(int dtype, const MlpArgs& a, hipStream_t stream, const char* 
     const bool stream_weights = group_bytes > AN_LDS;
     // of a masked head with at most seven valid columns only those are computed here, else all (what lies past them needs one of its own)
     const int outputs = N <= 7 ? N : a.out_stride;
-    if (stream_weights && !all_256 && outputs <= AN_ROUND_OUT && a.batch > 64 * cus && a.batch <= AN_ROUND_ROWS * cus) {
+    const bool short_stack = NL <= 3 && outputs > 4 && outputs <= 16;
+    if ((stream_weights || short_stack) && !all_256 && outputs <= AN_ROUND_OUT && a.batch > 64 * cus && a.batch <= AN_ROUND_ROWS * cus) {
         const void* kernel = dtype == SP_F16 ? (const void*)mlp_round_kernel<SP_F16> : (const void*)mlp_round_kernel<SP_BF16>;
         int rc = ensure_dynamic_lds(kernel, AN_ROUND_LDS);
         if (rc != SP_OK) return rc;

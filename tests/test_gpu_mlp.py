@@ -276,7 +276,8 @@ def test_a_single_hidden_layer_of_256_on_both_sides_of_its_lines(LY, dims, mask,
 
 @pytest.mark.parametrize("dims,mask", [([48, 256, 256, 32, 64], 4), ([48, 256, 256, 32, 64], 9), ([64, 256, 224, 128, 6], 0), ([128, 192, 192, 192, 12], 5),
                                        ([128, 256, 256, 32], 0), ([112, 256, 256, 256, 24], 17), ([128, 256, 256, 64], 20), ([128] * 7 + [30], 0),
-                                       ([256, 256, 16], 0), ([32, 64, 64, 64, 10], 0), ([128, 64, 64], 3)])
+                                       ([256, 256, 16], 0), ([32, 64, 64, 64, 10], 0), ([128, 64, 64], 3), ([256, 192, 10], 0), ([32, 64, 64, 5], 0),
+                                       ([48, 128, 16], 7)])
 def test_a_round_of_128_rows_per_unit(LY, dims, mask):
     """Between 64 and 128 rows per compute unit other forms run than below and above: the rows of a batch just behind the first line and
     just in front of the second give the bits they give as part of one behind it, a row of NaNs among them, with biases and without, and
