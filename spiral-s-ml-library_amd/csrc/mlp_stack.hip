@@ -272,8 +272,10 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
         int row = tile * ST_ROWS + r;
         row = row < a.batch ? row : a.batch - 1;
         const float* xr = a.x + (long)row * k0 + 4 * q;
-        // (a load that only some lanes take part in is waited for where the others go on: at most the last one is of that kind.
-        // 108-64-32, 48 rows: 5 k cycles for the inputs with every load of that kind.)
+        // (a load that only some lanes take part in is waited for where the others go on.  Up to eight of them: at most the last one is of
+        // that kind, 108-64-32, 48 rows, 5 k cycles for the inputs otherwise.  Up to four: the branches cost more, 32-16-64 relu, 7280 rows x 16
+        // 12.7 us without them, 13.5 with, 60-16-16-4 17024 rows 8.0, 8.4 -- but where every block is whole.)
+        constexpr bool WHOLE = !PARTS && (HT == 8 || FULL);
         if (!PARTS && k0 < 16) {
 #pragma unroll
             for (int j = 0; j < HT; ++j) x[j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -282,7 +284,7 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
         }
 #pragma unroll
         for (int j = 0; j < HT; ++j) {
-            if (!PARTS && 16 * j + 16 <= k0) {
+            if (WHOLE && 16 * j + 16 <= k0) {
                 x[j] = *reinterpret_cast<const f32x4*>(xr + 16 * j);
             } else {
                 x[j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -322,7 +324,10 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
             const unsigned per_kt = a.per_kt[l];
             for (int b = wave; b < kt * nt; b += waves) {
                 int tile, block;
-                if (b < kt * whole) {
+                if (nt == 1) {
+                    tile = 0;
+                    block = b;
+                } else if (b < kt * whole) {
                     const int turn = b >> log_group, group = (int)((unsigned)turn * per_kt >> 16);
                     tile = (group << log_group) + (b & ((1 << log_group) - 1));
                     block = turn - group * kt;
