@@ -265,7 +265,6 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
     const int waves = blockDim.x >> 6;
     const int r = lane & 15, q = lane >> 4;
     const int e = blockIdx.y;
-    const float NEG_INF = -__builtin_inff();
     const int layers = a.n_layers, k0 = a.dims[0], kt0 = (k0 + 15) >> 4;
 
     auto load_x = [&](int tile, f32x4 (&x)[HT]) {
@@ -538,7 +537,6 @@ __global__ __launch_bounds__(SF_MAX_THREADS) void stack_features_kernel(const fl
     const int acts_bytes = planes * PLANE;
     const int row0 = blockIdx.x * (ST_ROWS * R);
     const unsigned lds0 = (unsigned)(size_t)lds;
-    const float NEG_INF = -__builtin_inff();
     auto width = [&](int l) { return (int)((unsigned)(widths >> (8 * l)) & 0xffu) << 2; };
     auto outputs_of = [&](int l) { return l + 1 < NL ? width(l + 1) : N; };
     const int K0 = width(0);
@@ -840,7 +838,7 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
                 if (l > 0 && dims[l] / 16 > most_tiles) most_tiles = dims[l] / 16;
             }
             const int waves = most_tiles < 4 ? 4 : most_tiles > 8 ? 8 : most_tiles;
-            for (int l = 0; l < n_layers; ++l) units += (dims[l] + 31) / 32 * (((l + 1 < n_layers ? dims[l + 1] : a.mask_size) + 15) / 16 + waves - 1) / waves;
+            for (int l = 0; l < n_layers; ++l) units += (dims[l] + 31) / 32 * ((((l + 1 < n_layers ? dims[l + 1] : a.mask_size) + 15) / 16 + waves - 1) / waves);
             const int planes = widest > 64 ? 2 : 1, ring_at = 2 * planes * rt * ST_ROWS * 256 + SF_UNIFORMS;
             int slots = (ST_LDS - ring_at) / (waves * SF_UNIT);
             slots = slots < SF_SLOTS ? slots : SF_SLOTS;
