@@ -1276,6 +1276,8 @@ struct GemmKernelNames {
         register_kernel("gemm_bf16_256x256", (const void*)gemm_abt_kernel<SP_BF16, SP_F32, 256, 256, 2, 4>, 512);
         register_kernel("gemm_f16_256x256", (const void*)gemm_abt_kernel<SP_F16, SP_F32, 256, 256, 2, 4>, 512);
         register_kernel("gemm_bf16_128x128", (const void*)gemm_abt_kernel<SP_BF16, SP_F32, 128, 128, 2, 2>, 256);
+        register_kernel("gemm_bf16_128x64", (const void*)gemm_abt_kernel<SP_BF16, SP_F32, 128, 64, 2, 2, 2, 2, true>, 256);
+        register_kernel("gemm_bf16_128x96", (const void*)gemm_abt_kernel<SP_BF16, SP_F32, 128, 96, 4, 1, 2, 2, true>, 256);
         register_kernel("gemm_f32_64x64", (const void*)gemm_abt_kernel<SP_F32, SP_F32, 64, 64, 2, 2>, 256);
         register_kernel("gemm_bf16_256x256_4w", (const void*)gemm_abt_w4_kernel<SP_BF16, SP_F32>, 256);
         register_kernel("gemm_f16_256x256_4w", (const void*)gemm_abt_w4_kernel<SP_F16, SP_F32>, 256);

@@ -740,6 +740,16 @@ __global__ __launch_bounds__(256) void mlp_split_kernel(const void* x_first, con
     }
 }
 
+namespace {
+struct MlpKernelNames {
+    MlpKernelNames() {
+        register_kernel("mlp_forward_256", (const void*)mlp_h256_kernel<SP_F16, 8, 1>, 512);
+        register_kernel("mlp_forward_256_4w", (const void*)mlp_h256_kernel<SP_F16, 4, 1>, 256);
+        register_kernel("mlp_forward_256_split", (const void*)mlp_split_kernel<SP_F16, 1>, 256);
+    }
+} mlp_kernel_names;
+}  // namespace
+
 }  // namespace sp
 
 using namespace sp;

@@ -1034,7 +1034,12 @@ namespace {
 struct MlpAnyKernelNames {
     MlpAnyKernelNames() {
         register_kernel("mlp_forward", (const void*)mlp_features_kernel<SP_F16, 1>, AN_FEATURES_THREADS);
+        register_kernel("mlp_forward_64_rows", (const void*)mlp_features_kernel<SP_F16, 4>, AN_FEATURES_THREADS);
         register_kernel("mlp_forward_wide", (const void*)mlp_rows_kernel<SP_F16, 16, false, 8>, 512);
+        register_kernel("mlp_forward_wide_4w", (const void*)mlp_rows_kernel<SP_F16, 16, false, 4>, 256);
+        register_kernel("mlp_forward_wide_stream", (const void*)mlp_rows_kernel<SP_F16, 16, true, 8>, 512);
+        register_kernel("mlp_forward_wide_128", (const void*)mlp_rows_kernel<SP_F16, 8, false, 8>, 512);
+        register_kernel("mlp_forward_round", (const void*)mlp_round_kernel<SP_F16>, AN_ROUND_WAVES * 64);
     }
 } mlp_any_kernel_names;
 }  // namespace

@@ -912,6 +912,9 @@ extern "C" int sp_stack_forward_f32(const void* x, int32_t n_layers, const void*
 namespace {
 struct MlpStackKernelNames {
     MlpStackKernelNames() {
+        register_kernel("stack_forward_f32_few", (const void*)stack_features_kernel<1, false>, SF_MAX_THREADS);
+        register_kernel("stack_forward_f32_few_regret", (const void*)stack_features_kernel<1, true>, SF_MAX_THREADS);
+        register_kernel("stack_forward_f32_few_2", (const void*)stack_features_kernel<2, false>, SF_MAX_THREADS);
         register_kernel("stack_forward_f32", (const void*)mlp_stack_kernel<4, false, true>, ST_MAX_THREADS);
         register_kernel("stack_forward_f32_regret", (const void*)mlp_stack_kernel<4, true, true>, ST_MAX_THREADS);
         register_kernel("stack_forward_f32_parts", (const void*)mlp_stack_kernel<4, false, true, true>, ST_PARTS_THREADS);

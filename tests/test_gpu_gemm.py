@@ -139,6 +139,29 @@ def test_tiles_of_128_by_64_and_96_are_exact(MM, dtype, m, n, k, tile):
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("e,m,n,k,tile", [(16, 600, 276, 8, (128, 64)), (4, 2568, 273, 8, (128, 64)), (7, 1160, 358, 32, (128, 64)), (7, 2464, 138, 8, (128, 64)),
+                                          (4, 2552, 279, 392, (128, 96)), (4, 2536, 263, 264, (128, 96)), (16, 1736, 68, 312, (128, 96)), (16, 1968, 65, 272, (128, 96))])
+def test_batches_on_tiles_of_128_by_64_and_96_are_their_members(MM, dtype, e, m, n, k, tile):
+    """A batch on the tiles between the 128 and 64 wide ones, at one row or column past a tile: integer operands give every member what a plain
+    launch of it gives, with and without an A that all share, bias + ReLU and beta, and nothing in front of or behind C is touched."""
+    announce("gemm batch tile %s %s %d x %dx%dx%d" % (tile, dtype, e, m, n, k))
+    cfg = MM.matmul_config_batched(e, m, n, k, TORCH[dtype])
+    assert (cfg["m_tile"], cfg["n_tile"]) == tile
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    b = dev(rng.integers(-1, 2, size=(e, n, k)).astype(np.float32), TORCH[dtype])
+    bias, pad = dev(rng.integers(-5, 6, size=n).astype(np.float32)), 64
+    for shared in (False, True):
+        a = dev(rng.integers(-2, 3, size=(m, k) if shared else (e, m, k)).astype(np.float32), TORCH[dtype])
+        for out, beta, add in (("f32", 0.0, None), (dtype, 0.0, bias), ("f32", 2.0, bias)):
+            buf = torch.full((pad + e * m * n + pad,), -77.0, dtype=TORCH[out], device="cuda")
+            c = buf[pad:pad + e * m * n].view(e, m, n)
+            c.copy_(dev(rng.integers(-4, 5, size=(e, m, n)).astype(np.float32)))
+            want = [MM.matmul_abt(a if shared else a[i], b[i], c=c[i].clone(), bias=add, relu=add is not None, beta=beta) for i in range(e)]
+            MM.matmul_abt_batched(a, b, c=c, bias=add, relu=add is not None, beta=beta)
+            assert torch.equal(c, torch.stack(want)) and (buf[:pad] == -77).all() and (buf[-pad:] == -77).all()
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("m,n,k", [(8370, 332, 8), (8449, 333, 184), (8449, 333, 200), (51392, 16, 120), (55244, 30, 328), (58332, 9, 32)])
 def test_reading_c_may_change_the_tile_but_not_the_sums(MM, dtype, m, n, k):
     """Where beta takes another tile than the same call without: C of zeros gives the bits of beta = 0."""
@@ -147,6 +170,17 @@ def test_reading_c_may_change_the_tile_but_not_the_sums(MM, dtype, m, n, k):
     a, b = (torch.randn((r, k), generator=g, device="cuda").to(TORCH[dtype]) for r in (m, n))
     want = MM.matmul_abt(a, b, c=torch.full((m, n), float("nan"), device="cuda"))
     assert torch.equal(MM.matmul_abt(a, b, c=torch.zeros((m, n), device="cuda"), beta=1.0), want)
+
+
+@pytest.mark.parametrize("name,threads", [("gemm_bf16_128x64", 256), ("gemm_bf16_128x96", 256), ("mlp_forward", 1024), ("mlp_forward_64_rows", 1024),
+                                          ("mlp_forward_wide", 512), ("mlp_forward_wide_4w", 256), ("mlp_forward_wide_stream", 512), ("mlp_forward_wide_128", 512),
+                                          ("mlp_forward_round", 512), ("mlp_forward_256", 512), ("mlp_forward_256_4w", 256), ("mlp_forward_256_split", 256),
+                                          ("stack_forward_f32_few", 512), ("stack_forward_f32_few_regret", 512), ("stack_forward_f32_few_2", 512)])
+def test_kernels_have_names_and_the_registers_of_their_workgroups(name, threads):
+    """512 registers a SIMD, shared by the waves that a workgroup puts on each."""
+    from ml import _lib
+    info = _lib.kernel_info(name)
+    assert info["threads_per_block"] == threads and 0 < info["vgprs"] <= 512 // max(1, threads // 256) and info["max_blocks_per_cu"] >= 1
 
 
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])

@@ -328,6 +328,53 @@ def test_past_a_narrow_mask_are_zeros_behind_a_256_wide_layer(LY, mask, dtype):
         assert (policy[:, mask:] == 0).all()
 
 
+@pytest.mark.parametrize("dims,mask", [([64, 128, 64], 5), ([64, 128, 64], 11), ([64, 128, 64], 32), ([64, 128, 64], 40), ([48, 96, 40], 20), ([32, 160, 63], 13),
+                                       ([128, 192, 256, 192, 64], 17), ([128, 192, 256, 192, 64], 3), ([128, 192, 256, 192, 64], 47)])
+@pytest.mark.parametrize("rows", ["40", "66", "130"])
+def test_masked_columns_of_rows_wider_than_the_head(LY, dims, mask, rows):
+    """Without logits the valid columns alone are computed and the rest of a row, of whole 16-byte pieces or not, follows: bit for bit the
+    policy and the actions of the call that writes the logits, in every kernel (rows per compute unit from 66 up), in front of and behind
+    nothing, and the oracle's."""
+    announce("mlp masked rows %s mask=%d rows %s" % (dims, mask, rows))
+    batch = int(rows) if rows == "40" else int(rows) * torch.cuda.get_device_properties(0).multi_processor_count + 5
+    rng = np.random.default_rng(sum(dims) + mask)
+    for dtype, head in (("f16", "regret_matching"), ("bf16", "softmax_regret_matching"), ("f16", "softmax")):
+        x, ws, u = make_problem(rng, batch, dims, dtype)
+        t, n = TORCH[dtype], dims[-1]
+        xd, wd, ud = dev(x, t), [dev(w, t) for w in ws], dev(u)
+        buf = torch.full((64 + batch * n + 64,), -9.0, device="cuda")
+        policy = buf[64:64 + batch * n].view(batch, n)
+        _, action = LY.mlp_forward(xd, wd, None, head, ud, mask, policy_out=policy)
+        full_p, full_a, _ = LY.mlp_forward(xd, wd, None, head, ud, mask, True)
+        assert torch.equal(policy, full_p) and torch.equal(action, full_a)
+        assert (buf[:64] == -9).all() and (buf[-64:] == -9).all() and (policy[:, mask:] == 0).all()
+        want, _, _ = olayers.mlp_forward(x, ws, None, HEAD_CODE[head], u, dtype, mask)
+        assert ogemm.rel_frobenius(host(policy), want) < 2e-4          # (the bound of the other stacks)
+        assert (host(action) == orow.discrete_sampling(host(policy), u)).all()
+
+
+@pytest.mark.parametrize("dims,mask", [([64, 128, 4], 0), ([32, 64, 64], 3), ([64, 128, 16], 0), ([32, 160, 64], 0), ([48, 64, 64], 40), ([128, 192, 256, 192, 4], 0),
+                                       ([128, 192, 256, 192, 64], 0), ([128, 192, 256, 192, 64], 21), ([64, 256, 4], 0)])
+@pytest.mark.parametrize("rows", [2, 66, 132])
+def test_heads_of_any_width_draw_their_own_uniforms(LY, dims, mask, rows):
+    """A Philox stream in place of the tensor of uniforms in every kernel of these stacks: the policy's bits and the actions of the run that
+    reads what sp_philox_uniforms hands out for the rows."""
+    from ml import _lib, primitives
+    announce("mlp philox any width %s mask=%d rows %d" % (dims, mask, rows))
+    batch = rows * torch.cuda.get_device_properties(0).multi_processor_count - 32
+    rng = np.random.default_rng(sum(dims) + mask + rows)
+    x, ws, _ = make_problem(rng, batch, dims, "bf16")
+    xd, wd = dev(x, torch.bfloat16), [dev(w, torch.bfloat16) for w in ws]
+    for cfg in (primitives.philox(_lib.PHILOX_LAYER, blocks_per_grid=32, rows_per_block=batch // 32, offset=8), primitives.philox(_lib.PHILOX_GRID, blocks_per_grid=24)):
+        u = primitives.philox_uniforms(cfg, batch, dims[-1])
+        assert u.unique().numel() > batch // 2
+        for head in ("regret_matching", "softmax"):
+            want = LY.mlp_forward(xd, wd, None, head, u, mask)
+            got = LY.mlp_forward(xd, wd, None, head, None, mask, rng=cfg)
+            assert all(torch.equal(g, w) for g, w in zip(got, want))
+    assert (host(got[1]) == orow.discrete_sampling(host(got[0]), host(u))).all()
+
+
 @pytest.mark.parametrize("dims,head,mask,batch,dtype,with_bias", [
     ([32, 256, 256, 256, 3], "softmax_regret_matching", 0, 16384, "f16", False),     # the benchmark's policy network
     ([32, 256, 256, 256, 3], "softmax", 0, 1, "bf16", False),                        # a single row
