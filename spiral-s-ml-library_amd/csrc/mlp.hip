@@ -834,10 +834,11 @@ extern "C" int sp_mlp_forward(int dtype, const void* x, int32_t n_layers, const 
     // leaves the registers (64-256-6 97 rows 5.2 / 6.4, 16384 5.4 / 7.7, 24000 5.5 / 11.6, 300000 42 / 46; 64-256-10 97 rows 11.4 / 6.6, 300000
     // 107 / 48) -- for up to four only as far as a round of 128 rows a unit goes (32-256-4 24000 rows 5.2 / 7.4, 40000 8.6 / 7.6, 300000 36
     // / 22), and not where half of the first layer's four chunks is padding and the units hold 64 rows at most (128-256-4 4096 rows 7.3 / 6.5,
-    // 24000 8.9 / 10.3; 256-256-4 4096 rows 7.1 / 7.7).
+    // 24000 8.9 / 10.3; 256-256-4 4096 rows 7.1 / 7.7), for more than four outputs 16 (128-256-8 2000 rows 7.5 / 6.7, 10000 7.2 / 7.5).
     const bool one_hidden = n_layers == 2;
     if (one_hidden)
-        h256 = h256 && a.nout <= 8 && (a.nout > 4 || (batch <= 128l * cus && (wide || dims[0] <= 64 || dims[0] > 128)));
+        h256 = h256 && a.nout <= 8 && (a.nout > 4 || batch <= 128l * cus) &&
+               !(!wide && dims[0] > 64 && dims[0] <= 128 && (a.nout <= 4 || batch <= 16l * cus));
     // up to 32 outputs: one round of 128 rows a unit against two of 64 (128-256-256-256-24 24620 rows 24.1 / 27.0)
     const int most_out = wide && batch <= 128l * cus && a.nout == dims[n_layers] ? 32 : 16;
     if (!h256 || a.nout > most_out) {

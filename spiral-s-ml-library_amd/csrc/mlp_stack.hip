@@ -323,7 +323,7 @@ __global__ __launch_bounds__(PARTS ? ST_PARTS_THREADS : ST_MAX_THREADS, HT == 4 
             const unsigned per_kt = a.per_kt[l];
             for (int b = wave; b < kt * nt; b += waves) {
                 int tile, block;
-                if (nt == 1) {
+                if (!FULL && nt == 1) {
                     tile = 0;
                     block = b;
                 } else if (b < kt * whole) {

@@ -251,7 +251,7 @@ def test_a_hidden_sum_that_is_no_number_becomes_zero(LY, dims, mask, rows_per_un
 
 @pytest.mark.parametrize("dims,mask,few,many", [([32, 256, 4], 0, "64", "128+1"), ([64, 256, 64], 4, "64+1", "129"), ([80, 256, 3], 0, "64", "64+1"),
                                                 ([128, 256, 2], 0, "128", "128+1"), ([256, 256, 4], 0, "64+1", "130"), ([16, 256, 8], 0, "64", "64+1"),
-                                                ([144, 256, 8], 5, "3", "140"), ([64, 256, 64], 8, "64", "200"), ([64, 256, 12], 9, "64", "129")])
+                                                ([144, 256, 8], 5, "3", "140"), ([112, 256, 7], 0, "16", "16+1"), ([64, 256, 64], 8, "64", "200"), ([64, 256, 12], 9, "64", "129")])
 def test_a_single_hidden_layer_of_256_on_both_sides_of_its_lines(LY, dims, mask, few, many):
     """Which kernel such a stack runs on goes by the outputs, the inputs and the rows per compute unit: the rows of a batch in front of a
     line give the bits they give as part of one behind it, with and without biases, against the oracle."""
