@@ -33,7 +33,6 @@ PyObject* g_array = nullptr;
 PyObject* g_pointer = nullptr;
 PyObject* g_cast = nullptr;
 PyObject* g_byref = nullptr;
-PyObject* g_philox = nullptr;     // the ctypes structure that stands for sp_philox_t
 
 // ---- arguments: what the caller's objects become; false with an exception set if they do not fit ----
 constexpr Py_ssize_t MOST = 16;   // elements of a host array given as a list or tuple that need no allocation
@@ -148,6 +147,17 @@ bool unwrapped(PyObject* o, PyObject* type, const Take& take) {
     return ok;
 }
 
+// What a function is bound to, in a capsule that the function object holds.
+struct Bound {
+    void* fn;
+    PyObject* stream;             // the ctypes structure that stands for sp_philox_t
+    const char* name;
+    PyObject* function = nullptr; // the function object itself: what the tape records
+    Bound(void* fn, PyObject* stream, const char* name) : fn(fn), stream(Py_NewRef(stream)), name(name) {}
+    Bound(const Bound&) = delete;
+    ~Bound() { Py_DECREF(stream); }
+};
+
 // HOST_INTS: of an entry point whose const int32_t* are host arrays.  Those that take arrays of addresses take the widths of a stack
 // beside them; everywhere else a const int32_t* is device memory.
 template <typename T, bool HOST_INTS, typename = void>
@@ -156,7 +166,7 @@ struct Arg;
 template <typename T, bool HOST_INTS>
 struct Arg<T, HOST_INTS, std::enable_if_t<std::is_integral_v<T>>> {
     T value = 0;
-    bool load(PyObject* o) {
+    bool load(PyObject* o, const Bound&) {
         unsigned long long v = 0;
         if (PyLong_Check(o) ? !as_integer(o, v) : !unwrapped(o, scalar_type<T>(), [&](PyObject* x) { return as_integer(x, v); })) return false;
         value = (T)v;
@@ -167,7 +177,7 @@ struct Arg<T, HOST_INTS, std::enable_if_t<std::is_integral_v<T>>> {
 template <typename T, bool HOST_INTS>
 struct Arg<T, HOST_INTS, std::enable_if_t<std::is_floating_point_v<T>>> {
     T value = 0;
-    bool load(PyObject* o) {
+    bool load(PyObject* o, const Bound&) {
         double v = 0;
         auto number = [&](PyObject* x) {
             v = PyFloat_AsDouble(x);
@@ -184,7 +194,7 @@ template <typename T, bool HOST_INTS>
 struct Arg<T*, HOST_INTS, std::enable_if_t<!std::is_pointer_v<std::remove_const_t<T>> && !std::is_same_v<T, const sp_philox_t> &&
                                            !(HOST_INTS && std::is_same_v<T, const int32_t>)>> {
     T* value = nullptr;
-    bool load(PyObject* o) {
+    bool load(PyObject* o, const Bound&) {
         void* p = nullptr;
         if (o != Py_None && !PyLong_Check(o)) {
             const int is_pointer = PyObject_IsInstance(o, g_pointer);
@@ -242,7 +252,7 @@ struct Arg<T*, HOST_INTS, std::enable_if_t<std::is_pointer_v<std::remove_const_t
         value = n <= (size_t)MOST ? few : (T*)buffer.view.buf;
         return true;
     }
-    bool load(PyObject* o) {
+    bool load(PyObject* o, const Bound&) {
         if (PyTuple_Check(o) || PyList_Check(o)) return list(o);
         if (o == Py_None) return true;
         PyObject* const type = ADDRESSES ? g_void_p : g_int32;
@@ -278,20 +288,20 @@ struct Arg<const sp_philox_t*, HOST_INTS> {
         value = (const sp_philox_t*)buffer.view.buf;
         return true;
     }
-    bool load(PyObject* o) {
+    bool load(PyObject* o, const Bound& bound) {
         if (o == Py_None) return true;
-        if (PyObject_TypeCheck(o, (PyTypeObject*)g_philox)) return memory(o);
+        if (PyObject_TypeCheck(o, (PyTypeObject*)bound.stream)) return memory(o);
         const char* const what = "a random stream is None or a PhiloxConfig";
         if ((PyObject*)Py_TYPE(o) == g_byref) {
-            PyObject* target = referred(o, g_philox, what);
+            PyObject* target = referred(o, bound.stream, what);
             if (target == nullptr) return false;
             const bool ok = memory(target);
             Py_DECREF(target);
             return ok;
         }
-        const int is_array = is_of(o, g_array, g_philox);
+        const int is_array = is_of(o, g_array, bound.stream);
         if (is_array != 0) return is_array > 0 && memory(o);
-        const int is_pointer = is_of(o, g_pointer, g_philox);
+        const int is_pointer = is_of(o, g_pointer, bound.stream);
         if (is_pointer == 0) return refuse(o, what);
         void* p = nullptr;
         if (is_pointer < 0 || !pointed_to(o, p)) return false;
@@ -313,13 +323,6 @@ void refuse_argument(int number) {
 }
 
 // ---- one function per entry point ----
-// What a function is bound to, in a capsule that the function object holds.
-struct Bound {
-    void* fn;
-    PyObject* function;           // the function object itself: what the tape records
-    const char* name;
-};
-
 template <typename F>
 struct Entry;
 template <typename... A>
@@ -329,7 +332,7 @@ struct Entry<int(A...)> {
     template <size_t... I>
     static PyObject* run(const Bound& bound, PyObject* const* given, std::index_sequence<I...>) {
         std::tuple<Arg<A, HOST_INTS>...> args;
-        if (int at = 0; !((++at, std::get<I>(args).load(given[I])) && ...)) {
+        if (int at = 0; !((++at, std::get<I>(args).load(given[I], bound)) && ...)) {
             refuse_argument(at);
             return nullptr;
         }
@@ -369,14 +372,14 @@ struct Entry<int(A...)> {
     X(sp_mlp_forward) X(sp_mlp_pack_weights) X(sp_mlp_forward_packed) X(sp_mlp_forward_ensemble) X(sp_ensemble_binarize)            \
     X(sp_stack_forward_f32)
 
-bool bind_one(void* library, PyObject* functions, const char* name, PyCFunction call, PyMethodDef& def) {
+bool bind_one(void* library, PyObject* stream, PyObject* functions, const char* name, PyCFunction call, PyMethodDef& def) {
     void* const fn = dlsym(library, name);
     if (fn == nullptr) {
         PyErr_Format(PyExc_RuntimeError, "the library has no %s", name);
         return false;
     }
     def = PyMethodDef{name, call, METH_FASTCALL, nullptr};
-    Bound* const bound = new (std::nothrow) Bound{fn, nullptr, name};
+    Bound* const bound = new (std::nothrow) Bound(fn, stream, name);
     if (bound == nullptr) {
         PyErr_NoMemory();
         return false;
@@ -396,7 +399,7 @@ bool bind_one(void* library, PyObject* functions, const char* name, PyCFunction 
 }
 
 // bind(path, stream): a dict of the functions behind the library at `path`, which the process keeps; `stream`: the ctypes structure
-// that stands for sp_philox_t.
+// that stands for sp_philox_t in their calls.
 PyObject* bind(PyObject*, PyObject* const* given, Py_ssize_t n) {
     if (n != 2 || !PyType_Check(given[1])) return PyErr_Format(PyExc_TypeError, "bind takes a path and a structure type");
     const char* p = PyUnicode_AsUTF8(given[0]);
@@ -424,7 +427,6 @@ PyObject* bind(PyObject*, PyObject* const* given, Py_ssize_t n) {
     }
     Py_DECREF(ctypes);
     if (!found) return nullptr;
-    Py_XSETREF(g_philox, Py_NewRef(given[1]));
     void* library = dlopen(p, RTLD_NOW | RTLD_LOCAL);
     if (library == nullptr) return PyErr_Format(PyExc_RuntimeError, "%s", dlerror());
     PyObject* functions = PyDict_New();
@@ -436,7 +438,7 @@ PyObject* bind(PyObject*, PyObject* const* given, Py_ssize_t n) {
 #undef SP_ID
     };
     static PyMethodDef defs[COUNT];
-#define SP_BIND(name) ok = ok && bind_one(library, functions, #name, (PyCFunction)(void (*)(void))&Entry<std::remove_pointer_t<decltype(&::name)>>::call, defs[ID_##name]);
+#define SP_BIND(name) ok = ok && bind_one(library, given[1], functions, #name, (PyCFunction)(void (*)(void))&Entry<std::remove_pointer_t<decltype(&::name)>>::call, defs[ID_##name]);
     SP_LAUNCHES(SP_BIND)
 #undef SP_BIND
     if (!ok) {

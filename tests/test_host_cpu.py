@@ -190,3 +190,16 @@ def test_each_library_keeps_its_own_functions(tmp_path):
     functions = L._host.bind(other, L.PhiloxConfig)
     assert refused_before == -2 and functions["sp_map_f32"](1, P, P, -1, None) == -42
     assert L.lib.sp_map_f32(1, P, P, -1, None) == -2 and functions["sp_row_map_i32"](6, P, P, 8, 8, None) == -42
+
+
+def test_each_library_keeps_its_own_structure():
+    """A second module with a structure of its own for random streams, or this one loaded again, leaves the first one's as it was."""
+    class Other(C.Structure):
+        _fields_ = L.PhiloxConfig._fields_
+    functions = L._host.bind(L.lib._cdll._name, Other)
+    assert reaches(stack(rng=bad_stream()), AT_THE_STREAM)
+    other = Other.from_buffer_copy(bad_stream())
+    assert reaches(stack(fn=functions["sp_mlp_forward"], rng=other), AT_THE_STREAM)
+    for fn, rng in ((L.lib.sp_mlp_forward, other), (functions["sp_mlp_forward"], bad_stream())):
+        with pytest.raises(WRONG):
+            stack(fn=fn, rng=rng)
