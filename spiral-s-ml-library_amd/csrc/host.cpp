@@ -231,16 +231,23 @@ struct Arg<T*, HOST_INTS, std::enable_if_t<std::is_pointer_v<std::remove_const_t
             }
         }
         for (Py_ssize_t i = 0; i < n; ++i) {
-            PyObject* e = PySequence_Fast_GET_ITEM(o, i);
+            if (i >= PySequence_Fast_GET_SIZE(o)) {        // (an element's __index__ may shorten the list)
+                PyErr_SetString(PyExc_RuntimeError, "a list of arguments changed its size");
+                return false;
+            }
+            PyObject* e = Py_NewRef(PySequence_Fast_GET_ITEM(o, i));
+            bool ok;
             if constexpr (ADDRESSES) {
                 void* p = nullptr;
-                if (!as_address(e, p)) return false;
+                ok = as_address(e, p);
                 elements[i] = (Element)p;
             } else {
                 unsigned long long v = 0;
-                if (!as_integer(e, v)) return false;
+                ok = as_integer(e, v);
                 elements[i] = (Element)v;
             }
+            Py_DECREF(e);
+            if (!ok) return false;
         }
         value = elements;
         return true;

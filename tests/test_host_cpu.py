@@ -203,3 +203,14 @@ def test_each_library_keeps_its_own_structure():
     for fn, rng in ((L.lib.sp_mlp_forward, other), (functions["sp_mlp_forward"], bad_stream())):
         with pytest.raises(WRONG):
             stack(fn=fn, rng=rng)
+
+
+def test_lists_may_change_while_they_are_read():
+    class Shortens:
+        def __index__(self):
+            dims.clear()
+            return 64
+    dims = [32]
+    dims += [Shortens(), 4]
+    with pytest.raises(RuntimeError, match="changed its size"):
+        stack(dims=dims)
